@@ -168,7 +168,7 @@ def main():
     plan = runner.describe_plan()
     quantized = "quantizedRows=1" in plan or "rankRows16=1" in plan       # a ranking kernel runs in front of the walk
     plan_fields = dict(item.split("=", 1) for item in plan.split() if "=" in item)
-    kernel = ("WalkRowsTiledKernel" if " tileSize=1 " not in plan else "WalkRowsLdsKernel") if "rows_lds" in plan else \
+    kernel = ("WalkRowsTiledKernel" if " tileSize=1 " not in plan and " tiling=0 " not in plan else "WalkRowsLdsKernel") if "rows_lds" in plan else \
         ("WalkGlobalKernel" if "global_walk" in plan else "WalkTreeParallelKernel")
     # the rank-quantised path reads the f32 rows in its binning kernel: both kernels count for the HBM roofline
     hbm_ms = walk_ms + bin_ms if quantized else walk_ms

@@ -435,7 +435,7 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
   const Forest forest = NormalizeToLessThan(input);
   if (profile && profile->hits.size() != forest.trees.size()) throw Error("hit-count profile does not match the forest");
   if (plan.kernel == LaunchPlan::Kernel::kGlobalWalk) {
-    if (plan.tileSize > 1) throw Error("tile sizes above 1 need the row-parallel LDS kernel; this forest has a tree too big for LDS");
+    if (plan.WalkTile() > 1) throw Error("tile sizes above 1 need the row-parallel LDS kernel; this forest has a tree too big for LDS");
     return PackForGlobalWalk(forest, plan);
   }
   const int K = plan.interleave;
@@ -459,10 +459,10 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
     throw Error("rank-quantised rows need the row-parallel kernel with 64 rows per block");
   if (plan.rankRows16 && (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.quantizedRows || plan.featureOffsetInWords))
     throw Error("two-byte rank rows need the row-parallel kernel (and exclude one-byte ranks and word offsets)");
-  const int T = plan.tileSize;
-  if (T < 1 || T > kMaxTileSize)
-    throw Error("tile size " + std::to_string(T) + " is not supported: the device kernels walk tiles of 1 to " +
+  if (plan.tileSize < 1 || plan.tileSize > kMaxTileSize)
+    throw Error("tile size " + std::to_string(plan.tileSize) + " is not supported: the device kernels walk tiles of 1 to " +
                 std::to_string(kMaxTileSize) + " nodes");
+  const int T = plan.WalkTile();
   if (plan.deferTails && (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || T != 1 || plan.quantizedRows || plan.rankRows16 ||
                           plan.featureOffsetInWords || forest.numClasses > 0 || !profile))
     throw Error("deferred tails need a profile and the scalar row-parallel kernel on float32 rows of a model without classes");
@@ -888,7 +888,7 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
 }
 
 Tree UnpackTree(const PackedModel &pm, int32_t treeIndex) {
-  if (pm.plan.tileSize > 1) throw Error("tiled models are checked through their walks, not unpacked");
+  if (pm.plan.WalkTile() > 1) throw Error("tiled models are checked through their walks, not unpacked");
   if (pm.plan.kernel == LaunchPlan::Kernel::kGlobalWalk) {
     for (const DeviceGlobalTree &gt : pm.globalTrees) {
       if (gt.origin != treeIndex) continue;

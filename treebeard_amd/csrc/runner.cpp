@@ -315,7 +315,7 @@ void InferenceRunner::SetGroupStaging(int32_t mode) {
 bool InferenceRunner::DirectStaging() const {
   const LaunchPlan &plan = m_model.plan;
   if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds) return false; // (only the row-parallel walks have the form)
-  if (plan.tileSize > 1 || plan.rankRows16) return true;                 // (the tiled walk and the walk on two-byte ranks have no other)
+  if (plan.WalkTile() > 1 || plan.rankRows16) return true;                // (the tiled walk and the walk on two-byte ranks have no other)
   if (m_groupStaging != 0) return m_groupStaging == 2;
   // Measured on MI355X (28 to 520 features, 600 to 1000 trees): 5 to 15 % faster with two blocks per CU,
   // 2 to 4 % slower with one, whose wait for the copy nothing covers.  (LDS is handed out in coarse pieces.)
@@ -327,7 +327,7 @@ hipError_t InferenceRunner::LaunchWalk(const WalkParams &p, hipStream_t stream) 
   if (plan.kernel == LaunchPlan::Kernel::kGlobalWalk) return LaunchWalkGlobal(p, plan.interleave, stream);
   if (plan.kernel == LaunchPlan::Kernel::kTreeParallel)
     return LaunchWalkTreeParallel(p, plan.interleave, m_model.LdsBytes(), stream);
-  if (plan.tileSize > 1) return LaunchWalkRowsTiled(p, plan.tileSize, plan.interleave, m_model.LdsBytes(), stream);
+  if (plan.WalkTile() > 1) return LaunchWalkRowsTiled(p, plan.WalkTile(), plan.interleave, m_model.LdsBytes(), stream);
   const int tileMode = plan.rankRows16 ? 3 : plan.quantizedRows ? 2 : (plan.featureOffsetInWords ? 1 : 0);
   return LaunchWalkRowsLds(p, plan.interleave, tileMode, m_model.LdsBytes(), stream);
 }
@@ -704,7 +704,7 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
     timed.push_back(Timed{original, 0.0});
     // Peeled walks (deferred tails) of the same shapes: they need a hit-count profile; without one from the caller
     // the rows of this batch are profiled (leaf ids of up to 4096 rows, counted on the host).
-    if (!original.deferTails && m_forest.numClasses == 0 && original.tileSize == 1) {
+    if (!original.deferTails && m_forest.numClasses == 0 && original.WalkTile() == 1) {
       if (!m_profile) m_profile = CollectProfile(deviceInputs, std::min<int64_t>(rows, 4096));
       const size_t shapes = timed.size();
       for (size_t i = 0; i < shapes; ++i) {
@@ -753,7 +753,7 @@ std::string InferenceRunner::DescribePlan() const {
   if (p.peelWalks) {
     if (p.kernel == LaunchPlan::Kernel::kTreeParallel) peel = "ignored(tree_parallel)";
     else if (p.kernel == LaunchPlan::Kernel::kGlobalWalk) peel = "ignored(global_walk)";
-    else if (p.tileSize > 1 || p.deferTails) peel = "1";
+    else if (p.WalkTile() > 1 || p.deferTails) peel = "1";
     else if (m_forest.numClasses > 0) peel = "ignored(classes)";
     else if (p.quantizedRows || p.rankRows16) peel = "ignored(ranks)";
     else if (p.featureOffsetInWords) peel = "ignored(words)";

@@ -389,7 +389,7 @@ int32_t tbmi_set_plan(intptr_t h, int32_t rowsPerBlock, int32_t treeThreads, int
         // peeled walks keep their form where the new shape has room for it (the caller's group size gives up the
         // stub column's and the queues' share)
         plan.deferTails = false;
-        if (plan.peelWalks && r->Profile() && plan.tileSize == 1 && DeferTailsFit(r->GetForest(), &plan)) plan.deferTails = true;
+        if (plan.peelWalks && r->Profile() && plan.WalkTile() == 1 && DeferTailsFit(r->GetForest(), &plan)) plan.deferTails = true;
         r->Repack(plan);
         return 0;
       },
@@ -402,6 +402,7 @@ int32_t tbmi_set_tree_parallel_plan(intptr_t h, int32_t rowsPerBlock, int32_t tr
       [&] {
         InferenceRunner *r = Runner(h);
         LaunchPlan plan = r->Model().plan;
+        if (plan.tileSize > 1) throw Error("tile sizes above 1 need the row-parallel kernel on float32 rows");
         plan.kernel = LaunchPlan::Kernel::kTreeParallel;
         plan.deferTails = false;
         plan.featureOffsetInWords = false;

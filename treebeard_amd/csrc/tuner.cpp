@@ -91,7 +91,12 @@ LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoSche
   if (walk.tileSize < 1 || walk.tileSize > kMaxTileSize)
     throw Error("tile size " + std::to_string(walk.tileSize) + " is not supported: the device kernels walk tiles of 1 to " +
                 std::to_string(kMaxTileSize) + " nodes");
-  LaunchPlan plan = ChooseScalarPlan(forest, batchSize, ov, limits, walk.tileSize);
+  if (walk.tileSize > 1 && (int64_t)(forest.numFeatures + 1) * 64 * 4 > 0xFFFF)
+    throw Error("tile sizes above 1 need a row tile below 64 KB: " + std::to_string(forest.numFeatures) + " features are too many");
+  LaunchPlan wanted;
+  wanted.tileSize = walk.tileSize;
+  wanted.tiling = walk.tiling;
+  LaunchPlan plan = ChooseScalarPlan(forest, batchSize, ov, limits, wanted.WalkTile());
   plan.tileSize = walk.tileSize;
   plan.tiling = walk.tiling;
   plan.peelWalks = walk.peelWalks;
@@ -101,7 +106,7 @@ LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoSche
 }
 
 bool DeferTailsFit(const Forest &forest, LaunchPlan *plan) {
-  if (plan->kernel != LaunchPlan::Kernel::kRowParallelLds || plan->tileSize != 1 || plan->quantizedRows || plan->rankRows16 ||
+  if (plan->kernel != LaunchPlan::Kernel::kRowParallelLds || plan->WalkTile() != 1 || plan->quantizedRows || plan->rankRows16 ||
       plan->featureOffsetInWords || forest.numClasses > 0)
     return false;
   // every wave's queue comes out of the tree group's share of LDS
@@ -115,7 +120,7 @@ bool DeferTailsFit(const Forest &forest, LaunchPlan *plan) {
 
 namespace {
 
-// tileSize > 1: the plan must be the row-parallel kernel on f32 rows with byte offsets (tiles hold byte offsets
+// tileSize > 1 (tiles chosen by a profile): the plan must be the row-parallel kernel on f32 rows with byte offsets (tiles hold byte offsets
 // into a row tile below 64 KB), and groups are sized for tiles, which take three to eight times the bytes of
 // scalar nodes.
 LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAutoScheduleOptions *ov,
@@ -131,8 +136,6 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     // two blocks per CU while 24 KB remain for a group, byte offsets below 64 KB
     auto tileBytes = [&](int32_t r) { return (int64_t)(forest.numFeatures + 1) * r * 4; };
     while (rb > 64 && (tileBytes(rb) > 0xFFFF || limits.ldsBytesPerBlock / 2 - tileBytes(rb) < 24 * 1024)) rb /= 2;
-    if (tileBytes(rb) > 0xFFFF)
-      throw Error("tile sizes above 1 need a row tile below 64 KB: " + std::to_string(forest.numFeatures) + " features are too many");
     plan.rowsPerBlock = rb;
     plan.treeThreads = std::max(1, 1024 / rb);
     if (ov && ov->numTreeThreads > 0) plan.treeThreads = std::max(1, std::min(ov->numTreeThreads, 1024 / rb));
@@ -294,7 +297,7 @@ std::vector<LaunchPlan> CandidatePlans(const Forest &forest, int64_t batchSize, 
   std::vector<LaunchPlan> out;
   LaunchPlan base = ChoosePlan(forest, batchSize, nullptr, limits, walk);
   out.push_back(base);
-  if (base.tileSize > 1) { // block shapes and interleave factors of the tiled walk
+  if (base.WalkTile() > 1) { // block shapes and interleave factors of the tiled walk
     for (int32_t rb : {64, 128, 256})
       for (int32_t k : {1, 2, 4}) {
         LaunchPlan p = base;
@@ -305,7 +308,7 @@ std::vector<LaunchPlan> CandidatePlans(const Forest &forest, int64_t batchSize, 
         if (tile > 0xFFFF) continue;
         const int64_t meet = forest.numClasses > 0 ? (int64_t)rb * p.treeThreads * 8 : 0;
         int64_t group = std::min<int64_t>(65536, limits.ldsBytesPerBlock / 2 - tile - meet - 2048);
-        if (group < TiledGroupNeed(forest, base.tileSize)) continue;
+        if (group < TiledGroupNeed(forest, base.WalkTile())) continue;
         if (base.treeSlices > 1) group = std::min<int64_t>(group, base.groupBytes);
         p.groupBytes = (int32_t)(group & ~15);
         bool dup = false;
