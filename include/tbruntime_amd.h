@@ -123,7 +123,8 @@ TBAMD_EXPORT int32_t tbmi_run_device(intptr_t runner, const float *deviceInputs,
  * work queued after it sees their results: no synchronisation is needed on either side.  All calls on one
  * runner share its device buffers (the packed model, partial sums, rank-quantised rows); the library records
  * an event behind the kernels of every call made here, and the next call on this runner - on another stream,
- * or through an entry point that uses the runner's own stream - waits for it on the device, while calls that
+ * or through an entry point that uses the runner's own stream - waits for it on the device (after a call on the
+ * default stream: for what that stream holds when the next call is made elsewhere), while calls that
  * re-pack the model (tbmi_set_*_plan, tbmi_autotune), grow the buffers (the first call, and a call with more
  * rows than any before it, allocates) or delete the runner wait for it on the host.  Calls on one runner are
  * therefore ordered, never concurrent; use one runner per stream for kernels that should overlap.  One caller

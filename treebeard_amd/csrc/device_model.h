@@ -133,6 +133,19 @@ struct RankChunkDesc {
   uint32_t tableBegin, tableEntries;
 };
 
+// Three levels of a tree in one 48-byte piece (three 16-byte loads), for walks whose cost is the latency of dependent
+// loads: slot 0 is the top node, slots 1-2 its children, slots 3-6 theirs, the eight children below those are the
+// tops of further blocks.  A leaf (feature kFewRowsLeaf) ends the walk in whatever slot it sits; the children of
+// slots 3-6 that exist (bit 2 * (slot - 3) + side of `exits`) follow each other from block `firstChild`.
+struct DeviceFewRowsBlock {
+  float value[7];       // split threshold, or the prediction on a leaf
+  uint32_t firstChild;
+  uint16_t feature[7];
+  uint16_t exits;
+};
+static_assert(sizeof(DeviceFewRowsBlock) == 48, "three 16-byte loads");
+constexpr uint32_t kFewRowsLeaf = 0xFFFFu;
+
 struct DeviceGroup {
   uint32_t nodeBegin;   // first node of the group in the packed node array
   uint32_t nodeCount;   // multiple of 2 so that the group is a whole number of 16-byte pieces

@@ -53,6 +53,7 @@ struct WalkParams {
   int32_t *leafIds = nullptr;     // [rows][numTrees]
   const int32_t *nodeOrigin = nullptr;
   const int32_t *slotTree = nullptr;
+  hipEvent_t done = nullptr;      // recorded when this kernel completes (kLaunchersRecordEvents)
 };
 
 // From this many tree slices on, small batches are finalized by a wave per (row, class); classifiers then need
@@ -70,7 +71,36 @@ struct FinalizeParams {
   int8_t *classOut = nullptr;  // multiclass: arg-max class id
   float *margins = nullptr;    // optional [rows][classes] per-class sums
   float *probabilities = nullptr; // optional [rows][classes] softmax
+  hipEvent_t done = nullptr;
 };
+
+// Batches of a few rows: one launch that also finishes (no partial sums, no finalize kernel).
+struct FewRowsParams {
+  const float *x = nullptr;                   // rows x numFeatures, row-major; device memory or pinned host memory
+  const DeviceFewRowsBlock *blocks = nullptr; // PackFewRows
+  const int32_t *classBegin = nullptr;
+  int64_t rows = 0;
+  int32_t numFeatures = 0, numTrees = 0, numClasses = 0;
+  int32_t transform = 0;
+  double initialValue = 0.0;
+  float *out = nullptr;                       // as in FinalizeParams
+  int8_t *classOut = nullptr;
+  float *margins = nullptr;
+  float *probabilities = nullptr;
+  hipEvent_t done = nullptr;
+};
+
+#if defined(__HIP__)
+inline constexpr bool kLaunchersRecordEvents = true;
+// How many rows of such a forest LaunchFewRows takes sooner than the launch plans do (0: never).
+int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth);
+hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream);
+#else
+// (host-only builds of the runner, under the sanitizers, link stand-ins of the launchers below and have no others)
+inline constexpr bool kLaunchersRecordEvents = false;
+inline int64_t FewRowsLimit(int32_t, int32_t, int32_t, int32_t) { return 0; }
+inline hipError_t LaunchFewRows(const FewRowsParams &, hipStream_t) { return hipErrorNotSupported; }
+#endif
 
 // Row-parallel walk over LDS-staged tree groups: block = s.rowsPerBlock * s.treeThreads lanes.
 // `interleave` in {1,2,4,8}; `tileMode`: 0 f32 tile with byte offsets, 1 f32 tile with offsets in units of

@@ -8,6 +8,9 @@
 // result initialisation and sigmoid).
 #include "kernels.h"
 
+#include <hip/hip_ext.h>
+
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 
@@ -1214,6 +1217,28 @@ RankRows16Kernel(const float *__restrict__ x, const float *__restrict__ tables, 
   }
 }
 
+// A row's class sums -> class id (arg-max of the f32 sums, ties to the larger id) and, on request, the f32 sums and
+// their softmax.
+__device__ __forceinline__ void FinishClasses(const double *sums, int C, int64_t row, float *out, int8_t *classOut,
+                                              float *margins, float *probabilities) {
+  float best = -INFINITY;
+  int bestClass = 0;
+  double maxMargin = -INFINITY;
+  for (int c = 0; c < C; ++c) {
+    const float m = (float)sums[c];
+    if (margins) margins[row * C + c] = m;
+    if (!(best > m)) { best = m; bestClass = c; }
+    maxMargin = sums[c] > maxMargin ? sums[c] : maxMargin;
+  }
+  if (classOut) classOut[row] = (int8_t)bestClass;
+  if (out) out[row] = (float)bestClass;
+  if (probabilities) {
+    double z = 0.0;
+    for (int c = 0; c < C; ++c) z += exp(sums[c] - maxMargin);
+    for (int c = 0; c < C; ++c) probabilities[row * C + c] = (float)(exp(sums[c] - maxMargin) / z);
+  }
+}
+
 // ---------------------------------------------------------------------------
 // Sums the tree-slice partials of each row (in slice order, starting from the
 // initial value), then applies the output transform.  Multiclass rows get the
@@ -1284,6 +1309,104 @@ __global__ void __launch_bounds__(256) FinalizeWideKernel(const FinalizeParams p
   if (lane == 0) p.partial[((int64_t)p.treeSlices * p.rows + row) * Cn + c] = margin - p.initialValue;
 }
 
+// ---------------------------------------------------------------------------
+// A few rows: one launch, one lane per (row, tree).  What such a batch waits for is latency - of the launches, of
+// staging tree groups in LDS and of the dependent node reads - so nothing is staged but the rows and nothing is left
+// to a second kernel: a lane reads a tree three levels at a time (one 48-byte block, three 16-byte loads in flight
+// together, so a walk of 8 levels waits for three loads of L2 latency instead of nine), leaves its leaf value in LDS,
+// and a wave per (row, class) adds them in a fixed order.  One row through 1000 trees of depth 8 took 15.2 us a call
+// with the tree-parallel kernel and its finalize launch.
+// ---------------------------------------------------------------------------
+constexpr int64_t kFewRowsWork = (int64_t)3 << 20; // (row, tree, block of three levels) visits, see FewRowsLimit
+
+struct FewRowsShape {
+  int rowsPerBlock, threads;
+  size_t leafStride, ldsBytes; // floats per tree in the leaf array; LDS of a block
+};
+
+FewRowsShape ShapeOfFewRows(int64_t rows, int numFeatures, int numTrees, int numClasses) {
+  FewRowsShape s;
+  s.rowsPerBlock = (int)std::max<int64_t>(1, (rows + 255) / 256); // a block per compute unit before blocks take more rows
+  s.threads = (int)std::min<int64_t>(1024, ((int64_t)s.rowsPerBlock * numTrees + 63) / 64 * 64);
+  if (s.threads < 64) s.threads = 64;
+  s.leafStride = (size_t)s.rowsPerBlock | 1; // (odd: the lanes that add a row's leaves read different banks)
+  s.ldsBytes = ((size_t)numTrees * s.leafStride + (size_t)s.rowsPerBlock * numFeatures) * sizeof(float);
+  s.ldsBytes = ((s.ldsBytes + 7) & ~(size_t)7) + (size_t)s.rowsPerBlock * std::max(1, numClasses) * sizeof(double);
+  return s;
+}
+
+__global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int rowsPerBlock, int leafStride) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int tid = threadIdx.x, threads = blockDim.x;
+  const int T = p.numTrees, F = p.numFeatures, R = rowsPerBlock;
+  const int Cn = p.numClasses > 0 ? p.numClasses : 1;
+  const int64_t row0 = (int64_t)blockIdx.x * R;
+  const int valid = p.rows - row0 < R ? (int)(p.rows - row0) : R;
+  float *leaves = reinterpret_cast<float *>(lds);
+  float *rowTile = leaves + (size_t)T * leafStride;
+  double *sums = reinterpret_cast<double *>((reinterpret_cast<uintptr_t>(rowTile + (size_t)R * F) + 7) & ~(uintptr_t)7);
+  const U32x4 *blocks = reinterpret_cast<const U32x4 *>(p.blocks);
+  const int items = valid * T; // item i: row i % valid of tree i / valid (lanes of a wave share the top of a tree)
+
+  // the first trees' top blocks are requested before the rows are staged
+  U32x4 q0{}, q1{}, q2{};
+  if (tid < items) {
+    const U32x4 *b = blocks + (size_t)(tid / valid) * 3;
+    q0 = b[0], q1 = b[1], q2 = b[2];
+  }
+  {
+    const float *src = p.x + row0 * F;
+    for (int e = tid; e < valid * F; e += threads) rowTile[e] = src[e];
+  }
+  __syncthreads();
+  for (int i = tid; i < items; i += threads) {
+    const int t = i / valid, r = i - t * valid;
+    const float *row = rowTile + r * F;
+    if (i != tid) {
+      const U32x4 *b = blocks + (size_t)t * 3;
+      q0 = b[0], q1 = b[1], q2 = b[2];
+    }
+    float leaf;
+    for (;;) {
+      const uint32_t f0 = q2.x & 0xFFFFu;
+      leaf = AsFloat(q0.x);
+      if (f0 == kFewRowsLeaf) break;
+      const bool right0 = !(row[f0] < leaf); // (NaN goes right)
+      const uint32_t f1 = right0 ? q2.y & 0xFFFFu : q2.x >> 16;
+      leaf = AsFloat(right0 ? q0.z : q0.y);
+      if (f1 == kFewRowsLeaf) break;
+      const bool right1 = !(row[f1] < leaf);
+      const uint32_t pair = right0 ? (q2.w << 16) | (q2.z >> 16) : (q2.z << 16) | (q2.y >> 16); // features of slots 3, 4 or 5, 6
+      const uint32_t f2 = right1 ? pair >> 16 : pair & 0xFFFFu;
+      leaf = AsFloat(right0 ? (right1 ? q1.z : q1.y) : (right1 ? q1.x : q0.w));
+      if (f2 == kFewRowsLeaf) break;
+      const bool right2 = !(row[f2] < leaf);
+      const uint32_t exit = (right0 ? 4u : 0u) + (right1 ? 2u : 0u) + (right2 ? 1u : 0u);
+      const uint32_t child = q1.w + (uint32_t)__popc((q2.w >> 16) & ((1u << exit) - 1u));
+      const U32x4 *b = blocks + (size_t)child * 3;
+      q0 = b[0], q1 = b[1], q2 = b[2];
+    }
+    leaves[(size_t)t * leafStride + r] = leaf;
+  }
+  __syncthreads();
+  // a wave per (row, class): lanes take trees in turn, a butterfly adds the lanes
+  const int lane = tid & 63;
+  for (int pair = tid >> 6; pair < valid * Cn; pair += threads >> 6) {
+    const int r = pair / Cn, c = pair - r * Cn;
+    const int end = p.numClasses > 0 ? p.classBegin[c + 1] : T;
+    double sum = 0.0;
+    for (int t = (p.numClasses > 0 ? p.classBegin[c] : 0) + lane; t < end; t += 64) sum += (double)leaves[(size_t)t * leafStride + r];
+    for (int m = 1; m <= 32; m <<= 1) sum += ShuffleXor(sum, m); // (ascending: see ShuffleXor)
+    const double margin = p.initialValue + sum;
+    if (lane != 0) continue;
+    if (p.numClasses == 0) p.out[row0 + r] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
+    else sums[pair] = margin;
+  }
+  if (p.numClasses == 0) return;
+  __syncthreads();
+  if (tid < valid) FinishClasses(sums + tid * Cn, Cn, row0 + tid, p.out, p.classOut, p.margins, p.probabilities);
+}
+
 // The ceiling on dynamic LDS is an attribute of each kernel on each device: it is raised once per kernel and
 // device, to the whole 160 KB, instead of on every launch (a runtime call that small batches would pay for each
 // time).  Two threads that meet here for the first time both make the call, which is harmless.
@@ -1299,14 +1422,23 @@ template <auto Kernel> hipError_t AllowFullLds() {
   return e;
 }
 
+// Launches a kernel; `done` (may be null) is recorded by the kernel's own completion, which costs a small call 1.4 us
+// less than an event recorded behind it (a packet of its own), and waiting for it 2.3 us less than a wait for the stream.
+template <typename... Params, typename... Args>
+hipError_t StartKernel(void (*kernel)(Params...), dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream, hipEvent_t done,
+                       Args... args) {
+  if (done) hipExtLaunchKernelGGL(kernel, grid, block, (uint32_t)ldsBytes, stream, nullptr, done, 0, static_cast<Params>(args)...);
+  else kernel<<<grid, block, ldsBytes, stream>>>(static_cast<Params>(args)...);
+  return hipGetLastError();
+}
+
 template <int K, int PF, int W, int V>
 hipError_t LaunchWalkVariant(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream) {
   hipError_t e = AllowFullLds<&WalkRowsLdsKernel<K, PF, W, V>>();
   if (e != hipSuccess) return e;
-  WalkRowsLdsKernel<K, PF, W, V><<<grid, block, ldsBytes, stream>>>(p.x, p.nodes16, p.bundles, p.bundleRoots, p.groups, p.s, p.out, p.classOut,
-                                                                    p.partial, p.leafIds, p.nodeOrigin, p.slotTree,
-                                                                    reinterpret_cast<const U32x2 *>(p.tailNodes), p.tailOrigin);
-  return hipGetLastError();
+  return StartKernel(&WalkRowsLdsKernel<K, PF, W, V>, grid, block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles, p.bundleRoots,
+                     p.groups, p.s, p.out, p.classOut, p.partial, p.leafIds, p.nodeOrigin, p.slotTree,
+                     reinterpret_cast<const U32x2 *>(p.tailNodes), p.tailOrigin);
 }
 
 template <int K, int PF, int W>
@@ -1391,9 +1523,8 @@ template <int T, int K, int V>
 hipError_t LaunchTiledVariant(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream) {
   hipError_t e = AllowFullLds<&WalkRowsTiledKernel<T, K, V>>();
   if (e != hipSuccess) return e;
-  WalkRowsTiledKernel<T, K, V><<<grid, block, ldsBytes, stream>>>(p.x, p.nodes16, p.bundles, p.groups, p.s, p.out, p.classOut, p.partial,
-                                                                  p.leafIds, p.nodeOrigin, p.slotTree);
-  return hipGetLastError();
+  return StartKernel(&WalkRowsTiledKernel<T, K, V>, grid, block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles, p.groups, p.s, p.out,
+                     p.classOut, p.partial, p.leafIds, p.nodeOrigin, p.slotTree);
 }
 
 template <int T, int K>
@@ -1443,15 +1574,13 @@ hipError_t LaunchTreeParallelKP(const WalkParams &p, dim3 grid, dim3 block, size
   if (p.leafIds) {
     hipError_t e = AllowFullLds<&WalkTreeParallelKernel<K, PF, true>>();
     if (e != hipSuccess) return e;
-    WalkTreeParallelKernel<K, PF, true><<<grid, block, ldsBytes, stream>>>(p.x, p.nodes16, p.bundles, p.groups, p.s, p.out,
-                                                                          p.partial, p.leafIds, p.nodeOrigin, p.slotTree);
-  } else {
-    hipError_t e = AllowFullLds<&WalkTreeParallelKernel<K, PF, false>>();
-    if (e != hipSuccess) return e;
-    WalkTreeParallelKernel<K, PF, false><<<grid, block, ldsBytes, stream>>>(p.x, p.nodes16, p.bundles, p.groups, p.s, p.out,
-                                                                           p.partial, nullptr, nullptr, nullptr);
+    return StartKernel(&WalkTreeParallelKernel<K, PF, true>, grid, block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles, p.groups, p.s,
+                       p.out, p.partial, p.leafIds, p.nodeOrigin, p.slotTree);
   }
-  return hipGetLastError();
+  hipError_t e = AllowFullLds<&WalkTreeParallelKernel<K, PF, false>>();
+  if (e != hipSuccess) return e;
+  return StartKernel(&WalkTreeParallelKernel<K, PF, false>, grid, block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles, p.groups, p.s,
+                     p.out, p.partial, nullptr, nullptr, nullptr);
 }
 
 template <int K>
@@ -1486,10 +1615,10 @@ namespace {
 template <int K>
 hipError_t LaunchGlobalK(const WalkParams &p, dim3 grid, dim3 block, hipStream_t stream) {
   if (p.leafIds)
-    WalkGlobalKernel<K, true><<<grid, block, 0, stream>>>(p.x, p.globalNodes, p.globalTrees, p.s, p.out, p.partial, p.leafIds);
-  else
-    WalkGlobalKernel<K, false><<<grid, block, 0, stream>>>(p.x, p.globalNodes, p.globalTrees, p.s, p.out, p.partial, nullptr);
-  return hipGetLastError();
+    return StartKernel(&WalkGlobalKernel<K, true>, grid, block, 0, stream, p.done, p.x, p.globalNodes, p.globalTrees, p.s, p.out, p.partial,
+                       p.leafIds);
+  return StartKernel(&WalkGlobalKernel<K, false>, grid, block, 0, stream, p.done, p.x, p.globalNodes, p.globalTrees, p.s, p.out, p.partial,
+                     nullptr);
 }
 } // namespace
 
@@ -1573,21 +1702,40 @@ hipError_t LaunchRankRows16(const float *x, const float *tables, const RankFeatu
   return hipGetLastError();
 }
 
+// Items a compute unit walks cost about 20 cycles of its address path per 16-byte gather of 64 lanes; up to about
+// 4 us of that the form stays ahead of the launch plans, whose batches of this size take 12 to 15 us.
+int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth) {
+  if (numTrees < 1) return 0;
+  const int64_t rounds = depth / 3 + 1;
+  int64_t rows = kFewRowsWork / ((int64_t)numTrees * rounds);
+  while (rows > 0 && ShapeOfFewRows(rows, numFeatures, numTrees, numClasses).ldsBytes > 64 * 1024) rows /= 2;
+  return rows;
+}
+
+hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream) {
+  if (p.rows <= 0) return hipSuccess;
+  const FewRowsShape s = ShapeOfFewRows(p.rows, p.numFeatures, p.numTrees, p.numClasses);
+  if (p.numTrees < 1 || s.ldsBytes > 64 * 1024) return hipErrorInvalidValue;
+  if (p.numClasses == 0 ? !p.out : !(p.out || p.classOut || p.margins || p.probabilities)) return hipErrorInvalidValue;
+  const int64_t blocks = (p.rows + s.rowsPerBlock - 1) / s.rowsPerBlock;
+  return StartKernel(&FewRowsKernel, dim3((unsigned)blocks), dim3((unsigned)s.threads), s.ldsBytes, stream, p.done, p, s.rowsPerBlock,
+                     (int)s.leafStride);
+}
+
 hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
   const int Cn = p.numClasses > 0 ? p.numClasses : 1;
   FinalizeParams q = p;
   if (p.treeSlices >= kWideFinalizeSlices && p.rows * Cn <= 65536) { // few rows, many slices: a wave per (row, class)
     const int64_t waves = p.rows * Cn;
-    FinalizeWideKernel<<<dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream>>>(p);
-    hipError_t e = hipGetLastError();
+    hipError_t e = StartKernel(&FinalizeWideKernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream,
+                               p.numClasses == 0 ? p.done : nullptr, p);
     if (e != hipSuccess || p.numClasses == 0) return e;
     q.partial = p.partial + (int64_t)p.treeSlices * p.rows * Cn; // the class sums now sit in the spare slot
     q.treeSlices = 1;
   }
   const int64_t blocks = (q.rows + 255) / 256;
-  FinalizeKernel<<<dim3((unsigned)blocks), dim3(256), 0, stream>>>(q);
-  return hipGetLastError();
+  return StartKernel(&FinalizeKernel, dim3((unsigned)blocks), dim3(256), 0, stream, q.done, q);
 }
 
 } // namespace tbamd

@@ -422,6 +422,53 @@ PackedModel PackForGlobalWalk(const Forest &forest, const LaunchPlan &plan) {
 
 } // namespace
 
+FewRowsModel PackFewRows(const Forest &input) {
+  FewRowsModel fm;
+  if (input.numFeatures >= (int32_t)kFewRowsLeaf) return fm;
+  const Forest forest = NormalizeToLessThan(input);
+  const int32_t Cn = std::max(1, forest.numClasses);
+  std::vector<int32_t> order(forest.trees.size());
+  std::iota(order.begin(), order.end(), 0);
+  auto classOf = [&](int32_t t) { return forest.numClasses > 0 ? forest.trees[(size_t)t].classId : 0; };
+  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) { return classOf(a) < classOf(b); });
+  fm.classBegin.assign((size_t)Cn + 1, (int32_t)order.size());
+  for (size_t i = order.size(); i-- > 0;)
+    for (int32_t c = classOf(order[i]); c >= 0 && fm.classBegin[(size_t)c] > (int32_t)i; --c) fm.classBegin[(size_t)c] = (int32_t)i;
+  fm.blocks.resize(order.size());
+  struct Top { int32_t node; size_t block; };
+  std::vector<Top> queue;
+  for (size_t i = 0; i < order.size(); ++i) {
+    const Tree &tree = forest.trees[(size_t)order[i]];
+    queue.assign(1, Top{0, i});
+    for (size_t head = 0; head < queue.size(); ++head) {
+      DeviceFewRowsBlock b{};
+      for (uint16_t &f : b.feature) f = (uint16_t)kFewRowsLeaf; // (slots below a leaf are never reached)
+      b.firstChild = (uint32_t)fm.blocks.size();
+      int32_t at[7] = {queue[head].node, -1, -1, -1, -1, -1, -1};
+      for (int s = 0; s < 7; ++s) {
+        if (at[s] < 0) continue;
+        const int32_t n = at[s];
+        b.value[s] = tree.value[(size_t)n];
+        if (tree.IsLeaf(n)) continue;
+        b.feature[s] = (uint16_t)tree.feature[(size_t)n];
+        for (int side = 0; side < 2; ++side) {
+          const int32_t child = side == 0 ? tree.left[(size_t)n] : tree.right[(size_t)n];
+          if (s < 3) {
+            at[2 * s + 1 + side] = child;
+          } else {
+            b.exits = (uint16_t)(b.exits | 1u << (2 * (s - 3) + side));
+            queue.push_back(Top{child, fm.blocks.size()});
+            fm.blocks.emplace_back();
+          }
+        }
+      }
+      fm.blocks[queue[head].block] = b;
+      if (fm.blocks.size() > 0x7FFFFFF0u) throw Error("forest has too many nodes");
+    }
+  }
+  return fm;
+}
+
 PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile) {
   // Plans also come out of files: every field is brought into its range before anything is computed from it.
   if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds && plan.kernel != LaunchPlan::Kernel::kTreeParallel &&

@@ -145,6 +145,15 @@ struct PackedModel {
   size_t LdsBytes() const; // row tile + the largest group (+ reduction scratch)
 };
 
+// The forest as blocks of three levels, for batches of a few rows (LaunchFewRows): trees ordered by class, block t
+// is the top of tree t, classBegin[c] the first tree of class c (one class without classes).  Independent of the launch plan.
+struct FewRowsModel {
+  std::vector<DeviceFewRowsBlock> blocks;
+  std::vector<int32_t> classBegin; // max(1, classes) + 1 entries
+};
+// Empty when a feature index does not fit the block's 16 bits.
+FewRowsModel PackFewRows(const Forest &forest);
+
 // Largest number of distinct split thresholds any one feature has (after comparison normalisation).
 int32_t MaxThresholdsPerFeature(const Forest &forest);
 

@@ -1,6 +1,7 @@
 #include "runner.h"
 
 #include <algorithm>
+#include <cstring>
 #include <mutex>
 #include <sstream>
 #include <vector>
@@ -62,6 +63,7 @@ InferenceRunner::InferenceRunner(Forest forest, const CompilerOptions &options,
     m_walk.peelWalks = m_profile && gPeeledWalks;
     m_model = PackForest(m_forest, ChoosePlan(m_forest, m_options.batchSize, gpuOptions, m_limits, m_walk), m_profile.get());
     UploadModel();
+    UploadFewRows();
   } catch (...) { // a constructor that throws gets no destructor call: give back what was created
     Release();
     throw;
@@ -79,6 +81,7 @@ InferenceRunner::InferenceRunner(Forest forest, const CompilerOptions &options, 
     m_walk.peelWalks = plan.peelWalks;
     m_model = PackForest(m_forest, plan, m_profile.get());
     UploadModel();
+    UploadFewRows();
   } catch (...) {
     Release();
     throw;
@@ -117,15 +120,24 @@ void InferenceRunner::InitDevice() {
   Check(hipEventCreate(&m_evStart), "hipEventCreate");
   Check(hipEventCreate(&m_evStop), "hipEventCreate");
   Check(hipEventCreateWithFlags(&m_asyncDone, hipEventDisableTiming), "hipEventCreate");
+  Check(hipEventCreateWithFlags(&m_callDone, hipEventDisableTiming), "hipEventCreate");
+}
+
+void InferenceRunner::RecordAsyncCall() {
+  if (m_asyncRecorded) return;
+  Check(hipEventRecord(m_asyncDone, m_asyncStream), "hipEventRecord");
+  m_asyncRecorded = true;
 }
 
 void InferenceRunner::OrderAfterAsyncCall(hipStream_t stream) {
   if (!m_asyncPending || stream == m_asyncStream) return; // (calls on one stream are ordered by the stream)
+  RecordAsyncCall();
   Check(hipStreamWaitEvent(stream, m_asyncDone, 0), "hipStreamWaitEvent");
 }
 
 void InferenceRunner::WaitForAsyncCall() {
   if (!m_asyncPending) return;
+  RecordAsyncCall();
   Check(hipEventSynchronize(m_asyncDone), "hipEventSynchronize");
   m_asyncPending = false;
 }
@@ -133,9 +145,15 @@ void InferenceRunner::WaitForAsyncCall() {
 InferenceRunner::~InferenceRunner() { Release(); }
 
 void InferenceRunner::Release() noexcept {
-  if (m_asyncPending) (void)hipEventSynchronize(m_asyncDone); // kernels of an asynchronous call still read the model
+  if (m_asyncPending) { // kernels of an asynchronous call still read the model
+    if (!m_asyncRecorded) (void)hipEventRecord(m_asyncDone, m_asyncStream);
+    (void)hipEventSynchronize(m_asyncDone);
+  }
   if (m_stream) (void)hipStreamSynchronize(m_stream);
   FreeModel();
+  (void)hipFree(m_dFewRows);
+  (void)hipFree(m_dFewRowsClasses);
+  if (m_smallHost) (void)hipHostFree(m_smallHost);
   (void)hipFree(m_dPartial);
   (void)hipFree(m_dRanks);
   (void)hipFree(m_dStageIn);
@@ -148,6 +166,7 @@ void InferenceRunner::Release() noexcept {
   if (m_evStart) (void)hipEventDestroy(m_evStart);
   if (m_evStop) (void)hipEventDestroy(m_evStop);
   if (m_asyncDone) (void)hipEventDestroy(m_asyncDone);
+  if (m_callDone) (void)hipEventDestroy(m_callDone);
 
   if (m_stream) (void)hipStreamDestroy(m_stream);
 }
@@ -214,6 +233,19 @@ void InferenceRunner::UploadModel() {
   }
 }
 
+void InferenceRunner::UploadFewRows() {
+  if (m_forest.trees.empty()) return;
+  int32_t depth = 0;
+  for (const Tree &tree : m_forest.trees) depth = std::max(depth, tree.Depth());
+  const int64_t limit = FewRowsLimit(m_forest.numFeatures, (int32_t)m_forest.trees.size(), m_forest.numClasses, depth);
+  if (limit < 1) return;
+  const FewRowsModel model = PackFewRows(m_forest);
+  if (model.blocks.empty()) return;
+  m_dFewRows = Upload(model.blocks, "upload few-rows blocks");
+  m_dFewRowsClasses = Upload(model.classBegin, "upload class ranges");
+  m_fewRowsLimit = limit;
+}
+
 void InferenceRunner::Repack(const LaunchPlan &plan) {
   PackedModel next = PackForest(m_forest, plan, m_profile.get());
   // refuse before anything is freed: a plan that fails leaves the runner as it was
@@ -268,9 +300,11 @@ void InferenceRunner::EnsureRanks(int64_t rows) {
   m_ranksBytes = need;
 }
 
-InferenceRunner::Workspace InferenceRunner::OwnWorkspace(int64_t rows, hipStream_t stream) {
-  EnsurePartial(rows);
-  EnsureRanks(rows);
+InferenceRunner::Workspace InferenceRunner::OwnWorkspace(int64_t rows, hipStream_t stream, bool planKernels) {
+  if (planKernels || !TakesFewRows(rows)) {
+    EnsurePartial(rows);
+    EnsureRanks(rows);
+  }
   // An asynchronous call on another stream may still use these buffers: `stream` waits for it on the device.
   OrderAfterAsyncCall(stream);
   Workspace ws;
@@ -364,8 +398,27 @@ WalkParams InferenceRunner::MakeWalkParams(const float *deviceInputs, int64_t ro
 }
 
 void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out, int8_t *classOut, float *margins,
-                             float *probabilities, int32_t *leafIds, hipStream_t stream, const Workspace &ws) {
+                             float *probabilities, int32_t *leafIds, hipStream_t stream, const Workspace &ws, hipEvent_t done) {
   if (rows <= 0) return;
+  if (!leafIds && TakesFewRows(rows)) {
+    FewRowsParams f;
+    f.x = deviceInputs;
+    f.blocks = m_dFewRows;
+    f.classBegin = m_dFewRowsClasses;
+    f.rows = rows;
+    f.numFeatures = m_forest.numFeatures;
+    f.numTrees = (int32_t)m_forest.trees.size();
+    f.numClasses = m_forest.numClasses;
+    f.transform = m_forest.transform == Transform::kSigmoid ? 1 : 0;
+    f.initialValue = m_forest.initialValue;
+    f.out = out;
+    f.classOut = classOut;
+    f.margins = margins;
+    f.probabilities = probabilities;
+    f.done = done;
+    Check(LaunchFewRows(f, stream), "launch few-rows kernel");
+    return;
+  }
   WalkParams p = MakeWalkParams(PrepareRows(deviceInputs, rows, ws.ranks, stream), rows);
   // A classifier whose trees all sit in one slice needs no second kernel when only the class id is wanted:
   // the row-parallel kernels keep the running arg-max themselves.
@@ -380,6 +433,7 @@ void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out
     p.nodeOrigin = m_dNodeOrigin;
     p.slotTree = m_dSlotTree;
   }
+  p.done = finalize ? nullptr : done;
   Check(LaunchWalk(p, stream), "launch walk kernel");
   if (finalize) {
     FinalizeParams f;
@@ -393,8 +447,10 @@ void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out
     f.classOut = classOut;
     f.margins = margins;
     f.probabilities = probabilities;
+    f.done = done;
     Check(LaunchFinalize(f, stream), "launch finalize kernel");
   }
+  if (done && !kLaunchersRecordEvents) Check(hipEventRecord(done, stream), "hipEventRecord");
 }
 
 void InferenceRunner::RunDevice(const float *deviceInputs, void *deviceResults, int64_t rows) {
@@ -402,14 +458,12 @@ void InferenceRunner::RunDevice(const float *deviceInputs, void *deviceResults, 
   const Workspace ws = OwnWorkspace(rows, m_stream);
   if (gMeasureGpuKernelTime) Check(hipEventRecord(m_evStart, m_stream), "hipEventRecord");
   for (int i = 0; i < runs; ++i) {
-    if (ClassIdsAsInt8())
-      Launch(deviceInputs, rows, nullptr, static_cast<int8_t *>(deviceResults), nullptr, nullptr, nullptr, m_stream, ws);
-    else
-      Launch(deviceInputs, rows, static_cast<float *>(deviceResults), nullptr, nullptr, nullptr, nullptr, m_stream, ws);
+    LaunchPredictions(deviceInputs, rows, deviceResults, m_stream, ws, m_callDone);
   }
   if (gMeasureGpuKernelTime) Check(hipEventRecord(m_evStop, m_stream), "hipEventRecord");
-  Check(hipStreamSynchronize(m_stream), "inference kernels");
+  if (rows > 0) Check(hipEventSynchronize(m_callDone), "inference kernels");
   if (gMeasureGpuKernelTime) {
+    Check(hipEventSynchronize(m_evStop), "inference kernels");
     float ms = 0.f;
     Check(hipEventElapsedTime(&ms, m_evStart, m_evStop), "hipEventElapsedTime");
     m_lastKernelMicros = (int64_t)(ms * 1000.0);
@@ -423,12 +477,13 @@ void InferenceRunner::RunDeviceOnStream(const float *deviceInputs, void *deviceR
   // The runner's own stream is idle here (every entry point that uses it waits for it before returning); an
   // earlier asynchronous call may still be running on another stream and uses the same buffers.
   const Workspace ws = OwnWorkspace(rows, stream);
-  if (ClassIdsAsInt8())
-    Launch(deviceInputs, rows, nullptr, static_cast<int8_t *>(deviceResults), nullptr, nullptr, nullptr, stream, ws);
-  else
-    Launch(deviceInputs, rows, static_cast<float *>(deviceResults), nullptr, nullptr, nullptr, nullptr, stream, ws);
-  Check(hipEventRecord(m_asyncDone, stream), "hipEventRecord");
+  // The event costs a small call 1.4 us, and calls on one stream need none.  The default stream is there as long as
+  // the process is, so its event can wait until a call comes on another stream; a stream of the caller's may be
+  // destroyed before that.
+  const bool record = stream != nullptr;
+  LaunchPredictions(deviceInputs, rows, deviceResults, stream, ws, record ? m_asyncDone : nullptr);
   m_asyncStream = stream;
+  m_asyncRecorded = record;
   m_asyncPending = true;
 }
 
@@ -438,8 +493,9 @@ void InferenceRunner::RunDeviceNoAlloc(const float *deviceInputs, void *deviceRe
   if (rows < 0) throw Error("negative row count");
   if (rows == 0) return;
   if (!deviceInputs || !deviceResults) throw Error("null device buffer");
-  const size_t partialBytes = FusesArgmax() ? 0 : (PartialBytes(rows) + 255) & ~(size_t)255; // (no partial sums when the walk keeps the arg-max)
-  const size_t ranksBytes = RanksBytes(rows);
+  const bool few = TakesFewRows(rows);
+  const size_t partialBytes = few || FusesArgmax() ? 0 : (PartialBytes(rows) + 255) & ~(size_t)255; // (no partial sums when the walk keeps the arg-max)
+  const size_t ranksBytes = few ? 0 : RanksBytes(rows);
   if (partialBytes + ranksBytes > kNoAllocScratchBytes)
     throw Error("this launch plan needs " + std::to_string(partialBytes + ranksBytes) + " bytes of scratch memory for " +
                 std::to_string(rows) + " rows; the fixed array of the no-allocation entry point holds " +
@@ -450,22 +506,19 @@ void InferenceRunner::RunDeviceNoAlloc(const float *deviceInputs, void *deviceRe
   ws.ranks = base + partialBytes;
   // Every partial sum the finalize kernel reads and every rank the walk reads is written earlier in
   // this same call, so nothing has to be cleared between calls.
-  if (ClassIdsAsInt8())
-    Launch(deviceInputs, rows, nullptr, static_cast<int8_t *>(deviceResults), nullptr, nullptr, nullptr, stream, ws);
-  else
-    Launch(deviceInputs, rows, static_cast<float *>(deviceResults), nullptr, nullptr, nullptr, nullptr, stream, ws);
+  LaunchPredictions(deviceInputs, rows, deviceResults, stream, ws);
 }
 
 void InferenceRunner::RunDeviceMulticlass(const float *deviceInputs, int64_t rows, int8_t *classIds, float *margins,
                                           float *probabilities) {
   if (m_forest.numClasses == 0) throw Error("model is not a multiclass classifier");
-  Launch(deviceInputs, rows, nullptr, classIds, margins, probabilities, nullptr, m_stream, OwnWorkspace(rows, m_stream));
-  Check(hipStreamSynchronize(m_stream), "inference kernels");
+  Launch(deviceInputs, rows, nullptr, classIds, margins, probabilities, nullptr, m_stream, OwnWorkspace(rows, m_stream), m_callDone);
+  if (rows > 0) Check(hipEventSynchronize(m_callDone), "inference kernels");
 }
 
 void InferenceRunner::DumpLeafIds(const float *deviceInputs, int32_t *deviceLeafIds, int64_t rows) {
   // results of the prediction itself are discarded
-  const Workspace ws = OwnWorkspace(rows, m_stream);
+  const Workspace ws = OwnWorkspace(rows, m_stream, true);
   float *scratch = nullptr;
   Check(hipMalloc(reinterpret_cast<void **>(&scratch), std::max<int64_t>(rows, 1) * sizeof(float)), "allocate scratch");
   try {
@@ -497,6 +550,9 @@ void InferenceRunner::RunHost(const void *hostInputs, void *hostResults, int64_t
 
 namespace {
 
+// Host batches up to this many bytes of rows are read by the kernel where they lie in pinned memory.
+constexpr size_t kSmallHostBytes = (size_t)512 << 10;
+
 // True when the runtime knows the address as pinned (or registered) host memory, which DMA reads
 // directly; pageable memory makes the query fail, and that error must not linger.
 bool IsPinnedHost(const void *ptr) {
@@ -512,9 +568,22 @@ bool IsPinnedHost(const void *ptr) {
 
 void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, int64_t rows) {
   if (rows <= 0) return;
-  EnsureStaging(rows);
   const size_t rowBytes = (size_t)m_forest.numFeatures * sizeof(float);
   const size_t totalBytes = (size_t)rows * rowBytes;
+  // A few rows: the kernel reads them out of pinned host memory itself and leaves the results there - one launch and
+  // one wait instead of two copies around the kernels (each row is read once, so a copy to the device buys nothing).
+  if (!gMeasureGpuKernelTime && TakesFewRows(rows) && totalBytes <= kSmallHostBytes) {
+    if (!m_smallHost) Check(hipHostMalloc(&m_smallHost, kSmallHostBytes + (size_t)m_fewRowsLimit * sizeof(float), hipHostMallocDefault), "allocate pinned staging");
+    float *in = static_cast<float *>(m_smallHost);
+    void *results = static_cast<char *>(m_smallHost) + kSmallHostBytes;
+    std::memcpy(in, hostInputs, totalBytes);
+    OrderAfterAsyncCall(m_stream);
+    LaunchPredictions(in, rows, results, m_stream, Workspace(), m_callDone);
+    Check(hipEventSynchronize(m_callDone), "inference kernels");
+    std::memcpy(hostResults, results, (size_t)rows * ReturnTypeBytes());
+    return;
+  }
+  EnsureStaging(rows);
   // Large batches go through in pieces: the copy of piece i+1 (on its own stream) overlaps the kernels
   // of piece i.  Rows are independent, so the pieces give the same results as one launch.
   if (gMeasureGpuKernelTime || totalBytes < ((size_t)16 << 20) || rows < 2 * 4096) {
@@ -559,10 +628,7 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
       Check(hipMemcpyAsync(dIn, src, (size_t)count * rowBytes, hipMemcpyHostToDevice, m_copyStream), "copy inputs");
       Check(hipEventRecord(m_pieceReady[p], m_copyStream), "hipEventRecord");
       Check(hipStreamWaitEvent(m_stream, m_pieceReady[p], 0), "hipStreamWaitEvent");
-      if (ClassIdsAsInt8())
-        Launch(dIn, count, nullptr, static_cast<int8_t *>(m_dStageOut) + first, nullptr, nullptr, nullptr, m_stream, ws);
-      else
-        Launch(dIn, count, static_cast<float *>(m_dStageOut) + first, nullptr, nullptr, nullptr, nullptr, m_stream, ws);
+      LaunchPredictions(dIn, count, static_cast<char *>(m_dStageOut) + first * ReturnTypeBytes(), m_stream, ws);
     }
     Check(hipStreamSynchronize(m_stream), "inference kernels");
   }
@@ -572,7 +638,7 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
 void InferenceRunner::TimeKernels(const float *deviceInputs, void *deviceResults, int64_t rows, int32_t runs,
                                   double *walkMs, double *finalizeMs, double *binMs) {
   runs = std::max(1, runs);
-  const Workspace ws = OwnWorkspace(rows, m_stream);
+  const Workspace ws = OwnWorkspace(rows, m_stream, true);
   const bool fused = FusesArgmax();
   const bool finalize = NeedsFinalize() && !fused;
   float ms = 0.f;
@@ -773,6 +839,7 @@ std::string InferenceRunner::DescribePlan() const {
      << " staging=" << (DirectStaging() ? "direct" : "registers")
      << " peelWalks=" << peel << " treesTiledByProfile=" << m_model.treesTiledByProfile
      << " lockStepSteps=" << m_model.lockStepSteps << " profiledSteps=" << m_model.profiledSteps
+     << " fewRowsLimit=" << m_fewRowsLimit
      << " treesDeferred=" << m_model.treesDeferred << " deferredEntriesPerRow=" << m_model.deferredEntriesPerRow;
   return os.str();
 }

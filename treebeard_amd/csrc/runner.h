@@ -72,6 +72,11 @@ public:
                    double *finalizeMs, double *binMs);
   // Re-packs the model for another launch plan (used by the timed search).
   void Repack(const LaunchPlan &plan);
+  // A plan the caller chose: every call runs it, small batches included.
+  void PinPlan(const LaunchPlan &plan) {
+    Repack(plan);
+    m_planPinned = true;
+  }
   // Timed search over CandidatePlans(); keeps the fastest.  Returns its time in ms.  A runner without a hit-count
   // profile profiles up to 4096 of the rows itself, so that peeled walks can be among the candidates.
   double AutoTune(const float *deviceInputs, int64_t rows);
@@ -107,12 +112,17 @@ private:
   void RunHostChunk(const void *hostInputs, void *hostResults, int64_t rows);
   void InitDevice();
   // Ordering of calls that share the runner's buffers (see RunDeviceOnStream).
+  void RecordAsyncCall();                        // the event behind the last asynchronous call, if it has none yet
   void OrderAfterAsyncCall(hipStream_t stream); // device-side: `stream` waits for the last asynchronous call
   void WaitForAsyncCall();                       // host-side: returns when the last asynchronous call has finished
   void UploadModel();
+  void UploadFewRows();
   void FreeModel();
   void EnsurePartial(int64_t rows);
   void EnsureStaging(int64_t rows);
+  // Batches of a few rows go through LaunchFewRows, whatever the launch plan, unless the caller pinned a plan or asked
+  // for peeled walks.
+  bool TakesFewRows(int64_t rows) const { return rows <= m_fewRowsLimit && !m_planPinned && !m_model.plan.peelWalks; }
   void EnsureRanks(int64_t rows);
   // Device memory the kernels of one call use beyond inputs and outputs.
   struct Workspace {
@@ -121,7 +131,8 @@ private:
   };
   // Allocating callers: grows the runner's own buffers to hold `rows` rows and orders `stream`, on which the
   // caller is about to launch, behind an asynchronous call that may still use them.
-  Workspace OwnWorkspace(int64_t rows, hipStream_t stream);
+  // `planKernels`: the call runs the launch plan's kernels however few rows it has.
+  Workspace OwnWorkspace(int64_t rows, hipStream_t stream, bool planKernels = false);
   size_t PartialBytes(int64_t rows) const;
   size_t RanksBytes(int64_t rows) const;
   // Rank-quantised plans: runs the binning kernel and returns the buffer the walk kernel reads.
@@ -133,8 +144,15 @@ private:
   }
   WalkParams MakeWalkParams(const float *deviceInputs, int64_t rows) const;
   hipError_t LaunchWalk(const WalkParams &p, hipStream_t stream) const;
+  // `done` (may be null) is recorded behind the last kernel.
   void Launch(const float *deviceInputs, int64_t rows, float *out, int8_t *classOut, float *margins,
-              float *probabilities, int32_t *leafIds, hipStream_t stream, const Workspace &ws);
+              float *probabilities, int32_t *leafIds, hipStream_t stream, const Workspace &ws, hipEvent_t done = nullptr);
+  // The predictions alone, as RunInference returns them (ReturnTypeBytes() per row).
+  void LaunchPredictions(const float *deviceInputs, int64_t rows, void *results, hipStream_t stream, const Workspace &ws,
+                         hipEvent_t done = nullptr) {
+    if (ClassIdsAsInt8()) Launch(deviceInputs, rows, nullptr, static_cast<int8_t *>(results), nullptr, nullptr, nullptr, stream, ws, done);
+    else Launch(deviceInputs, rows, static_cast<float *>(results), nullptr, nullptr, nullptr, nullptr, stream, ws, done);
+  }
 
   Forest m_forest;
   std::unique_ptr<HitCountProfile> m_profile;
@@ -152,9 +170,15 @@ private:
   size_t m_pinnedBytes = 0;
   std::unique_ptr<ParallelCopier> m_copier;
   hipEvent_t m_evStart = nullptr, m_evStop = nullptr;
+  hipEvent_t m_callDone = nullptr;  // behind the kernels of a call that waits for them
   hipEvent_t m_asyncDone = nullptr; // recorded behind the kernels of the last RunDeviceOnStream call
   hipStream_t m_asyncStream = nullptr;
-  bool m_asyncPending = false;
+  bool m_asyncPending = false, m_asyncRecorded = false;
+  bool m_planPinned = false;
+  int64_t m_fewRowsLimit = 0;
+  DeviceFewRowsBlock *m_dFewRows = nullptr;
+  int32_t *m_dFewRowsClasses = nullptr;
+  void *m_smallHost = nullptr;      // pinned host memory the few-rows kernel reads rows from and leaves results in
 
   DeviceGlobalNode *m_dGlobalNodes = nullptr;
   DeviceGlobalTree *m_dGlobalTrees = nullptr;

@@ -390,7 +390,7 @@ int32_t tbmi_set_plan(intptr_t h, int32_t rowsPerBlock, int32_t treeThreads, int
         // stub column's and the queues' share)
         plan.deferTails = false;
         if (plan.peelWalks && r->Profile() && plan.WalkTile() == 1 && DeferTailsFit(r->GetForest(), &plan)) plan.deferTails = true;
-        r->Repack(plan);
+        r->PinPlan(plan);
         return 0;
       },
       -1);
@@ -415,7 +415,7 @@ int32_t tbmi_set_tree_parallel_plan(intptr_t h, int32_t rowsPerBlock, int32_t tr
         if (groupBytes > 0) plan.groupBytes = groupBytes;
         else plan.groupBytes = std::min(plan.groupBytes, 256 * plan.ThreadsPerBlock());
         if (treeSlices > 0) plan.treeSlices = treeSlices;
-        r->Repack(plan);
+        r->PinPlan(plan);
         return 0;
       },
       -1);
@@ -436,7 +436,7 @@ int32_t tbmi_set_global_walk_plan(intptr_t h, int32_t rowsPerBlock, int32_t inte
         plan.interleave = interleave > 0 ? interleave : 4;
         plan.treeSlices = treeSlices > 0 ? treeSlices : 1;
         plan.groupBytes = 0;
-        r->Repack(plan);
+        r->PinPlan(plan);
         return 0;
       },
       -1);
@@ -460,7 +460,7 @@ int32_t tbmi_set_quantized_plan(intptr_t h, int32_t treeThreads, int32_t interle
         if (groupBytes > 0) plan.groupBytes = groupBytes;
         else plan.groupBytes = std::min(plan.groupBytes, 256 * plan.ThreadsPerBlock());
         plan.treeSlices = treeSlices > 0 ? treeSlices : 1;
-        r->Repack(plan);
+        r->PinPlan(plan);
         return 0;
       },
       -1);
@@ -484,7 +484,7 @@ int32_t tbmi_set_rank16_plan(intptr_t h, int32_t rowsPerBlock, int32_t treeThrea
         if (groupBytes > 0) plan.groupBytes = groupBytes;
         else plan.groupBytes = std::min(plan.groupBytes, 256 * plan.ThreadsPerBlock());
         plan.treeSlices = treeSlices > 0 ? treeSlices : 1;
-        r->Repack(plan);
+        r->PinPlan(plan);
         return 0;
       },
       -1);
