@@ -54,17 +54,42 @@ struct WalkParams {
   const int32_t *nodeOrigin = nullptr;
   const int32_t *slotTree = nullptr;
   hipEvent_t done = nullptr;      // recorded when this kernel completes (kLaunchersRecordEvents)
+  // Row-parallel walk on f32 or one-byte rank rows, kLaunchersSplitEvenly: `splitBlocks` blocks (0: one per row block and
+  // tree slice) share the units row block x tree group evenly; partial holds SplitLine::Slots slots.
+  int32_t splitBlocks = 0;
 };
 
 // From this many tree slices on, small batches are finalized by a wave per (row, class); classifiers then need
 // one spare slot of [rows][classes] doubles behind the last slice of the partial sums.
 constexpr int kWideFinalizeSlices = 16;
 
+// Row blocks x tree groups as one line of units, cut into equal parts for `blocks` <= units blocks.
+struct SplitLine {
+  int64_t units;
+  int32_t groups, blocks;
+#if defined(__HIP__)
+  __host__ __device__
+#endif
+  int64_t FirstUnit(int64_t block) const { return block * units / blocks; }
+#if defined(__HIP__)
+  __host__ __device__
+#endif
+  int64_t FirstBlock(int64_t rowBlock) const { return ((rowBlock * groups + 1) * blocks - 1) / units; } // (the owner of its first unit)
+#if defined(__HIP__)
+  __host__ __device__
+#endif
+  int Parts(int64_t rowBlock) const { return (int)(((rowBlock + 1) * groups * blocks - 1) / units - FirstBlock(rowBlock)) + 1; }
+  // The most parts any row block has.
+  static int64_t Slots(int64_t blocks, int64_t rowBlocks) { return (blocks + rowBlocks - 1) / rowBlocks + (blocks % rowBlocks ? 1 : 0); }
+};
+
 struct FinalizeParams {
   double *partial = nullptr;   // [slices (+ 1 spare, see kWideFinalizeSlices)][rows][max(1, classes)]
   int64_t rows = 0;
   int32_t numClasses = 0;
   int32_t treeSlices = 1;      // number of partial sums per (row, class)
+  int32_t splitBlocks = 0;     // a split walk: its blocks, rows per block and tree groups (treeSlices: slots)
+  int32_t rowsPerBlock = 0, groups = 0;
   double initialValue = 0.0;
   int32_t transform = 0;
   float *out = nullptr;        // regression / binary prediction, may be null for multiclass
@@ -92,12 +117,14 @@ struct FewRowsParams {
 
 #if defined(__HIP__)
 inline constexpr bool kLaunchersRecordEvents = true;
+inline constexpr bool kLaunchersSplitEvenly = true;
 // How many rows of such a forest LaunchFewRows takes sooner than the launch plans do (0: never).
 int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth);
 hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream);
 #else
 // (host-only builds of the runner, under the sanitizers, link stand-ins of the launchers below and have no others)
 inline constexpr bool kLaunchersRecordEvents = false;
+inline constexpr bool kLaunchersSplitEvenly = false;
 inline int64_t FewRowsLimit(int32_t, int32_t, int32_t, int32_t) { return 0; }
 inline hipError_t LaunchFewRows(const FewRowsParams &, hipStream_t) { return hipErrorNotSupported; }
 #endif

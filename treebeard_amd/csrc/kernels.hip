@@ -146,18 +146,20 @@ __device__ __forceinline__ void StageRows(const float *__restrict__ src, int val
 // the classifiers' running arg-max (WalkScalars::fuseArgmax).
 enum WalkVariant : int { kWalkPlain = 0, kWalkDump = 1, kWalkDefer = 2, kWalkFuse = 3 };
 
+// Groups [gBegin, gEnd) of one row block: everything a block of the row-parallel walk does.  `slice` names the slot of
+// the partial sums this part fills.
 template <int K, int PF, int kMode, int kVariant>
-__global__ void __launch_bounds__(1024)
-WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16,
-                  const DeviceBundle *__restrict__ bundles, const DeviceNode *__restrict__ bundleRoots,
-                  const DeviceGroup *__restrict__ groups,
-                  const WalkScalars s, float *__restrict__ out, int8_t *__restrict__ classOut,
-                  double *__restrict__ partial, int32_t *__restrict__ leafIds, const int32_t *__restrict__ nodeOrigin,
-                  const int32_t *__restrict__ slotTree, const U32x2 *__restrict__ tailNodes, const int32_t *__restrict__ tailOrigin) {
+__device__ __forceinline__ void
+WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int slice,
+             const float *__restrict__ x, const uint4 *__restrict__ nodes16,
+             const DeviceBundle *__restrict__ bundles, const DeviceNode *__restrict__ bundleRoots,
+             const DeviceGroup *__restrict__ groups,
+             const WalkScalars &s, float *__restrict__ out, int8_t *__restrict__ classOut,
+             double *__restrict__ partial, int32_t *__restrict__ leafIds, const int32_t *__restrict__ nodeOrigin,
+             const int32_t *__restrict__ slotTree, const U32x2 *__restrict__ tailNodes, const int32_t *__restrict__ tailOrigin) {
   constexpr bool kDump = kVariant == kWalkDump, kDefer = kVariant == kWalkDefer, kFuse = kVariant == kWalkFuse;
   // LDS: [tree group nodes | transposed row tile].  The group sits at LDS
   // address 0 so that node pointers are LDS addresses as stored.
-  extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x;
   const int threads = blockDim.x;
   const int RB = s.rowsPerBlock;
@@ -166,9 +168,26 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
   // uniform inside a wave (RB is a multiple of 64); readfirstlane tells the compiler so
   const int tt = __builtin_amdgcn_readfirstlane(tid / RB);
   const int F = s.numFeatures;
-  const int64_t row0 = (int64_t)blockIdx.x * RB;
+  const int64_t row0 = rowBlock * RB;
   const int64_t remaining = s.rows - row0;
   const int valid = remaining < RB ? (int)remaining : RB;
+
+  // Direct staging: a group is copied by global -> LDS loads (lane i of a wave-wide load leaves its 16 bytes at base +
+  // 16 i, lanes switched off write nothing): no staging registers, no LDS store instructions.  The block waits for its
+  // own copy; the CU's other block walks meanwhile, which is why launch plans ask for this form only when two blocks
+  // fit a CU.
+#define TBAMD_COPY_GROUP(GRP)                                                                                          \
+  {                                                                                                                    \
+    const U32x4 *src = reinterpret_cast<const U32x4 *>(nodes16) + ((GRP).nodeBegin >> 1);                              \
+    const int pieces = (int)((GRP).nodeCount >> 1);                                                                    \
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);                                                         \
+    for (int first = wave * 64; first < pieces; first += threads)                                                      \
+      if (first + (tid & 63) < pieces)                                                                                 \
+        __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + first + (tid & 63)),   \
+                                         (__attribute__((address_space(3))) void *)(lds + (uint32_t)first * 16u), 16, 0, 0); \
+  }
+  // the first group is on its way while the rows are staged
+  if (PF == 0 && gBegin < gEnd) TBAMD_COPY_GROUP(groups[gBegin])
 
   uint32_t column; // LDS address of this row's feature 0
   if (IsRankTile(kMode)) {
@@ -176,7 +195,7 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
     // column is filled here), or two bytes each as [row block][feature pair][row][2], pad feature included.
     typedef uint32_t Piece __attribute__((ext_vector_type(4)));
     const int tileBytes = kMode == kTileRankU8 ? F * RB : ((F + 2) >> 1) * RB * 4;
-    const Piece *src = reinterpret_cast<const Piece *>(reinterpret_cast<const uint8_t *>(x) + (int64_t)blockIdx.x * tileBytes);
+    const Piece *src = reinterpret_cast<const Piece *>(reinterpret_cast<const uint8_t *>(x) + rowBlock * tileBytes);
     Piece *dst = reinterpret_cast<Piece *>(lds + s.groupRegionBytes);
     const int pieces = tileBytes >> 4;
     for (int base = 0; base < pieces; base += threads * kStageUnroll) {
@@ -215,9 +234,6 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
   const uint32_t laneTag = (uint32_t)(tid & 63) << 26;            // a queue entry: lane << 26 | tail index
   uint32_t queued = 0;                                            // entries in the queue (the same in every lane)
 
-  const int slice = blockIdx.y;
-  const int gBegin = (int)(((int64_t)s.numGroups * slice) / s.treeSlices);
-  const int gEnd = (int)(((int64_t)s.numGroups * (slice + 1)) / s.treeSlices);
   const int C = s.numClasses;
   const int64_t row = row0 + lane;
   double *partialRow = partial ? partial + ((int64_t)slice * s.rows + row) * (C > 0 ? C : 1) : nullptr;
@@ -321,7 +337,7 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
 
   for (int g = gBegin; g < gEnd; ++g) {
     const DeviceGroup grp = groups[g];
-    __syncthreads(); // rows staged / previous group no longer read
+    if (PF > 0 || g > gBegin) __syncthreads(); // rows staged / previous group no longer read
     if (PF > 0) {
       U32x4 *dst = reinterpret_cast<U32x4 *>(lds);
       const int pieces = (int)(grp.nodeCount >> 1);
@@ -331,17 +347,7 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
         if (idx < pieces) dst[idx] = fetched[i];
       }
     } else {
-      // Direct staging: the group is copied by global -> LDS loads (lane i of a wave-wide load leaves its 16 bytes
-      // at base + 16 i, lanes switched off write nothing): no staging registers, no LDS store instructions.  The
-      // block waits for its own copy; the CU's other block walks meanwhile, which is why launch plans ask for
-      // this form only when two blocks fit a CU.
-      const U32x4 *src = reinterpret_cast<const U32x4 *>(nodes16) + (grp.nodeBegin >> 1);
-      const int pieces = (int)(grp.nodeCount >> 1);
-      const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-      for (int first = wave * 64; first < pieces; first += threads)
-        if (first + (tid & 63) < pieces)
-          __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void *)(src + first + (tid & 63)),
-                                           (__attribute__((address_space(3))) void *)(lds + (uint32_t)first * 16u), 16, 0, 0);
+      if (g > gBegin) TBAMD_COPY_GROUP(grp)
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     }
     __syncthreads();
@@ -482,9 +488,62 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
     const double margin = s.initialValue + acc;
     out[row] = (float)(s.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
   }
+#undef TBAMD_COPY_GROUP
 #undef TBAMD_FLUSH_CLASS
 #undef TBAMD_PREFETCH_GROUP
 #undef TBAMD_WALK_QUEUE
+}
+
+template <int K, int PF, int kMode, int kVariant>
+__global__ void __launch_bounds__(1024)
+WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16,
+                  const DeviceBundle *__restrict__ bundles, const DeviceNode *__restrict__ bundleRoots,
+                  const DeviceGroup *__restrict__ groups,
+                  const WalkScalars s, float *__restrict__ out, int8_t *__restrict__ classOut,
+                  double *__restrict__ partial, int32_t *__restrict__ leafIds, const int32_t *__restrict__ nodeOrigin,
+                  const int32_t *__restrict__ slotTree, const U32x2 *__restrict__ tailNodes, const int32_t *__restrict__ tailOrigin) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const int slice = blockIdx.y;
+  const int gBegin = (int)(((int64_t)s.numGroups * slice) / s.treeSlices);
+  const int gEnd = (int)(((int64_t)s.numGroups * (slice + 1)) / s.treeSlices);
+  WalkRowBlock<K, PF, kMode, kVariant>(lds, blockIdx.x, gBegin, gEnd, slice, x, nodes16, bundles, bundleRoots, groups, s, out, classOut,
+                                       partial, leafIds, nodeOrigin, slotTree, tailNodes, tailOrigin);
+}
+
+// ---------------------------------------------------------------------------
+// The row-parallel walk for batches of a few rounds of blocks.  Row blocks x tree groups are one line of units, cut
+// into as many equal parts as blocks run at once: no last round that is nearly empty (65537 rows in blocks of 256 x 2
+// tree slices are 514 blocks for 512 places, which took twice the time of 512), and a block stages the rows of the row
+// blocks its part touches, one or two.  Part p of a row block leaves its sums in slot p of the partial sums, which the
+// finalize kernel adds in order.  (Adding them in the block that comes last, found with a ticket, was measured: the
+// write-through stores, the ticket and the reads are three round trips to memory, 5 to 12 us where the finalize launch
+// takes 4.)
+// ---------------------------------------------------------------------------
+template <int K, int kMode>
+// (80 SGPRs: with the 16 the trap handler takes, 8 waves per SIMD - two blocks of 16 waves - leave each wave 100; at 88 one
+// block per CU ran, 40 % slower)
+__global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80)))
+WalkRowsSplitKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16,
+                    const DeviceBundle *__restrict__ bundles, const DeviceNode *__restrict__ bundleRoots,
+                    const DeviceGroup *__restrict__ groups, const WalkScalars s, double *__restrict__ partial) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  const SplitLine line{((s.rows + s.rowsPerBlock - 1) / s.rowsPerBlock) * s.numGroups, s.numGroups, (int)gridDim.x};
+  WalkScalars own = s;
+  int64_t unit = line.FirstUnit(blockIdx.x);
+  const int64_t unitEnd = line.FirstUnit((int64_t)blockIdx.x + 1);
+  while (unit < unitEnd) {
+    // (what the walk computes from these is computed again for every row block, not kept in registers across them)
+    asm volatile("" : "+s"(own.rowsPerBlock), "+s"(own.numFeatures), "+s"(own.treeThreads), "+s"(own.groupRegionBytes));
+    const int64_t rowBlock = unit / line.groups;
+    const int gBegin = (int)(unit - rowBlock * line.groups);
+    const int64_t left = unitEnd - rowBlock * line.groups;
+    const int gEnd = (int)(left < line.groups ? left : line.groups);
+    WalkRowBlock<K, 0, kMode, kWalkPlain>(lds, rowBlock, gBegin, gEnd, (int)((int64_t)blockIdx.x - line.FirstBlock(rowBlock)), x, nodes16,
+                                          bundles, bundleRoots, groups, own, nullptr, nullptr, partial, nullptr, nullptr, nullptr, nullptr,
+                                          nullptr);
+    unit += gEnd - gBegin;
+    __syncthreads(); // the rows' tile and the group are rewritten
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -1217,28 +1276,6 @@ RankRows16Kernel(const float *__restrict__ x, const float *__restrict__ tables, 
   }
 }
 
-// A row's class sums -> class id (arg-max of the f32 sums, ties to the larger id) and, on request, the f32 sums and
-// their softmax.
-__device__ __forceinline__ void FinishClasses(const double *sums, int C, int64_t row, float *out, int8_t *classOut,
-                                              float *margins, float *probabilities) {
-  float best = -INFINITY;
-  int bestClass = 0;
-  double maxMargin = -INFINITY;
-  for (int c = 0; c < C; ++c) {
-    const float m = (float)sums[c];
-    if (margins) margins[row * C + c] = m;
-    if (!(best > m)) { best = m; bestClass = c; }
-    maxMargin = sums[c] > maxMargin ? sums[c] : maxMargin;
-  }
-  if (classOut) classOut[row] = (int8_t)bestClass;
-  if (out) out[row] = (float)bestClass;
-  if (probabilities) {
-    double z = 0.0;
-    for (int c = 0; c < C; ++c) z += exp(sums[c] - maxMargin);
-    for (int c = 0; c < C; ++c) probabilities[row * C + c] = (float)(exp(sums[c] - maxMargin) / z);
-  }
-}
-
 // ---------------------------------------------------------------------------
 // Sums the tree-slice partials of each row (in slice order, starting from the
 // initial value), then applies the output transform.  Multiclass rows get the
@@ -1247,48 +1284,120 @@ __device__ __forceinline__ void FinishClasses(const double *sums, int C, int64_t
 // src/mlir/LowerReduceOps.cpp:148-187) and, on request, the sums and their
 // softmax.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) FinalizeKernel(const FinalizeParams p) {
-  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (row >= p.rows) return;
-  const int C = p.numClasses;
-  if (C == 0) {
-    double margin = p.initialValue;
-    for (int s = 0; s < p.treeSlices; ++s) margin += p.partial[(int64_t)s * p.rows + row];
-    p.out[row] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
-    return;
-  }
+// A row's class sums -> class id (arg-max of the f32 sums, ties to the larger id) and, on request, the f32 sums and
+// their softmax.
+template <typename SumOf> // class -> its sum
+__device__ __forceinline__ void FinishClasses(SumOf sumOf, int C, int64_t row, float *out, int8_t *classOut, float *margins,
+                                              float *probabilities) {
   float best = -INFINITY;
   int bestClass = 0;
   double maxMargin = -INFINITY;
   for (int c = 0; c < C; ++c) {
-    double margin = p.initialValue;
-    for (int s = 0; s < p.treeSlices; ++s) margin += p.partial[((int64_t)s * p.rows + row) * C + c];
-    const float m = (float)margin;
-    if (p.margins) p.margins[row * C + c] = m;
+    const double sum = sumOf(c);
+    const float m = (float)sum;
+    if (margins) margins[row * C + c] = m;
     if (!(best > m)) { best = m; bestClass = c; }
-    maxMargin = margin > maxMargin ? margin : maxMargin;
+    maxMargin = sum > maxMargin ? sum : maxMargin;
   }
-  if (p.classOut) p.classOut[row] = (int8_t)bestClass;
-  if (p.out) p.out[row] = (float)bestClass;
-  if (p.probabilities) {
+  if (classOut) classOut[row] = (int8_t)bestClass;
+  if (out) out[row] = (float)bestClass;
+  if (probabilities) {
     double z = 0.0;
-    for (int c = 0; c < C; ++c) {
-      double margin = p.initialValue;
-      for (int s = 0; s < p.treeSlices; ++s) margin += p.partial[((int64_t)s * p.rows + row) * C + c];
-      z += exp(margin - maxMargin);
-    }
-    for (int c = 0; c < C; ++c) {
-      double margin = p.initialValue;
-      for (int s = 0; s < p.treeSlices; ++s) margin += p.partial[((int64_t)s * p.rows + row) * C + c];
-      p.probabilities[row * C + c] = (float)(exp(margin - maxMargin) / z);
-    }
+    for (int c = 0; c < C; ++c) z += exp(sumOf(c) - maxMargin);
+    for (int c = 0; c < C; ++c) probabilities[row * C + c] = (float)(exp(sumOf(c) - maxMargin) / z);
   }
+}
+
+// How many slots of the partial sums hold parts of a row.
+__device__ __forceinline__ int PartsOfRow(const FinalizeParams &p, int64_t row) {
+  if (p.splitBlocks == 0) return p.treeSlices;
+  return SplitLine{((p.rows + p.rowsPerBlock - 1) / p.rowsPerBlock) * p.groups, p.groups, p.splitBlocks}.Parts(row / p.rowsPerBlock);
+}
+
+__global__ void __launch_bounds__(256) FinalizeKernel(const FinalizeParams p) {
+  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (row >= p.rows) return;
+  const int parts = PartsOfRow(p, row);
+  double margin = p.initialValue;
+#pragma unroll 4
+  for (int s = 0; s < parts; ++s) margin += p.partial[(int64_t)s * p.rows + row];
+  p.out[row] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
+}
+
+// Classifiers: the block's rows x classes are read as they lie (coalesced; a lane per row read a line per class and all
+// of them three times: 13 us for 65537 rows x 8 classes x 2 slices), meet in LDS, and the rows are finished there.
+constexpr int kFinalizeLds = 4096; // doubles of sums a block holds
+
+__global__ void __launch_bounds__(256) FinalizeClassesKernel(const FinalizeParams p, int rowsPerBlock) {
+  extern __shared__ __align__(16) unsigned char lds[];
+  double *sums = reinterpret_cast<double *>(lds); // [row][class], rows an odd number of doubles apart
+  const int C = p.numClasses, stride = C | 1;
+  double *rowMax = sums + rowsPerBlock * stride, *rowZ = rowMax + rowsPerBlock;
+  const int64_t row0 = (int64_t)blockIdx.x * rowsPerBlock;
+  const int valid = p.rows - row0 < rowsPerBlock ? (int)(p.rows - row0) : rowsPerBlock;
+  const int tid = threadIdx.x, threads = blockDim.x;
+  for (int e = tid; e < valid * C; e += threads) {
+    const int r = e / C, c = e - r * C;
+    const int parts = PartsOfRow(p, row0 + r);
+    double margin = p.initialValue;
+    for (int s = 0; s < parts; ++s) margin += p.partial[((int64_t)s * p.rows + row0) * C + e];
+    sums[r * stride + c] = margin;
+    if (p.margins) p.margins[row0 * C + e] = (float)margin;
+  }
+  __syncthreads();
+  for (int r = tid; r < valid; r += threads) {
+    float best = -INFINITY;
+    int bestClass = 0;
+    double maxMargin = -INFINITY;
+    for (int c = 0; c < C; ++c) {
+      const double margin = sums[r * stride + c];
+      const float m = (float)margin;
+      if (!(best > m)) { best = m; bestClass = c; }
+      maxMargin = margin > maxMargin ? margin : maxMargin;
+    }
+    if (p.classOut) p.classOut[row0 + r] = (int8_t)bestClass;
+    if (p.out) p.out[row0 + r] = (float)bestClass;
+    rowMax[r] = maxMargin;
+  }
+  if (!p.probabilities) return;
+  __syncthreads();
+  for (int e = tid; e < valid * C; e += threads) {
+    const int r = e / C, at = r * stride + (e - r * C);
+    sums[at] = exp(sums[at] - rowMax[r]);
+  }
+  __syncthreads();
+  for (int r = tid; r < valid; r += threads) {
+    double z = 0.0;
+    for (int c = 0; c < C; ++c) z += sums[r * stride + c];
+    rowZ[r] = z;
+  }
+  __syncthreads();
+  for (int e = tid; e < valid * C; e += threads) {
+    const int r = e / C;
+    p.probabilities[row0 * C + e] = (float)(sums[r * stride + (e - r * C)] / rowZ[r]);
+  }
+}
+
+// More classes than a block's LDS holds sums of: a lane per row adds the parts again each time a sum is needed.
+__global__ void __launch_bounds__(256) FinalizeManyClassesKernel(const FinalizeParams p) {
+  const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (row >= p.rows) return;
+  const int parts = PartsOfRow(p, row);
+  FinishClasses(
+      [&](int c) {
+        double margin = p.initialValue;
+        for (int s = 0; s < parts; ++s) margin += p.partial[((int64_t)s * p.rows + row) * p.numClasses + c];
+        return margin;
+      },
+      p.numClasses, row, p.out, p.classOut, p.margins, p.probabilities);
 }
 
 // Small batches split over many tree slices (kWideFinalizeSlices or more): one wave per (row, class).  The lanes fetch the slice
 // partials side by side (one memory latency instead of one per slice), each adds its slices in slice
 // order, and a fixed butterfly combines the lanes - the order of additions depends only on the number
 // of slices.
+constexpr int64_t kWideFinalizeItems = 8192; // (65536 took 15 us for 8192 rows x 8 classes)
+
 __global__ void __launch_bounds__(256) FinalizeWideKernel(const FinalizeParams p) {
   const int lane = threadIdx.x & 63;
   const int64_t item = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -1297,14 +1406,15 @@ __global__ void __launch_bounds__(256) FinalizeWideKernel(const FinalizeParams p
   const int64_t row = item / Cn;
   const int c = (int)(item - row * Cn);
   double sum = 0.0;
-  for (int s = lane; s < p.treeSlices; s += 64) sum += p.partial[((int64_t)s * p.rows + row) * Cn + c];
+  const int parts = PartsOfRow(p, row);
+  for (int s = lane; s < parts; s += 64) sum += p.partial[((int64_t)s * p.rows + row) * Cn + c];
   for (int m = 1; m <= 32; m <<= 1) sum += ShuffleXor(sum, m); // (ascending: see ShuffleXor)
   const double margin = p.initialValue + sum;
   if (p.numClasses == 0) {
     if (lane == 0) p.out[row] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
     return;
   }
-  // classifiers: the class sum goes into the spare slot behind the last slice; FinalizeKernel (1 slice, reading
+  // classifiers: the class sum goes into the spare slot behind the last slice; FinalizeClassesKernel (1 slice, reading
   // that slot) does the rest.  The slices themselves stay as they are, so the launch can be repeated.
   if (lane == 0) p.partial[((int64_t)p.treeSlices * p.rows + row) * Cn + c] = margin - p.initialValue;
 }
@@ -1404,7 +1514,7 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
   }
   if (p.numClasses == 0) return;
   __syncthreads();
-  if (tid < valid) FinishClasses(sums + tid * Cn, Cn, row0 + tid, p.out, p.classOut, p.margins, p.probabilities);
+  if (tid < valid) FinishClasses([&](int c) { return sums[tid * Cn + c]; }, Cn, row0 + tid, p.out, p.classOut, p.margins, p.probabilities);
 }
 
 // The ceiling on dynamic LDS is an attribute of each kernel on each device: it is raised once per kernel and
@@ -1441,6 +1551,17 @@ hipError_t LaunchWalkVariant(const WalkParams &p, dim3 grid, dim3 block, size_t 
                      reinterpret_cast<const U32x2 *>(p.tailNodes), p.tailOrigin);
 }
 
+template <int K, int W>
+hipError_t LaunchSplit(const WalkParams &p, dim3 block, size_t ldsBytes, hipStream_t stream) {
+  const int64_t rowBlocks = (p.s.rows + p.s.rowsPerBlock - 1) / p.s.rowsPerBlock;
+  if (p.splitBlocks < 1 || p.splitBlocks > rowBlocks * p.s.numGroups || !p.partial || p.leafIds || p.s.deferTails || p.s.fuseArgmax)
+    return hipErrorInvalidValue;
+  hipError_t e = AllowFullLds<&WalkRowsSplitKernel<K, W>>();
+  if (e != hipSuccess) return e;
+  return StartKernel(&WalkRowsSplitKernel<K, W>, dim3((unsigned)p.splitBlocks), block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles,
+                     p.bundleRoots, p.groups, p.s, p.partial);
+}
+
 template <int K, int PF, int W>
 hipError_t LaunchWalkKP(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream) {
   if (p.leafIds) { // (the dump kernel walks every bundle to its full depth and leaves the arg-max to the finalize kernel)
@@ -1458,6 +1579,7 @@ hipError_t LaunchWalkKP(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBy
 
 template <int K, int W>
 hipError_t LaunchWalkK(const WalkParams &p, int prefetch, dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream) {
+  if (p.splitBlocks) return LaunchSplit<K, W>(p, block, ldsBytes, stream);
   if (p.directStaging) return LaunchWalkKP<K, 0, W>(p, grid, block, ldsBytes, stream);
   if (prefetch <= 4) return LaunchWalkKP<K, 4, W>(p, grid, block, ldsBytes, stream);
   if (prefetch <= 8) return LaunchWalkKP<K, 8, W>(p, grid, block, ldsBytes, stream);
@@ -1483,6 +1605,7 @@ namespace {
 // Outputs the walk kernels dereference must be there: a fused epilogue writes p.out (or p.classOut), everything
 // else goes through p.partial.
 bool OutputsConsistent(const WalkParams &p) {
+  if (p.splitBlocks) return true; // (LaunchSplit)
   if (p.s.fuseArgmax) return p.s.numClasses > 0 && p.s.treeSlices == 1 && (p.out || p.classOut);
   if (p.s.numClasses > 0 || p.s.treeSlices > 1) return p.partial != nullptr;
   return p.out != nullptr || p.partial != nullptr;
@@ -1507,6 +1630,7 @@ hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, 
     return LaunchWalkW<kTileRankU8>(p, interleave, prefetch, grid, block, ldsBytes, stream);
   case kTileRankU16: // (tree groups always go straight from global memory into LDS)
     if ((int64_t)((p.s.numFeatures + 2) / 2) * RB * 4 > 0x10000) return hipErrorInvalidValue; // byte offsets
+    if (p.splitBlocks) return hipErrorInvalidValue; // (the plan search tries this form on full batches only)
     switch (interleave) {
     case 1: return LaunchWalkKP<1, 0, kTileRankU16>(p, grid, block, ldsBytes, stream);
     case 2: return LaunchWalkKP<2, 0, kTileRankU16>(p, grid, block, ldsBytes, stream);
@@ -1726,13 +1850,24 @@ hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
   const int Cn = p.numClasses > 0 ? p.numClasses : 1;
   FinalizeParams q = p;
-  if (p.treeSlices >= kWideFinalizeSlices && p.rows * Cn <= 65536) { // few rows, many slices: a wave per (row, class)
+  if (p.treeSlices >= kWideFinalizeSlices && p.rows * Cn <= kWideFinalizeItems) { // few rows, many slices: a wave per (row, class)
     const int64_t waves = p.rows * Cn;
     hipError_t e = StartKernel(&FinalizeWideKernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream,
                                p.numClasses == 0 ? p.done : nullptr, p);
     if (e != hipSuccess || p.numClasses == 0) return e;
     q.partial = p.partial + (int64_t)p.treeSlices * p.rows * Cn; // the class sums now sit in the spare slot
     q.treeSlices = 1;
+    q.splitBlocks = 0;
+  }
+  if (q.numClasses > 0) {
+    // (rows of a block: as many as LDS holds, fewer where that leaves compute units without a block)
+    const int64_t perBlock = std::max<int64_t>(1, std::min<int64_t>({256, kFinalizeLds / (q.numClasses | 1), std::max<int64_t>(8, q.rows / 512)}));
+    const int64_t blocks = (q.rows + perBlock - 1) / perBlock;
+    const size_t ldsBytes = (size_t)perBlock * ((size_t)(q.numClasses | 1) + 2) * sizeof(double);
+    if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
+    if (ldsBytes > 64 * 1024)
+      return StartKernel(&FinalizeManyClassesKernel, dim3((unsigned)((q.rows + 255) / 256)), dim3(256), 0, stream, q.done, q);
+    return StartKernel(&FinalizeClassesKernel, dim3((unsigned)blocks), dim3(256), ldsBytes, stream, q.done, q, (int)perBlock);
   }
   const int64_t blocks = (q.rows + 255) / 256;
   return StartKernel(&FinalizeKernel, dim3((unsigned)blocks), dim3(256), 0, stream, q.done, q);

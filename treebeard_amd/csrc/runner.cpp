@@ -257,11 +257,12 @@ void InferenceRunner::Repack(const LaunchPlan &plan) {
   UploadModel();
 }
 
-size_t InferenceRunner::PartialBytes(int64_t rows) const {
-  if (!NeedsFinalize()) return 0;
+size_t InferenceRunner::PartialBytes(int64_t rows, bool split) const {
+  const int32_t splitBlocks = split ? SplitBlocks(rows) : 0;
+  if (split ? splitBlocks == 0 : !NeedsFinalize()) return 0;
+  size_t slots = split ? (size_t)SplitLine::Slots(splitBlocks, RowBlocks(rows)) : (size_t)m_model.PartialCount();
   // (+ the spare slot the wide finalize of a classifier leaves its class sums in)
-  const size_t slots = (size_t)m_model.PartialCount() +
-                       (m_forest.numClasses > 0 && m_model.PartialCount() >= kWideFinalizeSlices ? 1 : 0);
+  if (m_forest.numClasses > 0 && slots >= (size_t)kWideFinalizeSlices) ++slots;
   return slots * (size_t)rows * (size_t)std::max(1, m_forest.numClasses) * sizeof(double);
 }
 
@@ -276,8 +277,29 @@ size_t InferenceRunner::RanksBytes(int64_t rows) const {
   return (size_t)((rows + 63) / 64) * 64 * (size_t)m_forest.numFeatures;
 }
 
-void InferenceRunner::EnsurePartial(int64_t rows) {
-  const size_t need = PartialBytes(rows);
+int32_t InferenceRunner::SplitBlocks(int64_t rows) const {
+  const LaunchPlan &plan = m_model.plan;
+  if (!kLaunchersSplitEvenly || plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.WalkTile() > 1 || plan.rankRows16 ||
+      plan.deferTails)
+    return 0;
+  const int64_t blocks = RowBlocks(rows) * plan.treeSlices;
+  const int64_t perCu = std::max<int64_t>(1, std::min<int64_t>(2048 / plan.ThreadsPerBlock(),
+                                                               m_limits.ldsBytesPerBlock / (int64_t)(m_model.LdsBytes() + 512)));
+  const int64_t places = perCu * m_limits.computeUnits; // blocks that run at once
+  if (blocks <= places || blocks % places == 0) return 0;
+  WalkShape shape;
+  shape.rowBlocks = RowBlocks(rows);
+  shape.rowsPerBlock = plan.rowsPerBlock;
+  shape.numFeatures = m_forest.numFeatures;
+  shape.levels = (double)m_model.lockStepSteps;
+  shape.groups = (double)m_model.groups.size();
+  shape.computeUnits = m_limits.computeUnits;
+  shape.blocksPerUnit = (int32_t)perCu;
+  if (SplitWalkMicros(shape) >= SlicedWalkMicros(shape, plan.treeSlices)) return 0;
+  return (int32_t)std::min<int64_t>(places, RowBlocks(rows) * (int64_t)m_model.groups.size());
+}
+
+void InferenceRunner::EnsurePartial(size_t need) {
   if (need <= m_partialBytes) return;
   WaitForAsyncCall();
   Check(hipStreamSynchronize(m_stream), "hipStreamSynchronize");
@@ -302,7 +324,7 @@ void InferenceRunner::EnsureRanks(int64_t rows) {
 
 InferenceRunner::Workspace InferenceRunner::OwnWorkspace(int64_t rows, hipStream_t stream, bool planKernels) {
   if (planKernels || !TakesFewRows(rows)) {
-    EnsurePartial(rows);
+    EnsurePartial(std::max(PartialBytes(rows, false), PartialBytes(rows, true)));
     EnsureRanks(rows);
   }
   // An asynchronous call on another stream may still use these buffers: `stream` waits for it on the device.
@@ -397,6 +419,33 @@ WalkParams InferenceRunner::MakeWalkParams(const float *deviceInputs, int64_t ro
   return p;
 }
 
+bool InferenceRunner::SetOutputs(WalkParams &p, float *out, int8_t *classOut, float *margins, float *probabilities, bool leafIds,
+                                 const Workspace &ws) const {
+  p.splitBlocks = ws.split && !leafIds ? SplitBlocks(p.s.rows) : 0;
+  if (p.splitBlocks) {
+    p.partial = ws.partial;
+    return true;
+  }
+  // A classifier whose trees all sit in one slice needs no second kernel when only the class id is wanted:
+  // the row-parallel kernels keep the running arg-max themselves.
+  const bool fused = FusesArgmax() && !margins && !probabilities && !leafIds;
+  const bool finalize = NeedsFinalize() && !fused;
+  p.s.fuseArgmax = fused ? 1 : 0;
+  p.out = finalize ? nullptr : out;
+  p.classOut = fused ? classOut : nullptr;
+  p.partial = finalize ? ws.partial : nullptr;
+  return finalize;
+}
+
+void InferenceRunner::SetParts(FinalizeParams &f, const WalkParams &p) const {
+  f.treeSlices = m_model.PartialCount();
+  if (p.splitBlocks == 0) return;
+  f.splitBlocks = p.splitBlocks;
+  f.rowsPerBlock = p.s.rowsPerBlock;
+  f.groups = p.s.numGroups;
+  f.treeSlices = (int32_t)SplitLine::Slots(p.splitBlocks, RowBlocks(p.s.rows));
+}
+
 void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out, int8_t *classOut, float *margins,
                              float *probabilities, int32_t *leafIds, hipStream_t stream, const Workspace &ws, hipEvent_t done) {
   if (rows <= 0) return;
@@ -420,14 +469,7 @@ void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out
     return;
   }
   WalkParams p = MakeWalkParams(PrepareRows(deviceInputs, rows, ws.ranks, stream), rows);
-  // A classifier whose trees all sit in one slice needs no second kernel when only the class id is wanted:
-  // the row-parallel kernels keep the running arg-max themselves.
-  const bool fused = FusesArgmax() && !margins && !probabilities && !leafIds;
-  const bool finalize = NeedsFinalize() && !fused;
-  p.s.fuseArgmax = fused ? 1 : 0;
-  p.out = finalize ? nullptr : out;
-  p.classOut = fused ? classOut : nullptr;
-  p.partial = finalize ? ws.partial : nullptr;
+  const bool finalize = SetOutputs(p, out, classOut, margins, probabilities, leafIds != nullptr, ws);
   if (leafIds) {
     p.leafIds = leafIds;
     p.nodeOrigin = m_dNodeOrigin;
@@ -440,7 +482,7 @@ void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out
     f.partial = ws.partial;
     f.rows = rows;
     f.numClasses = m_forest.numClasses;
-    f.treeSlices = m_model.PartialCount();
+    SetParts(f, p);
     f.initialValue = m_forest.initialValue;
     f.transform = p.s.transform;
     f.out = out;
@@ -494,14 +536,17 @@ void InferenceRunner::RunDeviceNoAlloc(const float *deviceInputs, void *deviceRe
   if (rows == 0) return;
   if (!deviceInputs || !deviceResults) throw Error("null device buffer");
   const bool few = TakesFewRows(rows);
-  const size_t partialBytes = few || FusesArgmax() ? 0 : (PartialBytes(rows) + 255) & ~(size_t)255; // (no partial sums when the walk keeps the arg-max)
   const size_t ranksBytes = few ? 0 : RanksBytes(rows);
+  auto padded = [](size_t bytes) { return (bytes + 255) & ~(size_t)255; };
+  Workspace ws;
+  size_t partialBytes = few ? 0 : padded(PartialBytes(rows, true));
+  ws.split = partialBytes > 0 && partialBytes + ranksBytes <= kNoAllocScratchBytes; // (an even split may need more partial sums)
+  if (!ws.split) partialBytes = few || FusesArgmax() ? 0 : padded(PartialBytes(rows, false)); // (none when the walk keeps the arg-max)
   if (partialBytes + ranksBytes > kNoAllocScratchBytes)
     throw Error("this launch plan needs " + std::to_string(partialBytes + ranksBytes) + " bytes of scratch memory for " +
                 std::to_string(rows) + " rows; the fixed array of the no-allocation entry point holds " +
                 std::to_string(kNoAllocScratchBytes) + ": pass fewer rows per call or use tbmi_run_device_async");
   unsigned char *base = ScratchOfCurrentDevice();
-  Workspace ws;
   ws.partial = reinterpret_cast<double *>(base);
   ws.ranks = base + partialBytes;
   // Every partial sum the finalize kernel reads and every rank the walk reads is written earlier in
@@ -614,6 +659,7 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
       }
       if (!m_copier) m_copier.reset(new ParallelCopier((int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()))));
     }
+    (void)OwnWorkspace((rows - 1) % perPiece + 1, m_stream); // (the last piece is shorter and may be split another way)
     const Workspace ws = OwnWorkspace(perPiece, m_stream); // the pieces run one after the other on the runner's stream
     int p = 0;
     for (int64_t first = 0; first < rows; first += perPiece, ++p) {
@@ -639,8 +685,6 @@ void InferenceRunner::TimeKernels(const float *deviceInputs, void *deviceResults
                                   double *walkMs, double *finalizeMs, double *binMs) {
   runs = std::max(1, runs);
   const Workspace ws = OwnWorkspace(rows, m_stream, true);
-  const bool fused = FusesArgmax();
-  const bool finalize = NeedsFinalize() && !fused;
   float ms = 0.f;
   if (binMs) *binMs = 0.0;
   const float *walkInputs = deviceInputs;
@@ -653,10 +697,8 @@ void InferenceRunner::TimeKernels(const float *deviceInputs, void *deviceResults
     if (binMs) *binMs = ms / runs;
   }
   WalkParams p = MakeWalkParams(walkInputs, rows);
-  p.s.fuseArgmax = fused ? 1 : 0;
-  p.out = finalize || (fused && ClassIdsAsInt8()) ? nullptr : static_cast<float *>(deviceResults);
-  p.classOut = fused && ClassIdsAsInt8() ? static_cast<int8_t *>(deviceResults) : nullptr;
-  p.partial = finalize ? ws.partial : nullptr;
+  const bool finalize = SetOutputs(p, ClassIdsAsInt8() ? nullptr : static_cast<float *>(deviceResults),
+                                   ClassIdsAsInt8() ? static_cast<int8_t *>(deviceResults) : nullptr, nullptr, nullptr, false, ws);
   Check(hipEventRecord(m_evStart, m_stream), "hipEventRecord");
   for (int i = 0; i < runs; ++i) Check(LaunchWalk(p, m_stream), "launch walk kernel");
   Check(hipEventRecord(m_evStop, m_stream), "hipEventRecord");
@@ -669,7 +711,7 @@ void InferenceRunner::TimeKernels(const float *deviceInputs, void *deviceResults
     f.partial = ws.partial;
     f.rows = rows;
     f.numClasses = m_forest.numClasses;
-    f.treeSlices = m_model.PartialCount();
+    SetParts(f, p);
     f.initialValue = m_forest.initialValue;
     f.transform = p.s.transform;
     if (ClassIdsAsInt8()) f.classOut = static_cast<int8_t *>(deviceResults);

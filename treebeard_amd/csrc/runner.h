@@ -118,7 +118,7 @@ private:
   void UploadModel();
   void UploadFewRows();
   void FreeModel();
-  void EnsurePartial(int64_t rows);
+  void EnsurePartial(size_t bytes);
   void EnsureStaging(int64_t rows);
   // Batches of a few rows go through LaunchFewRows, whatever the launch plan, unless the caller pinned a plan or asked
   // for peeled walks.
@@ -128,13 +128,18 @@ private:
   struct Workspace {
     double *partial = nullptr; // [PartialCount()][rows][max(1, classes)] when NeedsFinalize()
     uint8_t *ranks = nullptr;  // rank-quantised rows when the plan uses them
+    bool split = true;         // room for a walk split evenly (SplitBlocks)
   };
   // Allocating callers: grows the runner's own buffers to hold `rows` rows and orders `stream`, on which the
   // caller is about to launch, behind an asynchronous call that may still use them.
   // `planKernels`: the call runs the launch plan's kernels however few rows it has.
   Workspace OwnWorkspace(int64_t rows, hipStream_t stream, bool planKernels = false);
-  size_t PartialBytes(int64_t rows) const;
+  size_t PartialBytes(int64_t rows, bool split) const;
   size_t RanksBytes(int64_t rows) const;
+  // Blocks that share row blocks x tree groups evenly (WalkParams::splitBlocks), 0 where the launch is a block per row
+  // block and tree slice.
+  int32_t SplitBlocks(int64_t rows) const;
+  int64_t RowBlocks(int64_t rows) const { return (rows + m_model.plan.rowsPerBlock - 1) / m_model.plan.rowsPerBlock; }
   // Rank-quantised plans: runs the binning kernel and returns the buffer the walk kernel reads.
   const float *PrepareRows(const float *deviceInputs, int64_t rows, uint8_t *ranks, hipStream_t stream);
   bool NeedsFinalize() const { return m_model.plan.treeSlices > 1 || m_forest.numClasses > 0; }
@@ -143,6 +148,9 @@ private:
     return m_forest.numClasses > 0 && m_model.plan.treeSlices == 1 && m_model.plan.kernel == LaunchPlan::Kernel::kRowParallelLds;
   }
   WalkParams MakeWalkParams(const float *deviceInputs, int64_t rows) const;
+  // Sets the outputs of a walk; true when the finalize kernel has to follow.
+  void SetParts(FinalizeParams &f, const WalkParams &p) const; // which partial sums the walk `p` leaves
+  bool SetOutputs(WalkParams &p, float *out, int8_t *classOut, float *margins, float *probabilities, bool leafIds, const Workspace &ws) const;
   hipError_t LaunchWalk(const WalkParams &p, hipStream_t stream) const;
   // `done` (may be null) is recorded behind the last kernel.
   void Launch(const float *deviceInputs, int64_t rows, float *out, int8_t *classOut, float *margins,

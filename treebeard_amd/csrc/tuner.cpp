@@ -1,6 +1,7 @@
 #include "tuner.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace tbamd {
 
@@ -22,6 +23,15 @@ bool RowTileFits(int32_t numFeatures, int32_t rowsPerBlock, int32_t ldsBytes, bo
   return true;
 }
 
+
+// A block that takes `share` of the forest through its rows, with `together` blocks on its compute unit.
+double BlockMicros(const WalkShape &w, double share, int together) {
+  const double rowBytes = (double)w.rowsPerBlock * w.numFeatures * 4;
+  const double stage = 2.0 + (together > 1 ? rowBytes * together * w.computeUnits / 4e6 : rowBytes / 20e3);
+  const double walk = w.levels * (w.rowsPerBlock / 64.0) * 5.4 / 2400.0;
+  return stage + share * (together * walk + w.groups * (together > 1 ? 0.9 : 1.35));
+}
+constexpr double kFinalizeMicros = 5.0;
 
 int64_t BiggestTreeNodes(const Forest &forest) {
   int64_t biggest = 0;
@@ -84,6 +94,24 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
 int64_t TiledGroupNeed(const Forest &forest, int tileSize) {
   return BiggestTiledTreeBytes(forest, tileSize) + 2 * (int64_t)TileBytes(tileSize) + 16;
 }
+}
+
+double SlicedWalkMicros(const WalkShape &w, int32_t treeSlices) {
+  const int64_t places = (int64_t)w.computeUnits * w.blocksPerUnit, blocks = w.rowBlocks * treeSlices;
+  const double share = std::ceil(std::max(1.0, w.groups) / treeSlices) / std::max(1.0, w.groups); // (whole groups)
+  double us = 0.0;
+  if (const int64_t rounds = blocks / places) // (blocks of later rounds no longer march in step)
+    us += (1.0 + 0.88 * (double)(rounds - 1)) * BlockMicros(w, share, w.blocksPerUnit);
+  if (const int64_t rest = blocks % places) // the last round: spread over the units, alone on them if they suffice
+    us += BlockMicros(w, share, (int)((rest + w.computeUnits - 1) / w.computeUnits));
+  return us + (treeSlices > 1 ? kFinalizeMicros : 0.0);
+}
+
+double SplitWalkMicros(const WalkShape &w) {
+  const double share = (double)w.rowBlocks / ((double)w.computeUnits * w.blocksPerUnit); // of the forest, per block
+  // (a part that straddles row blocks stages the rows of each; whole groups only; 3 % for blocks that march in step)
+  const double rounded = w.groups > 0 ? std::ceil(share * w.groups) / w.groups : share;
+  return BlockMicros(w, rounded * 1.03, w.blocksPerUnit) + std::ceil(share) * BlockMicros(w, 0.0, w.blocksPerUnit) + kFinalizeMicros;
 }
 
 LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoScheduleOptions *ov,
@@ -279,9 +307,23 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   const int64_t totalBytes = (int64_t)forest.NumNodes() * kNodeBytes;
   int64_t groups = std::max<int64_t>(1, (totalBytes + plan.groupBytes - 1) / plan.groupBytes);
   int64_t slices = 1;
-  const int64_t wantBlocks = 2LL * limits.computeUnits;
-  if (rowBlocks < wantBlocks) slices = (wantBlocks + rowBlocks - 1) / rowBlocks;
-  slices = std::min<int64_t>(slices, std::max<int64_t>(1, totalBytes / 16384)); // >= 16 KB of trees per slice
+  if (rowBlocks < 2LL * limits.computeUnits) {
+    WalkShape shape;
+    shape.rowBlocks = rowBlocks;
+    shape.rowsPerBlock = rb;
+    shape.numFeatures = forest.numFeatures;
+    for (const Tree &tree : forest.trees) shape.levels += tree.Depth();
+    shape.computeUnits = limits.computeUnits;
+    shape.blocksPerUnit = budget == halfLds ? 2 : 1;
+    double best = 0.0;
+    // (at least 16 KB of trees per slice)
+    for (int64_t s = 1; s <= std::min<int64_t>(64, std::max<int64_t>(1, totalBytes / 16384)); ++s) {
+      shape.groups = (double)std::max<int64_t>(groups, s);
+      double us = SlicedWalkMicros(shape, (int32_t)s);
+      if (rowBlocks * s > shape.computeUnits * shape.blocksPerUnit) us = std::min(us, SplitWalkMicros(shape)); // (as the launch will choose)
+      if (s == 1 || us < best) best = us, slices = s;
+    }
+  }
   if (slices > groups) { // more, smaller groups so that every slice has one
     int64_t perSlice = std::max<int64_t>((totalBytes + slices - 1) / slices + 4096, need);
     if (perSlice < plan.groupBytes) plan.groupBytes = (int32_t)((perSlice + 15) & ~15);

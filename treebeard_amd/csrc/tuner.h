@@ -25,6 +25,22 @@ struct WalkOptions {
   bool peelWalks = false;
 };
 
+// What a row-parallel walk over `rowBlocks` row blocks takes on the device, in microseconds: enough to choose between
+// launch shapes of one plan, not to predict a time.  Fitted to MI355X timings of 100 to 1000 trees on 10 to 90 features
+// and 2048 to 200000 rows: a lock-step level of 64 rows occupies a compute unit's LDS for 5.4 cycles, shared by the
+// blocks on it; a tree group costs 1.35 us of copy and barriers that a second block hides but for 0.9; partial sums
+// cost a finalize launch of 5 us.
+struct WalkShape {
+  int64_t rowBlocks = 1;
+  int32_t rowsPerBlock = 256, numFeatures = 1;
+  double levels = 0.0;        // lock-step levels of one row over the whole forest
+  double groups = 1.0;        // tree groups of the whole forest
+  int32_t computeUnits = 256;
+  int32_t blocksPerUnit = 2;  // that run at once
+};
+double SlicedWalkMicros(const WalkShape &shape, int32_t treeSlices); // a block per row block and tree slice
+double SplitWalkMicros(const WalkShape &shape);                      // row blocks x groups split evenly over the blocks that run at once
+
 // Analytic choice; `overrides` (may be null) pins what the caller set.  Tile sizes above 1 always get the
 // row-parallel kernel on f32 rows (the only one that walks tiles) and fail when its row tile does not fit.
 LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoScheduleOptions *overrides,
