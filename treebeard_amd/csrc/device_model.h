@@ -146,6 +146,24 @@ struct DeviceFewRowsBlock {
 static_assert(sizeof(DeviceFewRowsBlock) == 48, "three 16-byte loads");
 constexpr uint32_t kFewRowsLeaf = 0xFFFFu;
 
+// Rank-quantised rows of up to 2047 features, trees of up to 255 splits: 4-byte nodes that a wave streams through LDS of
+// its own.  node = test << 24 | child pair << 16 | feature << 5: a row whose rank is below `test` (threshold index + 1)
+// goes to word 2 * pair of the tree, the others to word 2 * pair + 1; word 0 is the root, word 1 unused.  A leaf holds
+// its place: as a left child it tests the pad feature (rank 0) against 1, as a right child anything against 0.  The
+// leaves a walk of the bundle's depth reaches with its last step are never read as nodes: they have no words.
+// Predictions stand in an array of their own, one place per word (the last leaves' included).
+struct alignas(64) DeviceStreamBundle { // (whole words: one scalar load)
+  uint32_t wordBegin;     // multiple of 4; word 0 is the root of a tree of one leaf, which fills empty places
+  uint32_t piecesDepth;   // 16-byte pieces << 16 | depth of the deepest tree
+  uint32_t roots[4];      // byte offsets of trees 2 * k (low half) and 2 * k + 1, which the two halves of a wave walk
+  uint32_t valueBegin[8]; // of every tree, in the array of predictions (entry 0 is 0.0: the empty places')
+  uint32_t reserved[2];
+};
+constexpr int kStreamMaxChains = 4;          // trees a lane walks side by side (2 or 4); two lanes share a bundle's trees
+constexpr uint32_t kStreamBundleBytes = 4096;
+constexpr int32_t kStreamMaxFeatures = 2047;
+constexpr int32_t kStreamRows = 32;          // rows of a block: a rank byte each, 32 per feature
+
 struct DeviceGroup {
   uint32_t nodeBegin;   // first node of the group in the packed node array
   uint32_t nodeCount;   // multiple of 2 so that the group is a whole number of 16-byte pieces

@@ -115,18 +115,41 @@ struct FewRowsParams {
   hipEvent_t done = nullptr;
 };
 
+// Rank-quantised rows (the output of LaunchBinRows) against bundles each wave streams on its own.
+struct RankStreamParams {
+  const uint8_t *ranks = nullptr;
+  const uint32_t *words = nullptr; // PackRankStream
+  const float *values = nullptr;
+  const DeviceStreamBundle *bundles = nullptr;
+  int64_t rows = 0;
+  int32_t numFeatures = 0, numBundles = 0;
+  int32_t chains = kStreamMaxChains;
+  int32_t slices = 1;              // blocks that share a row block's bundles
+  int32_t transform = 0;
+  double initialValue = 0.0;
+  float *out = nullptr;            // one slice
+  double *partial = nullptr;       // [slices][rows] otherwise
+  hipEvent_t done = nullptr;
+};
+
 #if defined(__HIP__)
 inline constexpr bool kLaunchersRecordEvents = true;
 inline constexpr bool kLaunchersSplitEvenly = true;
 // How many rows of such a forest LaunchFewRows takes sooner than the launch plans do (0: never).
 int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth);
 hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream);
+inline constexpr bool kHaveRankStream = true;
+int32_t RankStreamSlices(int64_t rows, int32_t numFeatures, int32_t numBundles, int32_t computeUnits);
+hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream);
 #else
 // (host-only builds of the runner, under the sanitizers, link stand-ins of the launchers below and have no others)
 inline constexpr bool kLaunchersRecordEvents = false;
 inline constexpr bool kLaunchersSplitEvenly = false;
 inline int64_t FewRowsLimit(int32_t, int32_t, int32_t, int32_t) { return 0; }
 inline hipError_t LaunchFewRows(const FewRowsParams &, hipStream_t) { return hipErrorNotSupported; }
+inline constexpr bool kHaveRankStream = false;
+inline int32_t RankStreamSlices(int64_t, int32_t, int32_t, int32_t) { return 1; }
+inline hipError_t LaunchRankStream(const RankStreamParams &, hipStream_t) { return hipErrorNotSupported; }
 #endif
 
 // Row-parallel walk over LDS-staged tree groups: block = s.rowsPerBlock * s.treeThreads lanes.

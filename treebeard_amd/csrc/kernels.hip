@@ -1517,6 +1517,138 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
   if (tid < valid) FinishClasses([&](int c) { return sums[tid * Cn + c]; }, Cn, row0 + tid, p.out, p.classOut, p.margins, p.probabilities);
 }
 
+// ---------------------------------------------------------------------------
+// Wide rows, rank-quantised: a block keeps 32 rows of one byte per feature in LDS (64 KB at 2000 features) and every
+// wave streams its own bundles of four trees through 8 KB of its own, two bundles deep: while one is walked the next is
+// on its way from L2 (direct global -> LDS loads), so no wave waits for a copy or for another wave - the tree groups of
+// the row-parallel kernel, which all waves of a block copy, wait for and walk together with nothing else on the CU to
+// cover it, kept the LDS pipes 36 % busy.  The two halves of a wave walk two trees over the same 32 rows, each lane two
+// chains; 32 rows instead of 64 leave the room (twelve waves x two buffers), and 4-byte nodes halve what a bundle takes:
+// a step is a 4-byte node read and a one-byte rank read.  Leaf values stay in global memory, one gather per tree, issued
+// a bundle ahead of its use.  What bounds it is the latency of the two dependent LDS reads of a step at twelve waves a CU.
+// 262144 rows x 2000 features, 1000 trees of depth 8 (ranks included in neither): 1362 us with tree groups; here 996 with
+// two chains a lane, 914 with four and without words for the last level's leaves, 883 with two levels per loop turn, 800
+// with LDS reads awaited one by one.  20000 rows 94 -> 77 us.
+// ---------------------------------------------------------------------------
+constexpr int kStreamMaxWaves = 16;
+
+int StreamWaves(int32_t numFeatures) {
+  const int64_t tile = ((int64_t)(numFeatures + 1) * kStreamRows + 15) & ~(int64_t)15;
+  return (int)std::min<int64_t>(kStreamMaxWaves, (160 * 1024 - tile) / (2 * kStreamBundleBytes));
+}
+
+template <int K> // chains
+__global__ void __launch_bounds__(kStreamMaxWaves * 64)
+RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__ words, const float *__restrict__ values,
+                 const DeviceStreamBundle *__restrict__ bundles, int64_t rows, int F, int numBundles, int slices, int transform,
+                 double initialValue, float *__restrict__ out, double *__restrict__ partial) {
+  extern __shared__ __align__(16) unsigned char lds[]; // [feature][32 rows] ranks, pad feature included | two bundles per wave
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int waves = blockDim.x >> 6;
+  // The two halves of a 64-row rank tile share its cache lines: their blocks are 8 apart in launch order (same XCD).
+  const uint32_t linear = blockIdx.x;
+  const int64_t block = (int64_t)(linear >> 4) * 16 + (int64_t)((linear & 7u) * 2u + ((linear >> 3) & 1u));
+  if (block * kStreamRows >= rows) return;
+  const uint32_t tileBytes = ((uint32_t)(F + 1) * kStreamRows + 15u) & ~15u;
+  const uint32_t mine = tileBytes + (uint32_t)wave * (2u * kStreamBundleBytes); // this wave's two bundles
+  // 16 bytes per lane to LDS address DST + 16 * lane.  (Not the builtin: while one of those is outstanding the compiler
+  // awaits LDS reads only all together, and here one nearly always is.  The waits for these copies are the explicit ones.)
+#define TBAMD_STREAM_COPY(SRC, DST)                                                                                    \
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(SRC), "s"(DST) : "memory", "m0");
+  {
+    const uint8_t *src = ranks + (block >> 1) * F * 64 + (block & 1) * kStreamRows;
+    const int pieces = F * 2; // piece p: half (p & 1) of the 32 bytes of feature p / 2
+    for (int first = wave * 64; first < pieces; first += waves * 64) {
+      const int p = first + lane;
+      if (p < pieces) TBAMD_STREAM_COPY(src + (int64_t)(p >> 1) * 64 + (p & 1) * 16, (uint32_t)first * 16u)
+    }
+    if (tid < kStreamRows / 4) *reinterpret_cast<uint32_t *>(lds + (uint32_t)F * kStreamRows + tid * 4) = 0; // pad feature
+  }
+  const int first = (int)((int64_t)numBundles * blockIdx.y / slices), last = (int)((int64_t)numBundles * (blockIdx.y + 1) / slices);
+#define TBAMD_STREAM_BUNDLE(BD, BUFFER)                                                                                \
+  {                                                                                                                    \
+    const U32x4 *src = reinterpret_cast<const U32x4 *>(words + (BD).wordBegin);                                        \
+    const int pieces = (int)((BD).piecesDepth >> 16);                                                                  \
+    for (int q = 0; q < pieces; q += 64)                                                                               \
+      if (q + lane < pieces) TBAMD_STREAM_COPY(src + q + lane, (BUFFER) + (uint32_t)q * 16u)                           \
+  }
+  // descriptors are requested two bundles ahead
+  int b = first + wave;
+  DeviceStreamBundle bd{}, nextBd{};
+  if (b < last) {
+    bd = bundles[b];
+    if (b + waves < last) nextBd = bundles[b + waves];
+    TBAMD_STREAM_BUNDLE(bd, mine)
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads(); // the rows are there; from here on the waves run on their own
+
+  const uint32_t row = (uint32_t)lane & 31u;
+  const bool upper = lane >= 32;
+  double acc = 0.0;
+  float leaf[K];
+  uint32_t at[K]; // where the leaf values of the bundle before lie (entry 0: none)
+#pragma unroll
+  for (int k = 0; k < K; ++k) leaf[k] = 0.0f, at[k] = 0u;
+  uint32_t buffer = mine;
+  for (; b < last; b += waves) {
+    const DeviceStreamBundle afterBd = bundles[b + 2 * waves < last ? b + 2 * waves : b];
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this bundle, and the leaf values of the one before the last
+#pragma unroll
+    for (int k = 0; k < K; ++k) acc += (double)leaf[k];
+#pragma unroll
+    for (int k = 0; k < K; ++k) leaf[k] = values[at[k]];
+    const uint32_t other = buffer == mine ? mine + kStreamBundleBytes : mine;
+    if (b + waves < last) TBAMD_STREAM_BUNDLE(nextBd, other)
+    // (the descriptor's scalar load is done here: it would have the same effect on the LDS reads' waits)
+    asm volatile("" ::"s"(afterBd.wordBegin), "s"(afterBd.valueBegin[7]));
+    uint32_t left[K], right[K], addr[K]; // where the two words of a tree's pair 0 lie
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      left[k] = buffer + ((bd.roots[k] >> (upper ? 16 : 0)) & 0xFFFFu);
+      right[k] = left[k] + 4u;
+      addr[k] = left[k];
+    }
+    const int depth = (int)(bd.piecesDepth & 0xFFFFu);
+#pragma unroll 2
+    for (int d = 0; d < depth; ++d) {
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        const uint32_t node = *(const __attribute__((address_space(3))) uint32_t *)(uintptr_t)addr[k];
+        const uint32_t rank = LdsLoadByte((node & 0xFFE0u) | row);
+        addr[k] = (((node >> 16) & 0xFFu) << 3) + (rank < (node >> 24) ? left[k] : right[k]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < K; ++k) at[k] = (upper ? bd.valueBegin[2 * k + 1] : bd.valueBegin[2 * k]) + ((addr[k] - left[k]) >> 2);
+    bd = nextBd;
+    nextBd = afterBd;
+    buffer = other;
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc += (double)leaf[k];
+#pragma unroll
+  for (int k = 0; k < K; ++k) acc += (double)values[at[k]];
+#undef TBAMD_STREAM_BUNDLE
+#undef TBAMD_STREAM_COPY
+  acc += ShuffleXor(acc, 32);
+  __syncthreads(); // nobody reads ranks any more
+  double *meet = reinterpret_cast<double *>(lds); // [wave][row]
+  if (lane < kStreamRows) meet[wave * kStreamRows + lane] = acc;
+  __syncthreads();
+  if (tid >= kStreamRows || block * kStreamRows + tid >= rows) return;
+  double sum = 0.0;
+  for (int w = 0; w < waves; ++w) sum += meet[w * kStreamRows + tid];
+  const int64_t r = block * kStreamRows + tid;
+  if (partial) {
+    partial[(int64_t)blockIdx.y * rows + r] = sum;
+  } else {
+    const double margin = initialValue + sum;
+    out[r] = (float)(transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
+  }
+}
+
 // The ceiling on dynamic LDS is an attribute of each kernel on each device: it is raised once per kernel and
 // device, to the whole 160 KB, instead of on every launch (a runtime call that small batches would pay for each
 // time).  Two threads that meet here for the first time both make the call, which is harmless.
@@ -1844,6 +1976,29 @@ hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream) {
   const int64_t blocks = (p.rows + s.rowsPerBlock - 1) / s.rowsPerBlock;
   return StartKernel(&FewRowsKernel, dim3((unsigned)blocks), dim3((unsigned)s.threads), s.ldsBytes, stream, p.done, p, s.rowsPerBlock,
                      (int)s.leafStride);
+}
+
+// Slices fill the compute units while every wave of a block still has two bundles to overlap.
+int32_t RankStreamSlices(int64_t rows, int32_t numFeatures, int32_t numBundles, int32_t computeUnits) {
+  const int64_t blocks = (rows + kStreamRows - 1) / kStreamRows;
+  const int64_t most = numBundles / (2 * std::max(1, StreamWaves(numFeatures)));
+  return (int32_t)std::max<int64_t>(1, std::min<int64_t>({computeUnits / std::max<int64_t>(1, blocks), most, 64}));
+}
+
+hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
+  if (p.rows <= 0) return hipSuccess;
+  const int waves = StreamWaves(p.numFeatures);
+  if (waves < 1 || p.numFeatures > kStreamMaxFeatures || p.numBundles < 1 || (p.chains != 2 && p.chains != 4) || p.slices < 1 || p.slices > 65535) return hipErrorInvalidValue;
+  if (p.slices > 1 ? !p.partial : !p.out) return hipErrorInvalidValue;
+  const int64_t blocks = ((p.rows + kStreamRows - 1) / kStreamRows + 15) / 16 * 16;
+  const size_t ldsBytes = (((size_t)(p.numFeatures + 1) * kStreamRows + 15) & ~(size_t)15) + (size_t)waves * 2 * kStreamBundleBytes;
+  if (blocks > 0x7FFFFFFF || ldsBytes > 160 * 1024) return hipErrorInvalidValue;
+  const dim3 grid((unsigned)blocks, (unsigned)p.slices), block((unsigned)waves * 64);
+  hipError_t e = p.chains == 4 ? AllowFullLds<&RankStreamKernel<4>>() : AllowFullLds<&RankStreamKernel<2>>();
+  if (e != hipSuccess) return e;
+  return StartKernel(p.chains == 4 ? &RankStreamKernel<4> : &RankStreamKernel<2>, grid, block, ldsBytes, stream, p.done, p.ranks, p.words,
+                     p.values, p.bundles, p.rows, p.numFeatures, p.numBundles, p.slices, p.transform, p.initialValue,
+                     p.slices > 1 ? nullptr : p.out, p.slices > 1 ? p.partial : nullptr);
 }
 
 hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {

@@ -422,6 +422,96 @@ PackedModel PackForGlobalWalk(const Forest &forest, const LaunchPlan &plan) {
 
 } // namespace
 
+RankStreamModel PackRankStream(const Forest &input) {
+  RankStreamModel sm;
+  if (input.numClasses > 0 || input.numFeatures > kStreamMaxFeatures || input.trees.empty()) return sm;
+  const Forest forest = NormalizeToLessThan(input);
+  const std::vector<std::vector<float>> ranks = ThresholdsPerFeature(forest);
+  for (auto &sorted : ranks)
+    if (sorted.size() > 254) return sm;
+  std::vector<int32_t> order(forest.trees.size()), depth(forest.trees.size());
+  for (size_t t = 0; t < forest.trees.size(); ++t) {
+    if (forest.trees[t].NumNodes() > 511) return sm;
+    depth[t] = forest.trees[t].Depth();
+  }
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+    return depth[(size_t)a] != depth[(size_t)b] ? depth[(size_t)a] < depth[(size_t)b]
+                                                : forest.trees[(size_t)a].NumNodes() < forest.trees[(size_t)b].NumNodes();
+  });
+  auto leafWord = [&](uint32_t pair, bool right) { return (right ? 0u : 1u << 24) | pair << 16 | (uint32_t)forest.numFeatures << 5; };
+  // words of a tree's image in a bundle of `deepest` levels: the children of level deepest - 1 have none
+  auto wordsOf = [&](int32_t t, int32_t deepest) {
+    const Tree &tree = forest.trees[(size_t)t];
+    std::vector<int32_t> level{0};
+    uint32_t words = 2;
+    for (int32_t d = 0; d + 1 < deepest && !level.empty(); ++d) {
+      std::vector<int32_t> below;
+      for (int32_t n : level)
+        if (!tree.IsLeaf(n)) below.insert(below.end(), {tree.left[(size_t)n], tree.right[(size_t)n]});
+      words += (uint32_t)below.size();
+      level.swap(below);
+    }
+    return words;
+  };
+  auto pack = [&](int32_t chains) {
+    sm = RankStreamModel();
+    sm.chains = chains;
+    sm.values.push_back(0.0f);
+    for (size_t next = 0; next < order.size();) {
+      // as many trees as fit, each with the words the deepest of them (the last: they come by depth) asks for
+      size_t count = 0;
+      for (size_t n = 1; n <= (size_t)(2 * chains) && next + n <= order.size(); ++n) {
+        uint32_t words = 2 + 3;
+        for (size_t k = 0; k < n; ++k) words += wordsOf(order[next + k], depth[(size_t)order[next + n - 1]]);
+        if (words * 4 > kStreamBundleBytes && n > 1) break; // (a tree alone always fits)
+        count = n;
+      }
+      const int32_t deepest = depth[(size_t)order[next + count - 1]];
+      DeviceStreamBundle b{};
+      b.wordBegin = (uint32_t)sm.words.size();
+      sm.words.insert(sm.words.end(), {leafWord(0, false), 0u}); // the empty tree
+      for (size_t k = 0; k < count; ++k) {
+        const int32_t t = order[next + k];
+        const Tree &tree = forest.trees[(size_t)t];
+        const size_t at = sm.words.size(), valueAt = sm.values.size();
+        const uint32_t limit = wordsOf(t, deepest);
+        b.roots[k / 2] |= (uint32_t)(at - b.wordBegin) * 4 << (16 * (k & 1));
+        b.valueBegin[k] = (uint32_t)valueAt;
+        sm.words.resize(at + limit, 0u);
+        sm.values.resize(valueAt + tree.NumNodes() + 1, 0.0f);
+        struct Place { int32_t node; uint32_t word; };
+        std::vector<Place> queue{{0, 0}};
+        uint32_t pairs = 1;
+        for (size_t head = 0; head < queue.size(); ++head) { // breadth first: the last level's words come last
+          const auto [n, word] = queue[head];
+          if (tree.IsLeaf(n)) {
+            if (word < limit) sm.words[at + word] = leafWord(word / 2, word & 1u);
+            sm.values[valueAt + word] = tree.value[(size_t)n];
+            continue;
+          }
+          const auto &sorted = ranks[(size_t)tree.feature[(size_t)n]];
+          const uint32_t test = (uint32_t)(std::lower_bound(sorted.begin(), sorted.end(), tree.value[(size_t)n]) - sorted.begin()) + 1;
+          if (word >= limit) throw Error("internal error: a split without a word");
+          sm.words[at + word] = test << 24 | pairs << 16 | (uint32_t)tree.feature[(size_t)n] << 5;
+          queue.push_back({tree.left[(size_t)n], 2 * pairs});
+          queue.push_back({tree.right[(size_t)n], 2 * pairs + 1});
+          ++pairs;
+        }
+      }
+      while (sm.words.size() % 4) sm.words.push_back(0u);
+      b.piecesDepth = (uint32_t)((sm.words.size() - b.wordBegin) / 4) << 16 | (uint32_t)deepest;
+      if (sm.words.size() > 0x7FFFFFF0u) throw Error("forest has too many nodes");
+      sm.bundles.push_back(b);
+      next += count;
+    }
+  };
+  // four chains where bundles of eight trees are mostly full: a chain of empty places costs what any other does
+  pack(kStreamMaxChains);
+  if (sm.bundles.size() * 6 > order.size() + 6) pack(2);
+  return sm;
+}
+
 FewRowsModel PackFewRows(const Forest &input) {
   FewRowsModel fm;
   if (input.numFeatures >= (int32_t)kFewRowsLeaf) return fm;

@@ -154,6 +154,16 @@ struct FewRowsModel {
 // Empty when a feature index does not fit the block's 16 bits.
 FewRowsModel PackFewRows(const Forest &forest);
 
+// A forest on rank-quantised rows as bundles for LaunchRankStream; empty where the form cannot hold it (classes, too many
+// features or thresholds, a tree of more than 255 splits).
+struct RankStreamModel {
+  std::vector<uint32_t> words;
+  std::vector<float> values;
+  std::vector<DeviceStreamBundle> bundles; // by depth
+  int32_t chains = kStreamMaxChains;       // trees per bundle: twice as many
+};
+RankStreamModel PackRankStream(const Forest &forest);
+
 // Largest number of distinct split thresholds any one feature has (after comparison normalisation).
 int32_t MaxThresholdsPerFeature(const Forest &forest);
 

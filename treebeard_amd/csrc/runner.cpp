@@ -181,6 +181,13 @@ void InferenceRunner::FreeModel() {
   (void)hipFree(m_dBinTable);
   (void)hipFree(m_dRankFeatures);
   (void)hipFree(m_dRankChunks);
+  (void)hipFree(m_dStreamWords);
+  (void)hipFree(m_dStreamValues);
+  (void)hipFree(m_dStreamBundles);
+  m_dStreamWords = nullptr;
+  m_dStreamValues = nullptr;
+  m_dStreamBundles = nullptr;
+  m_streamBundles = 0;
   (void)hipFree(m_dTailNodes);
   (void)hipFree(m_dTailOrigin);
   m_dTailNodes = nullptr;
@@ -217,6 +224,16 @@ void InferenceRunner::UploadModel() {
   m_dNodeOrigin = Upload(m_model.nodeOrigin, "upload node origins");
   m_dSlotTree = Upload(m_model.slotTree, "upload slot table");
   if (m_model.plan.quantizedRows) m_dBinTable = Upload(m_model.binThresholds, "upload threshold table");
+  if (kHaveRankStream && m_model.plan.quantizedRows) {
+    const RankStreamModel stream = PackRankStream(m_forest);
+    if (!stream.bundles.empty()) {
+      m_dStreamWords = Upload(stream.words, "upload stream words");
+      m_dStreamValues = Upload(stream.values, "upload stream values");
+      m_dStreamBundles = Upload(stream.bundles, "upload stream bundles");
+      m_streamBundles = (int32_t)stream.bundles.size();
+      m_streamChains = stream.chains;
+    }
+  }
   if (m_model.plan.deferTails) {
     m_dTailNodes = Upload(m_model.tailNodes, "upload tail nodes");
     m_dTailOrigin = Upload(m_model.tailOrigin, "upload tail node origins");
@@ -258,6 +275,10 @@ void InferenceRunner::Repack(const LaunchPlan &plan) {
 }
 
 size_t InferenceRunner::PartialBytes(int64_t rows, bool split) const {
+  if (split && StreamsBundles()) {
+    const int32_t slices = StreamSlices(rows);
+    return slices > 1 ? (size_t)slices * (size_t)rows * sizeof(double) : 0;
+  }
   const int32_t splitBlocks = split ? SplitBlocks(rows) : 0;
   if (split ? splitBlocks == 0 : !NeedsFinalize()) return 0;
   size_t slots = split ? (size_t)SplitLine::Slots(splitBlocks, RowBlocks(rows)) : (size_t)m_model.PartialCount();
@@ -446,6 +467,46 @@ void InferenceRunner::SetParts(FinalizeParams &f, const WalkParams &p) const {
   f.treeSlices = (int32_t)SplitLine::Slots(p.splitBlocks, RowBlocks(p.s.rows));
 }
 
+bool InferenceRunner::LaunchWalkFor(const float *walkInputs, int64_t rows, FinalizeParams &f, int32_t *leafIds, hipStream_t stream,
+                                    const Workspace &ws, hipEvent_t done) {
+  f.partial = ws.partial;
+  f.rows = rows;
+  f.numClasses = m_forest.numClasses;
+  f.initialValue = m_forest.initialValue;
+  f.transform = m_forest.transform == Transform::kSigmoid ? 1 : 0;
+  if (StreamsBundles() && !leafIds) {
+    RankStreamParams p;
+    p.ranks = reinterpret_cast<const uint8_t *>(walkInputs);
+    p.words = m_dStreamWords;
+    p.values = m_dStreamValues;
+    p.bundles = m_dStreamBundles;
+    p.rows = rows;
+    p.numFeatures = m_forest.numFeatures;
+    p.numBundles = m_streamBundles;
+    p.chains = m_streamChains;
+    p.slices = ws.split ? StreamSlices(rows) : 1;
+    p.transform = f.transform;
+    p.initialValue = f.initialValue;
+    p.out = f.out;
+    p.partial = ws.partial;
+    f.treeSlices = p.slices;
+    p.done = p.slices > 1 ? nullptr : done;
+    Check(LaunchRankStream(p, stream), "launch rank-stream kernel");
+    return p.slices > 1;
+  }
+  WalkParams p = MakeWalkParams(walkInputs, rows);
+  const bool finalize = SetOutputs(p, f.out, f.classOut, f.margins, f.probabilities, leafIds != nullptr, ws);
+  if (leafIds) {
+    p.leafIds = leafIds;
+    p.nodeOrigin = m_dNodeOrigin;
+    p.slotTree = m_dSlotTree;
+  }
+  p.done = finalize ? nullptr : done;
+  Check(LaunchWalk(p, stream), "launch walk kernel");
+  if (finalize) SetParts(f, p);
+  return finalize;
+}
+
 void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out, int8_t *classOut, float *margins,
                              float *probabilities, int32_t *leafIds, hipStream_t stream, const Workspace &ws, hipEvent_t done) {
   if (rows <= 0) return;
@@ -468,30 +529,14 @@ void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out
     Check(LaunchFewRows(f, stream), "launch few-rows kernel");
     return;
   }
-  WalkParams p = MakeWalkParams(PrepareRows(deviceInputs, rows, ws.ranks, stream), rows);
-  const bool finalize = SetOutputs(p, out, classOut, margins, probabilities, leafIds != nullptr, ws);
-  if (leafIds) {
-    p.leafIds = leafIds;
-    p.nodeOrigin = m_dNodeOrigin;
-    p.slotTree = m_dSlotTree;
-  }
-  p.done = finalize ? nullptr : done;
-  Check(LaunchWalk(p, stream), "launch walk kernel");
-  if (finalize) {
-    FinalizeParams f;
-    f.partial = ws.partial;
-    f.rows = rows;
-    f.numClasses = m_forest.numClasses;
-    SetParts(f, p);
-    f.initialValue = m_forest.initialValue;
-    f.transform = p.s.transform;
-    f.out = out;
-    f.classOut = classOut;
-    f.margins = margins;
-    f.probabilities = probabilities;
-    f.done = done;
+  FinalizeParams f;
+  f.out = out;
+  f.classOut = classOut;
+  f.margins = margins;
+  f.probabilities = probabilities;
+  f.done = done;
+  if (LaunchWalkFor(PrepareRows(deviceInputs, rows, ws.ranks, stream), rows, f, leafIds, stream, ws, done))
     Check(LaunchFinalize(f, stream), "launch finalize kernel");
-  }
   if (done && !kLaunchersRecordEvents) Check(hipEventRecord(done, stream), "hipEventRecord");
 }
 
@@ -541,7 +586,7 @@ void InferenceRunner::RunDeviceNoAlloc(const float *deviceInputs, void *deviceRe
   Workspace ws;
   size_t partialBytes = few ? 0 : padded(PartialBytes(rows, true));
   ws.split = partialBytes > 0 && partialBytes + ranksBytes <= kNoAllocScratchBytes; // (an even split may need more partial sums)
-  if (!ws.split) partialBytes = few || FusesArgmax() ? 0 : padded(PartialBytes(rows, false)); // (none when the walk keeps the arg-max)
+  if (!ws.split) partialBytes = few || FusesArgmax() || StreamsBundles() ? 0 : padded(PartialBytes(rows, false)); // (none when the walk keeps the arg-max)
   if (partialBytes + ranksBytes > kNoAllocScratchBytes)
     throw Error("this launch plan needs " + std::to_string(partialBytes + ranksBytes) + " bytes of scratch memory for " +
                 std::to_string(rows) + " rows; the fixed array of the no-allocation entry point holds " +
@@ -696,26 +741,18 @@ void InferenceRunner::TimeKernels(const float *deviceInputs, void *deviceResults
     Check(hipEventElapsedTime(&ms, m_evStart, m_evStop), "hipEventElapsedTime");
     if (binMs) *binMs = ms / runs;
   }
-  WalkParams p = MakeWalkParams(walkInputs, rows);
-  const bool finalize = SetOutputs(p, ClassIdsAsInt8() ? nullptr : static_cast<float *>(deviceResults),
-                                   ClassIdsAsInt8() ? static_cast<int8_t *>(deviceResults) : nullptr, nullptr, nullptr, false, ws);
+  FinalizeParams f;
+  if (ClassIdsAsInt8()) f.classOut = static_cast<int8_t *>(deviceResults);
+  else f.out = static_cast<float *>(deviceResults);
+  bool finalize = false;
   Check(hipEventRecord(m_evStart, m_stream), "hipEventRecord");
-  for (int i = 0; i < runs; ++i) Check(LaunchWalk(p, m_stream), "launch walk kernel");
+  for (int i = 0; i < runs; ++i) finalize = LaunchWalkFor(walkInputs, rows, f, nullptr, m_stream, ws, nullptr);
   Check(hipEventRecord(m_evStop, m_stream), "hipEventRecord");
   Check(hipStreamSynchronize(m_stream), "walk kernel");
   Check(hipEventElapsedTime(&ms, m_evStart, m_evStop), "hipEventElapsedTime");
   if (walkMs) *walkMs = ms / runs;
   if (finalizeMs) *finalizeMs = 0.0;
   if (finalize) {
-    FinalizeParams f;
-    f.partial = ws.partial;
-    f.rows = rows;
-    f.numClasses = m_forest.numClasses;
-    SetParts(f, p);
-    f.initialValue = m_forest.initialValue;
-    f.transform = p.s.transform;
-    if (ClassIdsAsInt8()) f.classOut = static_cast<int8_t *>(deviceResults);
-    else f.out = static_cast<float *>(deviceResults);
     Check(hipEventRecord(m_evStart, m_stream), "hipEventRecord");
     for (int i = 0; i < runs; ++i) Check(LaunchFinalize(f, m_stream), "launch finalize kernel");
     Check(hipEventRecord(m_evStop, m_stream), "hipEventRecord");

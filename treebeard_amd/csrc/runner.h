@@ -142,6 +142,12 @@ private:
   int64_t RowBlocks(int64_t rows) const { return (rows + m_model.plan.rowsPerBlock - 1) / m_model.plan.rowsPerBlock; }
   // Rank-quantised plans: runs the binning kernel and returns the buffer the walk kernel reads.
   const float *PrepareRows(const float *deviceInputs, int64_t rows, uint8_t *ranks, hipStream_t stream);
+  // Rank-quantised rows go through LaunchRankStream where the forest has the form, unless the caller pinned a plan.
+  bool StreamsBundles() const { return m_streamBundles > 0 && !m_planPinned; }
+  int32_t StreamSlices(int64_t rows) const { return RankStreamSlices(rows, m_forest.numFeatures, m_streamBundles, m_limits.computeUnits); }
+  // The walk behind PrepareRows, with its outputs set; true when the finalize kernel (`f`) has to follow.
+  bool LaunchWalkFor(const float *walkInputs, int64_t rows, FinalizeParams &f, int32_t *leafIds, hipStream_t stream, const Workspace &ws,
+                     hipEvent_t done);
   bool NeedsFinalize() const { return m_model.plan.treeSlices > 1 || m_forest.numClasses > 0; }
   // Classifier, one tree slice, row-parallel LDS kernel: the walk kernel can store the class id itself.
   bool FusesArgmax() const {
@@ -185,6 +191,10 @@ private:
   bool m_planPinned = false;
   int64_t m_fewRowsLimit = 0;
   DeviceFewRowsBlock *m_dFewRows = nullptr;
+  uint32_t *m_dStreamWords = nullptr;     // rank-quantised plans: bundles for LaunchRankStream
+  float *m_dStreamValues = nullptr;
+  DeviceStreamBundle *m_dStreamBundles = nullptr;
+  int32_t m_streamBundles = 0, m_streamChains = 0;
   int32_t *m_dFewRowsClasses = nullptr;
   void *m_smallHost = nullptr;      // pinned host memory the few-rows kernel reads rows from and leaves results in
 
