@@ -158,11 +158,14 @@ void InferenceRunner::Release() noexcept {
   (void)hipFree(m_dRanks);
   (void)hipFree(m_dStageIn);
   (void)hipFree(m_dStageOut);
-  for (void *buf : m_pinned)
-    if (buf) (void)hipHostFree(buf);
-  for (auto &ev : m_pieceReady)
-    if (ev) (void)hipEventDestroy(ev);
-  if (m_copyStream) (void)hipStreamDestroy(m_copyStream);
+  for (HostSlot &slot : m_hostSlots) {
+    if (slot.rows) (void)hipHostFree(slot.rows);
+    if (slot.results) (void)hipHostFree(slot.results);
+    if (slot.copied) (void)hipEventDestroy(slot.copied);
+    if (slot.done) (void)hipEventDestroy(slot.done);
+  }
+  for (hipStream_t stream : m_hostStreams)
+    if (stream) (void)hipStreamDestroy(stream);
   if (m_evStart) (void)hipEventDestroy(m_evStart);
   if (m_evStop) (void)hipEventDestroy(m_evStop);
   if (m_asyncDone) (void)hipEventDestroy(m_asyncDone);
@@ -331,8 +334,7 @@ void InferenceRunner::EnsurePartial(size_t need) {
   m_partialBytes = need;
 }
 
-void InferenceRunner::EnsureRanks(int64_t rows) {
-  const size_t need = RanksBytes(rows);
+void InferenceRunner::EnsureRanks(size_t need) {
   if (need <= m_ranksBytes) return;
   WaitForAsyncCall();
   Check(hipStreamSynchronize(m_stream), "hipStreamSynchronize");
@@ -346,7 +348,7 @@ void InferenceRunner::EnsureRanks(int64_t rows) {
 InferenceRunner::Workspace InferenceRunner::OwnWorkspace(int64_t rows, hipStream_t stream, bool planKernels) {
   if (planKernels || !TakesFewRows(rows)) {
     EnsurePartial(std::max(PartialBytes(rows, false), PartialBytes(rows, true)));
-    EnsureRanks(rows);
+    EnsureRanks(RanksBytes(rows));
   }
   // An asynchronous call on another stream may still use these buffers: `stream` waits for it on the device.
   OrderAfterAsyncCall(stream);
@@ -382,6 +384,27 @@ void InferenceRunner::EnsureStaging(int64_t rows) {
   Check(hipMalloc(reinterpret_cast<void **>(&m_dStageIn), (size_t)rows * m_forest.numFeatures * sizeof(float)), "allocate input staging");
   Check(hipMalloc(&m_dStageOut, (size_t)rows * sizeof(float)), "allocate output staging");
   m_stageRows = rows;
+}
+
+void InferenceRunner::EnsureHostSlots(int64_t count, int64_t rows, bool staged) {
+  const auto grow = [](void *&buffer, size_t &have, size_t bytes) {
+    if (bytes <= have) return;
+    have = 0;
+    if (buffer) (void)hipHostFree(buffer);
+    buffer = nullptr;
+    Check(hipHostMalloc(&buffer, bytes, hipHostMallocDefault), "allocate pinned staging");
+    have = bytes;
+  };
+  for (int64_t i = 0; i < std::min<int64_t>(count, kHostSlots); ++i) {
+    HostSlot &slot = m_hostSlots[i];
+    if (staged) grow(slot.rows, slot.rowBytes, (size_t)rows * m_forest.numFeatures * sizeof(float));
+    grow(slot.results, slot.resultBytes, (size_t)rows * sizeof(float));
+    if (count == 1) return; // (goes through on the runner's own stream)
+    for (hipEvent_t *event : {&slot.copied, &slot.done})
+      if (!*event) Check(hipEventCreateWithFlags(event, hipEventDisableTiming), "hipEventCreate");
+  }
+  for (hipStream_t &stream : m_hostStreams)
+    if (!stream) Check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
 }
 
 void InferenceRunner::SetGroupStaging(int32_t mode) {
@@ -643,6 +666,33 @@ namespace {
 // Host batches up to this many bytes of rows are read by the kernel where they lie in pinned memory.
 constexpr size_t kSmallHostBytes = (size_t)512 << 10;
 
+// How a host batch is cut: pieces of about 4 MB (73 us of the link, which cover the 10 us this thread needs for a piece), at
+// least 1024 rows (fewer take the kernels as long) as long as those fit 16 MB; a quarter and half a piece first, because
+// nothing overlaps their copies, and what is left at the end as two thirds and one third, because nothing overlaps the last
+// piece's kernels.
+constexpr size_t kHostPieceBytes = (size_t)4 << 20, kHostPartBytes = (size_t)1 << 20;
+// Calls of this many bytes write the pinned buffers past the caches: the caches do not hold both the rows and the buffers
+// any more, and a line that is not read before it is written saves a third of the memory traffic.
+constexpr size_t kStreamedHostBytes = (size_t)16 << 20;
+struct HostPieces {
+  int64_t rows, most, count; // `most`: rows of the largest piece
+  HostPieces(int64_t allRows, size_t rowBytes) : rows(allRows) {
+    const int64_t fit = (int64_t)((4 * kHostPieceBytes) / rowBytes);
+    most = std::min(std::max<int64_t>((int64_t)(kHostPieceBytes / rowBytes), 1024), fit);
+    most = std::max<int64_t>(256, most / 256 * 256);
+    if (rows <= most) most = rows, count = 1;
+    else count = 2 + (rows - most / 4 * 3 + most - 1) / most;
+  }
+  int64_t End(int64_t p) const {
+    if (p >= count - 1) return rows;
+    if (p == 0) return most / 4;
+    const int64_t begin = most / 4 * 3 + (p - 2) * most;
+    return p == count - 2 && p > 1 ? begin + std::min(most, ((rows - begin) * 2 / 3 + 63) / 64 * 64) : begin + most;
+  }
+  int64_t Begin(int64_t p) const { return p == 0 ? 0 : End(p - 1); }
+  int64_t Rows(int64_t p) const { return End(p) - Begin(p); }
+};
+
 // True when the runtime knows the address as pinned (or registered) host memory, which DMA reads
 // directly; pageable memory makes the query fail, and that error must not linger.
 bool IsPinnedHost(const void *ptr) {
@@ -674,56 +724,94 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
     return;
   }
   EnsureStaging(rows);
-  // Large batches go through in pieces: the copy of piece i+1 (on its own stream) overlaps the kernels
-  // of piece i.  Rows are independent, so the pieces give the same results as one launch.
-  if (gMeasureGpuKernelTime || totalBytes < ((size_t)16 << 20) || rows < 2 * 4096) {
+  if (gMeasureGpuKernelTime) {
     Check(hipMemcpyAsync(m_dStageIn, hostInputs, totalBytes, hipMemcpyHostToDevice, m_stream), "copy inputs");
     RunDevice(m_dStageIn, m_dStageOut, rows);
-  } else {
-    if (!m_copyStream) {
-      Check(hipStreamCreateWithFlags(&m_copyStream, hipStreamNonBlocking), "hipStreamCreate");
-      for (auto &ev : m_pieceReady) Check(hipEventCreateWithFlags(&ev, hipEventDisableTiming), "hipEventCreate");
-    }
-    // Pinned inputs are read by DMA where they lie, in 8 pieces.  Pageable inputs are first moved into
-    // one of two pinned buffers by a few host threads (one core copies slower than the link carries):
-    // pieces of about 16 MB, the host copy of piece i+1 overlapping the DMA of piece i.
-    const bool staged = !IsPinnedHost(hostInputs);
-    int64_t pieces = staged ? (int64_t)((totalBytes + ((size_t)16 << 20) - 1) >> 24) : 8;
-    pieces = std::max<int64_t>(2, std::min<int64_t>({pieces, (int64_t)kMaxPieces, rows / 4096}));
-    const int64_t perPiece = ((rows + pieces - 1) / pieces + 1023) / 1024 * 1024;
-    if (staged) {
-      const size_t pieceBytes = (size_t)perPiece * rowBytes;
-      if (pieceBytes > m_pinnedBytes) {
-        for (void *&buf : m_pinned) {
-          if (buf) (void)hipHostFree(buf);
-          buf = nullptr;
-        }
-        m_pinnedBytes = 0;
-        for (void *&buf : m_pinned) Check(hipHostMalloc(&buf, pieceBytes, hipHostMallocDefault), "allocate pinned staging");
-        m_pinnedBytes = pieceBytes;
-      }
-      if (!m_copier) m_copier.reset(new ParallelCopier((int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()))));
-    }
-    (void)OwnWorkspace((rows - 1) % perPiece + 1, m_stream); // (the last piece is shorter and may be split another way)
-    const Workspace ws = OwnWorkspace(perPiece, m_stream); // the pieces run one after the other on the runner's stream
-    int p = 0;
-    for (int64_t first = 0; first < rows; first += perPiece, ++p) {
-      const int64_t count = std::min(perPiece, rows - first);
-      float *dIn = m_dStageIn + first * m_forest.numFeatures;
-      const char *src = static_cast<const char *>(hostInputs) + (size_t)first * rowBytes;
-      if (staged) {
-        if (p >= 2) Check(hipEventSynchronize(m_pieceReady[p - 2]), "hipEventSynchronize"); // its buffer is free again
-        m_copier->Copy(m_pinned[p & 1], src, (size_t)count * rowBytes);
-        src = static_cast<const char *>(m_pinned[p & 1]);
-      }
-      Check(hipMemcpyAsync(dIn, src, (size_t)count * rowBytes, hipMemcpyHostToDevice, m_copyStream), "copy inputs");
-      Check(hipEventRecord(m_pieceReady[p], m_copyStream), "hipEventRecord");
-      Check(hipStreamWaitEvent(m_stream, m_pieceReady[p], 0), "hipStreamWaitEvent");
-      LaunchPredictions(dIn, count, static_cast<char *>(m_dStageOut) + first * ReturnTypeBytes(), m_stream, ws);
-    }
-    Check(hipStreamSynchronize(m_stream), "inference kernels");
+    Check(hipMemcpy(hostResults, m_dStageOut, (size_t)rows * ReturnTypeBytes(), hipMemcpyDeviceToHost), "copy results");
+    return;
   }
-  Check(hipMemcpy(hostResults, m_dStageOut, (size_t)rows * ReturnTypeBytes(), hipMemcpyDeviceToHost), "copy results");
+  // Rows go through in pieces: host threads move pageable rows into pinned memory (pinned ones are read where they lie),
+  // DMA takes them to the device, the kernels leave the results in pinned memory and this thread copies them out, all at
+  // the same time on different pieces.  Rows are independent, so the pieces give the same results as one launch.
+  const HostPieces pieces(rows, rowBytes);
+  const bool staged = !IsPinnedHost(hostInputs);
+  EnsureHostSlots(pieces.count, pieces.most, staged);
+  if (staged && !m_copier && totalBytes > kHostPartBytes)
+    m_copier.reset(new ParallelCopier((int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()))));
+  struct EndCall { // (an error leaves while rows are on their way)
+    InferenceRunner *runner;
+    ~EndCall() {
+      if (runner->m_copier) runner->m_copier->Finish();
+      if (failed)
+        for (hipStream_t stream : runner->m_hostStreams)
+          if (stream) (void)hipStreamSynchronize(stream);
+    }
+    bool failed = true;
+  } endCall{this};
+  const auto slotOf = [&](int64_t p) -> HostSlot & { return m_hostSlots[p % kHostSlots]; };
+  const auto source = [&](int64_t p) { return static_cast<const char *>(hostInputs) + (size_t)pieces.Begin(p) * rowBytes; };
+  const auto stageOf = [&](int64_t p) { return m_dStageIn + pieces.Begin(p) * m_forest.numFeatures; };
+  const auto bytesOf = [&](int64_t p) { return (size_t)pieces.Rows(p) * rowBytes; };
+  if (pieces.count == 1) {
+    const Workspace ws = OwnWorkspace(rows, m_stream);
+    // (1 MB of pageable rows at a time, half of that first: the host copy of one part covers the DMA of the part before)
+    const size_t firstPart = staged ? std::min(totalBytes, kHostPartBytes / 2) : totalBytes;
+    const auto partEnd = [&](size_t begin) { return begin == 0 ? firstPart : std::min(totalBytes, begin + kHostPartBytes); };
+    char *const to = staged ? static_cast<char *>(slotOf(0).rows) : nullptr;
+    const char *const from = static_cast<const char *>(hostInputs);
+    if (staged && m_copier)
+      for (size_t begin = 0; begin < totalBytes; begin = partEnd(begin)) m_copier->Append(to + begin, from + begin, partEnd(begin) - begin, false);
+    size_t part = 0;
+    for (size_t begin = 0; begin < totalBytes; begin = partEnd(begin), ++part) {
+      const size_t bytes = partEnd(begin) - begin;
+      if (staged && m_copier) m_copier->Await(part);
+      else if (staged) std::memcpy(to + begin, from + begin, bytes);
+      Check(hipMemcpyAsync(reinterpret_cast<char *>(m_dStageIn) + begin, (staged ? to : from) + begin, bytes, hipMemcpyHostToDevice, m_stream), "copy inputs");
+    }
+    LaunchPredictions(m_dStageIn, rows, slotOf(0).results, m_stream, ws, m_callDone);
+    Check(hipEventSynchronize(m_callDone), "inference kernels");
+    std::memcpy(hostResults, slotOf(0).results, (size_t)rows * ReturnTypeBytes());
+    endCall.failed = false;
+    return;
+  }
+  int64_t appended = 0, drained = 0;
+  const auto append = [&] { // the pool runs ahead of this loop as far as there are free slots
+    for (; staged && appended < pieces.count && appended < drained + kHostSlots; ++appended)
+      m_copier->Append(slotOf(appended).rows, source(appended), bytesOf(appended), totalBytes >= kStreamedHostBytes);
+  };
+  const auto drain = [&] {
+    HostSlot &slot = slotOf(drained);
+    Check(hipEventSynchronize(slot.done), "inference kernels");
+    std::memcpy(static_cast<char *>(hostResults) + pieces.Begin(drained) * ReturnTypeBytes(), slot.results,
+                (size_t)pieces.Rows(drained) * ReturnTypeBytes());
+    ++drained;
+  };
+  append();
+  // Copies go to two streams in turn, because each keeps its engine idle for 9 us (28 MB in pieces of 4 MB: 576 us on one
+  // stream, 520 on two), up to four of them ahead of the kernels, which run one piece after the other: launched on streams
+  // of their own they spoil each other's even split (262144 rows x 1000 trees of depth 8: 830 us for the whole call, 720
+  // here).  This thread waits for a copy and launches behind it; hipStreamWaitEvent would keep it for 18 us a piece.
+  // What bounds the call is the link (515 us for 28 MB), then the first piece's way in and the last one's way out.
+  // From pageable rows, 28 features: 262144 rows 950 -> 720 us; 16384 rows of 150 features 332 -> 275.
+  for (int64_t p : {(int64_t)0, (int64_t)1, pieces.count / 2, pieces.count - 2, pieces.count - 1}) // (every size there is)
+    (void)OwnWorkspace(pieces.Rows(p), m_stream);
+  const Workspace ws = OwnWorkspace(pieces.most, m_stream);
+  int64_t copies = 0;
+  for (int64_t p = 0; p < pieces.count; ++p) {
+    for (; copies < pieces.count && copies < p + kHostSlots / 2; ++copies) {
+      HostSlot &slot = slotOf(copies);
+      append();
+      if (staged) m_copier->Await((size_t)copies);
+      Check(hipMemcpyAsync(stageOf(copies), staged ? slot.rows : source(copies), bytesOf(copies), hipMemcpyHostToDevice, m_hostStreams[copies % kHostStreams]), "copy inputs");
+      Check(hipEventRecord(slot.copied, m_hostStreams[copies % kHostStreams]), "hipEventRecord");
+    }
+    HostSlot &slot = slotOf(p);
+    Check(hipEventSynchronize(slot.copied), "copy inputs");
+    LaunchPredictions(stageOf(p), pieces.Rows(p), slot.results, m_stream, ws, slot.done);
+    if (p - drained >= kHostSlots / 2 - 1) drain();
+  }
+  while (drained < pieces.count) drain();
+  endCall.failed = false;
 }
 
 void InferenceRunner::TimeKernels(const float *deviceInputs, void *deviceResults, int64_t rows, int32_t runs,

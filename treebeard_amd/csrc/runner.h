@@ -120,10 +120,11 @@ private:
   void FreeModel();
   void EnsurePartial(size_t bytes);
   void EnsureStaging(int64_t rows);
+  void EnsureHostSlots(int64_t count, int64_t rows, bool staged);
   // Batches of a few rows go through LaunchFewRows, whatever the launch plan, unless the caller pinned a plan or asked
   // for peeled walks.
   bool TakesFewRows(int64_t rows) const { return rows <= m_fewRowsLimit && !m_planPinned && !m_model.plan.peelWalks; }
-  void EnsureRanks(int64_t rows);
+  void EnsureRanks(size_t bytes);
   // Device memory the kernels of one call use beyond inputs and outputs.
   struct Workspace {
     double *partial = nullptr; // [PartialCount()][rows][max(1, classes)] when NeedsFinalize()
@@ -176,12 +177,15 @@ private:
   PackedModel m_model;
   int m_device = 0; // the device that was current at construction
   hipStream_t m_stream = nullptr;
-  hipStream_t m_copyStream = nullptr; // host-buffer entry point: copies of the next piece overlap the kernels
-  static constexpr int kMaxPieces = 64;
-  hipEvent_t m_pieceReady[kMaxPieces] = {};
-  // pageable inputs pass through two pinned buffers, filled by a few host threads
-  void *m_pinned[2] = {nullptr, nullptr};
-  size_t m_pinnedBytes = 0;
+  // Host-buffer entry points: a piece of the rows on its way through pinned memory, the device and back
+  struct HostSlot {
+    void *rows = nullptr, *results = nullptr; // pinned
+    size_t rowBytes = 0, resultBytes = 0;
+    hipEvent_t copied = nullptr, done = nullptr;
+  };
+  static constexpr int kHostSlots = 8, kHostStreams = 2;
+  HostSlot m_hostSlots[kHostSlots];
+  hipStream_t m_hostStreams[kHostStreams] = {};
   std::unique_ptr<ParallelCopier> m_copier;
   hipEvent_t m_evStart = nullptr, m_evStop = nullptr;
   hipEvent_t m_callDone = nullptr;  // behind the kernels of a call that waits for them
