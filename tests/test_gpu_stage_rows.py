@@ -28,6 +28,8 @@ def test_every_value_of_every_row_arrives(tmp_path, features):
     runner = make_runner(path, 4096)
     dx = torch.from_numpy(np.concatenate([np.zeros(1, np.float32), x.ravel()])).cuda()
     for rows_per_block, tree_threads in ((64, 16), (128, 6), (256, 4)):
+        if rows_per_block * features * 4 > 100 * 1024:                                # (does not fit a block's local memory)
+            continue
         runner.set_plan(rows_per_block, tree_threads, 2)
         for rows in (1, 63, 65, 257, 4129):
             out = torch.zeros(rows, device="cuda")

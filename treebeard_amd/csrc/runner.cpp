@@ -161,7 +161,6 @@ void InferenceRunner::Release() noexcept {
   for (HostSlot &slot : m_hostSlots) {
     if (slot.rows) (void)hipHostFree(slot.rows);
     if (slot.results) (void)hipHostFree(slot.results);
-    if (slot.copied) (void)hipEventDestroy(slot.copied);
     if (slot.done) (void)hipEventDestroy(slot.done);
   }
   for (hipStream_t stream : m_hostStreams)
@@ -400,8 +399,7 @@ void InferenceRunner::EnsureHostSlots(int64_t count, int64_t rows, bool staged) 
     if (staged) grow(slot.rows, slot.rowBytes, (size_t)rows * m_forest.numFeatures * sizeof(float));
     grow(slot.results, slot.resultBytes, (size_t)rows * sizeof(float));
     if (count == 1) return; // (goes through on the runner's own stream)
-    for (hipEvent_t *event : {&slot.copied, &slot.done})
-      if (!*event) Check(hipEventCreateWithFlags(event, hipEventDisableTiming), "hipEventCreate");
+    if (!slot.done) Check(hipEventCreateWithFlags(&slot.done, hipEventDisableTiming), "hipEventCreate");
   }
   for (hipStream_t &stream : m_hostStreams)
     if (!stream) Check(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking), "hipStreamCreate");
@@ -787,26 +785,27 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
     ++drained;
   };
   append();
-  // Copies go to two streams in turn, because each keeps its engine idle for 9 us (28 MB in pieces of 4 MB: 576 us on one
-  // stream, 520 on two), up to four of them ahead of the kernels, which run one piece after the other: launched on streams
-  // of their own they spoil each other's even split (262144 rows x 1000 trees of depth 8: 830 us for the whole call, 720
-  // here).  This thread waits for a copy and launches behind it; hipStreamWaitEvent would keep it for 18 us a piece.
+  // Two copies are under way at a time, on streams of their own, because each keeps its engine idle for 9 us (28 MB in
+  // pieces of 4 MB: 576 us on one stream, 520 on two).  The kernels run one piece after the other: launched on streams of
+  // their own they spoil each other's even split (262144 rows x 1000 trees of depth 8: 830 us for the whole call, 690 here).
+  // This thread waits for a copy and launches behind it: hipStreamWaitEvent would keep it for 18 us a piece, and an event
+  // behind a copy is a packet in a hardware queue, which waits for kernels where another stream of the process has the same
+  // queue (870 us beside two other open runners).
   // What bounds the call is the link (515 us for 28 MB), then the first piece's way in and the last one's way out.
-  // From pageable rows, 28 features: 262144 rows 950 -> 720 us; 16384 rows of 150 features 332 -> 275.
+  // From pageable rows, 28 features: 262144 rows 950 -> 690 us; 16384 rows of 150 features 335 -> 267.
   for (int64_t p : {(int64_t)0, (int64_t)1, pieces.count / 2, pieces.count - 2, pieces.count - 1}) // (every size there is)
     (void)OwnWorkspace(pieces.Rows(p), m_stream);
   const Workspace ws = OwnWorkspace(pieces.most, m_stream);
   int64_t copies = 0;
   for (int64_t p = 0; p < pieces.count; ++p) {
-    for (; copies < pieces.count && copies < p + kHostSlots / 2; ++copies) {
+    for (; copies < pieces.count && copies < p + kHostStreams; ++copies) {
       HostSlot &slot = slotOf(copies);
       append();
       if (staged) m_copier->Await((size_t)copies);
       Check(hipMemcpyAsync(stageOf(copies), staged ? slot.rows : source(copies), bytesOf(copies), hipMemcpyHostToDevice, m_hostStreams[copies % kHostStreams]), "copy inputs");
-      Check(hipEventRecord(slot.copied, m_hostStreams[copies % kHostStreams]), "hipEventRecord");
     }
     HostSlot &slot = slotOf(p);
-    Check(hipEventSynchronize(slot.copied), "copy inputs");
+    Check(hipStreamSynchronize(m_hostStreams[p % kHostStreams]), "copy inputs");
     LaunchPredictions(stageOf(p), pieces.Rows(p), slot.results, m_stream, ws, slot.done);
     if (p - drained >= kHostSlots / 2 - 1) drain();
   }

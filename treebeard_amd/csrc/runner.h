@@ -181,7 +181,7 @@ private:
   struct HostSlot {
     void *rows = nullptr, *results = nullptr; // pinned
     size_t rowBytes = 0, resultBytes = 0;
-    hipEvent_t copied = nullptr, done = nullptr;
+    hipEvent_t done = nullptr;
   };
   static constexpr int kHostSlots = 8, kHostStreams = 2;
   HostSlot m_hostSlots[kHostSlots];
