@@ -113,3 +113,31 @@ def test_calls_on_the_default_and_other_streams_follow_each_other(synth_model):
         runner.run_device_async(dx.data_ptr(), outs[0].data_ptr(), rows, None)
         runner.run_device(dx.data_ptr(), outs[1].data_ptr(), rows)
         np.testing.assert_allclose(outs[1].cpu().numpy(), expected[:rows], rtol=0, atol=ATOL_PROB)
+
+
+@pytest.mark.parametrize("classes,trees,features,depth", [(2, 2, 4, 3), (3, 3, 2, 6)])
+def test_more_rows_per_block_than_lanes(tmp_path, classes, trees, features, depth):
+    """Small classifiers whose limit gives a block more rows than it has lanes: every row's four outputs are written."""
+    rng = np.random.Generator(np.random.PCG64(classes))
+
+    def draw_split():
+        return rng.integers(0, features), rng.standard_normal()
+    path = str(tmp_path / "small.json")
+    synth.write_xgboost_json(path, [synth._grow_tree(rng, depth, lambda d, s: 1.0, draw_split, lambda: rng.normal()) for _ in range(trees)],
+                             features, objective="multi:softmax", num_class=classes, tree_info=[t % classes for t in range(trees)])
+    forest = model_io.load_xgboost_json(path)
+    runner = make_runner(path, 1024)
+    limit = limit_of(runner)
+    x = rng.standard_normal((393216, features), dtype=np.float32)
+    pred, sums = cpu_oracle.predict(forest, x, threads=8)
+    z = np.exp(sums.astype(np.float64) - sums.max(axis=1, keepdims=True))
+    dx = torch.from_numpy(x).cuda()
+    for rows in sorted({262144, 262145, limit, 393216}):
+        ids = torch.full((rows,), -1, dtype=torch.int8, device="cuda")
+        margins, probabilities = (torch.full((rows, classes), -1.0, device="cuda") for _ in range(2))
+        torch.cuda.synchronize()
+        runner.run_device_multiclass(dx.data_ptr(), rows, ids.data_ptr(), margins.data_ptr(), probabilities.data_ptr())
+        np.testing.assert_array_equal(ids.cpu().numpy().astype(np.float32), pred[:rows])
+        np.testing.assert_allclose(margins.cpu().numpy(), sums[:rows], rtol=RTOL_SUM, atol=1e-7)
+        np.testing.assert_allclose(probabilities.cpu().numpy(), (z / z.sum(axis=1, keepdims=True))[:rows], rtol=0, atol=ATOL_PROB)
+        close(forest, gpu_predict(runner, x[:rows]), pred[:rows])

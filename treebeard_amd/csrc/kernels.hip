@@ -1555,7 +1555,8 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
   }
   if (p.numClasses == 0) return;
   __syncthreads();
-  if (tid < valid) FinishClasses([&](int c) { return sums[tid * Cn + c]; }, Cn, row0 + tid, p.out, p.classOut, p.margins, p.probabilities);
+  for (int r = tid; r < valid; r += threads) // (a block of a small forest has more rows than lanes)
+    FinishClasses([&](int c) { return sums[r * Cn + c]; }, Cn, row0 + r, p.out, p.classOut, p.margins, p.probabilities);
 }
 
 // ---------------------------------------------------------------------------
