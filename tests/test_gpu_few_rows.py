@@ -116,8 +116,8 @@ def test_calls_on_the_default_and_other_streams_follow_each_other(synth_model):
 
 
 @pytest.mark.parametrize("classes,trees,features,depth", [(2, 2, 4, 3), (3, 3, 2, 6)])
-def test_more_rows_per_block_than_lanes(tmp_path, classes, trees, features, depth):
-    """Small classifiers whose limit gives a block more rows than it has lanes: every row's four outputs are written."""
+def test_small_classifiers_at_their_limit_and_far_beyond(tmp_path, classes, trees, features, depth):
+    """Few trees: a block has few waves for its rows.  Every row's four outputs are written, on both sides of the limit."""
     rng = np.random.Generator(np.random.PCG64(classes))
 
     def draw_split():
@@ -132,7 +132,7 @@ def test_more_rows_per_block_than_lanes(tmp_path, classes, trees, features, dept
     pred, sums = cpu_oracle.predict(forest, x, threads=8)
     z = np.exp(sums.astype(np.float64) - sums.max(axis=1, keepdims=True))
     dx = torch.from_numpy(x).cuda()
-    for rows in sorted({262144, 262145, limit, 393216}):
+    for rows in sorted({limit, limit + 1, 262144, 262145, 393216}):
         ids = torch.full((rows,), -1, dtype=torch.int8, device="cuda")
         margins, probabilities = (torch.full((rows, classes), -1.0, device="cuda") for _ in range(2))
         torch.cuda.synchronize()

@@ -5,6 +5,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+
 namespace tbamd {
 
 // Scalars of the row-parallel walk (passed by value, live in SGPRs).
@@ -115,6 +117,45 @@ struct FewRowsParams {
   hipEvent_t done = nullptr;
 };
 
+// How LaunchFewRows cuts a batch.
+struct FewRowsShape {
+  int rowsPerBlock, threads;
+  size_t leafStride, ldsBytes; // floats per tree in the leaf array; LDS of a block
+};
+constexpr size_t kFewRowsLds = 64 * 1024;
+inline FewRowsShape ShapeOfFewRows(int64_t rows, int numFeatures, int numTrees, int numClasses) {
+  FewRowsShape s;
+  s.rowsPerBlock = (int)std::max<int64_t>(1, (rows + 255) / 256); // a block per compute unit before blocks take more rows
+  s.threads = (int)std::min<int64_t>(1024, ((int64_t)s.rowsPerBlock * numTrees + 63) / 64 * 64);
+  if (s.threads < 64) s.threads = 64;
+  s.leafStride = (size_t)s.rowsPerBlock | 1; // (odd: the lanes that add a row's leaves read different banks)
+  s.ldsBytes = ((size_t)numTrees * s.leafStride + (size_t)s.rowsPerBlock * numFeatures) * sizeof(float);
+  s.ldsBytes = ((s.ldsBytes + 7) & ~(size_t)7) + (size_t)s.rowsPerBlock * std::max(1, numClasses) * sizeof(double);
+  return s;
+}
+
+// How many rows of such a forest LaunchFewRows takes sooner than the launch plans do (0: never).  Two costs grow with the
+// rows: the walks, about 20 cycles of a compute unit's address path per 16-byte gather of 64 lanes (4.5 us at kFewRowsWork
+// visits), and the sums, 0.4 us per (row, class) that a wave adds.  A forest of many trees ends at the first, one of few
+// trees (few waves a block) or many classes at the second.  Against it stand 7 us for the plans' launch and staging, 1.1 a
+// class and up to 4 for the walk: fitted to 72 forests of 1 to 400 trees and 0 to 12 classes, 250 to 400000 rows each.
+// Without the second term 393216 rows of two trees and two classes took 94 us here and 17 by the plan, 87381 rows of twelve
+// trees and six classes 68 and 14; with it no forest of the fit is more than 1.3 times the faster of the two forms.
+constexpr int64_t kFewRowsWork = (int64_t)3 << 20; // (row, tree, block of three levels) visits
+inline int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth) {
+  if (numTrees < 1) return 0;
+  const int64_t rounds = depth / 3 + 1;
+  const double planMicros = 7.0 + 1.1 * numClasses + std::min(4.0, (double)numTrees * depth / 100.0);
+  int64_t rows = kFewRowsWork / (numTrees * rounds);
+  while (rows > 0 && ShapeOfFewRows(rows, numFeatures, numTrees, numClasses).ldsBytes > kFewRowsLds) rows /= 2;
+  for (; rows > 0; rows = rows * 7 / 8) {
+    const FewRowsShape s = ShapeOfFewRows(rows, numFeatures, numTrees, numClasses);
+    const int64_t waves = s.threads / 64, sums = ((int64_t)s.rowsPerBlock * std::max(1, numClasses) + waves - 1) / waves;
+    if (4.5 + 4.5 * (double)(rows * numTrees * rounds) / (double)kFewRowsWork + 0.4 * (double)sums <= planMicros) break;
+  }
+  return rows;
+}
+
 // Rank-quantised rows (the output of LaunchBinRows) against bundles each wave streams on its own.
 struct RankStreamParams {
   const uint8_t *ranks = nullptr;
@@ -135,8 +176,6 @@ struct RankStreamParams {
 #if defined(__HIP__)
 inline constexpr bool kLaunchersRecordEvents = true;
 inline constexpr bool kLaunchersSplitEvenly = true;
-// How many rows of such a forest LaunchFewRows takes sooner than the launch plans do (0: never).
-int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth);
 hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream);
 inline constexpr bool kHaveRankStream = true;
 int32_t RankStreamSlices(int64_t rows, int32_t numFeatures, int32_t numBundles, int32_t computeUnits);
@@ -145,7 +184,6 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream);
 // (host-only builds of the runner, under the sanitizers, link stand-ins of the launchers below and have no others)
 inline constexpr bool kLaunchersRecordEvents = false;
 inline constexpr bool kLaunchersSplitEvenly = false;
-inline int64_t FewRowsLimit(int32_t, int32_t, int32_t, int32_t) { return 0; }
 inline hipError_t LaunchFewRows(const FewRowsParams &, hipStream_t) { return hipErrorNotSupported; }
 inline constexpr bool kHaveRankStream = false;
 inline int32_t RankStreamSlices(int64_t, int32_t, int32_t, int32_t) { return 1; }

@@ -1468,24 +1468,6 @@ __global__ void __launch_bounds__(256) FinalizeWideKernel(const FinalizeParams p
 // and a wave per (row, class) adds them in a fixed order.  One row through 1000 trees of depth 8 took 15.2 us a call
 // with the tree-parallel kernel and its finalize launch.
 // ---------------------------------------------------------------------------
-constexpr int64_t kFewRowsWork = (int64_t)3 << 20; // (row, tree, block of three levels) visits, see FewRowsLimit
-
-struct FewRowsShape {
-  int rowsPerBlock, threads;
-  size_t leafStride, ldsBytes; // floats per tree in the leaf array; LDS of a block
-};
-
-FewRowsShape ShapeOfFewRows(int64_t rows, int numFeatures, int numTrees, int numClasses) {
-  FewRowsShape s;
-  s.rowsPerBlock = (int)std::max<int64_t>(1, (rows + 255) / 256); // a block per compute unit before blocks take more rows
-  s.threads = (int)std::min<int64_t>(1024, ((int64_t)s.rowsPerBlock * numTrees + 63) / 64 * 64);
-  if (s.threads < 64) s.threads = 64;
-  s.leafStride = (size_t)s.rowsPerBlock | 1; // (odd: the lanes that add a row's leaves read different banks)
-  s.ldsBytes = ((size_t)numTrees * s.leafStride + (size_t)s.rowsPerBlock * numFeatures) * sizeof(float);
-  s.ldsBytes = ((s.ldsBytes + 7) & ~(size_t)7) + (size_t)s.rowsPerBlock * std::max(1, numClasses) * sizeof(double);
-  return s;
-}
-
 __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int rowsPerBlock, int leafStride) {
   extern __shared__ __align__(16) unsigned char lds[];
   const int tid = threadIdx.x, threads = blockDim.x;
@@ -1555,7 +1537,7 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
   }
   if (p.numClasses == 0) return;
   __syncthreads();
-  for (int r = tid; r < valid; r += threads) // (a block of a small forest has more rows than lanes)
+  for (int r = tid; r < valid; r += threads)
     FinishClasses([&](int c) { return sums[r * Cn + c]; }, Cn, row0 + r, p.out, p.classOut, p.margins, p.probabilities);
 }
 
@@ -2000,20 +1982,10 @@ hipError_t LaunchRankRows16(const float *x, const float *tables, const RankFeatu
   return hipGetLastError();
 }
 
-// Items a compute unit walks cost about 20 cycles of its address path per 16-byte gather of 64 lanes; up to about
-// 4 us of that the form stays ahead of the launch plans, whose batches of this size take 12 to 15 us.
-int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth) {
-  if (numTrees < 1) return 0;
-  const int64_t rounds = depth / 3 + 1;
-  int64_t rows = kFewRowsWork / ((int64_t)numTrees * rounds);
-  while (rows > 0 && ShapeOfFewRows(rows, numFeatures, numTrees, numClasses).ldsBytes > 64 * 1024) rows /= 2;
-  return rows;
-}
-
 hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
   const FewRowsShape s = ShapeOfFewRows(p.rows, p.numFeatures, p.numTrees, p.numClasses);
-  if (p.numTrees < 1 || s.ldsBytes > 64 * 1024) return hipErrorInvalidValue;
+  if (p.numTrees < 1 || s.ldsBytes > kFewRowsLds) return hipErrorInvalidValue;
   if (p.numClasses == 0 ? !p.out : !(p.out || p.classOut || p.margins || p.probabilities)) return hipErrorInvalidValue;
   const int64_t blocks = (p.rows + s.rowsPerBlock - 1) / s.rowsPerBlock;
   return StartKernel(&FewRowsKernel, dim3((unsigned)blocks), dim3((unsigned)s.threads), s.ldsBytes, stream, p.done, p, s.rowsPerBlock,
