@@ -6,9 +6,11 @@
 // model on the CPU with the kernels' addressing rules (group-relative node addresses, pre-multiplied
 // feature offsets, rank tiles, per-class partial sums, tree slices, finalize), reading every input and
 // writing every output element the kernels touch: a buffer sized or indexed wrongly by the host code is
-// reported by the sanitizer, and a wrongly packed model gives wrong predictions.  Test infrastructure only.
+// reported by the sanitizer, and a wrongly packed model gives wrong predictions.  A wait for an event that nothing has
+// recorded since the last wait ends the run.  Test infrastructure only.
 #include "kernels.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -91,9 +93,12 @@ hipError_t hipStreamDestroy(hipStream_t stream) {
   return hipSuccess;
 }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t, unsigned int) { return hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t event, unsigned int) {
+  if (*reinterpret_cast<int *>(event) == 0) std::abort(); // orders nothing
+  return hipSuccess;
+}
 hipError_t hipEventCreate(hipEvent_t *event) {
-  *event = reinterpret_cast<hipEvent_t>(new int(0));
+  *event = reinterpret_cast<hipEvent_t>(new int(0)); // (1: recorded, and not waited for since)
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *event, unsigned) { return hipEventCreate(event); }
@@ -101,8 +106,15 @@ hipError_t hipEventDestroy(hipEvent_t event) {
   delete reinterpret_cast<int *>(event);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t event, hipStream_t) {
+  *reinterpret_cast<int *>(event) = 1;
+  return hipSuccess;
+}
+hipError_t hipEventSynchronize(hipEvent_t event) {
+  if (*reinterpret_cast<int *>(event) == 0) std::abort(); // waits for nothing
+  *reinterpret_cast<int *>(event) = 0;
+  return hipSuccess;
+}
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
   static float fake = 1.0f; // every measurement a little longer than the last: plan searches keep the first
   fake += 0.001f;
@@ -119,7 +131,8 @@ hipError_t hipGetDevice(int *device) {
 }
 hipError_t hipGetDevicePropertiesR0600(hipDeviceProp_tR0600 *prop, int) {
   std::memset(prop, 0, sizeof(*prop));
-  prop->multiProcessorCount = 256;
+  const char *units = std::getenv("SHIM_COMPUTE_UNITS"); // (few of them: small batches already run in several rounds of blocks)
+  prop->multiProcessorCount = units ? std::atoi(units) : 256;
   prop->sharedMemPerBlock = 160 * 1024;
   return hipSuccess;
 }
@@ -134,6 +147,8 @@ hipError_t hipGetLastError(void) {
   return e;
 }
 
+long shimFewRows = 0, shimSplits = 0, shimStreams = 0; // launches of the forms that stand beside the launch plans' kernels
+
 } // extern "C"
 
 namespace tbamd {
@@ -146,16 +161,17 @@ uint32_t Bits(float v) {
   return u;
 }
 
-// One row through the slice's groups of an LDS-layout model.  `stride` is the node-offset distance between
+// What every launcher does with its parameters' event.
+hipError_t Launched(hipEvent_t done, hipStream_t stream) { return done ? hipEventRecord(done, stream) : hipSuccess; }
+
+// One row through groups [gBegin, gEnd) of an LDS-layout model.  `stride` is the node-offset distance between
 // two features; rankRows: x points at the rank tile [row block][feature][64 rows].
 // rankRows: 0 f32 rows, 1 one-byte ranks, 2 two-byte ranks ([row block][feature pair][row][2], `stride` = bytes of
 // one feature pair's column = rows per block x 4)
-void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64_t row, int slice, double *classSums,
+void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64_t row, int gBegin, int gEnd, double *classSums,
                 bool *classSeen) {
   const DeviceNode *nodes = reinterpret_cast<const DeviceNode *>(p.nodes16);
   const int F = p.s.numFeatures;
-  const int gBegin = (int)(((int64_t)p.s.numGroups * slice) / p.s.treeSlices);
-  const int gEnd = (int)(((int64_t)p.s.numGroups * (slice + 1)) / p.s.treeSlices);
   for (int g = gBegin; g < gEnd; ++g) {
     const DeviceGroup grp = p.groups[g];
     for (uint32_t b = 0; b < grp.bundleCount; ++b) {
@@ -255,24 +271,51 @@ void StoreRow(const WalkParams &p, int64_t row, int slice, const double *classSu
   }
 }
 
-hipError_t WalkLds(const WalkParams &p, int K, uint32_t stride, int rankRows) {
+// The walk's slots of the partial sums hold nothing yet: all of them can be written, and a part the walk leaves out shows.
+void ClearPartial(const WalkParams &p, int64_t slots) {
+  if (p.partial) std::fill_n(p.partial, slots * p.s.rows * std::max(1, p.s.numClasses), std::nan(""));
+}
+
+hipError_t WalkLds(const WalkParams &p, int K, uint32_t stride, int rankRows, hipStream_t stream) {
   if (K != 1 && K != 2 && K != 4 && K != 8) return hipErrorInvalidValue;
   if (p.s.treeSlices > 1 && !p.partial) std::abort(); // slices meet in the partial-sum buffer
   const int Cn = p.s.numClasses > 0 ? p.s.numClasses : 1;
   std::vector<double> sums((size_t)Cn);
   std::vector<char> seen((size_t)Cn);
-  for (int slice = 0; slice < p.s.treeSlices; ++slice)
-    for (int64_t row = 0; row < p.s.rows; ++row) {
+  const auto walk = [&](int64_t firstRow, int64_t lastRow, int gBegin, int gEnd, int slot) {
+    for (int64_t row = firstRow; row < lastRow; ++row) {
       std::fill(sums.begin(), sums.end(), 0.0);
-      WalkRowLds(p, K, stride, rankRows, row, slice, sums.data(), reinterpret_cast<bool *>(seen.data()));
-      StoreRow(p, row, slice, sums.data());
+      WalkRowLds(p, K, stride, rankRows, row, gBegin, gEnd, sums.data(), reinterpret_cast<bool *>(seen.data()));
+      StoreRow(p, row, slot, sums.data());
     }
-  return hipSuccess;
+  };
+  if (p.splitBlocks) { // parts of the line of row blocks x groups, each in a slot of its row block
+    const int64_t rowBlocks = (p.s.rows + p.s.rowsPerBlock - 1) / p.s.rowsPerBlock;
+    if (p.splitBlocks < 1 || p.splitBlocks > rowBlocks * p.s.numGroups || !p.partial || p.leafIds || p.s.deferTails || p.s.fuseArgmax)
+      return hipErrorInvalidValue;
+    ++shimSplits;
+    const SplitLine line{rowBlocks * p.s.numGroups, p.s.numGroups, p.splitBlocks};
+    const int64_t slots = SplitLine::Slots(p.splitBlocks, rowBlocks);
+    ClearPartial(p, slots);
+    for (int64_t block = 0; block < p.splitBlocks; ++block)
+      for (int64_t unit = line.FirstUnit(block), end = line.FirstUnit(block + 1); unit < end;) {
+        const int64_t rowBlock = unit / line.groups, first = rowBlock * p.s.rowsPerBlock, slot = block - line.FirstBlock(rowBlock);
+        const int gBegin = (int)(unit - rowBlock * line.groups), gEnd = (int)std::min<int64_t>(end - rowBlock * line.groups, line.groups);
+        if (slot < 0 || slot >= slots || slot >= line.Parts(rowBlock)) std::abort();
+        walk(first, std::min(p.s.rows, first + p.s.rowsPerBlock), gBegin, gEnd, (int)slot);
+        unit += gEnd - gBegin;
+      }
+    return Launched(p.done, stream);
+  }
+  ClearPartial(p, p.s.treeSlices);
+  for (int slice = 0; slice < p.s.treeSlices; ++slice)
+    walk(0, p.s.rows, (int)(((int64_t)p.s.numGroups * slice) / p.s.treeSlices), (int)(((int64_t)p.s.numGroups * (slice + 1)) / p.s.treeSlices), slice);
+  return Launched(p.done, stream);
 }
 
 } // namespace
 
-hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, size_t ldsBytes, hipStream_t) {
+hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, size_t ldsBytes, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
   const int RB = p.s.rowsPerBlock, TT = p.s.treeThreads;
   if (ldsBytes > 160 * 1024 || RB < 64 || (RB & (RB - 1)) || TT < 1 || RB * TT > 1024) return hipErrorInvalidValue;
@@ -280,10 +323,10 @@ hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, 
   const int prefetch = (int)((p.s.groupRegionBytes / 16 + RB * TT - 1) / (RB * TT));
   if (prefetch > 16) return hipErrorInvalidValue;
   if (tileMode == 2 && RB != 64) return hipErrorInvalidValue;
-  if (tileMode < 0 || tileMode > 3) return hipErrorInvalidValue;
+  if (tileMode < 0 || tileMode > 3 || (tileMode == 3 && p.splitBlocks)) return hipErrorInvalidValue;
   if (tileMode == 3 && (int64_t)((p.s.numFeatures + 2) / 2) * RB * 4 > 0x10000) return hipErrorInvalidValue;
   const uint32_t stride = tileMode == 0 || tileMode == 3 ? (uint32_t)RB * 4u : tileMode == 1 ? (uint32_t)RB : (uint32_t)RB / 4u;
-  return WalkLds(p, interleave, stride, tileMode == 3 ? 2 : tileMode == 2 ? 1 : 0);
+  return WalkLds(p, interleave, stride, tileMode == 3 ? 2 : tileMode == 2 ? 1 : 0, stream);
 }
 
 namespace {
@@ -344,7 +387,7 @@ uint32_t TileStepHost(const unsigned char *group, uint32_t groupBytes, uint32_t 
 
 } // namespace
 
-hipError_t LaunchWalkRowsTiled(const WalkParams &p, int tileSize, int interleave, size_t ldsBytes, hipStream_t) {
+hipError_t LaunchWalkRowsTiled(const WalkParams &p, int tileSize, int interleave, size_t ldsBytes, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
   const int RB = p.s.rowsPerBlock, TT = p.s.treeThreads, T = tileSize, K = interleave;
   if (ldsBytes > 160 * 1024 || RB < 64 || (RB & (RB - 1)) || TT < 1 || RB * TT > 1024) return hipErrorInvalidValue;
@@ -352,6 +395,7 @@ hipError_t LaunchWalkRowsTiled(const WalkParams &p, int tileSize, int interleave
   if (p.s.treeSlices < 1 || p.s.treeSlices > 65535) return hipErrorInvalidValue;
   if (T < 2 || T > kMaxTileSize || (K != 1 && K != 2 && K != 4)) return hipErrorInvalidValue;
   if (p.s.treeSlices > 1 && !p.partial) std::abort();
+  ClearPartial(p, p.s.treeSlices);
   const DeviceNode *nodes = reinterpret_cast<const DeviceNode *>(p.nodes16);
   const int F = p.s.numFeatures;
   const int Cn = p.s.numClasses > 0 ? p.s.numClasses : 1;
@@ -388,20 +432,20 @@ hipError_t LaunchWalkRowsTiled(const WalkParams &p, int tileSize, int interleave
       StoreRow(p, row, slice, sums.data());
     }
   }
-  return hipSuccess;
+  return Launched(p.done, stream);
 }
 
-hipError_t LaunchWalkTreeParallel(const WalkParams &p, int interleave, size_t ldsBytes, hipStream_t) {
+hipError_t LaunchWalkTreeParallel(const WalkParams &p, int interleave, size_t ldsBytes, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
   if (ldsBytes > 160 * 1024 || p.s.rowsPerBlock < 1 || p.s.treeLanes < 1) return hipErrorInvalidValue;
   const int threads = p.s.rowsPerBlock * p.s.treeLanes;
   if (threads > 1024 || threads % 64 != 0) return hipErrorInvalidValue;
   if (p.s.treeSlices < 1 || p.s.treeSlices > 65535) return hipErrorInvalidValue;
   if ((int)((p.s.groupRegionBytes / 16 + threads - 1) / threads) > 16) return hipErrorInvalidValue;
-  return WalkLds(p, interleave, 4u, 0);
+  return WalkLds(p, interleave, 4u, 0, stream);
 }
 
-hipError_t LaunchWalkGlobal(const WalkParams &p, int interleave, hipStream_t) {
+hipError_t LaunchWalkGlobal(const WalkParams &p, int interleave, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
   const int threads = p.s.rowsPerBlock;
   if (threads < 64 || threads > 1024 || threads % 64 != 0) return hipErrorInvalidValue;
@@ -426,7 +470,7 @@ hipError_t LaunchWalkGlobal(const WalkParams &p, int interleave, hipStream_t) {
       StoreRow(p, row, slice, sums.data());
     }
   }
-  return hipSuccess;
+  return Launched(p.done, stream);
 }
 
 hipError_t LaunchBinRows(const float *x, const float *table, uint8_t *ranks, int64_t rows, int numFeatures, int tableDepth,
@@ -488,41 +532,138 @@ hipError_t LaunchRankRows16(const float *x, const float *tables, const RankFeatu
   return hipSuccess;
 }
 
-hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t) {
+namespace {
+// A row's class sums -> the outputs asked for (ties go to the larger class id).
+void FinishRow(const double *sums, int C, int64_t row, float *out, int8_t *classOut, float *margins, float *probabilities) {
+  float best = -INFINITY;
+  int bestClass = 0;
+  double maxMargin = -INFINITY;
+  for (int c = 0; c < C; ++c) {
+    const float m = (float)sums[c];
+    if (margins) margins[row * C + c] = m;
+    if (!(best > m)) best = m, bestClass = c;
+    maxMargin = std::max(maxMargin, sums[c]);
+  }
+  if (classOut) classOut[row] = (int8_t)bestClass;
+  if (out) out[row] = (float)bestClass;
+  if (probabilities) {
+    double z = 0.0;
+    for (int c = 0; c < C; ++c) z += std::exp(sums[c] - maxMargin);
+    for (int c = 0; c < C; ++c) probabilities[row * C + c] = (float)(std::exp(sums[c] - maxMargin) / z);
+  }
+}
+
+float FinishMargin(double margin, int transform) { return (float)(transform == 1 ? 1.0 / (1.0 + std::exp(-margin)) : margin); }
+} // namespace
+
+hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
-  const int C = p.numClasses;
+  const int C = p.numClasses, Cn = std::max(1, C);
+  std::vector<double> sums((size_t)Cn);
   for (int64_t row = 0; row < p.rows; ++row) {
-    if (C == 0) {
-      double margin = p.initialValue;
-      for (int s = 0; s < p.treeSlices; ++s) margin += p.partial[(int64_t)s * p.rows + row];
-      p.out[row] = (float)(p.transform == 1 ? 1.0 / (1.0 + std::exp(-margin)) : margin);
-      continue;
+    int parts = p.treeSlices;
+    if (p.splitBlocks)
+      parts = SplitLine{((p.rows + p.rowsPerBlock - 1) / p.rowsPerBlock) * p.groups, p.groups, p.splitBlocks}.Parts(row / p.rowsPerBlock);
+    if (parts < 1 || parts > p.treeSlices) std::abort();
+    for (int c = 0; c < Cn; ++c) {
+      sums[(size_t)c] = p.initialValue;
+      for (int s = 0; s < parts; ++s) sums[(size_t)c] += p.partial[((int64_t)s * p.rows + row) * Cn + c];
+      // (the wide form leaves class sums in a spare slot behind the last one)
+      if (C > 0 && p.treeSlices >= kWideFinalizeSlices) p.partial[((int64_t)p.treeSlices * p.rows + row) * Cn + c] = sums[(size_t)c];
     }
-    float best = -INFINITY;
-    int bestClass = 0;
-    double maxMargin = -INFINITY;
-    std::vector<double> margins((size_t)C);
-    for (int c = 0; c < C; ++c) {
-      double margin = p.initialValue;
-      for (int s = 0; s < p.treeSlices; ++s) margin += p.partial[((int64_t)s * p.rows + row) * C + c];
-      margins[c] = margin;
-      const float m = (float)margin;
-      if (p.margins) p.margins[row * C + c] = m;
-      if (!(best > m)) {
-        best = m;
-        bestClass = c;
+    if (C == 0) p.out[row] = FinishMargin(sums[0], p.transform);
+    else FinishRow(sums.data(), C, row, p.out, p.classOut, p.margins, p.probabilities);
+  }
+  return Launched(p.done, stream);
+}
+
+// The kernel's blocks, lanes and LDS: a row no lane gets to, a leaf outside the block's array, a walk that runs out of the
+// blocks (heap memory here) all show.
+hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream) {
+  if (p.rows <= 0) return hipSuccess;
+  const FewRowsShape s = ShapeOfFewRows(p.rows, p.numFeatures, p.numTrees, p.numClasses);
+  if (p.numTrees < 1 || s.ldsBytes > kFewRowsLds) return hipErrorInvalidValue;
+  if (p.numClasses == 0 ? !p.out : !(p.out || p.classOut || p.margins || p.probabilities)) return hipErrorInvalidValue;
+  ++shimFewRows;
+  const int T = p.numTrees, F = p.numFeatures, R = s.rowsPerBlock, Cn = std::max(1, p.numClasses);
+  if (((T * s.leafStride + (size_t)R * F) * 4 + 7) / 8 * 8 + (size_t)R * Cn * 8 > s.ldsBytes) std::abort();
+  for (int64_t row0 = 0; row0 < p.rows; row0 += R) {
+    const int valid = (int)std::min<int64_t>(R, p.rows - row0);
+    std::vector<float> leaves((size_t)T * s.leafStride, std::nanf("")), rowTile(p.x + row0 * F, p.x + (row0 + valid) * F);
+    std::vector<double> sums((size_t)R * Cn);
+    for (int tid = 0; tid < s.threads; ++tid)
+      for (int i = tid; i < valid * T; i += s.threads) {
+        const int t = i / valid, r = i - t * valid;
+        size_t block = (size_t)t;
+        uint32_t slot = 0;
+        for (;;) {
+          const DeviceFewRowsBlock &b = p.blocks[block];
+          if (b.feature[slot] == kFewRowsLeaf) {
+            leaves[(size_t)t * s.leafStride + r] = b.value[slot];
+            break;
+          }
+          if (b.feature[slot] >= F) std::abort();
+          const uint32_t right = rowTile[(size_t)r * F + b.feature[slot]] < b.value[slot] ? 0u : 1u;
+          if (slot < 3) {
+            slot = 2 * slot + 1 + right;
+            continue;
+          }
+          const uint32_t exit = 2 * (slot - 3) + right;
+          if (!(b.exits >> exit & 1u)) std::abort();
+          block = b.firstChild + (uint32_t)__builtin_popcount(b.exits & ((1u << exit) - 1u));
+          slot = 0;
+        }
       }
-      maxMargin = std::max(maxMargin, margin);
-    }
-    if (p.classOut) p.classOut[row] = (int8_t)bestClass;
-    if (p.out) p.out[row] = (float)bestClass;
-    if (p.probabilities) {
-      double z = 0.0;
-      for (int c = 0; c < C; ++c) z += std::exp(margins[c] - maxMargin);
-      for (int c = 0; c < C; ++c) p.probabilities[row * C + c] = (float)(std::exp(margins[c] - maxMargin) / z);
+    for (int wave = 0; wave < s.threads / 64; ++wave)
+      for (int pair = wave; pair < valid * Cn; pair += s.threads / 64) {
+        const int r = pair / Cn, c = pair - r * Cn;
+        double margin = p.initialValue;
+        for (int t = p.numClasses > 0 ? p.classBegin[c] : 0, end = p.numClasses > 0 ? p.classBegin[c + 1] : T; t < end; ++t)
+          margin += (double)leaves[(size_t)t * s.leafStride + r];
+        if (p.numClasses == 0) p.out[row0 + r] = FinishMargin(margin, p.transform);
+        else sums[(size_t)pair] = margin;
+      }
+    for (int tid = 0; p.numClasses > 0 && tid < s.threads; ++tid)
+      for (int r = tid; r < valid; r += s.threads)
+        FinishRow(sums.data() + (size_t)r * Cn, Cn, row0 + r, p.out, p.classOut, p.margins, p.probabilities);
+  }
+  return Launched(p.done, stream);
+}
+
+hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
+  if (p.rows <= 0) return hipSuccess;
+  const int waves = StreamWaves(p.numFeatures), F = p.numFeatures;
+  if (waves < 1 || F > kStreamMaxFeatures || p.numBundles < 1 || (p.chains != 2 && p.chains != 4) || p.slices < 1 || p.slices > 65535)
+    return hipErrorInvalidValue;
+  if (p.slices > 1 ? !p.partial : !p.out) return hipErrorInvalidValue;
+  if ((((size_t)(F + 1) * kStreamRows + 15) & ~(size_t)15) + (size_t)waves * 2 * kStreamBundleBytes > 160 * 1024) return hipErrorInvalidValue;
+  ++shimStreams;
+  for (int slice = 0; slice < p.slices; ++slice) {
+    const int first = (int)((int64_t)p.numBundles * slice / p.slices), last = (int)((int64_t)p.numBundles * (slice + 1) / p.slices);
+    for (int64_t row = 0; row < p.rows; ++row) {
+      double sum = 0.0;
+      for (int b = first; b < last; ++b) {
+        const DeviceStreamBundle &bd = p.bundles[b];
+        const uint32_t words = (bd.piecesDepth >> 16) * 4, depth = bd.piecesDepth & 0xFFFFu;
+        if (words * 4 > kStreamBundleBytes || bd.wordBegin % 4) std::abort();
+        for (int k = 0; k < 2 * p.chains; ++k) {
+          const uint32_t root = (bd.roots[k / 2] >> (16 * (k & 1)) & 0xFFFFu) / 4;
+          uint32_t at = 0;
+          for (uint32_t d = 0; d < depth; ++d) {
+            if (root + at >= words) std::abort(); // a node outside the bundle
+            const uint32_t node = p.words[bd.wordBegin + root + at], f = node >> 5 & 0x7FFu;
+            if ((int)f > F || (node & 31u)) std::abort();
+            const uint32_t rank = (int)f == F ? 0u : p.ranks[((row / 64) * F + f) * 64 + row % 64];
+            at = 2 * (node >> 16 & 0xFFu) + (rank < node >> 24 ? 0u : 1u);
+          }
+          sum += (double)p.values[bd.valueBegin[k] + at];
+        }
+      }
+      if (p.slices > 1) p.partial[(int64_t)slice * p.rows + row] = sum;
+      else p.out[row] = FinishMargin(p.initialValue + sum, p.transform);
     }
   }
-  return hipSuccess;
+  return Launched(p.done, stream);
 }
 
 } // namespace tbamd

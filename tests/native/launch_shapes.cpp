@@ -2,6 +2,7 @@
 #include "kernels.h"
 
 #include <cstdio>
+#include <vector>
 
 using namespace tbamd;
 
@@ -34,8 +35,42 @@ static void FewRows() {
         }
 }
 
+// Parts of the line of row blocks x groups against the owners counted one by one.
+static void SplitLines() {
+  for (int64_t rowBlocks = 1; rowBlocks <= 70; rowBlocks += rowBlocks < 9 ? 1 : 7)
+    for (int groups = 1; groups <= 40; groups += groups < 6 ? 1 : 5)
+      for (int64_t blocks = 1; blocks <= rowBlocks * groups; blocks += blocks < 12 ? 1 : 1 + rowBlocks * groups / 23) {
+        const SplitLine line{rowBlocks * groups, groups, (int)blocks};
+        EXPECT(line.FirstUnit(0) == 0 && line.FirstUnit(blocks) == line.units, "%d groups %lld blocks", groups, (long long)blocks);
+        std::vector<int64_t> owner((size_t)line.units, -1);
+        for (int64_t b = 0; b < blocks; ++b)
+          for (int64_t u = line.FirstUnit(b); u < line.FirstUnit(b + 1); ++u) owner[(size_t)u] = b;
+        for (int64_t r = 0; r < rowBlocks; ++r) {
+          const int64_t first = owner[(size_t)(r * groups)], last = owner[(size_t)((r + 1) * groups - 1)];
+          EXPECT(first == line.FirstBlock(r) && last - first + 1 == line.Parts(r) && line.Parts(r) <= SplitLine::Slots(blocks, rowBlocks),
+                 "row block %lld of %lld, %d groups, %lld blocks", (long long)r, (long long)rowBlocks, groups, (long long)blocks);
+        }
+      }
+}
+
+// Every width of the form: the ranks and two bundles a wave fit LDS, and the slices never outnumber the bundles.
+static void Streams() {
+  for (int features = 1; features <= kStreamMaxFeatures; ++features) {
+    const int waves = StreamWaves(features);
+    EXPECT(waves >= 1 && waves <= kStreamMaxWaves && ((features + 1) * kStreamRows + 15) / 16 * 16 + waves * 2 * (int)kStreamBundleBytes <= 160 * 1024,
+           "%d features: %d waves", features, waves);
+    for (int bundles : {1, 2, 31, 125, 4000})
+      for (int64_t rows : {(int64_t)1, (int64_t)33, (int64_t)5000, (int64_t)1 << 20}) {
+        const int slices = RankStreamSlices(rows, features, bundles, 256);
+        EXPECT(slices >= 1 && slices <= 64 && (slices == 1 || slices * 2 * waves <= bundles), "%d features, %d bundles: %d slices", features, bundles, slices);
+      }
+  }
+}
+
 int main() {
   FewRows();
+  SplitLines();
+  Streams();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

@@ -112,6 +112,8 @@ int main(int argc, char **argv) {
         ++loaded;
         const LaunchPlan plan = ChoosePlan(forest, 4096, nullptr, limits);
         const PackedModel pm = PackForest(forest, plan);
+        (void)PackFewRows(forest);
+        (void)PackRankStream(forest);
         if (plan.kernel != LaunchPlan::Kernel::kGlobalWalk && !forest.trees.empty()) (void)UnpackTree(pm, 0);
         ++packed;
       } catch (const Error &) {

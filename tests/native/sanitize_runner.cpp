@@ -7,6 +7,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -17,6 +18,8 @@
 #include <random>
 #include <string>
 #include <vector>
+
+extern "C" long shimFewRows, shimSplits, shimStreams; // hip_host_shim.cpp
 
 namespace {
 
@@ -153,30 +156,50 @@ intptr_t MakeRunner(const Case &c, int32_t batch, bool int8Classes, int32_t tile
   return runner;
 }
 
+// The kernels of the runner's own launch plan, whatever forms take its calls otherwise (batches of a few rows, streamed
+// bundles): the plan the description names, pinned.
+void PinOwnPlan(intptr_t runner) {
+  char text[1024];
+  tbmi_describe_plan(runner, text, sizeof(text));
+  const auto field = [&](const char *name) {
+    const char *at = std::strstr(text, (std::string(" ") + name + "=").c_str());
+    return at ? std::atoi(at + std::strlen(name) + 2) : 0;
+  };
+  const int32_t rows = field("rowsPerBlock"), k = field("interleave"), bytes = field("groupBytes"), slices = field("treeSlices");
+  int32_t rc;
+  if (std::strstr(text, "kernel=tree_parallel")) rc = tbmi_set_tree_parallel_plan(runner, rows, field("treeLanes"), k, bytes, slices);
+  else if (std::strstr(text, "kernel=global_walk")) rc = tbmi_set_global_walk_plan(runner, rows, k, slices);
+  else if (field("quantizedRows")) rc = tbmi_set_quantized_plan(runner, field("treeThreads"), k, bytes, slices);
+  else if (field("rankRows16")) rc = tbmi_set_rank16_plan(runner, rows, field("treeThreads"), k, bytes, slices);
+  else rc = tbmi_set_plan(runner, rows, field("treeThreads"), k, bytes, slices);
+  EXPECT(rc == 0, "pinning %s", text);
+}
+
 // SANITIZE_QUICK=1: only the largest batch through the host entry points and the default plan through the
 // device entry points (the thread sanitizer's slower build looks at the copier threads, not at plan shapes).
 bool Quick() { return std::getenv("SANITIZE_QUICK") != nullptr; }
 
-void HostEntryPoints(const Case &c) {
+void HostEntryPoints(const Case &c, bool pinned = false) {
   const int64_t F = c.forest.numFeatures;
   // exact-size result buffers (heap, so that an overrun is seen), several batch sizes incl. the staged path
   for (int64_t rows : {(int64_t)1, (int64_t)63, (int64_t)1000, (int64_t)8192, c.rows}) {
     if (rows > c.rows || (Quick() && rows != c.rows)) continue;
     const intptr_t runner = MakeRunner(c, (int32_t)rows, false);
     if (!runner) continue;
+    if (pinned) PinOwnPlan(runner);
     std::vector<float> in(c.x.begin(), c.x.begin() + rows * F), out((size_t)rows, -1.f);
     RunInference(runner, in.data(), out.data());
     Compare(c, out.data(), 0, rows, "RunInference");
     RunInference(runner, in.data(), out.data()); // buffers reused
     Compare(c, out.data(), 0, rows, "RunInference again");
     // "pinned" input: memory the runtime knows as host memory is read where it lies
-    void *pinned = nullptr;
-    if (hipHostMalloc(&pinned, (size_t)rows * F * sizeof(float), 0) == hipSuccess) {
-      std::memcpy(pinned, in.data(), (size_t)rows * F * sizeof(float));
+    void *locked = nullptr;
+    if (hipHostMalloc(&locked, (size_t)rows * F * sizeof(float), 0) == hipSuccess) {
+      std::memcpy(locked, in.data(), (size_t)rows * F * sizeof(float));
       std::fill(out.begin(), out.end(), -1.f);
-      RunInference(runner, pinned, out.data());
+      RunInference(runner, locked, out.data());
       Compare(c, out.data(), 0, rows, "RunInference pinned");
-      (void)hipHostFree(pinned);
+      (void)hipHostFree(locked);
     }
     // any number of rows through a runner compiled for `rows`
     for (int64_t n : {(int64_t)0, rows / 3, rows, std::min(c.rows, rows * 2 + 5), c.rows}) {
@@ -193,6 +216,32 @@ void HostEntryPoints(const Case &c) {
     }
     DeleteInferenceRunner(runner);
   }
+}
+
+// Ids, sums and softmax of a classifier, together and one alone.
+void MulticlassOutputs(const Case &c, intptr_t runner, const float *dx, int64_t rows) {
+  if (c.forest.numClasses == 0) return;
+  const size_t values = (size_t)rows * (size_t)c.forest.numClasses;
+  int8_t *cls = nullptr;
+  float *margins = nullptr, *probs = nullptr;
+  EXPECT(hipMalloc((void **)&cls, (size_t)rows) == hipSuccess, "hipMalloc");
+  EXPECT(hipMalloc((void **)&margins, values * sizeof(float)) == hipSuccess, "hipMalloc");
+  EXPECT(hipMalloc((void **)&probs, values * sizeof(float)) == hipSuccess, "hipMalloc");
+  std::fill_n(margins, values, std::nanf(""));
+  std::fill_n(probs, values, std::nanf(""));
+  EXPECT(tbmi_run_device_multiclass(runner, dx, rows, cls, margins, probs) == 0, "tbmi_run_device_multiclass");
+  for (int64_t r = 0; r < rows; ++r) {
+    EXPECT((float)cls[r] == c.expected[r], "class id of row %lld", (long long)r);
+    double z = 0.0;
+    for (int64_t i = 0; i < c.forest.numClasses; ++i) z += probs[r * c.forest.numClasses + i];
+    EXPECT(std::fabs(z - 1.0) < 1e-5, "probabilities of row %lld", (long long)r);
+    EXPECT(margins[r * c.forest.numClasses + cls[r]] == *std::max_element(margins + r * c.forest.numClasses, margins + (r + 1) * c.forest.numClasses),
+           "sums of row %lld", (long long)r);
+  }
+  EXPECT(tbmi_run_device_multiclass(runner, dx, rows, nullptr, margins, nullptr) == 0, "tbmi_run_device_multiclass");
+  (void)hipFree(cls);
+  (void)hipFree(margins);
+  (void)hipFree(probs);
 }
 
 void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_t tilingType = 0, const char *profile = "",
@@ -251,6 +300,11 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
     EXPECT(tbmi_describe_plan(runner, big, sizeof(big)) > 0, "describe");
   };
   runAll("default plan");
+  MulticlassOutputs(c, runner, dx, rows);
+  if (tileSize == 1 && tilingType == 0) {
+    PinOwnPlan(runner);
+    runAll("default plan, pinned");
+  }
   if (tileSize > 1) { // block shapes of the tiled walk, the plan search, save and reload
     const int tiledPlans[][5] = {{64, 1, 1, 16384, 1}, {128, 8, 2, 32768, 3}, {256, 4, 4, 40960, 2}, {64, 16, 2, 24576, 5}, {128, 4, 1, 65536, 2}};
     for (auto &p : tiledPlans)
@@ -305,19 +359,7 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
   double best = 0;
   EXPECT(tbmi_autotune(runner, dx, rows < 96 ? rows : 96, &best) == 0, "tbmi_autotune");
   runAll("after the plan search");
-  if (multiclass) {
-    int8_t *cls = nullptr;
-    float *margins = nullptr, *probs = nullptr;
-    EXPECT(hipMalloc((void **)&cls, (size_t)rows) == hipSuccess, "hipMalloc");
-    EXPECT(hipMalloc((void **)&margins, (size_t)rows * c.forest.numClasses * sizeof(float)) == hipSuccess, "hipMalloc");
-    EXPECT(hipMalloc((void **)&probs, (size_t)rows * c.forest.numClasses * sizeof(float)) == hipSuccess, "hipMalloc");
-    EXPECT(tbmi_run_device_multiclass(runner, dx, rows, cls, margins, probs) == 0, "tbmi_run_device_multiclass");
-    EXPECT(tbmi_run_device_multiclass(runner, dx, rows, nullptr, margins, nullptr) == 0, "tbmi_run_device_multiclass");
-    for (int64_t r = 0; r < rows; ++r) EXPECT((float)cls[r] == c.expected[r], "class id of row %lld", (long long)r);
-    (void)hipFree(cls);
-    (void)hipFree(margins);
-    (void)hipFree(probs);
-  }
+  MulticlassOutputs(c, runner, dx, rows);
   const std::string file = std::string(std::getenv("TMPDIR") ? std::getenv("TMPDIR") : "/tmp") + "/sanitize_runner.tbamd";
   EXPECT(tbmi_save_compiled_model(runner, file.c_str()) == 0, "tbmi_save_compiled_model");
   const intptr_t again = tbmi_load_compiled_model(file.c_str(), 0);
@@ -331,6 +373,46 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
   (void)hipFree(dx);
   (void)hipFree(dout);
   (void)hipFree(dids);
+}
+
+// All of the case's rows in one device call through every entry point, on the default plan and on plans of several slices
+// (which a launch of many blocks splits evenly); calls on the default stream, another stream and the runner's own in turn.
+void WholeBatch(const Case &c) {
+  const int64_t rows = c.rows, F = c.forest.numFeatures;
+  const bool multiclass = c.forest.numClasses > 0;
+  const intptr_t runner = MakeRunner(c, (int32_t)rows, multiclass);
+  if (!runner) return;
+  hipStream_t other = nullptr;
+  EXPECT(hipStreamCreateWithFlags(&other, 0) == hipSuccess, "hipStreamCreateWithFlags");
+  float *dx = nullptr;
+  unsigned char *dout = nullptr;
+  const size_t resultBytes = (size_t)rows * (size_t)tbmi_result_bytes(runner);
+  EXPECT(hipMalloc((void **)&dx, (size_t)rows * F * sizeof(float)) == hipSuccess, "hipMalloc");
+  EXPECT(hipMalloc((void **)&dout, resultBytes) == hipSuccess, "hipMalloc");
+  std::memcpy(dx, c.x.data(), (size_t)rows * F * sizeof(float));
+  const int plans[][5] = {{0, 0, 0, 0, 0}, {64, 4, 2, 8192, 5}, {64, 16, 4, 16384, 2}, {128, 2, 1, 16384, 3}};
+  for (auto &p : plans) {
+    if (p[0] && tbmi_set_plan(runner, p[0], p[1], p[2], p[3], p[4]) != 0) continue;
+    const auto check = [&](int32_t rc, const char *what) {
+      if (rc != 0 && std::strstr(tbmi_last_error(), "scratch memory")) return;
+      EXPECT(rc == 0, "%s", what);
+      std::vector<float> got((size_t)rows);
+      for (int64_t r = 0; r < rows; ++r) got[r] = multiclass ? (float)(int8_t)dout[r] : reinterpret_cast<float *>(dout)[r];
+      Compare(c, got.data(), 0, rows, what);
+      std::memset(dout, 0x5A, resultBytes);
+    };
+    check(tbmi_run_device_async(runner, dx, dout, rows, nullptr), "async, default stream");
+    check(tbmi_run_device_async(runner, dx, dout, rows, other), "async, another stream");
+    check(tbmi_run_device(runner, dx, dout, rows), "run_device");
+    check(tbmi_run_device_async(runner, dx, dout, rows, nullptr), "async, default stream again");
+    check(tbmi_run_device_noalloc(runner, dx, dout, rows, other), "noalloc");
+    MulticlassOutputs(c, runner, dx, rows);
+  }
+  EXPECT(tbmi_run_device_async(runner, dx, dout, rows, nullptr) == 0, "async");
+  DeleteInferenceRunner(runner);
+  (void)hipFree(dx);
+  (void)hipFree(dout);
+  (void)hipStreamDestroy(other);
 }
 
 } // namespace
@@ -382,6 +464,7 @@ int main(int argc, char **argv) {
   // argv: pairs of <model.json> <rows>, or --mutate <compiled model> <iterations>
   if (argc == 4 && std::strcmp(argv[1], "--mutate") == 0) {
     if (int rc = MutatedCompiledModels(argv[2], std::atoi(argv[3]))) return rc;
+    std::printf("few-rows launches %ld\n", shimFewRows);
     std::printf("ok\n");
     return 0;
   }
@@ -398,6 +481,8 @@ int main(int argc, char **argv) {
     c.expected.resize((size_t)c.rows);
     for (int64_t r = 0; r < c.rows; ++r) c.expected[r] = Predict(c.forest, c.x.data() + r * F, nullptr);
     HostEntryPoints(c);
+    HostEntryPoints(c, true);
+    WholeBatch(c);
     DeviceEntryPoints(c, std::min<int64_t>(c.rows, 203));
     if (!Quick()) {
       const std::string profile =
@@ -425,6 +510,6 @@ int main(int argc, char **argv) {
   EXPECT(tbmi_run_device(0, nullptr, nullptr, 4) == -1, "null runner");
   EXPECT(CreateInferenceRunner("/nonexistent/model.json", "", 0) == 0, "missing options");
   if (gFailures) return 1;
-  std::printf("ok\n");
+  std::printf("launches: few-rows %ld, split %ld, stream %ld\nok\n", shimFewRows, shimSplits, shimStreams);
   return 0;
 }

@@ -163,6 +163,25 @@ def test_runner_under_address_sanitizer(tmp_path, synth_model, address_driver):
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+@pytest.mark.parametrize("units", ["4", "256"])
+def test_forms_beside_the_launch_plans_under_address_sanitizer(tmp_path, synth_model, address_driver, units):
+    """Batches of a few rows, evenly split launches (a chip of four compute units splits small ones) and streamed bundles of
+    one and of two slices: the three run, their packers, workspaces and index arithmetic under ASan + UBSan."""
+    import numpy as np
+    rng = np.random.Generator(np.random.PCG64(8))
+    trees = [synth._grow_tree(rng, 2, lambda d, s: 1.0, lambda: (rng.integers(0, 600), float(np.round(rng.normal(), 1))),
+                              lambda: rng.normal(0.0, 0.1)) for _ in range(600)]
+    wide = str(tmp_path / "wide_shallow.json")
+    synth.write_xgboost_json(wide, trees, 600)
+    env = dict(os.environ, SANITIZE_QUICK="1", SHIM_COMPUTE_UNITS=units, ASAN_OPTIONS="detect_leaks=1:abort_on_error=0", TMPDIR=str(tmp_path))
+    run = subprocess.run([address_driver, wide, "2701", _multiclass_model(tmp_path), "1301", synth_model(1), "2999"], capture_output=True,
+                         text=True, env=env, timeout=900)
+    assert run.returncode == 0, (run.stdout + run.stderr)[-4000:]
+    counts = [int(part.split()[-1]) for part in run.stdout.split("launches: ")[1].splitlines()[0].split(",")]
+    assert counts[0] > 0 and counts[2] > 0 and (counts[1] > 0 or units == "256"), run.stdout[-300:]
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 def test_runner_survives_mutated_compiled_models(tmp_path, synth_model, address_driver):
     """tbmi_load_compiled_model on compiled-model files whose header words (plan, batch size, return type, counts) and
     body were overwritten: refused with a message or loaded and run on a few rows, under ASan + UBSan."""

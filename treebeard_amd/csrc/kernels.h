@@ -55,8 +55,8 @@ struct WalkParams {
   int32_t *leafIds = nullptr;     // [rows][numTrees]
   const int32_t *nodeOrigin = nullptr;
   const int32_t *slotTree = nullptr;
-  hipEvent_t done = nullptr;      // recorded when this kernel completes (kLaunchersRecordEvents)
-  // Row-parallel walk on f32 or one-byte rank rows, kLaunchersSplitEvenly: `splitBlocks` blocks (0: one per row block and
+  hipEvent_t done = nullptr;      // recorded when this kernel completes
+  // Row-parallel walk on f32 or one-byte rank rows: `splitBlocks` blocks (0: one per row block and
   // tree slice) share the units row block x tree group evenly; partial holds SplitLine::Slots slots.
   int32_t splitBlocks = 0;
 };
@@ -173,22 +173,22 @@ struct RankStreamParams {
   hipEvent_t done = nullptr;
 };
 
-#if defined(__HIP__)
-inline constexpr bool kLaunchersRecordEvents = true;
-inline constexpr bool kLaunchersSplitEvenly = true;
+// Waves of a block of LaunchRankStream: as many as have room for two bundles each beside the rows' ranks.
+constexpr int kStreamMaxWaves = 16;
+inline int StreamWaves(int32_t numFeatures) {
+  const int64_t tile = ((int64_t)(numFeatures + 1) * kStreamRows + 15) & ~(int64_t)15;
+  return (int)std::min<int64_t>(kStreamMaxWaves, (160 * 1024 - tile) / (2 * kStreamBundleBytes));
+}
+// Slices fill the compute units while every wave of a block still has two bundles to overlap.
+inline int32_t RankStreamSlices(int64_t rows, int32_t numFeatures, int32_t numBundles, int32_t computeUnits) {
+  const int64_t blocks = (rows + kStreamRows - 1) / kStreamRows;
+  const int64_t most = numBundles / (2 * std::max(1, StreamWaves(numFeatures)));
+  return (int32_t)std::max<int64_t>(1, std::min<int64_t>({computeUnits / std::max<int64_t>(1, blocks), most, 64}));
+}
+
+// (Every launcher below records the `done` of its parameters behind its kernel.)
 hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream);
-inline constexpr bool kHaveRankStream = true;
-int32_t RankStreamSlices(int64_t rows, int32_t numFeatures, int32_t numBundles, int32_t computeUnits);
 hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream);
-#else
-// (host-only builds of the runner, under the sanitizers, link stand-ins of the launchers below and have no others)
-inline constexpr bool kLaunchersRecordEvents = false;
-inline constexpr bool kLaunchersSplitEvenly = false;
-inline hipError_t LaunchFewRows(const FewRowsParams &, hipStream_t) { return hipErrorNotSupported; }
-inline constexpr bool kHaveRankStream = false;
-inline int32_t RankStreamSlices(int64_t, int32_t, int32_t, int32_t) { return 1; }
-inline hipError_t LaunchRankStream(const RankStreamParams &, hipStream_t) { return hipErrorNotSupported; }
-#endif
 
 // Row-parallel walk over LDS-staged tree groups: block = s.rowsPerBlock * s.treeThreads lanes.
 // `interleave` in {1,2,4,8}; `tileMode`: 0 f32 tile with byte offsets, 1 f32 tile with offsets in units of

@@ -1554,13 +1554,6 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
 // two chains a lane, 914 with four and without words for the last level's leaves, 883 with two levels per loop turn, 800
 // with LDS reads awaited one by one.  20000 rows 94 -> 77 us.
 // ---------------------------------------------------------------------------
-constexpr int kStreamMaxWaves = 16;
-
-int StreamWaves(int32_t numFeatures) {
-  const int64_t tile = ((int64_t)(numFeatures + 1) * kStreamRows + 15) & ~(int64_t)15;
-  return (int)std::min<int64_t>(kStreamMaxWaves, (160 * 1024 - tile) / (2 * kStreamBundleBytes));
-}
-
 template <int K> // chains
 __global__ void __launch_bounds__(kStreamMaxWaves * 64)
 RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__ words, const float *__restrict__ values,
@@ -1990,13 +1983,6 @@ hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream) {
   const int64_t blocks = (p.rows + s.rowsPerBlock - 1) / s.rowsPerBlock;
   return StartKernel(&FewRowsKernel, dim3((unsigned)blocks), dim3((unsigned)s.threads), s.ldsBytes, stream, p.done, p, s.rowsPerBlock,
                      (int)s.leafStride);
-}
-
-// Slices fill the compute units while every wave of a block still has two bundles to overlap.
-int32_t RankStreamSlices(int64_t rows, int32_t numFeatures, int32_t numBundles, int32_t computeUnits) {
-  const int64_t blocks = (rows + kStreamRows - 1) / kStreamRows;
-  const int64_t most = numBundles / (2 * std::max(1, StreamWaves(numFeatures)));
-  return (int32_t)std::max<int64_t>(1, std::min<int64_t>({computeUnits / std::max<int64_t>(1, blocks), most, 64}));
 }
 
 hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {

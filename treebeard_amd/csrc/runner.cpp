@@ -226,7 +226,7 @@ void InferenceRunner::UploadModel() {
   m_dNodeOrigin = Upload(m_model.nodeOrigin, "upload node origins");
   m_dSlotTree = Upload(m_model.slotTree, "upload slot table");
   if (m_model.plan.quantizedRows) m_dBinTable = Upload(m_model.binThresholds, "upload threshold table");
-  if (kHaveRankStream && m_model.plan.quantizedRows) {
+  if (m_model.plan.quantizedRows) {
     const RankStreamModel stream = PackRankStream(m_forest);
     if (!stream.bundles.empty()) {
       m_dStreamWords = Upload(stream.words, "upload stream words");
@@ -302,7 +302,7 @@ size_t InferenceRunner::RanksBytes(int64_t rows) const {
 
 int32_t InferenceRunner::SplitBlocks(int64_t rows) const {
   const LaunchPlan &plan = m_model.plan;
-  if (!kLaunchersSplitEvenly || plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.WalkTile() > 1 || plan.rankRows16 ||
+  if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.WalkTile() > 1 || plan.rankRows16 ||
       plan.deferTails)
     return 0;
   const int64_t blocks = RowBlocks(rows) * plan.treeSlices;
@@ -558,7 +558,6 @@ void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out
   f.done = done;
   if (LaunchWalkFor(PrepareRows(deviceInputs, rows, ws.ranks, stream), rows, f, leafIds, stream, ws, done))
     Check(LaunchFinalize(f, stream), "launch finalize kernel");
-  if (done && !kLaunchersRecordEvents) Check(hipEventRecord(done, stream), "hipEventRecord");
 }
 
 void InferenceRunner::RunDevice(const float *deviceInputs, void *deviceResults, int64_t rows) {
