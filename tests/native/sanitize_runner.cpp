@@ -310,6 +310,10 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
     for (auto &p : tiledPlans)
       if (tbmi_set_plan(runner, p[0], p[1], p[2], p[3], p[4]) == 0) runAll("tiled plan");
     EXPECT(tbmi_set_tree_parallel_plan(runner, 4, 64, 1, 0, 1) == -1, "tree-parallel plan must refuse tiles");
+    EXPECT(tbmi_set_global_walk_plan(runner, 256, 4, 1) == -1, "global-walk plan must refuse tiles");
+    EXPECT(tbmi_set_quantized_plan(runner, 8, 4, 0, 1) == -1, "one-byte rank plan must refuse tiles");
+    EXPECT(tbmi_set_rank16_plan(runner, 64, 4, 4, 0, 1) == -1, "two-byte rank plan must refuse tiles");
+    if ((F + 1) * 512 * 4 > 0x10000) EXPECT(tbmi_set_plan(runner, 512, 2, 2, 0, 1) == -1, "a row tile of 64 KB must refuse tiles");
     double best = 0;
     EXPECT(tbmi_autotune(runner, dx, rows < 96 ? rows : 96, &best) == 0, "tbmi_autotune (tiled)"); // (a few rows: the search re-packs and launches hundreds of times)
     runAll("tiled, after the plan search");

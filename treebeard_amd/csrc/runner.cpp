@@ -276,6 +276,17 @@ void InferenceRunner::Repack(const LaunchPlan &plan) {
   UploadModel();
 }
 
+void InferenceRunner::PinPlan(const LaunchPlan &plan) {
+  if (plan.tileSize > 1) {
+    if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.quantizedRows || plan.rankRows16)
+      throw Error("tile sizes above 1 need the row-parallel kernel on float32 rows");
+    if ((int64_t)(m_forest.numFeatures + 1) * plan.rowsPerBlock * 4 > 0x10000)
+      throw Error("tile sizes above 1 need a row tile below 64 KB (tiles hold byte offsets): fewer rows per block");
+  }
+  Repack(plan);
+  m_planPinned = true;
+}
+
 size_t InferenceRunner::PartialBytes(int64_t rows, bool split) const {
   if (split && StreamsBundles()) {
     const int32_t slices = StreamSlices(rows);

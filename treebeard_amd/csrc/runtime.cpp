@@ -402,7 +402,6 @@ int32_t tbmi_set_tree_parallel_plan(intptr_t h, int32_t rowsPerBlock, int32_t tr
       [&] {
         InferenceRunner *r = Runner(h);
         LaunchPlan plan = r->Model().plan;
-        if (plan.tileSize > 1) throw Error("tile sizes above 1 need the row-parallel kernel on float32 rows");
         plan.kernel = LaunchPlan::Kernel::kTreeParallel;
         plan.deferTails = false;
         plan.featureOffsetInWords = false;
@@ -427,8 +426,7 @@ int32_t tbmi_set_global_walk_plan(intptr_t h, int32_t rowsPerBlock, int32_t inte
         InferenceRunner *r = Runner(h);
         LaunchPlan plan;
         plan.kernel = LaunchPlan::Kernel::kGlobalWalk;
-        // what the options asked of the walk stays in the plan: a tiled runner is refused by the packer (the
-        // global-memory walk has scalar nodes only) instead of quietly turning into a scalar walk
+        // what the options asked of the walk stays in the plan (a tiled runner is refused)
         plan.tileSize = r->Model().plan.tileSize;
         plan.tiling = r->Model().plan.tiling;
         plan.peelWalks = r->Model().plan.peelWalks;
