@@ -163,9 +163,10 @@ TBAMD_EXPORT int32_t tbmi_dump_leaf_ids(intptr_t runner, const float *deviceInpu
 TBAMD_EXPORT int32_t tbmi_time_kernels(intptr_t runner, const float *deviceInputs, void *deviceResults,
                                        int64_t rows, int32_t runs, double *walkMs, double *finalizeMs,
                                        double *binMs);
-/* Timed search over launch plans on the given rows; keeps the fastest plan. */
+/* Timed search over launch plans on the given rows; keeps the fastest plan and lets go of one pinned before. */
 TBAMD_EXPORT int32_t tbmi_autotune(intptr_t runner, const float *deviceInputs, int64_t rows, double *bestMs);
-/* Pins the row-parallel kernel: rowsPerBlock rows per block, treeThreads lanes per row (in different
+/* Pins the row-parallel kernel (every call runs a pinned plan, until tbmi_autotune or another plan; batches of a few rows
+ * and wide rows otherwise have forms of their own): rowsPerBlock rows per block, treeThreads lanes per row (in different
  * waves), interleave trees walked at once per lane, groupBytes of LDS per tree group, treeSlices blocks
  * per row block (values <= 0 keep the current choice; treeThreads <= 0 means 1). */
 TBAMD_EXPORT int32_t tbmi_set_plan(intptr_t runner, int32_t rowsPerBlock, int32_t treeThreads, int32_t interleave,

@@ -156,6 +156,12 @@ intptr_t MakeRunner(const Case &c, int32_t batch, bool int8Classes, int32_t tile
   return runner;
 }
 
+std::string Describe(intptr_t runner) {
+  char text[1024];
+  tbmi_describe_plan(runner, text, sizeof(text));
+  return text;
+}
+
 // The kernels of the runner's own launch plan, whatever forms take its calls otherwise (batches of a few rows, streamed
 // bundles): the plan the description names, pinned.
 void PinOwnPlan(intptr_t runner) {
@@ -362,6 +368,9 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
   if (tbmi_set_global_walk_plan(runner, 256, 4, 3) == 0) runAll("global walk plan");
   double best = 0;
   EXPECT(tbmi_autotune(runner, dx, rows < 96 ? rows : 96, &best) == 0, "tbmi_autotune");
+  const long fewBefore = shimFewRows;
+  EXPECT(tbmi_run_device(runner, dx, dout, 1) == 0 && (shimFewRows > fewBefore || std::strstr(Describe(runner).c_str(), " peelWalks=1 ")),
+         "the plan search ends a pinned plan's hold on small batches");
   runAll("after the plan search");
   MulticlassOutputs(c, runner, dx, rows);
   const std::string file = std::string(std::getenv("TMPDIR") ? std::getenv("TMPDIR") : "/tmp") + "/sanitize_runner.tbamd";

@@ -913,6 +913,8 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
   void *out = nullptr;
   Check(hipMalloc(&out, std::max<int64_t>(rows, 1) * sizeof(float)), "allocate tuning output");
   const LaunchPlan original = m_model.plan;
+  const bool pinned = m_planPinned;
+  m_planPinned = false; // (the search decides again)
   // Two rounds: every candidate with a few launches, then the best few (and the analytic plan the runner started
   // with) again with more launches, so that the plan kept is not one that merely had a lucky first timing.
   struct Timed { LaunchPlan plan; double ms; };
@@ -979,6 +981,7 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
     m_walk.peelWalks = best.peelWalks;
     Repack(best);
   } catch (...) {
+    m_planPinned = pinned;
     (void)hipFree(out);
     throw;
   }

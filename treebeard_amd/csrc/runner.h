@@ -72,11 +72,11 @@ public:
                    double *finalizeMs, double *binMs);
   // Re-packs the model for another launch plan (used by the timed search).
   void Repack(const LaunchPlan &plan);
-  // A plan the caller chose: every call runs it, small batches included.  A runner of tile size 2 or more takes the plans the
+  // A plan the caller chose: every call runs it, small batches included, until AutoTune.  A runner of tile size 2 or more takes the plans the
   // tiled walk has a form for and no others, also where its tiles are uniform and scalar nodes stand for them
   // (LaunchPlan::WalkTile): what a caller may pin does not depend on how tiles are walked.
   void PinPlan(const LaunchPlan &plan);
-  // Timed search over CandidatePlans(); keeps the fastest.  Returns its time in ms.  A runner without a hit-count
+  // Timed search over CandidatePlans(); keeps the fastest, which is not a pinned plan.  Returns its time in ms.  A runner without a hit-count
   // profile profiles up to 4096 of the rows itself, so that peeled walks can be among the candidates.
   double AutoTune(const float *deviceInputs, int64_t rows);
   // Peeled walks without a profile file: profiles up to 4096 of the given rows on the device (unless the runner
