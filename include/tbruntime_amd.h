@@ -159,7 +159,8 @@ TBAMD_EXPORT int32_t tbmi_run_device_multiclass(intptr_t runner, const float *de
 TBAMD_EXPORT int32_t tbmi_dump_leaf_ids(intptr_t runner, const float *deviceInputs, int32_t *deviceLeafIds,
                                         int64_t rows);
 /* Average kernel durations (ms) over `runs` launches each, measured with HIP events on the runner's stream:
- * the walk kernel, the finalize kernel and the rank-quantisation kernel (0 when the plan has none). */
+ * the walk kernel, the finalize kernel and the rank-quantisation kernel (0 where a call of `rows` rows runs none: a batch
+ * of a few rows is one kernel, reported as the walk). */
 TBAMD_EXPORT int32_t tbmi_time_kernels(intptr_t runner, const float *deviceInputs, void *deviceResults,
                                        int64_t rows, int32_t runs, double *walkMs, double *finalizeMs,
                                        double *binMs);

@@ -367,7 +367,9 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
     if (tbmi_set_rank16_plan(runner, p[0], p[1], p[2], p[3], p[4]) == 0) runAll("two-byte rank plan");
   if (tbmi_set_global_walk_plan(runner, 256, 4, 3) == 0) runAll("global walk plan");
   double best = 0;
+  const long fewInSearch = shimFewRows;
   EXPECT(tbmi_autotune(runner, dx, rows < 96 ? rows : 96, &best) == 0, "tbmi_autotune");
+  EXPECT((shimFewRows > fewInSearch) == !!std::strstr(Describe(runner).c_str(), " peelWalks=0 "), "the plan search times the kernel that takes its batch");
   const long fewBefore = shimFewRows;
   EXPECT(tbmi_run_device(runner, dx, dout, 1) == 0 && (shimFewRows > fewBefore || !std::strstr(Describe(runner).c_str(), " peelWalks=0 ")),
          "the plan search ends a pinned plan's hold on small batches");
@@ -395,6 +397,8 @@ void WholeBatch(const Case &c) {
   const bool multiclass = c.forest.numClasses > 0;
   const intptr_t runner = MakeRunner(c, (int32_t)rows, multiclass);
   if (!runner) return;
+  const std::string plan = Describe(runner);
+  const int64_t limit = std::atoll(plan.c_str() + plan.find("fewRowsLimit=") + std::strlen("fewRowsLimit="));
   hipStream_t other = nullptr;
   EXPECT(hipStreamCreateWithFlags(&other, 0) == hipSuccess, "hipStreamCreateWithFlags");
   float *dx = nullptr;
@@ -420,6 +424,17 @@ void WholeBatch(const Case &c) {
     check(tbmi_run_device_async(runner, dx, dout, rows, nullptr), "async, default stream again");
     check(tbmi_run_device_noalloc(runner, dx, dout, rows, other), "noalloc");
     MulticlassOutputs(c, runner, dx, rows);
+  }
+  double best = 0, walk = 0, fin = 0, bin = 0;
+  EXPECT(tbmi_autotune(runner, dx, std::min<int64_t>(rows, 300), &best) == 0, "tbmi_autotune");
+  for (int64_t n : {(int64_t)1, limit, limit + 1, rows}) { // what is timed is what a call runs
+    if (n < 1 || n > rows) continue;
+    const long few = shimFewRows, streams = shimStreams;
+    EXPECT(tbmi_run_device(runner, dx, dout, n) == 0, "run_device");
+    const long fewCall = shimFewRows - few, streamCall = shimStreams - streams;
+    EXPECT(fewCall == (n <= limit && std::strstr(Describe(runner).c_str(), " peelWalks=0 ")), "%lld rows, limit %lld", (long long)n, (long long)limit);
+    EXPECT(tbmi_time_kernels(runner, dx, dout, n, 1, &walk, &fin, &bin) == 0, "tbmi_time_kernels");
+    EXPECT(shimFewRows - few == 2 * fewCall && shimStreams - streams == 2 * streamCall, "kernels timed on %lld rows are not the call's", (long long)n);
   }
   EXPECT(tbmi_run_device_async(runner, dx, dout, rows, nullptr) == 0, "async");
   DeleteInferenceRunner(runner);

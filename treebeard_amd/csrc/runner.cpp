@@ -153,6 +153,9 @@ void InferenceRunner::Release() noexcept {
   FreeModel();
   (void)hipFree(m_dFewRows);
   (void)hipFree(m_dFewRowsClasses);
+  (void)hipFree(m_dStreamWords);
+  (void)hipFree(m_dStreamValues);
+  (void)hipFree(m_dStreamBundles);
   if (m_smallHost) (void)hipHostFree(m_smallHost);
   (void)hipFree(m_dPartial);
   (void)hipFree(m_dRanks);
@@ -183,13 +186,6 @@ void InferenceRunner::FreeModel() {
   (void)hipFree(m_dBinTable);
   (void)hipFree(m_dRankFeatures);
   (void)hipFree(m_dRankChunks);
-  (void)hipFree(m_dStreamWords);
-  (void)hipFree(m_dStreamValues);
-  (void)hipFree(m_dStreamBundles);
-  m_dStreamWords = nullptr;
-  m_dStreamValues = nullptr;
-  m_dStreamBundles = nullptr;
-  m_streamBundles = 0;
   (void)hipFree(m_dTailNodes);
   (void)hipFree(m_dTailOrigin);
   m_dTailNodes = nullptr;
@@ -226,16 +222,7 @@ void InferenceRunner::UploadModel() {
   m_dNodeOrigin = Upload(m_model.nodeOrigin, "upload node origins");
   m_dSlotTree = Upload(m_model.slotTree, "upload slot table");
   if (m_model.plan.quantizedRows) m_dBinTable = Upload(m_model.binThresholds, "upload threshold table");
-  if (m_model.plan.quantizedRows) {
-    const RankStreamModel stream = PackRankStream(m_forest);
-    if (!stream.bundles.empty()) {
-      m_dStreamWords = Upload(stream.words, "upload stream words");
-      m_dStreamValues = Upload(stream.values, "upload stream values");
-      m_dStreamBundles = Upload(stream.bundles, "upload stream bundles");
-      m_streamBundles = (int32_t)stream.bundles.size();
-      m_streamChains = stream.chains;
-    }
-  }
+  if (m_model.plan.quantizedRows) UploadStream();
   if (m_model.plan.deferTails) {
     m_dTailNodes = Upload(m_model.tailNodes, "upload tail nodes");
     m_dTailOrigin = Upload(m_model.tailOrigin, "upload tail node origins");
@@ -250,6 +237,19 @@ void InferenceRunner::UploadModel() {
       m_rankChunkFeatures = std::max(m_rankChunkFeatures, c.numFeatures);
     }
   }
+}
+
+void InferenceRunner::UploadStream() {
+  if (m_streamPacked) return; // (the bundles are the forest's, whatever the launch plan)
+  const RankStreamModel stream = PackRankStream(m_forest);
+  if (!stream.bundles.empty()) {
+    m_dStreamWords = Upload(stream.words, "upload stream words");
+    m_dStreamValues = Upload(stream.values, "upload stream values");
+    m_dStreamBundles = Upload(stream.bundles, "upload stream bundles");
+    m_streamBundles = (int32_t)stream.bundles.size();
+    m_streamChains = stream.chains;
+  }
+  m_streamPacked = true;
 }
 
 void InferenceRunner::UploadFewRows() {
@@ -824,11 +824,21 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
 }
 
 void InferenceRunner::TimeKernels(const float *deviceInputs, void *deviceResults, int64_t rows, int32_t runs,
-                                  double *walkMs, double *finalizeMs, double *binMs) {
+                                  double *walkMs, double *finalizeMs, double *binMs, bool planKernels) {
   runs = std::max(1, runs);
-  const Workspace ws = OwnWorkspace(rows, m_stream, true);
+  const Workspace ws = OwnWorkspace(rows, m_stream, planKernels);
   float ms = 0.f;
   if (binMs) *binMs = 0.0;
+  if (!planKernels && TakesFewRows(rows)) { // one kernel is the whole call
+    Check(hipEventRecord(m_evStart, m_stream), "hipEventRecord");
+    for (int i = 0; i < runs; ++i) LaunchPredictions(deviceInputs, rows, deviceResults, m_stream, ws);
+    Check(hipEventRecord(m_evStop, m_stream), "hipEventRecord");
+    Check(hipStreamSynchronize(m_stream), "few-rows kernel");
+    Check(hipEventElapsedTime(&ms, m_evStart, m_evStop), "hipEventElapsedTime");
+    if (walkMs) *walkMs = ms / runs;
+    if (finalizeMs) *finalizeMs = 0.0;
+    return;
+  }
   const float *walkInputs = deviceInputs;
   if (m_model.plan.quantizedRows || m_model.plan.rankRows16) {
     Check(hipEventRecord(m_evStart, m_stream), "hipEventRecord");
@@ -927,8 +937,8 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
     }
     double w = 0, f = 0, b = 0;
     try {
-      TimeKernels(deviceInputs, out, rows, 1, &w, &f, &b); // warm-up
-      TimeKernels(deviceInputs, out, rows, runs, &w, &f, &b);
+      TimeKernels(deviceInputs, out, rows, 1, &w, &f, &b, true); // warm-up
+      TimeKernels(deviceInputs, out, rows, runs, &w, &f, &b, true);
     } catch (const Error &) {
       (void)hipGetLastError(); // plan the launcher rejects (e.g. too few lanes to prefetch a group)
       return false;
@@ -939,16 +949,22 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
   LaunchPlan best = original;
   double bestMs = 1e300;
   try {
+    // (one-byte rank rows of a forest that streams its bundles run one kernel whatever the shape of the plan)
+    const auto streamed = [&](const LaunchPlan &plan) { return plan.quantizedRows && m_streamBundles > 0; };
+    const auto isTimed = [&](const LaunchPlan &plan) {
+      return streamed(plan) && std::any_of(timed.begin(), timed.end(), [&](const Timed &t) { return streamed(t.plan); });
+    };
     for (const LaunchPlan &cand : CandidatePlans(m_forest, rows, m_limits, m_walk)) {
       double ms = 0;
-      if (timePlan(cand, 3, &ms)) timed.push_back(Timed{m_model.plan, ms});
+      if (!isTimed(cand) && timePlan(cand, 3, &ms)) timed.push_back(Timed{m_model.plan, ms});
     }
     std::stable_sort(timed.begin(), timed.end(), [](const Timed &a, const Timed &b) { return a.ms < b.ms; });
     if (timed.size() > 6) timed.resize(6);
-    timed.push_back(Timed{original, 0.0});
+    if (!isTimed(original)) timed.push_back(Timed{original, 0.0});
     // Peeled walks (deferred tails) of the same shapes: they need a hit-count profile; without one from the caller
     // the rows of this batch are profiled (leaf ids of up to 4096 rows, counted on the host).
-    if (!original.deferTails && m_forest.numClasses == 0 && original.WalkTile() == 1) {
+    // (Not for a batch of a few rows: a peeled plan would keep it from its own form, which none of the plans timed here beats.)
+    if (!original.deferTails && m_forest.numClasses == 0 && original.WalkTile() == 1 && rows > m_fewRowsLimit) {
       if (!m_profile) m_profile = CollectProfile(deviceInputs, std::min<int64_t>(rows, 4096));
       const size_t shapes = timed.size();
       for (size_t i = 0; i < shapes; ++i) {
@@ -980,6 +996,10 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
       }
     m_walk.peelWalks = best.peelWalks;
     Repack(best);
+    if (TakesFewRows(rows)) { // calls of this batch run one kernel beside the plan: its time is theirs
+      TimeKernels(deviceInputs, out, rows, 1, &bestMs, nullptr, nullptr);
+      TimeKernels(deviceInputs, out, rows, 24, &bestMs, nullptr, nullptr);
+    }
   } catch (...) {
     m_planPinned = pinned;
     (void)hipFree(out);

@@ -66,10 +66,11 @@ public:
   // Parity check: original leaf node id reached by every (row, tree), int32[rows][numTrees].
   void DumpLeafIds(const float *deviceInputs, int32_t *deviceLeafIds, int64_t rows);
   // Average duration in milliseconds of the walk kernel, of the finalize kernel and of the
-  // rank-quantisation kernel (0 when the plan does not use them) over `runs` launches each,
-  // HIP events on the runner's stream.
+  // rank-quantisation kernel (0 when a call of `rows` rows does not run them) over `runs` launches each,
+  // HIP events on the runner's stream.  A batch of a few rows is one kernel, the "walk"; `planKernels`
+  // times the launch plan's kernels on it all the same.
   void TimeKernels(const float *deviceInputs, void *deviceResults, int64_t rows, int32_t runs, double *walkMs,
-                   double *finalizeMs, double *binMs);
+                   double *finalizeMs, double *binMs, bool planKernels = false);
   // Re-packs the model for another launch plan (used by the timed search).
   void Repack(const LaunchPlan &plan);
   // A plan the caller chose: every call runs it, small batches included, until AutoTune.  A runner of tile size 2 or more takes the plans the
@@ -77,7 +78,8 @@ public:
   // (LaunchPlan::WalkTile): what a caller may pin does not depend on how tiles are walked.
   void PinPlan(const LaunchPlan &plan);
   // Timed search over CandidatePlans(); keeps the fastest, which is not a pinned plan.  Returns its time in ms.  A runner without a hit-count
-  // profile profiles up to 4096 of the rows itself, so that peeled walks can be among the candidates.
+  // profile profiles up to 4096 of the rows itself, so that peeled walks can be among the candidates.  A batch of a few
+  // rows is searched with the plans' kernels, for larger ones, and returns the time of the kernel that takes it.
   double AutoTune(const float *deviceInputs, int64_t rows);
   // Peeled walks without a profile file: profiles up to 4096 of the given rows on the device (unless the runner
   // has a profile already) and re-packs the current plan with peeled walks where the plan has the form.
@@ -116,6 +118,7 @@ private:
   void WaitForAsyncCall();                       // host-side: returns when the last asynchronous call has finished
   void UploadModel();
   void UploadFewRows();
+  void UploadStream();
   void FreeModel();
   void EnsurePartial(size_t bytes);
   void EnsureStaging(int64_t rows);
@@ -143,7 +146,7 @@ private:
   // Rank-quantised plans: runs the binning kernel and returns the buffer the walk kernel reads.
   const float *PrepareRows(const float *deviceInputs, int64_t rows, uint8_t *ranks, hipStream_t stream);
   // Rank-quantised rows go through LaunchRankStream where the forest has the form, unless the caller pinned a plan.
-  bool StreamsBundles() const { return m_streamBundles > 0 && !m_planPinned; }
+  bool StreamsBundles() const { return m_model.plan.quantizedRows && m_streamBundles > 0 && !m_planPinned; }
   int32_t StreamSlices(int64_t rows) const { return RankStreamSlices(rows, m_forest.numFeatures, m_streamBundles, m_limits.computeUnits); }
   // The walk behind PrepareRows, with its outputs set; true when the finalize kernel (`f`) has to follow.
   bool LaunchWalkFor(const float *walkInputs, int64_t rows, FinalizeParams &f, int32_t *leafIds, hipStream_t stream, const Workspace &ws,
@@ -194,7 +197,8 @@ private:
   bool m_planPinned = false;
   int64_t m_fewRowsLimit = 0;
   DeviceFewRowsBlock *m_dFewRows = nullptr;
-  uint32_t *m_dStreamWords = nullptr;     // rank-quantised plans: bundles for LaunchRankStream
+  bool m_streamPacked = false;            // the first rank-quantised plan brings the bundles for LaunchRankStream
+  uint32_t *m_dStreamWords = nullptr;
   float *m_dStreamValues = nullptr;
   DeviceStreamBundle *m_dStreamBundles = nullptr;
   int32_t m_streamBundles = 0, m_streamChains = 0;
