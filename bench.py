@@ -48,7 +48,7 @@ def print_lds_read_costs():
 def plan_key(plan):
     """The fields of a plan description that decide which kernel runs and how (what a traffic figure is tied to)."""
     keep = ("kernel", "rowsPerBlock", "treeThreads", "treeLanes", "interleave", "groupBytes", "treeSlices", "quantizedRows",
-            "rankRows16", "tileSize", "staging", "peelWalks")
+            "rankRows16", "tileSize", "staging", "peelWalks", "batchKernel")
     fields = dict(item.split("=", 1) for item in plan.split() if "=" in item)
     return " ".join("%s=%s" % (k, fields[k]) for k in keep if k in fields)
 
@@ -60,7 +60,7 @@ def main():
     ap.add_argument("--warmup", type=int, default=3)
     ap.add_argument("--config", type=int, default=2, help="benchmark configuration 1..5 (default: the headline, 2)")
     ap.add_argument("--rows", type=int, default=0, help="override the batch size")
-    ap.add_argument("--tile-size", type=int, default=1, help="CompilerOptions tile size (2, 3, 4 run the tiled walk kernel)")
+    ap.add_argument("--tile-size", type=int, default=1, help="CompilerOptions tile size (with uniform tiling all sizes walk scalar nodes)")
     ap.add_argument("--group-staging", type=int, default=0, choices=[0, 1, 2],
                     help="how tree groups reach LDS: 0 by rule, 1 through prefetch registers, 2 direct global-to-LDS copies")
     ap.add_argument("--no-cpu-baseline", action="store_true")
@@ -168,8 +168,10 @@ def main():
     plan = runner.describe_plan()
     quantized = "quantizedRows=1" in plan or "rankRows16=1" in plan       # a ranking kernel runs in front of the walk
     plan_fields = dict(item.split("=", 1) for item in plan.split() if "=" in item)
-    kernel = ("WalkRowsTiledKernel" if " tileSize=1 " not in plan and " tiling=0 " not in plan else "WalkRowsLdsKernel") if "rows_lds" in plan else \
-        ("WalkGlobalKernel" if "global_walk" in plan else "WalkTreeParallelKernel")
+    kernel = {"few_rows": "FewRowsKernel", "rank_stream": "RankStreamKernel", "rows_lds_split": "WalkRowsSplitKernel",
+              "rows_lds": "WalkRowsLdsKernel", "rows_tiled": "WalkRowsTiledKernel", "tree_parallel": "WalkTreeParallelKernel",
+              "global_walk": "WalkGlobalKernel"}[plan_fields["batchKernel"]]
+    quantized = quantized and kernel != "FewRowsKernel"
     # the rank-quantised path reads the f32 rows in its binning kernel: both kernels count for the HBM roofline
     hbm_ms = walk_ms + bin_ms if quantized else walk_ms
     hbm_gbs = hbm_bytes_row * rows / (hbm_ms * 1e-3) / 1e9

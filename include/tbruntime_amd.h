@@ -198,6 +198,8 @@ TBAMD_EXPORT int32_t tbmi_set_rank16_plan(intptr_t runner, int32_t rowsPerBlock,
  * Results do not depend on it.  No counterpart in the reference (its GPU schedules cache trees with cooperative
  * loads, src/gpu/GPURepresentations.cpp:279-399). */
 TBAMD_EXPORT int32_t tbmi_set_group_staging(intptr_t runner, int32_t mode);
+/* The launch plan as `name=value` pairs; `batchKernel` names what a call of the compiled batch runs (few_rows, rank_stream,
+ * rows_lds_split, or the plan's own kernel), `walkTile` the nodes per tile the kernel walks.  Returns the full length. */
 TBAMD_EXPORT int32_t tbmi_describe_plan(intptr_t runner, char *buffer, int32_t length);
 /* Compile once, reload: saves the compiled model (forest + launch plan) of a runner to one file and
  * reopens it without the source model (batchSize <= 0 keeps the saved batch size).  Stands in for

@@ -420,7 +420,13 @@ void WholeBatch(const Case &c) {
     };
     check(tbmi_run_device_async(runner, dx, dout, rows, nullptr), "async, default stream");
     check(tbmi_run_device_async(runner, dx, dout, rows, other), "async, another stream");
+    const long few = shimFewRows, splits = shimSplits, streams = shimStreams;
     check(tbmi_run_device(runner, dx, dout, rows), "run_device");
+    const std::string ran = shimFewRows > few ? "few_rows" : shimStreams > streams ? "rank_stream" : shimSplits > splits ? "rows_lds_split" : "";
+    const std::string said = Describe(runner).substr(Describe(runner).find("batchKernel=") + std::strlen("batchKernel="));
+    EXPECT(ran.empty() ? said.compare(0, 9, "few_rows ") && said.compare(0, 12, "rank_stream ") && said.compare(0, 15, "rows_lds_split ")
+                       : said.compare(0, ran.size() + 1, ran + " ") == 0,
+           "batchKernel=%s, but the call ran %s", said.c_str(), ran.c_str());
     check(tbmi_run_device_async(runner, dx, dout, rows, nullptr), "async, default stream again");
     check(tbmi_run_device_noalloc(runner, dx, dout, rows, other), "noalloc");
     MulticlassOutputs(c, runner, dx, rows);

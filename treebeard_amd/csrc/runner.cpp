@@ -1009,6 +1009,17 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
   return bestMs;
 }
 
+const char *InferenceRunner::KernelOfBatch() const {
+  const LaunchPlan &p = m_model.plan;
+  const int64_t rows = m_options.batchSize;
+  if (TakesFewRows(rows)) return "few_rows";
+  if (StreamsBundles()) return "rank_stream";
+  if (SplitBlocks(rows) > 0) return "rows_lds_split";
+  if (p.kernel == LaunchPlan::Kernel::kTreeParallel) return "tree_parallel";
+  if (p.kernel == LaunchPlan::Kernel::kGlobalWalk) return "global_walk";
+  return p.WalkTile() > 1 ? "rows_tiled" : "rows_lds";
+}
+
 std::string InferenceRunner::DescribePlan() const {
   std::ostringstream os;
   const LaunchPlan &p = m_model.plan;
@@ -1034,11 +1045,11 @@ std::string InferenceRunner::DescribePlan() const {
      << " offsetsInWords=" << (p.featureOffsetInWords ? 1 : 0) << " quantizedRows=" << (p.quantizedRows ? 1 : 0) << " rankRows16=" << (p.rankRows16 ? 1 : 0)
      << " groups=" << m_model.groups.size()
      << " bundles=" << m_model.bundles.size() << " nodes=" << m_model.nodes.size()
-     << " ldsBytes=" << m_model.LdsBytes() << " tileSize=" << p.tileSize << " tiling=" << p.tiling
+     << " ldsBytes=" << m_model.LdsBytes() << " tileSize=" << p.tileSize << " tiling=" << p.tiling << " walkTile=" << p.WalkTile()
      << " staging=" << (DirectStaging() ? "direct" : "registers")
      << " peelWalks=" << peel << " treesTiledByProfile=" << m_model.treesTiledByProfile
      << " lockStepSteps=" << m_model.lockStepSteps << " profiledSteps=" << m_model.profiledSteps
-     << " fewRowsLimit=" << m_fewRowsLimit
+     << " batchKernel=" << KernelOfBatch() << " fewRowsLimit=" << m_fewRowsLimit
      << " treesDeferred=" << m_model.treesDeferred << " deferredEntriesPerRow=" << m_model.deferredEntriesPerRow;
   return os.str();
 }

@@ -105,6 +105,7 @@ public:
   const PackedModel &Model() const { return m_model; }
   const Forest &GetForest() const { return m_forest; }
   const HitCountProfile *Profile() const { return m_profile.get(); }
+  // The launch plan, and (`batchKernel`) what a call of the compiled batch runs: the plan's kernel or a form beside it.
   std::string DescribePlan() const;
   hipStream_t Stream() const { return m_stream; }
 
@@ -151,6 +152,7 @@ private:
   // The walk behind PrepareRows, with its outputs set; true when the finalize kernel (`f`) has to follow.
   bool LaunchWalkFor(const float *walkInputs, int64_t rows, FinalizeParams &f, int32_t *leafIds, hipStream_t stream, const Workspace &ws,
                      hipEvent_t done);
+  const char *KernelOfBatch() const;
   bool NeedsFinalize() const { return m_model.plan.treeSlices > 1 || m_forest.numClasses > 0; }
   // Classifier, one tree slice, row-parallel LDS kernel: the walk kernel can store the class id itself.
   bool FusesArgmax() const {
