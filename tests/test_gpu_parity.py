@@ -58,6 +58,41 @@ def is_multiclass(path, kind, num_features):
     return info[2] > 0
 
 
+def pin_own_plan(runner):
+    """Pins the launch plan the runner already has: its kernels then predict, where batches of a few rows and wide rows
+    otherwise run forms of their own."""
+    plan = dict(item.split("=", 1) for item in runner.describe_plan().split())
+    if plan["peelWalks"] != "0":
+        return                                        # (peeled walks run the plan's kernels on every batch)
+    rows, threads, lanes, k, group, slices = (int(plan[n]) for n in ("rowsPerBlock", "treeThreads", "treeLanes", "interleave", "groupBytes",
+                                                                     "treeSlices"))
+    if plan["kernel"] == "tree_parallel":
+        if plan["tileSize"] != "1":
+            return                                    # (uniform tiles on scalar nodes: setters take what tiles can walk)
+        runner.set_tree_parallel_plan(rows, lanes, k, group, slices)
+    elif plan["kernel"] == "global_walk":
+        if plan["tileSize"] != "1":
+            return
+        runner.set_global_walk_plan(rows, k, slices)
+    elif plan["quantizedRows"] == "1":
+        runner.set_quantized_plan(threads, k, group, slices)
+    else:
+        runner.set_plan(rows, threads, k, group, slices)
+    pinned = dict(item.split("=", 1) for item in runner.describe_plan().split())
+    assert pinned["batchKernel"] in ("rows_lds", "rows_lds_split", "rows_tiled", "tree_parallel", "global_walk"), pinned
+    same = ("kernel", "rowsPerBlock", "treeThreads", "treeLanes", "interleave", "groupBytes", "treeSlices", "quantizedRows", "walkTile")
+    assert [pinned[n] for n in same] == [plan[n] for n in same]
+
+
+def even_profile(path, forest):
+    """A hit-count profile that visits every leaf once: no tree is skewed, so its tiles are the uniform ones, walked as tiles."""
+    leaves = [int((forest.tree(t)[2] == -1).sum()) for t in range(forest.num_trees)]
+    with open(path, "w") as fh:
+        fh.write("%d, %d\n" % (forest.num_trees, max(leaves)))
+        fh.writelines(", ".join(["1, 0"] * n) + "\n" for n in leaves)
+    return str(path)
+
+
 def gpu_predict(runner, x):
     dx = torch.from_numpy(np.ascontiguousarray(x, dtype=np.float32)).cuda()
     rows = x.shape[0]
@@ -331,6 +366,8 @@ def test_small_batches_pick_the_tree_parallel_kernel(synth_model, k, rows):
     runner = make_runner(synth_model(k), rows)
     assert "kernel=tree_parallel" in runner.describe_plan()
     check_against_oracle(runner, forest, x)
+    pin_own_plan(runner)
+    check_against_oracle(runner, forest, x)
 
 
 def coarse_model(path, num_features, num_trees, num_class, seed):
@@ -514,7 +551,7 @@ def test_row_staging_alignment_and_ragged_tails(tmp_path, rows, features, offset
     flat = torch.zeros(rows * features + 8, dtype=torch.float32, device="cuda")
     flat[offset:offset + rows * features] = torch.from_numpy(x.reshape(-1)).cuda()
     out = torch.zeros(rows, dtype=torch.float32, device="cuda")
-    for setup in (lambda r: None, lambda r: r.set_plan(64, 2, 2, 16384, 1), lambda r: r.set_tree_parallel_plan(4, 16, 1, 16384, 1)):
+    for setup in (lambda r: None, pin_own_plan, lambda r: r.set_plan(64, 2, 2, 16384, 1), lambda r: r.set_tree_parallel_plan(4, 16, 1, 16384, 1)):
         runner = make_runner(path, rows)
         setup(runner)
         out.fill_(float("nan"))
@@ -712,8 +749,10 @@ def test_class_ties_go_to_the_larger_class_id(tmp_path, slices, tile_size):
     forest = model_io.load_xgboost_json(path)
     rows = 900
     x = rng.normal(size=(rows, 4)).astype(np.float32)
-    runner = make_tiled_runner(path, rows, tile_size, multiclass=True)
+    runner = make_tiled_runner(path, rows, tile_size, int(tile_size > 1), even_profile(tmp_path / "even.csv", forest) if tile_size > 1 else "",
+                               multiclass=True)
     runner.set_plan(64, 2, 2, 4096, slices)
+    assert " walkTile=%d " % tile_size in runner.describe_plan()
     _, sums = cpu_oracle.predict(forest, x)
     voted = np.isin(np.arange(6), info)
     margins = np.where(voted[None, :], sums, forest.initial_value).astype(np.float32)
@@ -752,6 +791,8 @@ def test_automatic_plan_over_feature_counts(tmp_path, features, rows, fine):
         assert ("quantizedRows=1" in plan) == (not fine), plan
     if features >= 3000:                                    # not even rank rows fit: a few f32 rows per block
         assert "kernel=tree_parallel" in plan, plan
+    check_against_oracle(runner, forest, x)
+    pin_own_plan(runner)
     check_against_oracle(runner, forest, x)
 
 
@@ -875,6 +916,8 @@ def test_random_forests_and_plans(tmp_path, seed):
     runner = make_runner(path, rows, gpu_options=gpu)
     runner.set_group_staging(int(rng.integers(0, 3)))     # tree groups by rule, through registers, or copied directly
     check_against_oracle(runner, forest, x)
+    pin_own_plan(runner)
+    check_against_oracle(runner, forest, x)
     kind = rng.integers(0, 5)
     try:
         if kind == 4:
@@ -919,6 +962,8 @@ def test_random_forests_tiles_and_peeled_walks(tmp_path, seed):
     except RuntimeError as error:        # rows too wide for the tiled walk's row tile
         assert tile > 1 and "tile" in str(error), str(error)
         return
+    check_against_oracle(runner, forest, x)
+    pin_own_plan(runner)
     check_against_oracle(runner, forest, x)
     if tile == 1 and rng.random() < 0.5:
         fresh = make_runner(path, rows)
@@ -1039,50 +1084,62 @@ def write_profile(path, forest, ids):
 
 @pytest.mark.parametrize("tile_size", [2, 3, 4, 5, 7, 8])
 @pytest.mark.parametrize("k,rows", [(1, 1024), (2, 4096), (3, 4096), (5, 2048)])
-def test_tiled_walk_selects_the_scalar_walks_leaves(synth_model, k, rows, tile_size):
-    """Set_tileSize > 1 runs the tiled kernel; its leaves are those of the scalar oracle and of the tiled CPU walk."""
+def test_tiled_walk_selects_the_scalar_walks_leaves(synth_model, tmp_path, k, rows, tile_size):
+    """The tiled kernel, which a profile asks for, and the scalar walk of uniform tiles: the leaves are those of the scalar
+    oracle and of the tiled CPU walk."""
     forest = model_io.load_xgboost_json(synth_model(k))
     x = synth.CONFIGS[k].batch_rows(rows, seed_offset=4)
-    runner = make_tiled_runner(synth_model(k), rows, tile_size, multiclass=k == 3)
-    assert " tileSize=%d " % tile_size in runner.describe_plan()
-    ids = gpu_leaf_ids(runner, x)
-    np.testing.assert_array_equal(ids, cpu_oracle.leaf_ids(forest, x))
-    np.testing.assert_array_equal(ids, cpu_oracle.TiledForest(forest, tile_size).leaf_ids(x))
-    check_against_oracle(runner, forest, x)
+    tiled_ids = cpu_oracle.TiledForest(forest, tile_size).leaf_ids(x)
+    for profile in ("", even_profile(tmp_path / "even.csv", forest)):
+        runner = make_tiled_runner(synth_model(k), rows, tile_size, 1 if profile else 0, profile, multiclass=k == 3)
+        plan = runner.describe_plan()
+        assert " tileSize=%d " % tile_size in plan and " walkTile=%d " % (tile_size if profile else 1) in plan and " treesTiledByProfile=0 " in plan
+        ids = gpu_leaf_ids(runner, x)
+        np.testing.assert_array_equal(ids, cpu_oracle.leaf_ids(forest, x))
+        np.testing.assert_array_equal(ids, tiled_ids)
+        check_against_oracle(runner, forest, x)
+        pin_own_plan(runner)
+        check_against_oracle(runner, forest, x)
 
 
 @pytest.mark.parametrize("tile_size", [2, 4, 8])
-def test_tiled_walk_on_the_reference_fixtures(plain_file, tile_size):
+def test_tiled_walk_on_the_reference_fixtures(plain_file, tmp_path, tile_size):
     for name in BENCHMARK_XGB:
         path = plain_file(benchmark_model(name))
         data = np.loadtxt(benchmark_csv(name), delimiter=",", dtype=np.float64)
         x, expected = data[:, :-1].astype(np.float32), data[:, -1]
         forest = model_io.load_xgboost_json(path)
-        runner = make_tiled_runner(path, x.shape[0], tile_size)
-        np.testing.assert_array_equal(gpu_leaf_ids(runner, x), cpu_oracle.leaf_ids(forest, x))
-        np.testing.assert_allclose(gpu_predict(runner, x), expected, rtol=RTOL_SUM, atol=ATOL_PROB)
+        for profile in ("", even_profile(tmp_path / "even.csv", forest)):
+            runner = make_tiled_runner(path, x.shape[0], tile_size, 1 if profile else 0, profile)
+            pin_own_plan(runner)
+            assert " walkTile=%d " % (tile_size if profile else 1) in runner.describe_plan()
+            np.testing.assert_array_equal(gpu_leaf_ids(runner, x), cpu_oracle.leaf_ids(forest, x))
+            np.testing.assert_allclose(gpu_predict(runner, x), expected, rtol=RTOL_SUM, atol=ATOL_PROB)
     for path in random_models()[::4]:
         forest = model_io.load_xgboost_json(path)
         x = np.random.default_rng(tile_size).random((777, forest.num_features), dtype=np.float32)
-        runner = make_tiled_runner(path, 777, tile_size)
-        np.testing.assert_array_equal(gpu_leaf_ids(runner, x), cpu_oracle.leaf_ids(forest, x))
-        np.testing.assert_array_equal(gpu_leaf_ids(runner, x), cpu_oracle.TiledForest(forest, tile_size).leaf_ids(x))
+        for profile in ("", even_profile(tmp_path / "even.csv", forest)):
+            runner = make_tiled_runner(path, 777, tile_size, 1 if profile else 0, profile)
+            np.testing.assert_array_equal(gpu_leaf_ids(runner, x), cpu_oracle.leaf_ids(forest, x))
+            np.testing.assert_array_equal(gpu_leaf_ids(runner, x), cpu_oracle.TiledForest(forest, tile_size).leaf_ids(x))
 
 
 @pytest.mark.parametrize("plan", [(64, 1, 1, 16384, 1), (128, 8, 2, 32768, 3), (256, 4, 4, 40960, 2), (64, 16, 2, 24576, 5)])
 @pytest.mark.parametrize("tile_size", [2, 3, 4, 6, 8])
-def test_tiled_launch_plans_agree(synth_model, tile_size, plan):
+def test_tiled_launch_plans_agree(synth_model, tmp_path, tile_size, plan):
     forest = model_io.load_xgboost_json(synth_model(2))
     x = synth.CONFIGS[2].batch_rows(1501, seed_offset=6)
     x[3, :] = np.inf
     x[4, :] = -np.inf
     x[5, :] = np.nan
-    runner = make_tiled_runner(synth_model(2), 1501, tile_size)
     if tile_size > 4 and plan[3] < 24576:        # the biggest tree of this model takes 18 KB in 64-byte tiles
         plan = (128, 2, 1, 32768, 1)
-    runner.set_plan(*plan)
-    assert " tileSize=%d " % tile_size in runner.describe_plan()
-    check_against_oracle(runner, forest, x)
+    for profile in ("", even_profile(tmp_path / "even.csv", forest)):
+        runner = make_tiled_runner(synth_model(2), 1501, tile_size, 1 if profile else 0, profile)
+        runner.set_plan(*plan)
+        assert " tileSize=%d " % tile_size in runner.describe_plan()
+        assert " walkTile=%d " % (tile_size if profile else 1) in runner.describe_plan()
+        check_against_oracle(runner, forest, x)
 
 
 def test_tile_sizes_the_kernels_do_not_walk_are_refused(synth_model):
@@ -1091,8 +1148,10 @@ def test_tile_sizes_the_kernels_do_not_walk_are_refused(synth_model):
     with pytest.raises(RuntimeError, match="row tile below 64 KB"):
         make_tiled_runner(synth_model(4), 64, 2)          # 2000 features: no tiled row tile
     runner = make_tiled_runner(synth_model(1), 64, 2)
-    with pytest.raises(RuntimeError, match="row-parallel kernel"):
-        runner.set_tree_parallel_plan(4, 64, 1, 0, 1)
+    for refused in (lambda: runner.set_tree_parallel_plan(4, 64, 1, 0, 1), lambda: runner.set_global_walk_plan(256, 4, 1),
+                    lambda: runner.set_quantized_plan(8, 4, 0, 1), lambda: runner.set_rank16_plan(64, 4, 4, 0, 1)):
+        with pytest.raises(RuntimeError, match="row-parallel kernel"):
+            refused()
 
 
 @pytest.mark.parametrize("tile_size,tiling_type,peel", [(4, 1, True), (4, 2, False), (2, 1, True), (3, 2, True), (1, 1, True)])

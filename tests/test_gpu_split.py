@@ -1,6 +1,6 @@
-"""Row blocks x tree groups split evenly over the blocks of a launch and finished in it: rows around the edges of row
-blocks and of rounds of blocks, tree slices, classifiers with and without sums, and repeated calls (the tickets of one
-call are the next one's)."""
+"""Row blocks x tree groups split evenly over the blocks of a launch, the parts added by the finalize kernel: rows around
+the edges of row blocks and of rounds of blocks, tree slices, classifiers with and without sums, repeated calls (the parts
+of one call lie where the last one's did)."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,7 @@ from oracle import cpu_oracle, model_io  # noqa: E402
 from treebeard_amd import synth  # noqa: E402
 
 from test_gpu_few_rows import close  # noqa: E402
-from test_gpu_parity import ATOL_PROB, RTOL_SUM, gpu_predict, make_runner  # noqa: E402
+from test_gpu_parity import ATOL_PROB, RTOL_SUM, gpu_predict, make_runner, pin_own_plan  # noqa: E402
 
 
 @pytest.mark.parametrize("plan", [(64, 16, 4, 16384, 2), (64, 4, 2, 8192, 5), (128, 8, 4, 32768, 3), (256, 4, 8, 16384, 1), (256, 2, 1, 40960, 4)])
@@ -57,5 +57,7 @@ def test_wide_rows_split_on_rank_tiles(synth_model):
         runner = make_runner(synth_model(4), batch)
         x = synth.CONFIGS[4].batch_rows(batch, seed_offset=6)
         expected = cpu_oracle.predict(forest, x, threads=8)[0]
-        for rows in (batch, batch - 1, 1000):
-            close(forest, gpu_predict(runner, x[:rows]), expected[:rows])
+        for pin in (lambda r: None, pin_own_plan):          # streamed bundles, then the rank tiles of the plan
+            pin(runner)
+            for rows in (batch, batch - 1, 1000):
+                close(forest, gpu_predict(runner, x[:rows]), expected[:rows])
