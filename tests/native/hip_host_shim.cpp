@@ -6,8 +6,9 @@
 // model on the CPU with the kernels' addressing rules (group-relative node addresses, pre-multiplied
 // feature offsets, rank tiles, per-class partial sums, tree slices, finalize), reading every input and
 // writing every output element the kernels touch: a buffer sized or indexed wrongly by the host code is
-// reported by the sanitizer, and a wrongly packed model gives wrong predictions.  A wait for an event that nothing has
-// recorded since the last wait ends the run.  Test infrastructure only.
+// reported by the sanitizer, and a wrongly packed model gives wrong predictions.  An asynchronous copy happens no sooner
+// than its stream is waited for or has something behind it, so a buffer that is given up too early shows; a wait for an event
+// that nothing has recorded since the last wait ends the run.  Test infrastructure only.
 #include "kernels.h"
 
 #include <algorithm>
@@ -22,6 +23,30 @@ namespace {
 std::mutex gMutex;
 std::map<const void *, std::pair<size_t, bool>> gAllocations; // pointer -> (bytes, pinned host)
 hipError_t gLastError = hipSuccess;
+
+struct Copy {
+  void *dst;
+  const void *src;
+  size_t bytes;
+};
+struct Stream {
+  long queued = 0, waited = 0; // pieces of work handed over, and how many of them the host has waited for
+  std::vector<Copy> copies;    // still to be done
+};
+std::map<hipStream_t, Stream> gStreams;
+struct Event {
+  bool recorded = false; // ... and not waited for since
+  hipStream_t stream = nullptr;
+  long at = 0;
+};
+Event &EventOf(hipEvent_t event) { return *reinterpret_cast<Event *>(event); }
+
+// (with gMutex held)
+void DoCopies(Stream &stream) {
+  for (const Copy &c : stream.copies)
+    if (c.bytes) std::memcpy(c.dst, c.src, c.bytes);
+  stream.copies.clear();
+}
 
 hipError_t Fail(hipError_t e) {
   gLastError = e;
@@ -45,6 +70,7 @@ hipError_t hipFree(void *ptr) {
   if (!ptr) return hipSuccess;
   {
     std::lock_guard<std::mutex> lock(gMutex);
+    for (auto &stream : gStreams) DoCopies(stream.second); // (the runtime waits too)
     if (!gAllocations.erase(ptr)) return Fail(hipErrorInvalidValue);
   }
   std::free(ptr);
@@ -67,8 +93,10 @@ hipError_t hipMemcpy(void *dst, const void *src, size_t bytes, hipMemcpyKind) {
   return hipSuccess;
 }
 
-hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind, hipStream_t) {
-  if (bytes) std::memcpy(dst, src, bytes);
+hipError_t hipMemcpyAsync(void *dst, const void *src, size_t bytes, hipMemcpyKind, hipStream_t stream) {
+  std::lock_guard<std::mutex> lock(gMutex);
+  ++gStreams[stream].queued;
+  gStreams[stream].copies.push_back(Copy{dst, src, bytes});
   return hipSuccess;
 }
 
@@ -89,30 +117,47 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *stream, unsigned int) {
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t stream) {
+  {
+    std::lock_guard<std::mutex> lock(gMutex);
+    DoCopies(gStreams[stream]);
+    gStreams.erase(stream);
+  }
   delete reinterpret_cast<int *>(stream);
   return hipSuccess;
 }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t stream) {
+  std::lock_guard<std::mutex> lock(gMutex);
+  Stream &s = gStreams[stream];
+  DoCopies(s);
+  s.waited = s.queued;
+  return hipSuccess;
+}
 hipError_t hipStreamWaitEvent(hipStream_t, hipEvent_t event, unsigned int) {
-  if (*reinterpret_cast<int *>(event) == 0) std::abort(); // orders nothing
+  if (!EventOf(event).recorded) std::abort(); // orders nothing
   return hipSuccess;
 }
 hipError_t hipEventCreate(hipEvent_t *event) {
-  *event = reinterpret_cast<hipEvent_t>(new int(0)); // (1: recorded, and not waited for since)
+  *event = reinterpret_cast<hipEvent_t>(new Event);
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t *event, unsigned) { return hipEventCreate(event); }
 hipError_t hipEventDestroy(hipEvent_t event) {
-  delete reinterpret_cast<int *>(event);
+  delete &EventOf(event);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t event, hipStream_t) {
-  *reinterpret_cast<int *>(event) = 1;
+hipError_t hipEventRecord(hipEvent_t event, hipStream_t stream) {
+  std::lock_guard<std::mutex> lock(gMutex);
+  DoCopies(gStreams[stream]);
+  EventOf(event) = Event{true, stream, gStreams[stream].queued};
   return hipSuccess;
 }
 hipError_t hipEventSynchronize(hipEvent_t event) {
-  if (*reinterpret_cast<int *>(event) == 0) std::abort(); // waits for nothing
-  *reinterpret_cast<int *>(event) = 0;
+  std::lock_guard<std::mutex> lock(gMutex);
+  Event &e = EventOf(event);
+  if (!e.recorded) std::abort(); // waits for nothing
+  e.recorded = false;
+  const auto stream = gStreams.find(e.stream);
+  if (stream != gStreams.end()) stream->second.waited = std::max(stream->second.waited, e.at);
   return hipSuccess;
 }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
@@ -147,6 +192,14 @@ hipError_t hipGetLastError(void) {
   return e;
 }
 
+// Streams with work that nobody has waited for, the default stream and `except` left out.
+int shimBusyStreams(hipStream_t except) {
+  std::lock_guard<std::mutex> lock(gMutex);
+  int busy = 0;
+  for (const auto &stream : gStreams) busy += stream.first && stream.first != except && stream.second.waited < stream.second.queued;
+  return busy;
+}
+long shimLaunchesToGo = -1; // launches until one fails (negative: none does)
 long shimFewRows = 0, shimSplits = 0, shimStreams = 0; // launches of the forms that stand beside the launch plans' kernels
 
 } // extern "C"
@@ -161,7 +214,15 @@ uint32_t Bits(float v) {
   return u;
 }
 
-// What every launcher does with its parameters' event.
+// A kernel starts behind its stream's copies ...
+bool Refused(hipStream_t stream) {
+  std::lock_guard<std::mutex> lock(gMutex);
+  if (shimLaunchesToGo >= 0 && shimLaunchesToGo-- == 0) return true;
+  DoCopies(gStreams[stream]);
+  ++gStreams[stream].queued;
+  return false;
+}
+// ... and records its parameters' event when it is done.
 hipError_t Launched(hipEvent_t done, hipStream_t stream) { return done ? hipEventRecord(done, stream) : hipSuccess; }
 
 // One row through groups [gBegin, gEnd) of an LDS-layout model.  `stride` is the node-offset distance between
@@ -317,6 +378,7 @@ hipError_t WalkLds(const WalkParams &p, int K, uint32_t stride, int rankRows, hi
 
 hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, size_t ldsBytes, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   const int RB = p.s.rowsPerBlock, TT = p.s.treeThreads;
   if (ldsBytes > 160 * 1024 || RB < 64 || (RB & (RB - 1)) || TT < 1 || RB * TT > 1024) return hipErrorInvalidValue;
   if (p.s.treeSlices < 1 || p.s.treeSlices > 65535) return hipErrorInvalidValue;
@@ -389,6 +451,7 @@ uint32_t TileStepHost(const unsigned char *group, uint32_t groupBytes, uint32_t 
 
 hipError_t LaunchWalkRowsTiled(const WalkParams &p, int tileSize, int interleave, size_t ldsBytes, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   const int RB = p.s.rowsPerBlock, TT = p.s.treeThreads, T = tileSize, K = interleave;
   if (ldsBytes > 160 * 1024 || RB < 64 || (RB & (RB - 1)) || TT < 1 || RB * TT > 1024) return hipErrorInvalidValue;
   if ((int64_t)(p.s.numFeatures + 1) * RB * 4 > 0x10000) return hipErrorInvalidValue;
@@ -437,6 +500,7 @@ hipError_t LaunchWalkRowsTiled(const WalkParams &p, int tileSize, int interleave
 
 hipError_t LaunchWalkTreeParallel(const WalkParams &p, int interleave, size_t ldsBytes, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   if (ldsBytes > 160 * 1024 || p.s.rowsPerBlock < 1 || p.s.treeLanes < 1) return hipErrorInvalidValue;
   const int threads = p.s.rowsPerBlock * p.s.treeLanes;
   if (threads > 1024 || threads % 64 != 0) return hipErrorInvalidValue;
@@ -447,6 +511,7 @@ hipError_t LaunchWalkTreeParallel(const WalkParams &p, int interleave, size_t ld
 
 hipError_t LaunchWalkGlobal(const WalkParams &p, int interleave, hipStream_t stream) {
   if (p.s.rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   const int threads = p.s.rowsPerBlock;
   if (threads < 64 || threads > 1024 || threads % 64 != 0) return hipErrorInvalidValue;
   if (interleave != 1 && interleave != 2 && interleave != 4 && interleave != 8) return hipErrorInvalidValue;
@@ -474,8 +539,9 @@ hipError_t LaunchWalkGlobal(const WalkParams &p, int interleave, hipStream_t str
 }
 
 hipError_t LaunchBinRows(const float *x, const float *table, uint8_t *ranks, int64_t rows, int numFeatures, int tableDepth,
-                         int chunkFeatures, hipStream_t) {
+                         int chunkFeatures, hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   if (chunkFeatures != 64) return hipErrorInvalidValue;
   if (tableDepth < 1 || tableDepth > 255 || ((tableDepth + 1) & tableDepth)) return hipErrorInvalidValue;
   const int64_t rowBlocks = (rows + 63) / 64;
@@ -495,8 +561,9 @@ hipError_t LaunchBinRows(const float *x, const float *table, uint8_t *ranks, int
 
 hipError_t LaunchRankRows16(const float *x, const float *tables, const RankFeatureDesc *features, const RankChunkDesc *chunks,
                             int numChunks, uint32_t maxChunkEntries, uint32_t maxChunkFeatures, uint16_t *ranks, int64_t rows,
-                            int numFeatures, int rowsPerBlock, hipStream_t) {
+                            int numFeatures, int rowsPerBlock, hipStream_t stream) {
   if (rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   if (numChunks < 1 || (size_t)maxChunkEntries * 4 + (size_t)maxChunkFeatures * 1025 * 4 + 16 > 160 * 1024 || rowsPerBlock < 64 ||
       rowsPerBlock % 64 != 0)
     return hipErrorInvalidValue;
@@ -558,6 +625,7 @@ float FinishMargin(double margin, int transform) { return (float)(transform == 1
 
 hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   const int C = p.numClasses, Cn = std::max(1, C);
   std::vector<double> sums((size_t)Cn);
   for (int64_t row = 0; row < p.rows; ++row) {
@@ -581,6 +649,7 @@ hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
 // blocks (heap memory here) all show.
 hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   const FewRowsShape s = ShapeOfFewRows(p.rows, p.numFeatures, p.numTrees, p.numClasses);
   if (p.numTrees < 1 || s.ldsBytes > kFewRowsLds) return hipErrorInvalidValue;
   if (p.numClasses == 0 ? !p.out : !(p.out || p.classOut || p.margins || p.probabilities)) return hipErrorInvalidValue;
@@ -632,6 +701,7 @@ hipError_t LaunchFewRows(const FewRowsParams &p, hipStream_t stream) {
 
 hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
+  if (Refused(stream)) return hipErrorLaunchFailure;
   const int waves = StreamWaves(p.numFeatures), F = p.numFeatures;
   if (waves < 1 || F > kStreamMaxFeatures || p.numBundles < 1 || (p.chains != 2 && p.chains != 4) || p.slices < 1 || p.slices > 65535)
     return hipErrorInvalidValue;

@@ -19,7 +19,8 @@
 #include <string>
 #include <vector>
 
-extern "C" long shimFewRows, shimSplits, shimStreams; // hip_host_shim.cpp
+extern "C" long shimFewRows, shimSplits, shimStreams, shimLaunchesToGo; // hip_host_shim.cpp
+extern "C" int shimBusyStreams(hipStream_t except);
 
 namespace {
 
@@ -105,7 +106,8 @@ struct Case {
   int64_t rows = 0;
 };
 
-void Compare(const Case &c, const float *got, int64_t first, int64_t rows, const char *what) {
+void Compare(const Case &c, const float *got, int64_t first, int64_t rows, const char *what, hipStream_t mine = nullptr) {
+  EXPECT(shimBusyStreams(mine) == 0, "%s returned with work under way", what);
   int64_t bad = 0;
   for (int64_t r = 0; r < rows; ++r) bad += !Close(got[r], c.expected[first + r]);
   EXPECT(bad == 0, "%s: %lld of %lld rows differ (%s)", what, (long long)bad, (long long)rows, c.path.c_str());
@@ -390,6 +392,34 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
   (void)hipFree(dids);
 }
 
+// Host calls whose n-th launch fails, of one piece and of several: nothing of theirs is under way when they return, and the
+// next call is right.
+void FailedCalls(const Case &c) {
+  const int64_t F = c.forest.numFeatures;
+  for (int64_t rows : {std::min<int64_t>(c.rows, 100), std::min<int64_t>(c.rows, 1500), c.rows}) {
+    const intptr_t runner = MakeRunner(c, (int32_t)rows, false);
+    if (!runner) continue;
+    PinOwnPlan(runner);
+    std::vector<float> out((size_t)rows);
+    void *locked = nullptr;
+    EXPECT(hipHostMalloc(&locked, (size_t)rows * F * sizeof(float), 0) == hipSuccess, "hipHostMalloc");
+    std::memcpy(locked, c.x.data(), (size_t)rows * F * sizeof(float));
+    for (const void *in : {static_cast<const void *>(c.x.data()), static_cast<const void *>(locked)})
+      for (long n = 0; n < 6; ++n) {
+        shimLaunchesToGo = n;
+        const int32_t rc = tbmi_run_host(runner, in, out.data(), rows);
+        EXPECT((rc != 0) == (shimLaunchesToGo < 0), "a failed launch is an error");
+        shimLaunchesToGo = -1;
+        EXPECT(shimBusyStreams(nullptr) == 0, "%lld rows, launch %ld failed: work under way", (long long)rows, n);
+        std::fill(out.begin(), out.end(), -1.f);
+        EXPECT(tbmi_run_host(runner, in, out.data(), rows) == 0, "the call after a failed one");
+        Compare(c, out.data(), 0, rows, "the call after a failed one");
+      }
+    (void)hipHostFree(locked);
+    DeleteInferenceRunner(runner);
+  }
+}
+
 // All of the case's rows in one device call through every entry point, on the default plan and on plans of several slices
 // (which a launch of many blocks splits evenly); calls on the default stream, another stream and the runner's own in turn.
 void WholeBatch(const Case &c) {
@@ -415,7 +445,7 @@ void WholeBatch(const Case &c) {
       EXPECT(rc == 0, "%s", what);
       std::vector<float> got((size_t)rows);
       for (int64_t r = 0; r < rows; ++r) got[r] = multiclass ? (float)(int8_t)dout[r] : reinterpret_cast<float *>(dout)[r];
-      Compare(c, got.data(), 0, rows, what);
+      Compare(c, got.data(), 0, rows, what, other);
       std::memset(dout, 0x5A, resultBytes);
     };
     check(tbmi_run_device_async(runner, dx, dout, rows, nullptr), "async, default stream");
@@ -517,6 +547,7 @@ int main(int argc, char **argv) {
     HostEntryPoints(c);
     HostEntryPoints(c, true);
     WholeBatch(c);
+    FailedCalls(c);
     DeviceEntryPoints(c, std::min<int64_t>(c.rows, 203));
     if (!Quick()) {
       const std::string profile =

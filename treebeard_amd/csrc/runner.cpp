@@ -732,10 +732,22 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
     return;
   }
   EnsureStaging(rows);
+  struct EndCall { // (an error leaves while rows and kernels are on their way, from and to memory of the caller's or of the next call's)
+    InferenceRunner *runner;
+    ~EndCall() {
+      if (runner->m_copier) runner->m_copier->Finish();
+      if (!failed) return;
+      for (hipStream_t stream : runner->m_hostStreams)
+        if (stream) (void)hipStreamSynchronize(stream);
+      (void)hipStreamSynchronize(runner->m_stream);
+    }
+    bool failed = true;
+  } endCall{this};
   if (gMeasureGpuKernelTime) {
     Check(hipMemcpyAsync(m_dStageIn, hostInputs, totalBytes, hipMemcpyHostToDevice, m_stream), "copy inputs");
     RunDevice(m_dStageIn, m_dStageOut, rows);
     Check(hipMemcpy(hostResults, m_dStageOut, (size_t)rows * ReturnTypeBytes(), hipMemcpyDeviceToHost), "copy results");
+    endCall.failed = false;
     return;
   }
   // Rows go through in pieces: host threads move pageable rows into pinned memory (pinned ones are read where they lie),
@@ -746,16 +758,6 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
   EnsureHostSlots(pieces.count, pieces.most, staged);
   if (staged && !m_copier && totalBytes > kHostPartBytes)
     m_copier.reset(new ParallelCopier((int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()))));
-  struct EndCall { // (an error leaves while rows are on their way)
-    InferenceRunner *runner;
-    ~EndCall() {
-      if (runner->m_copier) runner->m_copier->Finish();
-      if (failed)
-        for (hipStream_t stream : runner->m_hostStreams)
-          if (stream) (void)hipStreamSynchronize(stream);
-    }
-    bool failed = true;
-  } endCall{this};
   const auto slotOf = [&](int64_t p) -> HostSlot & { return m_hostSlots[p % kHostSlots]; };
   const auto source = [&](int64_t p) { return static_cast<const char *>(hostInputs) + (size_t)pieces.Begin(p) * rowBytes; };
   const auto stageOf = [&](int64_t p) { return m_dStageIn + pieces.Begin(p) * m_forest.numFeatures; };
