@@ -1,4 +1,5 @@
-// The host-side arithmetic of kernels.h that the launchers and the runner share, over its whole range.
+// The host-side arithmetic that the launchers and the runner share (kernels.h, host_copy.h), over its whole range.
+#include "host_copy.h"
 #include "kernels.h"
 
 #include <cstdio>
@@ -67,7 +68,31 @@ static void Streams() {
   }
 }
 
+// Host batches: pieces follow each other without gaps, none is empty or larger than its buffer, a buffer's piece has been
+// drained before the next one is copied into it, and the buffers of a runner stay under 64 MB (four rows at least each).
+static void HostBatches() {
+  for (size_t features : {1, 3, 8, 28, 250, 1000, 1024, 1025, 2000, 3000, 4096, 5003, 16000, 16384, 16385, 20000, 65535, 300000, 1 << 20, 3000000})
+    for (int64_t scale = 1; scale <= 4096; scale += scale < 24 ? 1 : scale / 3)
+      for (int64_t extra : {-1, 0, 1, 63, 64, 255}) {
+        const size_t rowBytes = features * 4;
+        const int64_t step = HostPieces((int64_t)1 << 40, rowBytes).most, rows = scale * step / 8 + extra;
+        if (rows < 1) continue;
+        const HostPieces p(rows, rowBytes);
+        EXPECT(p.count >= 1 && p.slots >= 4 && p.slots <= kHostSlots && p.slots / 2 - 1 + 2 <= p.slots - 1, "%zu features %lld rows", features, (long long)rows);
+        EXPECT((size_t)(p.slots * p.most) * rowBytes <= (size_t)64 << 20 || p.most <= 4, "%zu features %lld rows: %lld buffers of %lld rows", features,
+               (long long)rows, (long long)p.slots, (long long)p.most);
+        int64_t end = 0;
+        for (int64_t i = 0; i < p.count; ++i) {
+          EXPECT(p.Begin(i) == end && p.Rows(i) >= 1 && p.Rows(i) <= p.most, "%zu features %lld rows, piece %lld: %lld rows", features, (long long)rows,
+                 (long long)i, (long long)p.Rows(i));
+          end = p.End(i);
+        }
+        EXPECT(end == rows, "%zu features %lld rows", features, (long long)rows);
+      }
+}
+
 int main() {
+  HostBatches();
   FewRows();
   SplitLines();
   Streams();

@@ -2,6 +2,7 @@
 // about 10 GB/s out of memory, less than the link to the device, so the host-buffer entry point hands
 // the rows of a call to a small pool that lives as long as the runner.
 #pragma once
+#include <algorithm>
 #include <atomic>
 #include <condition_variable>
 #include <cstddef>
@@ -12,6 +13,34 @@
 #include <vector>
 
 namespace tbamd {
+
+// How a host batch is cut: pieces of about 4 MB (73 us of the link, which cover the 10 us the calling thread needs for a piece),
+// at least 1024 rows (fewer take the kernels as long) as long as those fit 16 MB; a quarter and half a piece first, because
+// nothing overlaps their copies, and what is left at the end as two thirds and one third, because nothing overlaps the last
+// piece's kernels.  The pieces take turns in `slots` pinned buffers: eight of 4 MB, fewer of larger ones (four are what two
+// copies under way, a piece in its kernels and one being filled need), so that they pin 32 MB, 64 for the widest rows.
+constexpr size_t kHostPieceBytes = (size_t)4 << 20, kHostPartBytes = (size_t)1 << 20;
+constexpr int kHostSlots = 8;
+struct HostPieces {
+  int64_t rows, most, count; // `most`: rows of the largest piece
+  int64_t slots;
+  HostPieces(int64_t allRows, size_t rowBytes) : rows(allRows) {
+    const int64_t fit = (int64_t)((4 * kHostPieceBytes) / rowBytes);
+    most = std::min(std::max<int64_t>((int64_t)(kHostPieceBytes / rowBytes), 1024), fit);
+    most = most >= 256 ? most / 256 * 256 : std::max<int64_t>(4, most); // (rows of 4 MB and more: four of them)
+    slots = std::max<int64_t>(4, std::min<int64_t>(kHostSlots, (int64_t)(kHostSlots * kHostPieceBytes / ((size_t)most * rowBytes))));
+    if (rows <= most) most = rows, count = 1;
+    else count = 2 + (rows - most / 4 * 3 + most - 1) / most;
+  }
+  int64_t End(int64_t p) const {
+    if (p >= count - 1) return rows;
+    if (p == 0) return most / 4;
+    const int64_t begin = most / 4 * 3 + (p - 2) * most;
+    return p == count - 2 && p > 1 ? begin + std::min(most, ((rows - begin) * 2 / 3 + 63) / 64 * 64) : begin + most;
+  }
+  int64_t Begin(int64_t p) const { return p == 0 ? 0 : End(p - 1); }
+  int64_t Rows(int64_t p) const { return End(p) - Begin(p); }
+};
 
 class ParallelCopier {
 public:

@@ -405,7 +405,7 @@ void InferenceRunner::EnsureHostSlots(int64_t count, int64_t rows, bool staged) 
     Check(hipHostMalloc(&buffer, bytes, hipHostMallocDefault), "allocate pinned staging");
     have = bytes;
   };
-  for (int64_t i = 0; i < std::min<int64_t>(count, kHostSlots); ++i) {
+  for (int64_t i = 0; i < count; ++i) {
     HostSlot &slot = m_hostSlots[i];
     if (staged) grow(slot.rows, slot.rowBytes, (size_t)rows * m_forest.numFeatures * sizeof(float));
     grow(slot.results, slot.resultBytes, (size_t)rows * sizeof(float));
@@ -674,33 +674,9 @@ namespace {
 // Host batches up to this many bytes of rows are read by the kernel where they lie in pinned memory.
 constexpr size_t kSmallHostBytes = (size_t)512 << 10;
 
-// How a host batch is cut: pieces of about 4 MB (73 us of the link, which cover the 10 us this thread needs for a piece), at
-// least 1024 rows (fewer take the kernels as long) as long as those fit 16 MB; a quarter and half a piece first, because
-// nothing overlaps their copies, and what is left at the end as two thirds and one third, because nothing overlaps the last
-// piece's kernels.
-constexpr size_t kHostPieceBytes = (size_t)4 << 20, kHostPartBytes = (size_t)1 << 20;
 // Calls of this many bytes write the pinned buffers past the caches: the caches do not hold both the rows and the buffers
 // any more, and a line that is not read before it is written saves a third of the memory traffic.
 constexpr size_t kStreamedHostBytes = (size_t)16 << 20;
-struct HostPieces {
-  int64_t rows, most, count; // `most`: rows of the largest piece
-  HostPieces(int64_t allRows, size_t rowBytes) : rows(allRows) {
-    const int64_t fit = (int64_t)((4 * kHostPieceBytes) / rowBytes);
-    most = std::min(std::max<int64_t>((int64_t)(kHostPieceBytes / rowBytes), 1024), fit);
-    most = std::max<int64_t>(256, most / 256 * 256);
-    if (rows <= most) most = rows, count = 1;
-    else count = 2 + (rows - most / 4 * 3 + most - 1) / most;
-  }
-  int64_t End(int64_t p) const {
-    if (p >= count - 1) return rows;
-    if (p == 0) return most / 4;
-    const int64_t begin = most / 4 * 3 + (p - 2) * most;
-    return p == count - 2 && p > 1 ? begin + std::min(most, ((rows - begin) * 2 / 3 + 63) / 64 * 64) : begin + most;
-  }
-  int64_t Begin(int64_t p) const { return p == 0 ? 0 : End(p - 1); }
-  int64_t Rows(int64_t p) const { return End(p) - Begin(p); }
-};
-
 // True when the runtime knows the address as pinned (or registered) host memory, which DMA reads
 // directly; pageable memory makes the query fail, and that error must not linger.
 bool IsPinnedHost(const void *ptr) {
@@ -755,10 +731,10 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
   // the same time on different pieces.  Rows are independent, so the pieces give the same results as one launch.
   const HostPieces pieces(rows, rowBytes);
   const bool staged = !IsPinnedHost(hostInputs);
-  EnsureHostSlots(pieces.count, pieces.most, staged);
+  EnsureHostSlots(std::min<int64_t>(pieces.count, pieces.slots), pieces.most, staged);
   if (staged && !m_copier && totalBytes > kHostPartBytes)
     m_copier.reset(new ParallelCopier((int)std::min(8u, std::max(1u, std::thread::hardware_concurrency()))));
-  const auto slotOf = [&](int64_t p) -> HostSlot & { return m_hostSlots[p % kHostSlots]; };
+  const auto slotOf = [&](int64_t p) -> HostSlot & { return m_hostSlots[p % pieces.slots]; };
   const auto source = [&](int64_t p) { return static_cast<const char *>(hostInputs) + (size_t)pieces.Begin(p) * rowBytes; };
   const auto stageOf = [&](int64_t p) { return m_dStageIn + pieces.Begin(p) * m_forest.numFeatures; };
   const auto bytesOf = [&](int64_t p) { return (size_t)pieces.Rows(p) * rowBytes; };
@@ -786,7 +762,7 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
   }
   int64_t appended = 0, drained = 0;
   const auto append = [&] { // the pool runs ahead of this loop as far as there are free slots
-    for (; staged && appended < pieces.count && appended < drained + kHostSlots; ++appended)
+    for (; staged && appended < pieces.count && appended < drained + pieces.slots; ++appended)
       m_copier->Append(slotOf(appended).rows, source(appended), bytesOf(appended), totalBytes >= kStreamedHostBytes);
   };
   const auto drain = [&] {
@@ -819,7 +795,7 @@ void InferenceRunner::RunHostChunk(const void *hostInputs, void *hostResults, in
     HostSlot &slot = slotOf(p);
     Check(hipStreamSynchronize(m_hostStreams[p % kHostStreams]), "copy inputs");
     LaunchPredictions(stageOf(p), pieces.Rows(p), slot.results, m_stream, ws, slot.done);
-    if (p - drained >= kHostSlots / 2 - 1) drain();
+    if (p - drained >= pieces.slots / 2 - 1) drain();
   }
   while (drained < pieces.count) drain();
   endCall.failed = false;

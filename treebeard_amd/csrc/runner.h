@@ -187,7 +187,7 @@ private:
     size_t rowBytes = 0, resultBytes = 0;
     hipEvent_t done = nullptr;
   };
-  static constexpr int kHostSlots = 8, kHostStreams = 2;
+  static constexpr int kHostStreams = 2;
   HostSlot m_hostSlots[kHostSlots];
   hipStream_t m_hostStreams[kHostStreams] = {};
   std::unique_ptr<ParallelCopier> m_copier;
