@@ -75,9 +75,12 @@ static void HostBatches() {
     for (int64_t scale = 1; scale <= 4096; scale += scale < 24 ? 1 : scale / 3)
       for (int64_t extra : {-1, 0, 1, 63, 64, 255}) {
         const size_t rowBytes = features * 4;
-        const int64_t step = HostPieces((int64_t)1 << 40, rowBytes).most, rows = scale * step / 8 + extra;
+        const int64_t least = scale % 3 == 0 ? 0 : 6144 << scale % 7; // (what a launch plan asks for)
+        const int64_t step = HostPieces((int64_t)1 << 40, rowBytes, least).most, rows = scale * step / 8 + extra;
         if (rows < 1) continue;
-        const HostPieces p(rows, rowBytes);
+        const HostPieces p(rows, rowBytes, least);
+        EXPECT(step >= std::min<int64_t>(least / 256 * 256, ((int64_t)16 << 20) / (int64_t)rowBytes / 256 * 256), "%zu features: pieces of %lld rows for %lld",
+               features, (long long)step, (long long)least);
         EXPECT(p.count >= 1 && p.slots >= 4 && p.slots <= kHostSlots && p.slots / 2 - 1 + 2 <= p.slots - 1, "%zu features %lld rows", features, (long long)rows);
         EXPECT((size_t)(p.slots * p.most) * rowBytes <= (size_t)64 << 20 || p.most <= 4, "%zu features %lld rows: %lld buffers of %lld rows", features,
                (long long)rows, (long long)p.slots, (long long)p.most);

@@ -15,7 +15,8 @@
 namespace tbamd {
 
 // How a host batch is cut: pieces of about 4 MB (73 us of the link, which cover the 10 us the calling thread needs for a piece),
-// at least 1024 rows (fewer take the kernels as long) as long as those fit 16 MB; a quarter and half a piece first, because
+// at least 1024 rows (fewer take the kernels as long) and `leastRows` (what the kernels need to work at their rate; two thirds of
+// the batch at most, so that something overlaps), as long as those fit 16 MB; a quarter and half a piece first, because
 // nothing overlaps their copies, and what is left at the end as two thirds and one third, because nothing overlaps the last
 // piece's kernels.  The pieces take turns in `slots` pinned buffers: eight of 4 MB, fewer of larger ones (four are what two
 // copies under way, a piece in its kernels and one being filled need), so that they pin 32 MB, 64 for the widest rows.
@@ -24,9 +25,9 @@ constexpr int kHostSlots = 8;
 struct HostPieces {
   int64_t rows, most, count; // `most`: rows of the largest piece
   int64_t slots;
-  HostPieces(int64_t allRows, size_t rowBytes) : rows(allRows) {
+  HostPieces(int64_t allRows, size_t rowBytes, int64_t leastRows = 0) : rows(allRows) {
     const int64_t fit = (int64_t)((4 * kHostPieceBytes) / rowBytes);
-    most = std::min(std::max<int64_t>((int64_t)(kHostPieceBytes / rowBytes), 1024), fit);
+    most = std::min(std::max<int64_t>({(int64_t)(kHostPieceBytes / rowBytes), 1024, std::min(leastRows, rows * 2 / 3)}), fit);
     most = most >= 256 ? most / 256 * 256 : std::max<int64_t>(4, most); // (rows of 4 MB and more: four of them)
     slots = std::max<int64_t>(4, std::min<int64_t>(kHostSlots, (int64_t)(kHostSlots * kHostPieceBytes / ((size_t)most * rowBytes))));
     if (rows <= most) most = rows, count = 1;

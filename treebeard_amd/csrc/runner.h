@@ -112,6 +112,7 @@ public:
 private:
   void Release() noexcept;
   void RunHostChunk(const void *hostInputs, void *hostResults, int64_t rows);
+  int64_t RowsForKernels() const; // rows of a piece of a host batch, if its kernels are to fill the device
   void InitDevice();
   // Ordering of calls that share the runner's buffers (see RunDeviceOnStream).
   void RecordAsyncCall();                        // the event behind the last asynchronous call, if it has none yet
