@@ -997,7 +997,8 @@ WalkTreeParallelKernel(const float *__restrict__ x, const uint4 *__restrict__ no
 // Global-memory walk: the fallback for forests with a tree that does not fit one LDS group.  One
 // lane per row; nodes (16 bytes, absolute child indices) and row values are read from global memory
 // through L1/L2, K trees at a time in lock step with an explicit leaf test.  Same accumulation,
-// class flush and tree-slice scheme as the LDS kernels.
+// class flush and tree-slice scheme as the LDS kernels.  65536 rows x 28 features, 40 trees of depth 16: 88 us, the texture
+// addressers 67 % busy with two gathers a level (node and value), the VALUs 12 %; the rest is the chain of dependent loads.
 // ---------------------------------------------------------------------------
 template <int K, bool kDump>
 __global__ void __launch_bounds__(1024)
@@ -1466,7 +1467,7 @@ __global__ void __launch_bounds__(256) FinalizeWideKernel(const FinalizeParams p
 // to a second kernel: a lane reads a tree three levels at a time (one 48-byte block, three 16-byte loads in flight
 // together, so a walk of 8 levels waits for three loads of L2 latency instead of nine), leaves its leaf value in LDS,
 // and a wave per (row, class) adds them in a fixed order.  One row through 1000 trees of depth 8 took 15.2 us a call
-// with the tree-parallel kernel and its finalize launch.
+// with the tree-parallel kernel and its finalize launch, 6.5 here (4.4 of them the kernel).
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int rowsPerBlock, int leafStride) {
   extern __shared__ __align__(16) unsigned char lds[];
@@ -1543,16 +1544,17 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
 
 // ---------------------------------------------------------------------------
 // Wide rows, rank-quantised: a block keeps 32 rows of one byte per feature in LDS (64 KB at 2000 features) and every
-// wave streams its own bundles of four trees through 8 KB of its own, two bundles deep: while one is walked the next is
+// wave streams its own bundles of eight trees through 8 KB of its own, two bundles deep: while one is walked the next is
 // on its way from L2 (direct global -> LDS loads), so no wave waits for a copy or for another wave - the tree groups of
 // the row-parallel kernel, which all waves of a block copy, wait for and walk together with nothing else on the CU to
-// cover it, kept the LDS pipes 36 % busy.  The two halves of a wave walk two trees over the same 32 rows, each lane two
-// chains; 32 rows instead of 64 leave the room (twelve waves x two buffers), and 4-byte nodes halve what a bundle takes:
-// a step is a 4-byte node read and a one-byte rank read.  Leaf values stay in global memory, one gather per tree, issued
-// a bundle ahead of its use.  What bounds it is the latency of the two dependent LDS reads of a step at twelve waves a CU.
-// 262144 rows x 2000 features, 1000 trees of depth 8 (ranks included in neither): 1362 us with tree groups; here 996 with
-// two chains a lane, 914 with four and without words for the last level's leaves, 883 with two levels per loop turn, 800
-// with LDS reads awaited one by one.  20000 rows 94 -> 77 us.
+// cover it, kept the LDS pipes 37 % busy.  The two halves of a wave walk different trees over the same 32 rows, each lane
+// four chains (two, in bundles of four trees, where bigger trees leave bundles of eight short); 32 rows instead of 64
+// leave the room (twelve waves x two buffers), and 4-byte nodes halve what a bundle takes: a step is a 4-byte node read
+// and a one-byte rank read.  Leaf values stay in global memory, one gather per tree, issued a bundle ahead of its use.
+// What bounds it is the latency of the two dependent LDS reads of a step at twelve waves a CU (LDS pipes 46 % busy, 13 %
+// of it bank conflicts of the rank reads; VALUs 62 %).
+// Walk of 262144 rows x 2000 features, 1000 trees of depth 8, on the same ranks: 1.33 ms with tree groups, 0.80-0.82 here;
+// of 20000 rows: 0.099 + 0.005 for the finalize kernel, 0.076 here.
 // ---------------------------------------------------------------------------
 template <int K> // chains
 __global__ void __launch_bounds__(kStreamMaxWaves * 64)

@@ -692,11 +692,11 @@ bool IsPinnedHost(const void *ptr) {
 
 // A plan made for a large batch has one tree slice: a piece of 4 MB, 146 row blocks of 28 features, then takes the walk of
 // 1000 trees of depth 8 as long (87 us) as one block for each of 256 compute units would.  Pieces of a block and a half per
-// unit and slice: host calls of 2^20 such rows 3.28 -> 2.40 ms (pinned 3.23 -> 2.34), 2^18 rows 1.04 -> 0.79,
-// 2^19 rows of eight classes on 54 features 2.80 -> 2.22; batches below 2^17 rows take as long as before.  One block a unit took up to a quarter longer than this, two
-// up to a third longer where the batch then was a single piece and 7 % less at best; three quarters of a batch in one piece
-// instead of two thirds (HostPieces) 8 % less for 2^17 rows and 12 % more for 90001 rows of eight classes.  What lost: pageable
-// 2^16 rows of 90 features, 0.57 -> 0.60.  Streamed bundles slice every piece anew.
+// unit and slice: host calls of 2^20 such rows 3.28 -> 2.40 ms (pinned 3.23 -> 2.34), 2^18 rows 1.04 -> 0.79, 2^19 rows of
+// eight classes on 54 features 2.80 -> 2.22; batches below 2^17 rows take as long as before, but for pageable 2^16 rows of 90
+// features (0.57 -> 0.60).  One block a unit took up to a quarter longer than this, two up to a third longer where the batch
+// then was a single piece and 7 % less at best; three quarters of a batch in one piece instead of two thirds (HostPieces)
+// 8 % less for 2^17 rows and 12 % more for 90001 rows of eight classes.  Streamed bundles slice every piece anew.
 int64_t InferenceRunner::RowsForKernels() const {
   if (StreamsBundles()) return 0;
   return (int64_t)m_limits.computeUnits * m_model.plan.rowsPerBlock * 3 / 2 / m_model.plan.treeSlices;
