@@ -200,6 +200,7 @@ int shimBusyStreams(hipStream_t except) {
   return busy;
 }
 long shimLaunchesToGo = -1; // launches until one fails (negative: none does)
+long shimNoLaunches = 0;    // every launch fails
 long shimFewRows = 0, shimSplits = 0, shimStreams = 0; // launches of the forms that stand beside the launch plans' kernels
 
 } // extern "C"
@@ -218,6 +219,7 @@ uint32_t Bits(float v) {
 bool Refused(hipStream_t stream) {
   std::lock_guard<std::mutex> lock(gMutex);
   if (shimLaunchesToGo >= 0 && shimLaunchesToGo-- == 0) return true;
+  if (shimNoLaunches) return true;
   DoCopies(gStreams[stream]);
   ++gStreams[stream].queued;
   return false;

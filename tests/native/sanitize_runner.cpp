@@ -19,7 +19,7 @@
 #include <string>
 #include <vector>
 
-extern "C" long shimFewRows, shimSplits, shimStreams, shimLaunchesToGo; // hip_host_shim.cpp
+extern "C" long shimFewRows, shimSplits, shimStreams, shimLaunchesToGo, shimNoLaunches; // hip_host_shim.cpp
 extern "C" int shimBusyStreams(hipStream_t except);
 
 namespace {
@@ -462,6 +462,15 @@ void WholeBatch(const Case &c) {
     MulticlassOutputs(c, runner, dx, rows);
   }
   double best = 0, walk = 0, fin = 0, bin = 0;
+  (void)tbmi_set_plan(runner, 64, 4, 2, 8192, 1);
+  const std::string before = Describe(runner);
+  for (int64_t n : {(int64_t)1, rows}) { // a search that fails leaves the plan and its pin (plans no launch of which succeeds are passed over)
+    shimNoLaunches = 1;
+    const int32_t failed = tbmi_autotune(runner, dx, n, &best);
+    shimNoLaunches = 0;
+    if (failed) EXPECT(Describe(runner) == before, "after a failed search: %s, before: %s", Describe(runner).c_str(), before.c_str());
+    else EXPECT(tbmi_set_plan(runner, 64, 4, 2, 8192, 1) == 0, "tbmi_set_plan");
+  }
   EXPECT(tbmi_autotune(runner, dx, std::min<int64_t>(rows, 300), &best) == 0, "tbmi_autotune");
   for (int64_t n : {(int64_t)1, limit, limit + 1, rows}) { // what is timed is what a call runs
     if (n < 1 || n > rows) continue;

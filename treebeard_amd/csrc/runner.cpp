@@ -991,8 +991,12 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
       TimeKernels(deviceInputs, out, rows, 24, &bestMs, nullptr, nullptr);
     }
   } catch (...) {
-    m_planPinned = pinned;
     (void)hipFree(out);
+    try {
+      Repack(original);
+    } catch (const Error &) { // (the error of the search is the one to report)
+    }
+    m_planPinned = pinned;
     throw;
   }
   (void)hipFree(out);
