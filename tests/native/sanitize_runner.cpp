@@ -392,6 +392,31 @@ void DeviceEntryPoints(const Case &c, int64_t rows, int32_t tileSize = 1, int32_
   (void)hipFree(dids);
 }
 
+// A runner made for a small batch, whose plan has many slices: the no-allocation entry point serves the batches that the few-rows
+// kernel can take, also above the limit up to which it is the faster form, where the plan's sums do not fit the fixed array.
+void NoAllocOfManySums(const Case &c) {
+  const intptr_t runner = MakeRunner(c, 512, c.forest.numClasses > 0);
+  if (!runner) return;
+  const std::string plan = Describe(runner);
+  const int64_t limit = std::atoll(plan.c_str() + plan.find("fewRowsLimit=") + std::strlen("fewRowsLimit="));
+  const long few = shimFewRows;
+  float *dx = nullptr;
+  void *out = nullptr;
+  const size_t resultBytes = (size_t)c.rows * (size_t)tbmi_result_bytes(runner);
+  EXPECT(limit < c.rows, "limit %lld", (long long)limit);
+  EXPECT(hipMalloc((void **)&dx, (size_t)c.rows * c.forest.numFeatures * sizeof(float)) == hipSuccess, "hipMalloc");
+  EXPECT(hipMalloc(&out, resultBytes) == hipSuccess, "hipMalloc");
+  std::memcpy(dx, c.x.data(), (size_t)c.rows * c.forest.numFeatures * sizeof(float));
+  EXPECT(tbmi_run_device_noalloc(runner, dx, out, c.rows, nullptr) == 0 && shimFewRows == few + 1, "noalloc of %lld rows, limit %lld",
+         (long long)c.rows, (long long)limit);
+  std::vector<float> got((size_t)c.rows);
+  for (int64_t r = 0; r < c.rows; ++r) got[r] = c.forest.numClasses > 0 ? (float)static_cast<int8_t *>(out)[r] : static_cast<float *>(out)[r];
+  Compare(c, got.data(), 0, c.rows, "noalloc of many sums");
+  (void)hipFree(dx);
+  (void)hipFree(out);
+  DeleteInferenceRunner(runner);
+}
+
 // Host calls whose n-th launch fails, of one piece and of several: nothing of theirs is under way when they return, and the
 // next call is right.
 void FailedCalls(const Case &c) {
@@ -553,6 +578,10 @@ int main(int argc, char **argv) {
     for (auto &v : c.x) v = normal(rng);
     c.expected.resize((size_t)c.rows);
     for (int64_t r = 0; r < c.rows; ++r) c.expected[r] = Predict(c.forest, c.x.data() + r * F, nullptr);
+    if (std::getenv("SANITIZE_NOALLOC")) {
+      NoAllocOfManySums(c);
+      continue;
+    }
     HostEntryPoints(c);
     HostEntryPoints(c, true);
     WholeBatch(c);

@@ -182,6 +182,20 @@ def test_forms_beside_the_launch_plans_under_address_sanitizer(tmp_path, synth_m
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_no_alloc_calls_of_many_class_sums(tmp_path, address_driver):
+    """40 trees voting for 40 classes, a plan of many slices: 26000 rows need 80 MB of partial sums, and none in the few-rows form."""
+    import numpy as np
+    rng = np.random.Generator(np.random.PCG64(9))
+    trees = [synth._grow_tree(rng, 8, lambda d, s: 1.0, lambda: (rng.integers(0, 4), float(np.round(rng.normal(), 2))),
+                              lambda: rng.normal(0.0, 0.1)) for _ in range(40)]
+    path = str(tmp_path / "manyclasses.json")
+    synth.write_xgboost_json(path, trees, 4, objective="multi:softmax", num_class=40, tree_info=list(range(40)))
+    env = dict(os.environ, SANITIZE_NOALLOC="1", ASAN_OPTIONS="detect_leaks=1:abort_on_error=0", TMPDIR=str(tmp_path))
+    run = subprocess.run([address_driver, path, "26000"], capture_output=True, text=True, env=env, timeout=600)
+    assert run.returncode == 0, (run.stdout + run.stderr)[-4000:]
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 def test_runner_survives_mutated_compiled_models(tmp_path, synth_model, address_driver):
     """tbmi_load_compiled_model on compiled-model files whose header words (plan, batch size, return type, counts) and
     body were overwritten: refused with a message or loaded and run on a few rows, under ASan + UBSan."""

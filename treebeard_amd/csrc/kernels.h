@@ -134,6 +134,15 @@ inline FewRowsShape ShapeOfFewRows(int64_t rows, int numFeatures, int numTrees, 
   return s;
 }
 
+// The most rows of such a forest LaunchFewRows is used for (0: none).
+constexpr int64_t kFewRowsWork = (int64_t)3 << 20; // (row, tree, block of three levels) visits
+inline int64_t FewRowsMost(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth) {
+  if (numTrees < 1) return 0;
+  int64_t rows = kFewRowsWork / ((int64_t)numTrees * (depth / 3 + 1));
+  while (rows > 0 && ShapeOfFewRows(rows, numFeatures, numTrees, numClasses).ldsBytes > kFewRowsLds) rows /= 2;
+  return rows;
+}
+
 // How many rows of such a forest LaunchFewRows takes sooner than the launch plans do (0: never).  Two costs grow with the
 // rows: the walks, about 20 cycles of a compute unit's address path per 16-byte gather of 64 lanes (4.5 us at kFewRowsWork
 // visits), and the sums, 0.4 us per (row, class) that a wave adds.  A forest of many trees ends at the first, one of few
@@ -141,17 +150,14 @@ inline FewRowsShape ShapeOfFewRows(int64_t rows, int numFeatures, int numTrees, 
 // class and up to 4 for the walk: fitted to 72 forests of 1 to 400 trees and 0 to 12 classes, 250 to 400000 rows each.
 // Without the second term 393216 rows of two trees and two classes took 94 us here and 17 by the plan, 87381 rows of twelve
 // trees and six classes 68 and 14; with it no forest of the fit is more than 1.3 times the faster of the two forms.
-constexpr int64_t kFewRowsWork = (int64_t)3 << 20; // (row, tree, block of three levels) visits
 inline int64_t FewRowsLimit(int32_t numFeatures, int32_t numTrees, int32_t numClasses, int32_t depth) {
-  if (numTrees < 1) return 0;
-  const int64_t rounds = depth / 3 + 1;
+  const int64_t visits = (int64_t)numTrees * (depth / 3 + 1);
   const double planMicros = 7.0 + 1.1 * numClasses + std::min(4.0, (double)numTrees * depth / 100.0);
-  int64_t rows = kFewRowsWork / (numTrees * rounds);
-  while (rows > 0 && ShapeOfFewRows(rows, numFeatures, numTrees, numClasses).ldsBytes > kFewRowsLds) rows /= 2;
+  int64_t rows = FewRowsMost(numFeatures, numTrees, numClasses, depth);
   for (; rows > 0; rows = rows * 7 / 8) {
     const FewRowsShape s = ShapeOfFewRows(rows, numFeatures, numTrees, numClasses);
     const int64_t waves = s.threads / 64, sums = ((int64_t)s.rowsPerBlock * std::max(1, numClasses) + waves - 1) / waves;
-    if (4.5 + 4.5 * (double)(rows * numTrees * rounds) / (double)kFewRowsWork + 0.4 * (double)sums <= planMicros) break;
+    if (4.5 + 4.5 * (double)(rows * visits) / (double)kFewRowsWork + 0.4 * (double)sums <= planMicros) break;
   }
   return rows;
 }

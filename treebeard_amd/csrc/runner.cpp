@@ -256,13 +256,14 @@ void InferenceRunner::UploadFewRows() {
   if (m_forest.trees.empty()) return;
   int32_t depth = 0;
   for (const Tree &tree : m_forest.trees) depth = std::max(depth, tree.Depth());
-  const int64_t limit = FewRowsLimit(m_forest.numFeatures, (int32_t)m_forest.trees.size(), m_forest.numClasses, depth);
-  if (limit < 1) return;
+  const int64_t most = FewRowsMost(m_forest.numFeatures, (int32_t)m_forest.trees.size(), m_forest.numClasses, depth);
+  if (most < 1) return;
   const FewRowsModel model = PackFewRows(m_forest);
   if (model.blocks.empty()) return;
   m_dFewRows = Upload(model.blocks, "upload few-rows blocks");
   m_dFewRowsClasses = Upload(model.classBegin, "upload class ranges");
-  m_fewRowsLimit = limit;
+  m_fewRowsLimit = FewRowsLimit(m_forest.numFeatures, (int32_t)m_forest.trees.size(), m_forest.numClasses, depth);
+  m_fewRowsMost = most;
 }
 
 void InferenceRunner::Repack(const LaunchPlan &plan) {
@@ -542,7 +543,7 @@ bool InferenceRunner::LaunchWalkFor(const float *walkInputs, int64_t rows, Final
 void InferenceRunner::Launch(const float *deviceInputs, int64_t rows, float *out, int8_t *classOut, float *margins,
                              float *probabilities, int32_t *leafIds, hipStream_t stream, const Workspace &ws, hipEvent_t done) {
   if (rows <= 0) return;
-  if (!leafIds && TakesFewRows(rows)) {
+  if (!leafIds && (ws.fewRows || TakesFewRows(rows))) {
     FewRowsParams f;
     f.x = deviceInputs;
     f.blocks = m_dFewRows;
@@ -618,7 +619,9 @@ void InferenceRunner::RunDeviceNoAlloc(const float *deviceInputs, void *deviceRe
   size_t partialBytes = few ? 0 : padded(PartialBytes(rows, true));
   ws.split = partialBytes > 0 && partialBytes + ranksBytes <= kNoAllocScratchBytes; // (an even split may need more partial sums)
   if (!ws.split) partialBytes = few || FusesArgmax() || StreamsBundles() ? 0 : padded(PartialBytes(rows, false)); // (none when the walk keeps the arg-max)
-  if (partialBytes + ranksBytes > kNoAllocScratchBytes)
+  // (a forest of few trees has a limit below what the form can take: there it stands in for plans the array cannot serve)
+  ws.fewRows = partialBytes + ranksBytes > kNoAllocScratchBytes && rows <= m_fewRowsMost && !m_planPinned && !m_model.plan.peelWalks;
+  if (!ws.fewRows && partialBytes + ranksBytes > kNoAllocScratchBytes)
     throw Error("this launch plan needs " + std::to_string(partialBytes + ranksBytes) + " bytes of scratch memory for " +
                 std::to_string(rows) + " rows; the fixed array of the no-allocation entry point holds " +
                 std::to_string(kNoAllocScratchBytes) + ": pass fewer rows per call or use tbmi_run_device_async");

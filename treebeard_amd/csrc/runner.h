@@ -134,6 +134,7 @@ private:
     double *partial = nullptr; // [PartialCount()][rows][max(1, classes)] when NeedsFinalize()
     uint8_t *ranks = nullptr;  // rank-quantised rows when the plan uses them
     bool split = true;         // room for a walk split evenly (SplitBlocks)
+    bool fewRows = false;      // no room for the plan's kernels: LaunchFewRows takes the batch, sooner or not
   };
   // Allocating callers: grows the runner's own buffers to hold `rows` rows and orders `stream`, on which the
   // caller is about to launch, behind an asynchronous call that may still use them.
@@ -198,7 +199,7 @@ private:
   hipStream_t m_asyncStream = nullptr;
   bool m_asyncPending = false, m_asyncRecorded = false;
   bool m_planPinned = false;
-  int64_t m_fewRowsLimit = 0;
+  int64_t m_fewRowsLimit = 0, m_fewRowsMost = 0;
   DeviceFewRowsBlock *m_dFewRows = nullptr;
   bool m_streamPacked = false;            // the first rank-quantised plan brings the bundles for LaunchRankStream
   uint32_t *m_dStreamWords = nullptr;
