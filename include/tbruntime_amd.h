@@ -137,8 +137,8 @@ TBAMD_EXPORT int32_t tbmi_run_device_async(intptr_t runner, const float *deviceI
  * rank-quantised rows of wide models) taken from one fixed device array of tbmi_noalloc_scratch_bytes()
  * bytes (32 MiB) that the library holds on every GPU it runs on.  It allocates, frees and synchronises
  * nothing.  A call whose plan needs more scratch memory than that for `rows` rows fails with a message
- * naming both sizes (pass fewer rows per call), unless the kernel of small batches, which needs none, can take it.  All calls on one GPU share the array: calls that overlap
- * in time on one GPU, from any runner or stream, race on it.  Because it may be captured into a graph this
+ * naming both sizes (pass fewer rows per call), unless the kernel of small batches, which needs none, can take
+ * it.  All calls on one GPU share the array: calls that overlap in time on one GPU, from any runner or stream, race on it.  Because it may be captured into a graph this
  * entry point records no event either: the caller keeps the runner alive and un-repacked (no tbmi_set_*_plan,
  * tbmi_autotune, DeleteInferenceRunner) until the kernels of its calls have finished.  The array costs every
  * process that loads the library 32 MiB of device memory per GPU it touches. */
