@@ -170,7 +170,7 @@ def main():
     plan_fields = dict(item.split("=", 1) for item in plan.split() if "=" in item)
     kernel = {"few_rows": "FewRowsKernel", "rank_stream": "RankStreamKernel", "rows_lds_split": "WalkRowsSplitKernel",
               "rows_lds": "WalkRowsLdsKernel", "rows_tiled": "WalkRowsTiledKernel", "tree_parallel": "WalkTreeParallelKernel",
-              "global_walk": "WalkGlobalKernel"}[plan_fields["batchKernel"]]
+              "global_walk": "WalkGlobalKernel", "deep_walk": "WalkRowsLdsKernel"}[plan_fields["batchKernel"]]
     quantized = quantized and kernel != "FewRowsKernel"
     # the rank-quantised path reads the f32 rows in its binning kernel: both kernels count for the HBM roofline
     hbm_ms = walk_ms + bin_ms if quantized else walk_ms

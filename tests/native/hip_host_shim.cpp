@@ -201,7 +201,7 @@ int shimBusyStreams(hipStream_t except) {
 }
 long shimLaunchesToGo = -1; // launches until one fails (negative: none does)
 long shimNoLaunches = 0;    // every launch fails
-long shimFewRows = 0, shimSplits = 0, shimStreams = 0; // launches of the forms that stand beside the launch plans' kernels
+long shimFewRows = 0, shimSplits = 0, shimStreams = 0, shimDeferred = 0; // launches of the forms that stand beside the launch plans' kernels
 
 } // extern "C"
 
@@ -273,7 +273,7 @@ void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64
           if (rankRows != 0 || stride == 0) std::abort();
           if (stop.value != stop.value) { // a NaN marks a stub; its payload is the tail index
             if (!bd.hasStubs || (stop.meta >> 16) + kNodeBytes != addr || (Bits(stop.value) & ~kStubIndexMask) != kStubValueBits ||
-                !p.tailNodes || !p.tailOrigin)
+                !p.tailNodes || (p.leafIds && !p.tailOrigin))
               std::abort();
             inTail = true;
             at = Bits(stop.value) & kStubIndexMask;
@@ -387,6 +387,7 @@ hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, 
   const int prefetch = (int)((p.s.groupRegionBytes / 16 + RB * TT - 1) / (RB * TT));
   if (prefetch > 16) return hipErrorInvalidValue;
   if (tileMode == 2 && RB != 64) return hipErrorInvalidValue;
+  if (p.s.deferTails) ++shimDeferred;
   if (tileMode < 0 || tileMode > 3 || (tileMode == 3 && p.splitBlocks)) return hipErrorInvalidValue;
   if (tileMode == 3 && (int64_t)((p.s.numFeatures + 2) / 2) * RB * 4 > 0x10000) return hipErrorInvalidValue;
   const uint32_t stride = tileMode == 0 || tileMode == 3 ? (uint32_t)RB * 4u : tileMode == 1 ? (uint32_t)RB : (uint32_t)RB / 4u;

@@ -19,7 +19,7 @@
 #include <string>
 #include <vector>
 
-extern "C" long shimFewRows, shimSplits, shimStreams, shimLaunchesToGo, shimNoLaunches; // hip_host_shim.cpp
+extern "C" long shimFewRows, shimSplits, shimStreams, shimDeferred, shimLaunchesToGo, shimNoLaunches; // hip_host_shim.cpp
 extern "C" int shimBusyStreams(hipStream_t except);
 
 namespace {
@@ -613,6 +613,6 @@ int main(int argc, char **argv) {
   EXPECT(tbmi_run_device(0, nullptr, nullptr, 4) == -1, "null runner");
   EXPECT(CreateInferenceRunner("/nonexistent/model.json", "", 0) == 0, "missing options");
   if (gFailures) return 1;
-  std::printf("launches: few-rows %ld, split %ld, stream %ld\nok\n", shimFewRows, shimSplits, shimStreams);
+  std::printf("launches: few-rows %ld, split %ld, stream %ld, deferred %ld\nok\n", shimFewRows, shimSplits, shimStreams, shimDeferred);
   return 0;
 }

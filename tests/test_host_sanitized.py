@@ -182,6 +182,23 @@ def test_forms_beside_the_launch_plans_under_address_sanitizer(tmp_path, synth_m
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_deep_walk_under_address_sanitizer(tmp_path, address_driver):
+    """Trees of more than 8190 nodes beside a single leaf and shallow ones: cut, packed and walked with deferred tails on every
+    entry point, the leaf-id dump and a pinned plan on the global-memory walk."""
+    import numpy as np
+    rng = np.random.Generator(np.random.PCG64(10))
+    grow = lambda depth, p: synth._grow_tree(rng, depth, lambda d, s: p, lambda: (rng.integers(0, 12), rng.normal()),
+                                             lambda: rng.normal(0.0, 0.1), force_root=depth > 0)
+    trees = [grow(13, 1.0), grow(14, 0.95), grow(0, 1.0), grow(3, 1.0), grow(12, 0.9)]
+    path = str(tmp_path / "deep.json")
+    synth.write_xgboost_json(path, trees, 12)
+    env = dict(os.environ, SANITIZE_QUICK="1", ASAN_OPTIONS="detect_leaks=1:abort_on_error=0", TMPDIR=str(tmp_path))
+    run = subprocess.run([address_driver, path, "31001"], capture_output=True, text=True, env=env, timeout=900)
+    assert run.returncode == 0, (run.stdout + run.stderr)[-4000:]
+    assert int(run.stdout.split("deferred ")[1].split()[0]) > 0, run.stdout[-300:]
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 def test_no_alloc_calls_of_many_class_sums(tmp_path, address_driver):
     """40 trees voting for 40 classes, a plan of many slices: 26000 rows need 80 MB of partial sums, and none in the few-rows form."""
     import numpy as np

@@ -73,8 +73,9 @@ constexpr uint32_t kNodeBytes = 8;
 constexpr uint32_t kDeferBytesPerWave = 512; // LDS of one wave's queue of deferred walks (LaunchPlan::deferTails)
 // Deferred tails: a tail node's meta word holds the index of its left child above kTailFeatureBits bits of feature
 // index; a queue entry holds a tail index below 6 bits of lane (bits 26 to 31).
-constexpr uint32_t kTailFeatureBits = 12;
-constexpr uint32_t kMaxTailNodes = 1u << 20;
+// (Eight bits: a row tile with byte offsets holds 64 rows of at most 255 features and the pad feature.)
+constexpr uint32_t kTailFeatureBits = 8;
+constexpr uint32_t kMaxTailNodes = 1u << 22;
 // A stub's value field: a quiet NaN whose low bits are the tail index.
 constexpr uint32_t kStubValueBits = 0x7FC00000u;
 constexpr uint32_t kStubIndexMask = kMaxTailNodes - 1u;

@@ -559,7 +559,23 @@ FewRowsModel PackFewRows(const Forest &input) {
   return fm;
 }
 
-PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile) {
+namespace {
+PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile, const std::vector<int32_t> *cuts);
+}
+
+PackedModel PackForest(const Forest &forest, const LaunchPlan &plan, const HitCountProfile *profile) {
+  return PackPlan(forest, plan, profile, nullptr);
+}
+
+PackedModel PackWithCuts(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &cuts) {
+  if (!plan.deferTails || cuts.size() != forest.trees.size()) throw Error("cut levels need a plan with deferred tails and one per tree");
+  return PackPlan(forest, plan, nullptr, &cuts);
+}
+
+namespace {
+constexpr uint32_t kPeeledTailNodes = 1u << 20; // below the cuts of a plan with a profile (8 MB: they stay in the caches)
+
+PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile, const std::vector<int32_t> *cuts) {
   // Plans also come out of files: every field is brought into its range before anything is computed from it.
   if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds && plan.kernel != LaunchPlan::Kernel::kTreeParallel &&
       plan.kernel != LaunchPlan::Kernel::kGlobalWalk)
@@ -601,7 +617,7 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
                 std::to_string(kMaxTileSize) + " nodes");
   const int T = plan.WalkTile();
   if (plan.deferTails && (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || T != 1 || plan.quantizedRows || plan.rankRows16 ||
-                          plan.featureOffsetInWords || forest.numClasses > 0 || !profile))
+                          plan.featureOffsetInWords || forest.numClasses > 0 || !(profile || cuts)))
     throw Error("deferred tails need a profile and the scalar row-parallel kernel on float32 rows of a model without classes");
   if (T > 1 && (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.quantizedRows || plan.rankRows16))
     throw Error("tile sizes above 1 need the row-parallel kernel on float32 rows");
@@ -701,7 +717,7 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
   std::vector<TiledTree> tiled(T > 1 ? numTrees : 0);
   std::vector<int32_t> depth(numTrees), peel(numTrees);
   std::vector<int32_t> fullDepth(numTrees, 0); // deferred tails: the tree's own depth (depth[] is then where its walk stops)
-  int64_t tailBudget = plan.deferTails && forest.numFeatures + 1 < (1 << kTailFeatureBits) ? (int64_t)kMaxTailNodes - 1 : 0;
+  int64_t tailBudget = plan.deferTails && forest.numFeatures + 1 < (1 << kTailFeatureBits) ? (int64_t)(cuts ? kMaxTailNodes : kPeeledTailNodes) - 1 : 0;
   std::vector<uint32_t> units(numTrees);
   for (size_t t = 0; t < numTrees; ++t) {
     const Tree &tree = forest.trees[t];
@@ -735,7 +751,9 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
     }
     peel[t] = plan.peelWalks && hits ? PeelDepth(*hits, leafLevel, depth[t]) : depth[t];
     fullDepth[t] = depth[t];
-    if (plan.deferTails) {
+    int32_t cut = cuts ? std::min((*cuts)[t], depth[t]) : depth[t];
+    double queued = 0.0; // (of the profiled rows, by the profile)
+    if (plan.deferTails && !cuts) {
       // Where the lock-step walk of this tree stops.  Costs in cycles of a compute unit per 64 rows: a lock-step
       // level is a node read (2.5 cycles while the level has at most 32 nodes, 4.3 for 64, 6.0 beyond) and a
       // feature read (2.4), as measured on MI355X; a deferred walk costs 20 to queue, fetch and hand back plus 20
@@ -758,12 +776,14 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
       double whole = 0.0;
       for (int32_t d = 0; d < depth[t]; ++d) whole += levelCost(d);
       double best = whole, head = 0.0;
-      int32_t cut = depth[t];
       for (int32_t d = 1; d < depth[t]; ++d) {
         head += levelCost(d - 1);
         const double cost = head + 2.0 + alive[(size_t)d] * ((depth[t] - d) * 20.0 + 20.0);
         if (cost < best && cost < 0.92 * whole) best = cost, cut = d;
       }
+      queued = alive[(size_t)cut];
+    }
+    if (cut < depth[t]) {
       bool nanLeaf = false; // (a NaN is what marks a stub)
       for (size_t i = 0; i < tree.NumNodes(); ++i) nanLeaf = nanLeaf || (tree.IsLeaf((int32_t)i) && tree.value[i] != tree.value[i]);
       if (cut < depth[t] && tailBudget > 0 && !nanLeaf) {
@@ -775,7 +795,7 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
         depth[t] = cut;
         peel[t] = cut;
         pm.treesDeferred += 1;
-        pm.deferredEntriesPerRow += alive[(size_t)cut];
+        pm.deferredEntriesPerRow += queued;
       }
     }
     pm.lockStepSteps += depth[t];
@@ -1023,6 +1043,7 @@ PackedModel PackForest(const Forest &input, const LaunchPlan &plan, const HitCou
   if (pm.bundleRoots.size() != pm.bundles.size() * (size_t)K) throw Error("internal error: bundle root table out of step");
   return pm;
 }
+} // namespace
 
 Tree UnpackTree(const PackedModel &pm, int32_t treeIndex) {
   if (pm.plan.WalkTile() > 1) throw Error("tiled models are checked through their walks, not unpacked");

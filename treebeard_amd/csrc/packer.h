@@ -176,6 +176,10 @@ int64_t BiggestTiledTreeBytes(const Forest &forest, int tileSize);
 // probability-based tiling and walk peeling.
 PackedModel PackForest(const Forest &forest, const LaunchPlan &plan, const HitCountProfile *profile = nullptr);
 
+// The same for a plan with deferTails whose cut levels are given (one per tree; the tree's depth or more: whole) instead of
+// weighed on a profile.
+PackedModel PackWithCuts(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &cuts);
+
 // Inverse of PackForest for tests: rebuilds (value, feature, left, right) of
 // original tree `tree` from the packed arrays.
 Tree UnpackTree(const PackedModel &model, int32_t tree);

@@ -156,6 +156,7 @@ void InferenceRunner::Release() noexcept {
   (void)hipFree(m_dStreamWords);
   (void)hipFree(m_dStreamValues);
   (void)hipFree(m_dStreamBundles);
+  FreeDeep();
   if (m_smallHost) (void)hipHostFree(m_smallHost);
   (void)hipFree(m_dPartial);
   (void)hipFree(m_dRanks);
@@ -210,6 +211,7 @@ void InferenceRunner::UploadModel() {
     m_model.plan.treeSlices = std::max(1, std::min<int32_t>(m_model.plan.treeSlices, (int32_t)m_model.globalTrees.size()));
     m_dGlobalNodes = Upload(m_model.globalNodes, "upload nodes");
     m_dGlobalTrees = Upload(m_model.globalTrees, "upload trees");
+    UploadDeep();
     return;
   }
   // treeSlices never exceeds the number of groups the packer produced
@@ -252,6 +254,37 @@ void InferenceRunner::UploadStream() {
   m_streamPacked = true;
 }
 
+void InferenceRunner::UploadDeep() {
+  if (m_deep.packed) return; // (the forest's, whatever the launch plan)
+  LaunchPlan plan;
+  std::vector<int32_t> cuts;
+  if (ChooseDeepWalk(m_forest, m_limits, &plan, &cuts)) {
+    try {
+      m_deep.model = PackWithCuts(m_forest, plan, cuts);
+      m_deep.nodes = Upload(m_deep.model.nodes, "upload nodes");
+      m_deep.bundles = Upload(m_deep.model.bundles, "upload bundles");
+      m_deep.bundleRoots = Upload(m_deep.model.bundleRoots, "upload bundle roots");
+      m_deep.groups = Upload(m_deep.model.groups, "upload groups");
+      m_deep.tailNodes = Upload(m_deep.model.tailNodes, "upload tail nodes");
+    } catch (...) {
+      FreeDeep();
+      throw;
+    }
+    m_deep.model.nodes = m_deep.model.bundleRoots = m_deep.model.tailNodes = {}; // (only the shape is needed on the host)
+    m_deep.model.nodeOrigin = m_deep.model.tailOrigin = {};
+  }
+  m_deep.packed = true;
+}
+
+void InferenceRunner::FreeDeep() {
+  (void)hipFree(m_deep.nodes);
+  (void)hipFree(m_deep.bundles);
+  (void)hipFree(m_deep.bundleRoots);
+  (void)hipFree(m_deep.groups);
+  (void)hipFree(m_deep.tailNodes);
+  m_deep = DeepWalk();
+}
+
 void InferenceRunner::UploadFewRows() {
   if (m_forest.trees.empty()) return;
   int32_t depth = 0;
@@ -291,6 +324,10 @@ void InferenceRunner::PinPlan(const LaunchPlan &plan) {
 size_t InferenceRunner::PartialBytes(int64_t rows, bool split) const {
   if (split && StreamsBundles()) {
     const int32_t slices = StreamSlices(rows);
+    return slices > 1 ? (size_t)slices * (size_t)rows * sizeof(double) : 0;
+  }
+  if (split && WalksDeep()) {
+    const int32_t slices = DeepSlices(rows);
     return slices > 1 ? (size_t)slices * (size_t)rows * sizeof(double) : 0;
   }
   const int32_t splitBlocks = split ? SplitBlocks(rows) : 0;
@@ -442,24 +479,24 @@ hipError_t InferenceRunner::LaunchWalk(const WalkParams &p, hipStream_t stream) 
   return LaunchWalkRowsLds(p, plan.interleave, tileMode, m_model.LdsBytes(), stream);
 }
 
-WalkParams InferenceRunner::MakeWalkParams(const float *deviceInputs, int64_t rows) const {
+WalkParams InferenceRunner::MakeWalkParams(const float *deviceInputs, int64_t rows, const PackedModel &model) const {
   WalkParams p;
   p.s.rows = rows;
   p.s.numFeatures = m_forest.numFeatures;
   p.s.numClasses = m_forest.numClasses;
-  p.s.numGroups = (int32_t)m_model.groups.size();
-  p.s.treeSlices = m_model.plan.treeSlices;
-  p.s.groupRegionBytes = m_model.GroupRegionBytes();
-  p.s.treeThreads = m_model.plan.treeThreads;
+  p.s.numGroups = (int32_t)model.groups.size();
+  p.s.treeSlices = model.plan.treeSlices;
+  p.s.groupRegionBytes = model.GroupRegionBytes();
+  p.s.treeThreads = model.plan.treeThreads;
   p.s.transform = m_forest.transform == Transform::kSigmoid ? 1 : 0;
   p.s.numTrees = (int32_t)m_forest.trees.size();
-  p.s.rowsPerBlock = m_model.plan.rowsPerBlock;
-  p.s.treeLanes = m_model.plan.treeLanes;
+  p.s.rowsPerBlock = model.plan.rowsPerBlock;
+  p.s.treeLanes = model.plan.treeLanes;
   p.s.initialValue = m_forest.initialValue;
-  p.peelWalks = m_model.plan.peelWalks;
-  p.s.deferTails = m_model.plan.deferTails ? 1 : 0;
-  p.s.tailDepth = (int32_t)m_model.maxTailDepth;
-  p.s.tileHops = m_model.maxTileHops;
+  p.peelWalks = model.plan.peelWalks;
+  p.s.deferTails = model.plan.deferTails ? 1 : 0;
+  p.s.tailDepth = (int32_t)model.maxTailDepth;
+  p.s.tileHops = model.maxTileHops;
   p.tailNodes = m_dTailNodes;
   p.tailOrigin = m_dTailOrigin;
   p.directStaging = DirectStaging();
@@ -527,7 +564,25 @@ bool InferenceRunner::LaunchWalkFor(const float *walkInputs, int64_t rows, Final
     Check(LaunchRankStream(p, stream), "launch rank-stream kernel");
     return p.slices > 1;
   }
-  WalkParams p = MakeWalkParams(walkInputs, rows);
+  if (WalksDeep() && !leafIds) {
+    const PackedModel &model = m_deep.model;
+    WalkParams p = MakeWalkParams(walkInputs, rows, model);
+    p.s.treeSlices = ws.split ? DeepSlices(rows) : 1;
+    p.directStaging = true;
+    p.nodes16 = reinterpret_cast<const uint4 *>(m_deep.nodes);
+    p.bundles = m_deep.bundles;
+    p.bundleRoots = m_deep.bundleRoots;
+    p.groups = m_deep.groups;
+    p.tailNodes = m_deep.tailNodes;
+    f.treeSlices = p.s.treeSlices;
+    const bool finalize = p.s.treeSlices > 1;
+    p.out = finalize ? nullptr : f.out;
+    p.partial = finalize ? ws.partial : nullptr;
+    p.done = finalize ? nullptr : done;
+    Check(LaunchWalkRowsLds(p, model.plan.interleave, 0, model.LdsBytes(), stream), "launch walk kernel");
+    return finalize;
+  }
+  WalkParams p = MakeWalkParams(walkInputs, rows, m_model);
   const bool finalize = SetOutputs(p, f.out, f.classOut, f.margins, f.probabilities, leafIds != nullptr, ws);
   if (leafIds) {
     p.leafIds = leafIds;
@@ -618,7 +673,7 @@ void InferenceRunner::RunDeviceNoAlloc(const float *deviceInputs, void *deviceRe
   Workspace ws;
   size_t partialBytes = few ? 0 : padded(PartialBytes(rows, true));
   ws.split = partialBytes > 0 && partialBytes + ranksBytes <= kNoAllocScratchBytes; // (an even split may need more partial sums)
-  if (!ws.split) partialBytes = few || FusesArgmax() || StreamsBundles() ? 0 : padded(PartialBytes(rows, false)); // (none when the walk keeps the arg-max)
+  if (!ws.split) partialBytes = few || FusesArgmax() || StreamsBundles() || WalksDeep() ? 0 : padded(PartialBytes(rows, false)); // (none when the walk keeps the arg-max)
   // (a forest of few trees has a limit below what the form can take: there it stands in for plans the array cannot serve)
   ws.fewRows = partialBytes + ranksBytes > kNoAllocScratchBytes && rows <= m_fewRowsMost && !m_planPinned && !m_model.plan.peelWalks;
   if (!ws.fewRows && partialBytes + ranksBytes > kNoAllocScratchBytes)
@@ -942,10 +997,14 @@ double InferenceRunner::AutoTune(const float *deviceInputs, int64_t rows) {
   LaunchPlan best = original;
   double bestMs = 1e300;
   try {
-    // (one-byte rank rows of a forest that streams its bundles run one kernel whatever the shape of the plan)
-    const auto streamed = [&](const LaunchPlan &plan) { return plan.quantizedRows && m_streamBundles > 0; };
+    // (one-byte rank rows of a forest that streams its bundles, and global-memory plans of one that walks with deferred
+    // tails, run one kernel whatever the shape of the plan)
+    const auto streamed = [&](const LaunchPlan &plan) {
+      return plan.kernel == LaunchPlan::Kernel::kGlobalWalk ? m_deep.nodes != nullptr : plan.quantizedRows && m_streamBundles > 0;
+    };
     const auto isTimed = [&](const LaunchPlan &plan) {
-      return streamed(plan) && std::any_of(timed.begin(), timed.end(), [&](const Timed &t) { return streamed(t.plan); });
+      return streamed(plan) &&
+             std::any_of(timed.begin(), timed.end(), [&](const Timed &t) { return streamed(t.plan) && t.plan.kernel == plan.kernel; });
     };
     for (const LaunchPlan &cand : CandidatePlans(m_forest, rows, m_limits, m_walk)) {
       double ms = 0;
@@ -1011,6 +1070,7 @@ const char *InferenceRunner::KernelOfBatch() const {
   const int64_t rows = m_options.batchSize;
   if (TakesFewRows(rows)) return "few_rows";
   if (StreamsBundles()) return "rank_stream";
+  if (WalksDeep()) return "deep_walk";
   if (SplitBlocks(rows) > 0) return "rows_lds_split";
   if (p.kernel == LaunchPlan::Kernel::kTreeParallel) return "tree_parallel";
   if (p.kernel == LaunchPlan::Kernel::kGlobalWalk) return "global_walk";

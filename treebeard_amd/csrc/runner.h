@@ -121,6 +121,8 @@ private:
   void UploadModel();
   void UploadFewRows();
   void UploadStream();
+  void UploadDeep();
+  void FreeDeep();
   void FreeModel();
   void EnsurePartial(size_t bytes);
   void EnsureStaging(int64_t rows);
@@ -151,6 +153,12 @@ private:
   // Rank-quantised rows go through LaunchRankStream where the forest has the form, unless the caller pinned a plan.
   bool StreamsBundles() const { return m_model.plan.quantizedRows && m_streamBundles > 0 && !m_planPinned; }
   int32_t StreamSlices(int64_t rows) const { return RankStreamSlices(rows, m_forest.numFeatures, m_streamBundles, m_limits.computeUnits); }
+  // Global-memory plans walk with deferred tails (ChooseDeepWalk) where the forest has the form, unless the caller pinned a plan.
+  bool WalksDeep() const { return m_model.plan.kernel == LaunchPlan::Kernel::kGlobalWalk && m_deep.nodes != nullptr && !m_planPinned; }
+  int32_t DeepSlices(int64_t rows) const {
+    const int64_t rb = m_deep.model.plan.rowsPerBlock;
+    return DeepWalkSlices((rows + rb - 1) / rb, (int64_t)m_deep.model.groups.size(), m_limits);
+  }
   // The walk behind PrepareRows, with its outputs set; true when the finalize kernel (`f`) has to follow.
   bool LaunchWalkFor(const float *walkInputs, int64_t rows, FinalizeParams &f, int32_t *leafIds, hipStream_t stream, const Workspace &ws,
                      hipEvent_t done);
@@ -160,7 +168,7 @@ private:
   bool FusesArgmax() const {
     return m_forest.numClasses > 0 && m_model.plan.treeSlices == 1 && m_model.plan.kernel == LaunchPlan::Kernel::kRowParallelLds;
   }
-  WalkParams MakeWalkParams(const float *deviceInputs, int64_t rows) const;
+  WalkParams MakeWalkParams(const float *deviceInputs, int64_t rows, const PackedModel &model) const;
   // Sets the outputs of a walk; true when the finalize kernel has to follow.
   void SetParts(FinalizeParams &f, const WalkParams &p) const; // which partial sums the walk `p` leaves
   bool SetOutputs(WalkParams &p, float *out, int8_t *classOut, float *margins, float *probabilities, bool leafIds, const Workspace &ws) const;
@@ -207,6 +215,13 @@ private:
   DeviceStreamBundle *m_dStreamBundles = nullptr;
   int32_t m_streamBundles = 0, m_streamChains = 0;
   int32_t *m_dFewRowsClasses = nullptr;
+  struct DeepWalk { // (the forest's, like the bundles above)
+    bool packed = false;
+    PackedModel model; // plan, groups and sizes; the arrays are on the device
+    DeviceNode *nodes = nullptr, *bundleRoots = nullptr, *tailNodes = nullptr;
+    DeviceBundle *bundles = nullptr;
+    DeviceGroup *groups = nullptr;
+  } m_deep;
   void *m_smallHost = nullptr;      // pinned host memory the few-rows kernel reads rows from and leaves results in
 
   DeviceGlobalNode *m_dGlobalNodes = nullptr;

@@ -133,6 +133,58 @@ LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoSche
   return plan;
 }
 
+// Blocks of 1024 lanes, two per compute unit: 256 rows while their tile takes up to 52 KB, else 128 or 64.  A tree group is
+// one bundle of two trees for every tree thread, and the trees are cut where that fills the block's half of LDS (a quarter
+// more: then some groups are a tree short, and fewer rows are queued).  65536 rows through 40 trees of depth 16 (22000
+// nodes each, every child splits again with probability 0.88): 92 us node by node from global memory, 25 here; cut levels
+// 7 / 8 / 9 / 10 / 11 27.8 / 27.4 / 26.2 / 24.9 / 29.2, one tree a lane at the same levels 31.2 / 30.2 / 29.0 / 28.0 / 28.1, four
+// 25.7 / 25.3 / 26.4 at levels 8 to 10.  70 features: 109 us -> 33 with 128 rows a block (40 with 64), 100 features 133 -> 36,
+// 150 features 177 -> 54.
+bool ChooseDeepWalk(const Forest &forest, const DeviceLimits &limits, LaunchPlan *plan, std::vector<int32_t> *cuts) {
+  if (forest.numClasses > 0 || forest.trees.empty() || forest.numFeatures + 1 >= (1 << kTailFeatureBits)) return false;
+  const auto tileBytes = [&](int32_t rows) { return (int64_t)(forest.numFeatures + 1) * rows * 4; };
+  int32_t rows = 256;
+  while (rows > 64 && tileBytes(rows) > 52 * 1024) rows /= 2;
+  *plan = LaunchPlan();
+  plan->rowsPerBlock = rows;
+  plan->treeThreads = 1024 / rows;
+  plan->interleave = 2;
+  plan->deferTails = true;
+  const int64_t queues = (int64_t)(plan->ThreadsPerBlock() / 64) * kDeferBytesPerWave;
+  const int64_t room = std::min<int64_t>(65536, limits.ldsBytesPerBlock / 2 - tileBytes(rows) - queues - 1024);
+  const int64_t bundles = (int64_t)plan->treeThreads * plan->interleave;
+  const int64_t mostTop = std::min(room * 5 / 4 / bundles, room) / kNodeBytes - 4;
+  if (mostTop < 31) return false;
+  int64_t tails = 0; // nodes below the cuts
+  cuts->clear();
+  for (const Tree &tree : forest.trees) {
+    int64_t top = 0;
+    int32_t depth = 0, cut = -1;
+    std::vector<int32_t> level{0}, below;
+    for (; !level.empty(); ++depth) {
+      if (cut < 0 && top + (int64_t)level.size() > mostTop) cut = depth - 1;
+      if (cut < 0) top += (int64_t)level.size();
+      below.clear();
+      for (int32_t n : level) {
+        if (tree.IsLeaf(n)) continue;
+        below.push_back(tree.left[n]);
+        below.push_back(tree.right[n]);
+      }
+      level.swap(below);
+    }
+    cuts->push_back(cut < 0 ? depth - 1 : cut);
+    tails += (int64_t)tree.NumNodes() - top + 64;
+  }
+  if (tails >= kMaxTailNodes) return false;
+  plan->groupBytes = (int32_t)(std::min<int64_t>(room, std::max<int64_t>((bundles * mostTop + 4) * kNodeBytes, 1024)) & ~15);
+  return true;
+}
+
+// One round of blocks.  More slices (each stages the rows again) took 30 us with 4 and 34 with 5 where 2 take 25, one 28.
+int32_t DeepWalkSlices(int64_t rowBlocks, int64_t groups, const DeviceLimits &limits) {
+  return (int32_t)std::max<int64_t>(1, std::min<int64_t>(2LL * limits.computeUnits / std::max<int64_t>(1, rowBlocks), groups));
+}
+
 bool DeferTailsFit(const Forest &forest, LaunchPlan *plan) {
   if (plan->kernel != LaunchPlan::Kernel::kRowParallelLds || plan->WalkTile() != 1 || plan->quantizedRows || plan->rankRows16 ||
       plan->featureOffsetInWords || forest.numClasses > 0)

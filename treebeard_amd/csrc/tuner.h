@@ -51,6 +51,13 @@ LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoSche
 // feature's column and the waves' queues take.  The caller sets the flag.
 bool DeferTailsFit(const Forest &forest, LaunchPlan *plan);
 
+// A forest with a tree too big for an LDS tree group (LaunchPlan::Kernel::kGlobalWalk), walked with deferred tails instead of
+// node by node from global memory: the tops of its trees fit.  Sets a plan for PackWithCuts and the level every tree is cut
+// at; false where the form cannot hold the forest (classes, rows too wide, too many nodes below the cuts).
+bool ChooseDeepWalk(const Forest &forest, const DeviceLimits &limits, LaunchPlan *plan, std::vector<int32_t> *cuts);
+// How many blocks share a row block's tree groups.
+int32_t DeepWalkSlices(int64_t rowBlocks, int64_t groups, const DeviceLimits &limits);
+
 // Candidate plans for the timed search (the analytic choice comes first).
 std::vector<LaunchPlan> CandidatePlans(const Forest &forest, int64_t batchSize, const DeviceLimits &limits,
                                        const WalkOptions &walk = WalkOptions());
