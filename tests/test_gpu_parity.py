@@ -1290,6 +1290,24 @@ def test_rows_too_wide_for_lds_walk_from_global_memory(tmp_path, features, rows)
     check_against_oracle(runner, forest, x)
 
 
+@pytest.mark.parametrize("slices", [15, 16, 17, 31])
+@pytest.mark.parametrize("rows", [1, 63, 65, 2048, 2049])
+def test_finalize_of_many_slices(synth_model, rows, slices):
+    """Class sums of a few rows over many tree slices, either side of the number of slices and of sums (2048 x 8) at which 64
+    sums a block take over."""
+    x = synth.CONFIGS[3].batch_rows(rows, seed_offset=9)
+    runner = make_runner(synth_model(3), rows)
+    runner.set_plan(64, 2, 2, 8192, slices)
+    assert "treeSlices=%d " % slices in runner.describe_plan()
+    forest = model_io.load_xgboost_json(synth_model(3))
+    check_against_oracle(runner, forest, x)
+    dx = torch.from_numpy(x).cuda()
+    margins = torch.zeros((rows, 8), dtype=torch.float32, device="cuda")
+    torch.cuda.synchronize()
+    runner.run_device_multiclass(dx.data_ptr(), rows, None, margins.data_ptr(), None)
+    np.testing.assert_allclose(margins.cpu().numpy(), cpu_oracle.predict(forest, x)[1], rtol=RTOL_SUM, atol=1e-7)
+
+
 def test_time_kernels_leaves_the_outputs_of_one_run(synth_model):
     """Repeated launches inside tbmi_time_kernels (wide finalize of a sliced classifier included) leave the same
     results as one tbmi_run_device."""

@@ -1367,7 +1367,8 @@ __global__ void __launch_bounds__(256) FinalizeKernel(const FinalizeParams p) {
 }
 
 // Classifiers: the block's rows x classes are read as they lie (coalesced; a lane per row read a line per class and all
-// of them three times: 13 us for 65537 rows x 8 classes x 2 slices), meet in LDS, and the rows are finished there.
+// of them three times: 13 us for 65537 rows x 8 classes x 2 slices), meet in LDS, and the rows are finished there.  A sum per
+// lane: blocks of 128 rows, whose lanes wait for memory four times in a row, took 4.7 us longer with sums and softmax.
 constexpr int kFinalizeLds = 4096; // doubles of sums a block holds
 
 __global__ void __launch_bounds__(256) FinalizeClassesKernel(const FinalizeParams p, int rowsPerBlock) {
@@ -1380,9 +1381,13 @@ __global__ void __launch_bounds__(256) FinalizeClassesKernel(const FinalizeParam
   const int tid = threadIdx.x, threads = blockDim.x;
   for (int e = tid; e < valid * C; e += threads) {
     const int r = e / C, c = e - r * C;
+    // (the first two parts are on their way while the divisions that count the parts run; a slot is there, filled or not)
+    const double *at = p.partial + row0 * C + e;
+    const double first = at[0], second = p.treeSlices > 1 ? at[p.rows * C] : 0.0;
     const int parts = PartsOfRow(p, row0 + r);
-    double margin = p.initialValue;
-    for (int s = 0; s < parts; ++s) margin += p.partial[((int64_t)s * p.rows + row0) * C + e];
+    double margin = p.initialValue + first;
+    if (parts > 1) margin += second;
+    for (int s = 2; s < parts; ++s) margin += at[(int64_t)s * p.rows * C];
     sums[r * stride + c] = margin;
     if (p.margins) p.margins[row0 * C + e] = (float)margin;
   }
@@ -1434,31 +1439,37 @@ __global__ void __launch_bounds__(256) FinalizeManyClassesKernel(const FinalizeP
       p.numClasses, row, p.out, p.classOut, p.margins, p.probabilities);
 }
 
-// Small batches split over many tree slices (kWideFinalizeSlices or more): one wave per (row, class).  The lanes fetch the slice
-// partials side by side (one memory latency instead of one per slice), each adds its slices in slice
-// order, and a fixed butterfly combines the lanes - the order of additions depends only on the number
-// of slices.
-constexpr int64_t kWideFinalizeItems = 8192; // (65536 took 15 us for 8192 rows x 8 classes)
+// Small batches split over many tree slices (kWideFinalizeSlices or more): 64 (row, class) sums a block, a lane each, and its
+// waves share the slices, so that a lane waits for few loads and a wave reads 512 contiguous bytes.  (A wave per sum, lanes
+// along the slices, read a 64-byte piece of memory for each of its 8 bytes: 4096 rows x 32 slices 3.0 us, 2.5 here; the call 15.1 and 13.9.)  Each wave
+// adds its slices in slice order, the waves are added in order: the order of additions depends on the number of slices alone.
+constexpr int64_t kWideFinalizeItems = 16384; // (a call of 2048 rows x 8 classes 33.3 us without, 31.5 with; 64000 sums 38.5 and 39.9)
+constexpr int kWideFinalizeWaves = 8;
 
-__global__ void __launch_bounds__(256) FinalizeWideKernel(const FinalizeParams p) {
-  const int lane = threadIdx.x & 63;
-  const int64_t item = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  const int Cn = p.numClasses > 0 ? p.numClasses : 1;
-  if (item >= p.rows * Cn) return; // (whole waves leave together)
-  const int64_t row = item / Cn;
-  const int c = (int)(item - row * Cn);
-  double sum = 0.0;
-  const int parts = PartsOfRow(p, row);
-  for (int s = lane; s < parts; s += 64) sum += p.partial[((int64_t)s * p.rows + row) * Cn + c];
-  for (int m = 1; m <= 32; m <<= 1) sum += ShuffleXor(sum, m); // (ascending: see ShuffleXor)
+__global__ void __launch_bounds__(kWideFinalizeWaves * 64) FinalizeWideKernel(const FinalizeParams p) {
+  __shared__ double meet[kWideFinalizeWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t items = p.rows * (p.numClasses > 0 ? p.numClasses : 1);
+  const int64_t item = (int64_t)blockIdx.x * 64 + lane;
+  if (item < items) {
+    const int parts = PartsOfRow(p, p.numClasses > 0 ? item / p.numClasses : item);
+    double sum = 0.0;
+#pragma unroll 4
+    for (int s = wave; s < parts; s += kWideFinalizeWaves) sum += p.partial[(int64_t)s * items + item];
+    meet[wave][lane] = sum;
+  }
+  __syncthreads();
+  if (wave != 0 || item >= items) return;
+  double sum = meet[0][lane];
+  for (int w = 1; w < kWideFinalizeWaves; ++w) sum += meet[w][lane];
   const double margin = p.initialValue + sum;
   if (p.numClasses == 0) {
-    if (lane == 0) p.out[row] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
+    p.out[item] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
     return;
   }
   // classifiers: the class sum goes into the spare slot behind the last slice; FinalizeClassesKernel (1 slice, reading
   // that slot) does the rest.  The slices themselves stay as they are, so the launch can be repeated.
-  if (lane == 0) p.partial[((int64_t)p.treeSlices * p.rows + row) * Cn + c] = margin - p.initialValue;
+  p.partial[(int64_t)p.treeSlices * items + item] = margin - p.initialValue;
 }
 
 // ---------------------------------------------------------------------------
@@ -2007,9 +2018,8 @@ hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
   const int Cn = p.numClasses > 0 ? p.numClasses : 1;
   FinalizeParams q = p;
-  if (p.treeSlices >= kWideFinalizeSlices && p.rows * Cn <= kWideFinalizeItems) { // few rows, many slices: a wave per (row, class)
-    const int64_t waves = p.rows * Cn;
-    hipError_t e = StartKernel(&FinalizeWideKernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, stream,
+  if (p.treeSlices >= kWideFinalizeSlices && p.rows * Cn <= kWideFinalizeItems) { // few rows, many slices
+    hipError_t e = StartKernel(&FinalizeWideKernel, dim3((unsigned)((p.rows * Cn + 63) / 64)), dim3(kWideFinalizeWaves * 64), 0, stream,
                                p.numClasses == 0 ? p.done : nullptr, p);
     if (e != hipSuccess || p.numClasses == 0) return e;
     q.partial = p.partial + (int64_t)p.treeSlices * p.rows * Cn; // the class sums now sit in the spare slot
@@ -2018,7 +2028,7 @@ hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   }
   if (q.numClasses > 0) {
     // (rows of a block: as many as LDS holds, fewer where that leaves compute units without a block)
-    const int64_t perBlock = std::max<int64_t>(1, std::min<int64_t>({256, kFinalizeLds / (q.numClasses | 1), std::max<int64_t>(8, q.rows / 512)}));
+    const int64_t perBlock = std::max<int64_t>(1, std::min<int64_t>({256, kFinalizeLds / (q.numClasses | 1), std::max<int64_t>(8, 256 / q.numClasses)}));
     const int64_t blocks = (q.rows + perBlock - 1) / perBlock;
     const size_t ldsBytes = (size_t)perBlock * ((size_t)(q.numClasses | 1) + 2) * sizeof(double);
     if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
