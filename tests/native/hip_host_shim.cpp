@@ -716,20 +716,24 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
     for (int64_t row = 0; row < p.rows; ++row) {
       double sum = 0.0;
       for (int b = first; b < last; ++b) {
-        const DeviceStreamBundle &bd = p.bundles[b];
-        const uint32_t words = (bd.piecesDepth >> 16) * 4, depth = bd.piecesDepth & 0xFFFFu;
-        if (words * 4 > kStreamBundleBytes || bd.wordBegin % 4) std::abort();
+        const uint32_t begin = p.bundles[b], words = kStreamBundleBytes / 4;
+        if (begin % 4) std::abort();
+        DeviceStreamHead heads[2];
+        std::memcpy(heads, p.words + begin, sizeof(heads));
+        const uint32_t depth = heads[0].depth;
+        if (heads[1].depth != depth || p.words[begin + words - 1] == 0xFFFFFFFFu) std::abort(); // (the copy reads that far)
         for (int k = 0; k < 2 * p.chains; ++k) {
-          const uint32_t root = (bd.roots[k / 2] >> (16 * (k & 1)) & 0xFFFFu) / 4;
+          const uint32_t root = heads[k & 1].roots[k / 2] / 4u;
+          if (root % 2) std::abort(); // (children are read two words at a time)
           uint32_t at = 0;
           for (uint32_t d = 0; d < depth; ++d) {
             if (root + at >= words) std::abort(); // a node outside the bundle
-            const uint32_t node = p.words[bd.wordBegin + root + at], f = node >> 5 & 0x7FFu;
+            const uint32_t node = p.words[begin + root + at], f = node >> 5 & 0x7FFu;
             if ((int)f > F || (node & 31u)) std::abort();
             const uint32_t rank = (int)f == F ? 0u : p.ranks[((row / 64) * F + f) * 64 + row % 64];
             at = 2 * (node >> 16 & 0xFFu) + (rank < node >> 24 ? 0u : 1u);
           }
-          sum += (double)p.values[bd.valueBegin[k] + at];
+          sum += (double)p.values[heads[k & 1].valueBegin[k / 2] + at];
         }
       }
       if (p.slices > 1) p.partial[(int64_t)slice * p.rows + row] = sum;

@@ -47,3 +47,25 @@ def test_streamed_bundles_match_the_oracle(tmp_path, features, trees, depth, spl
         call(dx.data_ptr(), out.data_ptr(), rows, stream.cuda_stream)
         stream.synchronize()
         close(forest, out.cpu().numpy(), expected)
+
+
+@pytest.mark.parametrize("trees", [3, 150])
+def test_workgroups_that_take_several_row_blocks(tmp_path, trees):
+    """More blocks of 32 rows than compute units: two and three per workgroup, the last of some only; three trees leave most
+    waves without a bundle, 150 leave them unequal numbers."""
+    rng = np.random.Generator(np.random.PCG64(trees))
+    features, levels = 600, 31
+    grid = np.sort(rng.standard_normal(levels)).astype(np.float32)
+    forest_trees = [synth._grow_tree(rng, 6, lambda d, s: 0.9, lambda: (rng.integers(0, features), grid[rng.integers(0, levels)]), rng.normal)
+                    for _ in range(trees)]
+    path = str(tmp_path / "wide.json")
+    synth.write_xgboost_json(path, forest_trees, features)
+    forest = model_io.load_xgboost_json(path)
+    runner = make_runner(path, 20000)
+    assert "quantizedRows=1" in runner.describe_plan()
+    x = rng.standard_normal((2 * 8192 + 4 * 32 + 5, features), dtype=np.float32)
+    expected = cpu_oracle.predict(forest, x)[0]
+    counts = [c for c in (8192, 8192 + 1, 8192 + 700, len(x)) if c > limit_of(runner)]
+    assert counts
+    for count in counts:
+        close(forest, gpu_predict(runner, x[:count]), expected[:count])

@@ -153,13 +153,17 @@ constexpr uint32_t kFewRowsLeaf = 0xFFFFu;
 // its place: as a left child it tests the pad feature (rank 0) against 1, as a right child anything against 0.  The
 // leaves a walk of the bundle's depth reaches with its last step are never read as nodes: they have no words.
 // Predictions stand in an array of their own, one place per word (the last leaves' included).
-struct alignas(64) DeviceStreamBundle { // (whole words: one scalar load)
-  uint32_t wordBegin;     // multiple of 4; word 0 is the root of a tree of one leaf, which fills empty places
-  uint32_t piecesDepth;   // 16-byte pieces << 16 | depth of the deepest tree
-  uint32_t roots[4];      // byte offsets of trees 2 * k (low half) and 2 * k + 1, which the two halves of a wave walk
-  uint32_t valueBegin[8]; // of every tree, in the array of predictions (entry 0 is 0.0: the empty places')
-  uint32_t reserved[2];
+//
+// A bundle's image begins with a DeviceStreamHead for each half of the wave that walks it, then the trees; it starts on a
+// 16-byte piece and the copy takes kStreamBundleBytes whatever its size (the words end with as many that belong to none).
+struct alignas(16) DeviceStreamHead {
+  uint16_t roots[4];      // byte offsets of the half's trees in the image
+  uint32_t depth;         // of the deepest tree of the bundle
+  uint32_t reserved;
+  uint32_t valueBegin[4]; // of every tree, in the array of predictions (entry 0 is 0.0: the empty places')
 };
+static_assert(sizeof(DeviceStreamHead) == 32, "two 16-byte LDS reads");
+constexpr uint32_t kStreamHeadWords = 2 * sizeof(DeviceStreamHead) / 4;
 constexpr int kStreamMaxChains = 4;          // trees a lane walks side by side (2 or 4); two lanes share a bundle's trees
 constexpr uint32_t kStreamBundleBytes = 4096;
 constexpr int32_t kStreamMaxFeatures = 2047;

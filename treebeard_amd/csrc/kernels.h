@@ -167,11 +167,12 @@ struct RankStreamParams {
   const uint8_t *ranks = nullptr;
   const uint32_t *words = nullptr; // PackRankStream
   const float *values = nullptr;
-  const DeviceStreamBundle *bundles = nullptr;
+  const uint32_t *bundles = nullptr; // first words
   int64_t rows = 0;
   int32_t numFeatures = 0, numBundles = 0;
   int32_t chains = kStreamMaxChains;
   int32_t slices = 1;              // blocks that share a row block's bundles
+  int32_t computeUnits = 256;
   int32_t transform = 0;
   double initialValue = 0.0;
   float *out = nullptr;            // one slice
@@ -181,6 +182,7 @@ struct RankStreamParams {
 
 // Waves of a block of LaunchRankStream: as many as have room for two bundles each beside the rows' ranks.
 constexpr int kStreamMaxWaves = 16;
+constexpr int kStreamTilePieces = 6; // 16-byte pieces of the next rows' ranks that a lane holds in registers
 inline int StreamWaves(int32_t numFeatures) {
   const int64_t tile = ((int64_t)(numFeatures + 1) * kStreamRows + 15) & ~(int64_t)15;
   return (int)std::min<int64_t>(kStreamMaxWaves, (160 * 1024 - tile) / (2 * kStreamBundleBytes));

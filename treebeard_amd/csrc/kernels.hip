@@ -1562,121 +1562,176 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
 // four chains (two, in bundles of four trees, where bigger trees leave bundles of eight short); 32 rows instead of 64
 // leave the room (twelve waves x two buffers), and 4-byte nodes halve what a bundle takes: a step is a 4-byte node read
 // and a one-byte rank read.  Leaf values stay in global memory, one gather per tree, issued a bundle ahead of its use.
-// What bounds it is the latency of the two dependent LDS reads of a step at twelve waves a CU (LDS pipes 46 % busy, 13 %
-// of it bank conflicts of the rank reads; VALUs 62 %).
-// Walk of 262144 rows x 2000 features, 1000 trees of depth 8, on the same ranks: 1.33 ms with tree groups, 0.80-0.82 here;
-// of 20000 rows: 0.099 + 0.005 for the finalize kernel, 0.076 here.
+//
+// With three waves a SIMD every wait in a wave's chain is seen.  So: the lane holds the word it stands on and reads both
+// children (8 bytes side by side, at the price of 4) together with the rank, one LDS round trip a level instead of two; a
+// bundle's roots and depth stand in its image, its place comes through a vector load (a scalar load took its latency every
+// bundle); and a workgroup stays, with the next rows' ranks on their way to registers while its last bundle is walked (it
+// has its compute unit's LDS to itself: nothing else walks while it loads).  Walk of 262144 rows x 2000 features, 1000 trees
+// of depth 8, on the same ranks: 1.33 ms with tree groups, 0.84 with two trips a level and a workgroup per 32 rows, 0.76
+// here, and the whole call 1.308 -> 1.223; 20000 rows 126 -> 120 us.  A level takes 0.067 ms (a wave's eight LDS reads and 20
+// VALU instructions in 34 cycles of its compute unit: LDS pipes 70 %, VALUs 60 % busy), the leaf values 0.065, the rest 0.16.
 // ---------------------------------------------------------------------------
 template <int K> // chains
 __global__ void __launch_bounds__(kStreamMaxWaves * 64)
 RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__ words, const float *__restrict__ values,
-                 const DeviceStreamBundle *__restrict__ bundles, int64_t rows, int F, int numBundles, int slices, int transform,
+                 const uint32_t *__restrict__ bundles, int64_t rows, int F, int numBundles, int slices, int transform,
                  double initialValue, float *__restrict__ out, double *__restrict__ partial) {
   extern __shared__ __align__(16) unsigned char lds[]; // [feature][32 rows] ranks, pad feature included | two bundles per wave
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int waves = blockDim.x >> 6;
   // The two halves of a 64-row rank tile share its cache lines: their blocks are 8 apart in launch order (same XCD).
-  const uint32_t linear = blockIdx.x;
-  const int64_t block = (int64_t)(linear >> 4) * 16 + (int64_t)((linear & 7u) * 2u + ((linear >> 3) & 1u));
-  if (block * kStreamRows >= rows) return;
+  const auto blockOf = [](uint32_t linear) { return (int64_t)(linear >> 4) * 16 + (int64_t)((linear & 7u) * 2u + ((linear >> 3) & 1u)); };
+  const uint32_t padded = (uint32_t)((rows + 16 * kStreamRows - 1) / (16 * kStreamRows)) * 16u;
+  const auto blockFrom = [&](uint32_t linear) { // the first that has rows, of those this workgroup takes
+    while (linear < padded && blockOf(linear) * kStreamRows >= rows) linear += gridDim.x;
+    return linear;
+  };
+  uint32_t linear = blockFrom(blockIdx.x);
+  if (linear >= padded) return;
   const uint32_t tileBytes = ((uint32_t)(F + 1) * kStreamRows + 15u) & ~15u;
   const uint32_t mine = tileBytes + (uint32_t)wave * (2u * kStreamBundleBytes); // this wave's two bundles
+  const int pieces = F * 2; // of a row block's ranks: piece p is half (p & 1) of the 32 bytes of feature p / 2
+  const auto pieceOf = [&](uint32_t of, int p) {
+    const int64_t block = blockOf(of);
+    return ranks + (block >> 1) * F * 64 + (block & 1) * kStreamRows + (int64_t)(p >> 1) * 64 + (p & 1) * 16;
+  };
   // 16 bytes per lane to LDS address DST + 16 * lane.  (Not the builtin: while one of those is outstanding the compiler
   // awaits LDS reads only all together, and here one nearly always is.  The waits for these copies are the explicit ones.)
 #define TBAMD_STREAM_COPY(SRC, DST)                                                                                    \
   asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(SRC), "s"(DST) : "memory", "m0");
-  {
-    const uint8_t *src = ranks + (block >> 1) * F * 64 + (block & 1) * kStreamRows;
-    const int pieces = F * 2; // piece p: half (p & 1) of the 32 bytes of feature p / 2
-    for (int first = wave * 64; first < pieces; first += waves * 64) {
-      const int p = first + lane;
-      if (p < pieces) TBAMD_STREAM_COPY(src + (int64_t)(p >> 1) * 64 + (p & 1) * 16, (uint32_t)first * 16u)
-    }
-    if (tid < kStreamRows / 4) *reinterpret_cast<uint32_t *>(lds + (uint32_t)F * kStreamRows + tid * 4) = 0; // pad feature
-  }
+  for (int p0 = wave * 64; p0 < pieces; p0 += waves * 64)
+    if (p0 + lane < pieces) TBAMD_STREAM_COPY(pieceOf(linear, p0 + lane), (uint32_t)p0 * 16u)
+  if (tid < kStreamRows / 4) *reinterpret_cast<uint32_t *>(lds + (uint32_t)F * kStreamRows + tid * 4) = 0; // pad feature
   const int first = (int)((int64_t)numBundles * blockIdx.y / slices), last = (int)((int64_t)numBundles * (blockIdx.y + 1) / slices);
-#define TBAMD_STREAM_BUNDLE(BD, BUFFER)                                                                                \
+  const auto bundlesOf = [&](int w) { return (last - first - w + waves - 1) / waves; }; // of wave w, per row block
+#define TBAMD_STREAM_BUNDLE(BEGIN, BUFFER)                                                                             \
   {                                                                                                                    \
-    const U32x4 *src = reinterpret_cast<const U32x4 *>(words + (BD).wordBegin);                                        \
-    const int pieces = (int)((BD).piecesDepth >> 16);                                                                  \
-    for (int q = 0; q < pieces; q += 64)                                                                               \
-      if (q + lane < pieces) TBAMD_STREAM_COPY(src + q + lane, (BUFFER) + (uint32_t)q * 16u)                           \
+    const U32x4 *src = reinterpret_cast<const U32x4 *>(words + (BEGIN)) + lane;                                        \
+    _Pragma("unroll") for (uint32_t q = 0; q < kStreamBundleBytes; q += 1024u)                                         \
+        TBAMD_STREAM_COPY(src + q / 16u, (BUFFER) + q)                                                                 \
   }
-  // descriptors are requested two bundles ahead
-  int b = first + wave;
-  DeviceStreamBundle bd{}, nextBd{};
-  if (b < last) {
-    bd = bundles[b];
-    if (b + waves < last) nextBd = bundles[b + waves];
-    TBAMD_STREAM_BUNDLE(bd, mine)
+  // The bundle walked next, and the one behind it; behind the last one comes the first, for the next row block.
+  const int begin = first + wave;
+  const auto after = [&](int b) { return b + waves < last ? b + waves : begin; };
+  // (The places of the bundles come through vector loads, a bundle ahead: a scalar load in flight would make every LDS read's
+  // wait one for it.  What else is to be known of a bundle stands in its image.)
+  uint32_t zero;
+  asm volatile("v_mov_b32 %0, 0" : "=v"(zero));
+  uint32_t nextBegin = 0;
+  if (begin < last) {
+    const uint32_t now = bundles[begin];
+    TBAMD_STREAM_BUNDLE(now, mine)
+    nextBegin = bundles[(uint32_t)after(begin) + zero];
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads(); // the rows are there; from here on the waves run on their own
+  __syncthreads(); // the rows are there; until they are through, the waves run on their own
 
   const uint32_t row = (uint32_t)lane & 31u;
   const bool upper = lane >= 32;
-  double acc = 0.0;
-  float leaf[K];
-  uint32_t at[K]; // where the leaf values of the bundle before lie (entry 0: none)
-#pragma unroll
-  for (int k = 0; k < K; ++k) leaf[k] = 0.0f, at[k] = 0u;
   uint32_t buffer = mine;
-  for (; b < last; b += waves) {
-    const DeviceStreamBundle afterBd = bundles[b + 2 * waves < last ? b + 2 * waves : b];
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this bundle, and the leaf values of the one before the last
+  for (uint32_t pass = 0;; ++pass) {
+    const uint32_t nextLinear = blockFrom(linear + gridDim.x);
+    const bool more = nextLinear < padded;
+    U32x4 nextRanks[kStreamTilePieces];
+#define TBAMD_STREAM_NEXT_ROWS                                                                                         \
+  _Pragma("unroll") for (int i = 0; i < kStreamTilePieces; ++i) {                                                      \
+    const int p = (i * waves + wave) * 64 + lane;                                                                      \
+    nextRanks[i] = *reinterpret_cast<const U32x4 *>(pieceOf(nextLinear, p < pieces ? p : pieces - 1));                 \
+  }
+    double acc = 0.0;
+    float leaf[K];
+    uint32_t at[K]; // where the leaf values of the bundle before lie (entry 0: none)
+#pragma unroll
+    for (int k = 0; k < K; ++k) leaf[k] = 0.0f, at[k] = 0u;
+    if (begin >= last && more) TBAMD_STREAM_NEXT_ROWS
+    for (int b = begin; b < last; b += waves) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); // this bundle, and the leaf values of the one before the last
+      const uint32_t follows = __builtin_amdgcn_readfirstlane(nextBegin);
+#pragma unroll
+      for (int k = 0; k < K; ++k) acc += (double)leaf[k];
+#pragma unroll
+      for (int k = 0; k < K; ++k) leaf[k] = values[at[k]];
+      const uint32_t other = buffer == mine ? mine + kStreamBundleBytes : mine;
+      if (b + waves < last || more) TBAMD_STREAM_BUNDLE(follows, other)
+      nextBegin = bundles[(uint32_t)after(after(b)) + zero];
+      if (b + waves >= last && more) TBAMD_STREAM_NEXT_ROWS
+      const U32x4 head = LdsLoadQuad(buffer + (upper ? (uint32_t)sizeof(DeviceStreamHead) : 0u));
+      const U32x4 valueBegin = LdsLoadQuad(buffer + (upper ? (uint32_t)sizeof(DeviceStreamHead) : 0u) + 16u);
+      const int depth = (int)__builtin_amdgcn_readfirstlane(head.z);
+      uint32_t tree[K], node[K]; // where the words of a tree lie, and the word the lane stands on
+#pragma unroll
+      for (int k = 0; k < K; ++k) {
+        tree[k] = buffer + (k & 1 ? head[k / 2] >> 16 : head[k / 2] & 0xFFFFu);
+        node[k] = *(const __attribute__((address_space(3))) uint32_t *)(uintptr_t)tree[k];
+      }
+      // (awaited here: in the loop the compiler would wait for them, and so for other chains' reads, at every level)
+#pragma unroll
+      for (int k = 0; k < K; ++k) asm volatile("" : "+v"(node[k]));
+#pragma unroll 2
+      for (int d = 1; d < depth; ++d) {
+        U32x2 children[K];
+        uint32_t rank[K];
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          rank[k] = LdsLoadByte((node[k] & 0xFFE0u) | row);
+          children[k] = LdsLoadNode((((node[k] >> 16) & 0xFFu) << 3) + tree[k]);
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          // (both children are read: left to itself the compiler reads one, when the rank is there)
+          asm volatile("" : "+v"(rank[k]), "+v"(children[k]));
+          node[k] = rank[k] < (node[k] >> 24) ? children[k].x : children[k].y;
+        }
+      }
+      uint32_t rank[K]; // (the last level's words are not there: only which they are counts)
+#pragma unroll
+      for (int k = 0; k < K; ++k) rank[k] = LdsLoadByte((node[k] & 0xFFE0u) | row);
+#pragma unroll
+      for (int k = 0; k < K; ++k) asm volatile("" : "+v"(rank[k]));
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        at[k] = valueBegin[k] + (depth > 0 ? ((node[k] >> 15) & 0x1FEu) + (rank[k] < (node[k] >> 24) ? 0u : 1u) : 0u);
+      buffer = other;
+    }
 #pragma unroll
     for (int k = 0; k < K; ++k) acc += (double)leaf[k];
 #pragma unroll
-    for (int k = 0; k < K; ++k) leaf[k] = values[at[k]];
-    const uint32_t other = buffer == mine ? mine + kStreamBundleBytes : mine;
-    if (b + waves < last) TBAMD_STREAM_BUNDLE(nextBd, other)
-    // (the descriptor's scalar load is done here: it would have the same effect on the LDS reads' waits)
-    asm volatile("" ::"s"(afterBd.wordBegin), "s"(afterBd.valueBegin[7]));
-    uint32_t left[K], right[K], addr[K]; // where the two words of a tree's pair 0 lie
+    for (int k = 0; k < K; ++k) acc += (double)values[at[k]];
+    acc += ShuffleXor(acc, 32);
+    // A wave's sums go where its last bundle was: its other buffer may hold the first one for the next rows.
+    const auto meetOf = [&](int w) {
+      const uint32_t walked = (uint32_t)bundlesOf(w) * (pass + 1u);
+      return reinterpret_cast<double *>(lds + tileBytes + (uint32_t)w * (2u * kStreamBundleBytes) + (walked & 1u ? 0u : kStreamBundleBytes));
+    };
+    if (lane < kStreamRows) meetOf(wave)[lane] = acc;
+    __syncthreads(); // the sums are there, nobody reads ranks any more
+    if (more) {
 #pragma unroll
-    for (int k = 0; k < K; ++k) {
-      left[k] = buffer + ((bd.roots[k] >> (upper ? 16 : 0)) & 0xFFFFu);
-      right[k] = left[k] + 4u;
-      addr[k] = left[k];
-    }
-    const int depth = (int)(bd.piecesDepth & 0xFFFFu);
-#pragma unroll 2
-    for (int d = 0; d < depth; ++d) {
-#pragma unroll
-      for (int k = 0; k < K; ++k) {
-        const uint32_t node = *(const __attribute__((address_space(3))) uint32_t *)(uintptr_t)addr[k];
-        const uint32_t rank = LdsLoadByte((node & 0xFFE0u) | row);
-        addr[k] = (((node >> 16) & 0xFFu) << 3) + (rank < (node >> 24) ? left[k] : right[k]);
+      for (int i = 0; i < kStreamTilePieces; ++i) {
+        const int p = (i * waves + wave) * 64 + lane;
+        if (p < pieces) *reinterpret_cast<U32x4 *>(lds + (uint32_t)p * 16u) = nextRanks[i];
       }
     }
-#pragma unroll
-    for (int k = 0; k < K; ++k) at[k] = (upper ? bd.valueBegin[2 * k + 1] : bd.valueBegin[2 * k]) + ((addr[k] - left[k]) >> 2);
-    bd = nextBd;
-    nextBd = afterBd;
-    buffer = other;
+    const int64_t r = blockOf(linear) * kStreamRows + tid;
+    if (tid < kStreamRows && r < rows) {
+      double sum = 0.0;
+      for (int w = 0; w < waves; ++w) sum += meetOf(w)[tid];
+      if (partial) {
+        partial[(int64_t)blockIdx.y * rows + r] = sum;
+      } else {
+        const double margin = initialValue + sum;
+        out[r] = (float)(transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
+      }
+    }
+    if (!more) return;
+    __syncthreads(); // the next rows are there, the sums are read
+    linear = nextLinear;
   }
-#pragma unroll
-  for (int k = 0; k < K; ++k) acc += (double)leaf[k];
-#pragma unroll
-  for (int k = 0; k < K; ++k) acc += (double)values[at[k]];
+#undef TBAMD_STREAM_NEXT_ROWS
 #undef TBAMD_STREAM_BUNDLE
 #undef TBAMD_STREAM_COPY
-  acc += ShuffleXor(acc, 32);
-  __syncthreads(); // nobody reads ranks any more
-  double *meet = reinterpret_cast<double *>(lds); // [wave][row]
-  if (lane < kStreamRows) meet[wave * kStreamRows + lane] = acc;
-  __syncthreads();
-  if (tid >= kStreamRows || block * kStreamRows + tid >= rows) return;
-  double sum = 0.0;
-  for (int w = 0; w < waves; ++w) sum += meet[w * kStreamRows + tid];
-  const int64_t r = block * kStreamRows + tid;
-  if (partial) {
-    partial[(int64_t)blockIdx.y * rows + r] = sum;
-  } else {
-    const double margin = initialValue + sum;
-    out[r] = (float)(transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
-  }
 }
 
 // The ceiling on dynamic LDS is an attribute of each kernel on each device: it is raised once per kernel and
@@ -2006,7 +2061,10 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
   const int64_t blocks = ((p.rows + kStreamRows - 1) / kStreamRows + 15) / 16 * 16;
   const size_t ldsBytes = (((size_t)(p.numFeatures + 1) * kStreamRows + 15) & ~(size_t)15) + (size_t)waves * 2 * kStreamBundleBytes;
   if (blocks > 0x7FFFFFFF || ldsBytes > 160 * 1024) return hipErrorInvalidValue;
-  const dim3 grid((unsigned)blocks, (unsigned)p.slices), block((unsigned)waves * 64);
+  if ((int64_t)p.numFeatures * 2 > (int64_t)waves * 64 * kStreamTilePieces) return hipErrorInvalidValue;
+  // (a workgroup has a compute unit's LDS to itself and goes on with other rows; multiples of 16 keep the XCDs' row blocks)
+  const int64_t groups = std::min<int64_t>(blocks, std::max(16, p.computeUnits / 16 * 16));
+  const dim3 grid((unsigned)groups, (unsigned)p.slices), block((unsigned)waves * 64);
   hipError_t e = p.chains == 4 ? AllowFullLds<&RankStreamKernel<4>>() : AllowFullLds<&RankStreamKernel<2>>();
   if (e != hipSuccess) return e;
   return StartKernel(p.chains == 4 ? &RankStreamKernel<4> : &RankStreamKernel<2>, grid, block, ldsBytes, stream, p.done, p.ranks, p.words,

@@ -462,22 +462,27 @@ RankStreamModel PackRankStream(const Forest &input) {
       // as many trees as fit, each with the words the deepest of them (the last: they come by depth) asks for
       size_t count = 0;
       for (size_t n = 1; n <= (size_t)(2 * chains) && next + n <= order.size(); ++n) {
-        uint32_t words = 2 + 3;
+        uint32_t words = kStreamHeadWords + 2 + 3;
         for (size_t k = 0; k < n; ++k) words += wordsOf(order[next + k], depth[(size_t)order[next + n - 1]]);
         if (words * 4 > kStreamBundleBytes && n > 1) break; // (a tree alone always fits)
         count = n;
       }
       const int32_t deepest = depth[(size_t)order[next + count - 1]];
-      DeviceStreamBundle b{};
-      b.wordBegin = (uint32_t)sm.words.size();
+      const uint32_t begin = (uint32_t)sm.words.size();
+      DeviceStreamHead heads[2]{};
+      for (DeviceStreamHead &head : heads) {
+        for (uint16_t &root : head.roots) root = kStreamHeadWords * 4; // (the empty tree)
+        head.depth = (uint32_t)deepest;
+      }
+      sm.words.resize(begin + kStreamHeadWords);
       sm.words.insert(sm.words.end(), {leafWord(0, false), 0u}); // the empty tree
       for (size_t k = 0; k < count; ++k) {
         const int32_t t = order[next + k];
         const Tree &tree = forest.trees[(size_t)t];
         const size_t at = sm.words.size(), valueAt = sm.values.size();
         const uint32_t limit = wordsOf(t, deepest);
-        b.roots[k / 2] |= (uint32_t)(at - b.wordBegin) * 4 << (16 * (k & 1));
-        b.valueBegin[k] = (uint32_t)valueAt;
+        heads[k & 1].roots[k / 2] = (uint16_t)((at - begin) * 4);
+        heads[k & 1].valueBegin[k / 2] = (uint32_t)valueAt;
         sm.words.resize(at + limit, 0u);
         sm.values.resize(valueAt + tree.NumNodes() + 1, 0.0f);
         struct Place { int32_t node; uint32_t word; };
@@ -500,11 +505,12 @@ RankStreamModel PackRankStream(const Forest &input) {
         }
       }
       while (sm.words.size() % 4) sm.words.push_back(0u);
-      b.piecesDepth = (uint32_t)((sm.words.size() - b.wordBegin) / 4) << 16 | (uint32_t)deepest;
+      std::memcpy(sm.words.data() + begin, heads, sizeof(heads));
       if (sm.words.size() > 0x7FFFFFF0u) throw Error("forest has too many nodes");
-      sm.bundles.push_back(b);
+      sm.bundles.push_back(begin);
       next += count;
     }
+    sm.words.resize(sm.words.size() + kStreamBundleBytes / 4, 0u);
   };
   // four chains where bundles of eight trees are mostly full: a chain of empty places costs what any other does
   pack(kStreamMaxChains);

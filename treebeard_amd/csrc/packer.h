@@ -159,7 +159,7 @@ FewRowsModel PackFewRows(const Forest &forest);
 struct RankStreamModel {
   std::vector<uint32_t> words;
   std::vector<float> values;
-  std::vector<DeviceStreamBundle> bundles; // by depth
+  std::vector<uint32_t> bundles;           // each one's first word; by depth
   int32_t chains = kStreamMaxChains;       // trees per bundle: twice as many
 };
 RankStreamModel PackRankStream(const Forest &forest);

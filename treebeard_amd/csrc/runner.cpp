@@ -554,6 +554,7 @@ bool InferenceRunner::LaunchWalkFor(const float *walkInputs, int64_t rows, Final
     p.numFeatures = m_forest.numFeatures;
     p.numBundles = m_streamBundles;
     p.chains = m_streamChains;
+    p.computeUnits = m_limits.computeUnits;
     p.slices = ws.split ? StreamSlices(rows) : 1;
     p.transform = f.transform;
     p.initialValue = f.initialValue;

@@ -212,7 +212,7 @@ private:
   bool m_streamPacked = false;            // the first rank-quantised plan brings the bundles for LaunchRankStream
   uint32_t *m_dStreamWords = nullptr;
   float *m_dStreamValues = nullptr;
-  DeviceStreamBundle *m_dStreamBundles = nullptr;
+  uint32_t *m_dStreamBundles = nullptr;
   int32_t m_streamBundles = 0, m_streamChains = 0;
   int32_t *m_dFewRowsClasses = nullptr;
   struct DeepWalk { // (the forest's, like the bundles above)
