@@ -25,6 +25,9 @@ struct WalkScalars {
   // Row-parallel kernels, classifiers with one tree slice: the kernel keeps the running arg-max of the class
   // sums (which arrive in ascending class order) and stores the class id itself; no partial sums, no finalize.
   int32_t fuseArgmax = 0;
+  // Row-parallel scalar walk of a classifier: bundle i of a group is tree thread i % treeThreads', and class c's trees are all
+  // tree thread c % treeThreads' (PackedModel::ownClasses).
+  int32_t ownClasses = 0;
   // Scalar row-parallel walk on an f32 tile with byte offsets: trees may end in stubs (device_model.h); the row
   // tile then has a column for the stub feature and every wave a queue of deferred walks behind it.
   int32_t deferTails = 0;

@@ -184,8 +184,9 @@ __device__ __forceinline__ void StageRows(const float *__restrict__ src, int val
 //
 // kVariant picks what is compiled in beside the plain walk (each costs the plain walk about a percent when it
 // is merely present): kWalkDump the leaf-id dump of the parity checks, kWalkDefer the deferred tails, kWalkFuse
-// the classifiers' running arg-max (WalkScalars::fuseArgmax).
-enum WalkVariant : int { kWalkPlain = 0, kWalkDump = 1, kWalkDefer = 2, kWalkFuse = 3 };
+// the classifiers' running arg-max (WalkScalars::fuseArgmax), kWalkOwn and kWalkOwnFuse classes of the tree threads' own
+// (WalkScalars::ownClasses; as a run-time branch of the plain walk it cost 1000 trees without classes 40 %: SGPRs).
+enum WalkVariant : int { kWalkPlain = 0, kWalkDump = 1, kWalkDefer = 2, kWalkFuse = 3, kWalkOwn = 4, kWalkOwnFuse = 5 };
 
 // Groups [gBegin, gEnd) of one row block: everything a block of the row-parallel walk does.  `slice` names the slot of
 // the partial sums this part fills.
@@ -198,7 +199,9 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
              const WalkScalars &s, float *__restrict__ out, int8_t *__restrict__ classOut,
              double *__restrict__ partial, int32_t *__restrict__ leafIds, const int32_t *__restrict__ nodeOrigin,
              const int32_t *__restrict__ slotTree, const U32x2 *__restrict__ tailNodes, const int32_t *__restrict__ tailOrigin) {
-  constexpr bool kDump = kVariant == kWalkDump, kDefer = kVariant == kWalkDefer, kFuse = kVariant == kWalkFuse;
+  constexpr bool kDump = kVariant == kWalkDump, kDefer = kVariant == kWalkDefer;
+  constexpr bool kFuse = kVariant == kWalkFuse || kVariant == kWalkOwnFuse;
+  const bool own = kVariant == kWalkOwn || kVariant == kWalkOwnFuse || (kDump && s.ownClasses);
   // LDS: [tree group nodes | transposed row tile].  The group sits at LDS
   // address 0 so that node pointers are LDS addresses as stored.
   const int tid = threadIdx.x;
@@ -282,12 +285,12 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
   // them in thread order.  Classifiers meet at class boundaries, while a tree group is live, so
   // their meeting area sits behind the row tile; otherwise the (then idle) group region is used.
   double *meet = reinterpret_cast<double *>(
-      C > 0 ? lds + ((s.groupRegionBytes + (kMode == kTileRankU16 ? (uint32_t)((F + 2) >> 1) * RB * 4u
+      C > 0 && !own ? lds + ((s.groupRegionBytes + (kMode == kTileRankU16 ? (uint32_t)((F + 2) >> 1) * RB * 4u
                                                                   : (uint32_t)(F + 1) * RB * (kMode == kTileRankU8 ? 1u : 4u)) + 7u) & ~7u)
             : lds);
 
   double acc = 0.0;
-  int curClass = 0;
+  int curClass = own ? tt : 0;
   float best = -INFINITY; // fuseArgmax: running maximum of the class sums and its class (tree thread 0)
   int bestClass = 0;
 
@@ -329,6 +332,21 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
     } else if (tt == 0 && lane < valid) {                                                                              \
       partialRow[curClass] = acc;                                                                                      \
       for (int c = curClass + 1; c < (UPTO); ++c) partialRow[c] = 0.0;                                                 \
+    }                                                                                                                  \
+    acc = 0.0;                                                                                                         \
+  }
+  // The same where the class is the tree thread's own: nobody to meet.
+#define TBAMD_FLUSH_OWN_CLASS(UPTO)                                                                                    \
+  {                                                                                                                    \
+    if (kFuse) {                                                                                                       \
+      const float m = (float)(s.initialValue + acc);                                                                   \
+      if (!(best > m)) { best = m; bestClass = curClass; }                                                             \
+      const float m0 = (float)s.initialValue;                                                                          \
+      for (int c = curClass + TT; c < (UPTO); c += TT)                                                                 \
+        if (!(best > m0)) { best = m0; bestClass = c; }                                                                \
+    } else if (lane < valid) {                                                                                         \
+      partialRow[curClass] = acc;                                                                                      \
+      for (int c = curClass + TT; c < (UPTO); c += TT) partialRow[c] = 0.0;                                            \
     }                                                                                                                  \
     acc = 0.0;                                                                                                         \
   }
@@ -401,7 +419,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
     uint32_t b0 = 0;
     while (b0 < grp.bundleCount) {
       uint32_t b1 = grp.bundleCount;
-      if (C > 0) {
+      if (C > 0 && !own) {
         // most groups vote for one class: the descriptor says so and no bundle has to be looked at
         const int cls = grp.uniformClass ? (int)grp.uniformClass - 1 : (int)bundles[grp.bundleBegin + b0].classId;
         if (cls != curClass) { // classes arrive in ascending order
@@ -415,6 +433,10 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
       }
       for (uint32_t b = b0 + tt; b < b1; b += TT) {
         const DeviceBundle bd = bundles[grp.bundleBegin + b];
+        if (own && (int)bd.classId != curClass) {
+          TBAMD_FLUSH_OWN_CLASS((int)bd.classId)
+          curClass = (int)bd.classId;
+        }
         uint32_t addr[K];
 #pragma unroll
         for (int k = 0; k < K; ++k) addr[k] = bd.root[k];
@@ -506,6 +528,26 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
   if (kDefer) // what is still queued is walked on now
     while (queued > 0u) TBAMD_WALK_QUEUE
 
+  if (own) {
+    TBAMD_FLUSH_OWN_CLASS(C)
+    if (!kFuse) return;
+    // each tree thread has the best of its own classes: the larger sum, or the larger class id of equal ones, as the running rule
+    __syncthreads();
+    float *bests = reinterpret_cast<float *>(lds);
+    int *classes = reinterpret_cast<int *>(lds) + threads;
+    bests[tid] = best;
+    classes[tid] = bestClass;
+    __syncthreads();
+    if (tt != 0 || lane >= valid) return;
+    for (int t = 1; t < TT; ++t) {
+      const float m = bests[t * RB + lane];
+      const int c = classes[t * RB + lane];
+      if (m > best || (m == best && c > bestClass)) { best = m; bestClass = c; }
+    }
+    if (classOut) classOut[row] = (int8_t)bestClass;
+    else out[row] = (float)bestClass;
+    return;
+  }
   if (C > 0) {
     TBAMD_FLUSH_CLASS(C)
     if (kFuse && tt == 0 && lane < valid) {
@@ -531,6 +573,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
   }
 #undef TBAMD_COPY_GROUP
 #undef TBAMD_FLUSH_CLASS
+#undef TBAMD_FLUSH_OWN_CLASS
 #undef TBAMD_PREFETCH_GROUP
 #undef TBAMD_WALK_QUEUE
 }
@@ -560,7 +603,7 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
 // write-through stores, the ticket and the reads are three round trips to memory, 5 to 12 us where the finalize launch
 // takes 4.)
 // ---------------------------------------------------------------------------
-template <int K, int kMode>
+template <int K, int kMode, int kVariant> // kWalkPlain or kWalkOwn
 // (80 SGPRs: with the 16 the trap handler takes, 8 waves per SIMD - two blocks of 16 waves - leave each wave 100; at 88 one
 // block per CU ran, 40 % slower)
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80)))
@@ -579,7 +622,7 @@ WalkRowsSplitKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes
     const int gBegin = (int)(unit - rowBlock * line.groups);
     const int64_t left = unitEnd - rowBlock * line.groups;
     const int gEnd = (int)(left < line.groups ? left : line.groups);
-    WalkRowBlock<K, 0, kMode, kWalkPlain>(lds, rowBlock, gBegin, gEnd, (int)((int64_t)blockIdx.x - line.FirstBlock(rowBlock)), x, nodes16,
+    WalkRowBlock<K, 0, kMode, kVariant>(lds, rowBlock, gBegin, gEnd, (int)((int64_t)blockIdx.x - line.FirstBlock(rowBlock)), x, nodes16,
                                           bundles, bundleRoots, groups, own, nullptr, nullptr, partial, nullptr, nullptr, nullptr, nullptr,
                                           nullptr);
     unit += gEnd - gBegin;
@@ -1773,9 +1816,9 @@ hipError_t LaunchSplit(const WalkParams &p, dim3 block, size_t ldsBytes, hipStre
   const int64_t rowBlocks = (p.s.rows + p.s.rowsPerBlock - 1) / p.s.rowsPerBlock;
   if (p.splitBlocks < 1 || p.splitBlocks > rowBlocks * p.s.numGroups || !p.partial || p.leafIds || p.s.deferTails || p.s.fuseArgmax)
     return hipErrorInvalidValue;
-  hipError_t e = AllowFullLds<&WalkRowsSplitKernel<K, W>>();
+  hipError_t e = p.s.ownClasses ? AllowFullLds<&WalkRowsSplitKernel<K, W, kWalkOwn>>() : AllowFullLds<&WalkRowsSplitKernel<K, W, kWalkPlain>>();
   if (e != hipSuccess) return e;
-  return StartKernel(&WalkRowsSplitKernel<K, W>, dim3((unsigned)p.splitBlocks), block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles,
+  return StartKernel(p.s.ownClasses ? &WalkRowsSplitKernel<K, W, kWalkOwn> : &WalkRowsSplitKernel<K, W, kWalkPlain>, dim3((unsigned)p.splitBlocks), block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles,
                      p.bundleRoots, p.groups, p.s, p.partial);
 }
 
@@ -1785,6 +1828,9 @@ hipError_t LaunchWalkKP(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBy
     if (p.s.fuseArgmax || (p.s.deferTails && W != kTileF32Bytes)) return hipErrorInvalidValue;
     return LaunchWalkVariant<K, PF, W, kWalkDump>(p, grid, block, ldsBytes, stream);
   }
+  if (p.s.ownClasses)
+    return p.s.fuseArgmax ? LaunchWalkVariant<K, PF, W, kWalkOwnFuse>(p, grid, block, ldsBytes, stream)
+                          : LaunchWalkVariant<K, PF, W, kWalkOwn>(p, grid, block, ldsBytes, stream);
   if (p.s.fuseArgmax) return LaunchWalkVariant<K, PF, W, kWalkFuse>(p, grid, block, ldsBytes, stream);
   // deferred tails are built for the f32 tile with byte offsets only (the packer makes stubs for no other plan)
   if (p.s.deferTails) {

@@ -40,7 +40,7 @@ size_t PackedModel::LdsBytes() const {
     const size_t waves = (size_t)(plan.ThreadsPerBlock() + 63) / 64;
     bytes = (bytes + 7) & ~(size_t)7;
     bytes += waves * 8 + (size_t)plan.rowsPerBlock * (numClasses > 0 ? numClasses : 1) * 8;
-  } else if (plan.treeThreads > 1 && numClasses > 0) {
+  } else if (plan.treeThreads > 1 && numClasses > 0 && !ownClasses) {
     bytes = (bytes + 7) & ~(size_t)7;
     bytes += (size_t)plan.ThreadsPerBlock() * 8; // classifiers: cross-wave pass behind the row tile
   }
@@ -976,7 +976,71 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     }
   };
 
-  size_t next = 0;
+  // Classes of the tree threads' own: rounds of a bundle for every tree thread, class c's on thread c % treeThreads.  Taken where
+  // the threads that wait for the others' classes lose less than the meetings: 2^20 rows x 54 features, 800 trees of depth 6,
+  // four tree threads: 8 classes 916 -> 847 us, 12 969 -> 862 (no levels of a tree thread idle), 11 955 -> 894 (13 a class), 7
+  // 917 -> 910 (27), 10 862 -> 890 (24), 9 941 -> 957 (48), 5 853 -> 1015 (144); 700 trees of depth 5, 7 classes 651 -> 615 (18).
+  std::vector<std::vector<int32_t>> rounds; // treeThreads * K trees each, -1: none
+  if (forest.numClasses >= plan.treeThreads && plan.treeThreads > 1 && T == 1 && plan.kernel == LaunchPlan::Kernel::kRowParallelLds) {
+    const size_t TT = (size_t)plan.treeThreads, C = (size_t)forest.numClasses;
+    std::vector<std::vector<int32_t>> ofClass(C);
+    for (int32_t t : order) ofClass[(size_t)forest.trees[(size_t)t].classId].push_back(t);
+    double levels = 0.0, idle = 0.0;
+    for (int32_t d : depth) levels += d;
+    bool fits = true;
+    for (size_t c0 = 0; c0 < C; c0 += TT) {
+      size_t most = 0;
+      for (size_t c = c0; c < std::min(C, c0 + TT); ++c) most = std::max(most, (ofClass[c].size() + K - 1) / K);
+      for (size_t i = 0; i < most; ++i) {
+        std::vector<int32_t> round(TT * K, -1);
+        uint32_t need = 0;
+        for (size_t c = c0; c < std::min(C, c0 + TT); ++c)
+          for (size_t k = 0; k < (size_t)K && i * K + k < ofClass[c].size(); ++k) {
+            const int32_t t = ofClass[c][i * K + k];
+            round[(c - c0) * K + k] = t;
+            need += units[(size_t)t];
+          }
+        for (int32_t t : round) idle += t < 0 ? levels / (double)numTrees : 0.0;
+        fits = fits && need + 2 <= groupCapacity - 1;
+        rounds.push_back(std::move(round));
+      }
+    }
+    pm.ownClasses = fits && !order.empty() && idle / (double)TT <= 20.0 * (double)C;
+  }
+  if (pm.ownClasses) {
+    const size_t TT = (size_t)plan.treeThreads;
+    for (size_t next = 0; next < rounds.size();) {
+      openGroup();
+      DeviceGroup &g = pm.groups.back();
+      for (; next < rounds.size(); ++next) {
+        uint32_t need = 0;
+        for (int32_t t : rounds[next]) need += t < 0 ? 0 : units[(size_t)t];
+        if (need > groupCapacity - 1 - ((uint32_t)pm.nodes.size() - g.nodeBegin)) break;
+        for (size_t thread = 0; thread < TT; ++thread) {
+          DeviceBundle b{};
+          b.firstSlot = (uint32_t)pm.slotTree.size();
+          for (int k = 0; k < K; ++k) {
+            const int32_t t = rounds[next][thread * K + (size_t)k];
+            pm.slotTree.push_back(t);
+            if (t < 0) continue; // (root 0: the null leaf)
+            const uint32_t base = (uint32_t)pm.nodes.size() - g.nodeBegin;
+            b.root[k] = (uint16_t)(base * kNodeBytes);
+            b.depth = b.peelDepth = std::max<uint32_t>(b.depth, (uint32_t)depth[(size_t)t]);
+            emitTree(t, base);
+          }
+          const int32_t any = rounds[next][thread * K];
+          // (a bundle without trees keeps its thread's class; every thread has one in the first round of its first classes)
+          b.classId = any >= 0 ? (uint16_t)forest.trees[(size_t)any].classId
+                      : pm.bundles.size() >= TT ? pm.bundles[pm.bundles.size() - TT].classId : (uint16_t)thread;
+          for (int k = 0; k < K; ++k) pm.bundleRoots.push_back(pm.nodes[g.nodeBegin + b.root[k] / kNodeBytes]);
+          pm.bundles.push_back(b);
+        }
+      }
+      closeGroup();
+    }
+  }
+
+  size_t next = pm.ownClasses ? order.size() : 0;
   while (next < order.size()) {
     openGroup();
     DeviceGroup &g = pm.groups.back();

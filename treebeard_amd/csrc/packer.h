@@ -96,6 +96,9 @@ struct PackedModel {
   // the f32 row-parallel walk takes level 0 from scalar registers instead of an LDS node read.
   std::vector<DeviceNode> bundleRoots;
   uint32_t maxGroupNodes = 0;
+  // Classifiers on scalar row-parallel plans: every class is one tree thread's, so that class sums need no meeting of the tree
+  // threads.  Groups are whole rounds of a bundle for every tree thread, bundles without trees among them.
+  bool ownClasses = false;
   // Tiled plans: how many trees were tiled by visit counts (the others breadth first), and the tile steps
   // one row takes over the whole forest: lock-step (deepest leaf of every tree) and, when a profile was
   // given, what the profiled rows need on average.
@@ -132,10 +135,10 @@ struct PackedModel {
   std::vector<RankChunkDesc> rankChunks;
 
   uint32_t PadFeatureOffset() const;
-  // LDS bytes of the tree-group region (regressors reuse it for the tree threads' cross-wave pass).
+  // LDS bytes of the tree-group region (regressors, and classifiers with classes of the tree threads' own, reuse it for the tree threads' cross-wave pass).
   uint32_t GroupRegionBytes() const {
     uint32_t bytes = maxGroupNodes * kNodeBytes;
-    if (plan.kernel == LaunchPlan::Kernel::kRowParallelLds && plan.treeThreads > 1 && numClasses == 0)
+    if (plan.kernel == LaunchPlan::Kernel::kRowParallelLds && plan.treeThreads > 1 && (numClasses == 0 || ownClasses))
       bytes = bytes > (uint32_t)plan.ThreadsPerBlock() * 8u ? bytes : (uint32_t)plan.ThreadsPerBlock() * 8u;
     return (bytes + 15u) & ~15u;
   }

@@ -497,6 +497,7 @@ WalkParams InferenceRunner::MakeWalkParams(const float *deviceInputs, int64_t ro
   p.s.deferTails = model.plan.deferTails ? 1 : 0;
   p.s.tailDepth = (int32_t)model.maxTailDepth;
   p.s.tileHops = model.maxTileHops;
+  p.s.ownClasses = model.ownClasses ? 1 : 0;
   p.tailNodes = m_dTailNodes;
   p.tailOrigin = m_dTailOrigin;
   p.directStaging = DirectStaging();
@@ -1108,7 +1109,8 @@ std::string InferenceRunner::DescribePlan() const {
      << " peelWalks=" << peel << " treesTiledByProfile=" << m_model.treesTiledByProfile
      << " lockStepSteps=" << m_model.lockStepSteps << " profiledSteps=" << m_model.profiledSteps
      << " batchKernel=" << KernelOfBatch() << " fewRowsLimit=" << m_fewRowsLimit
-     << " treesDeferred=" << m_model.treesDeferred << " deferredEntriesPerRow=" << m_model.deferredEntriesPerRow;
+     << " treesDeferred=" << m_model.treesDeferred << " deferredEntriesPerRow=" << m_model.deferredEntriesPerRow
+     << " ownClasses=" << (m_model.ownClasses ? 1 : 0);
   return os.str();
 }
 
