@@ -61,3 +61,24 @@ def test_wide_rows_split_on_rank_tiles(synth_model):
             pin(runner)
             for rows in (batch, batch - 1, 1000):
                 close(forest, gpu_predict(runner, x[:rows]), expected[:rows])
+
+
+def test_whole_rounds_of_many_slices_are_split_too(tmp_path):
+    """352 row blocks, for which the plan takes 48 slices (any number serves the split alike): 33 whole rounds of blocks."""
+    rng = np.random.Generator(np.random.PCG64(12))
+    trees = [synth._grow_tree(rng, 9, lambda d, s: 0.9, lambda: (rng.integers(0, 20), rng.normal()), rng.normal) for _ in range(500)]
+    path = str(tmp_path / "m.json")
+    synth.write_xgboost_json(path, trees, 20)
+    rows = 90000
+    runner = make_runner(path, rows)
+    plan = runner.describe_plan()
+    slices = int(plan.split("treeSlices=")[1].split()[0])
+    runner.set_plan(256, 4, 4, 51712, 48)
+    pinned = runner.describe_plan()
+    assert "batchKernel=rows_lds_split" in plan, plan
+    assert "treeSlices=48" not in pinned or "batchKernel=rows_lds_split" in pinned, (slices, pinned)
+    x = rng.standard_normal((rows, 20), dtype=np.float32)
+    got = gpu_predict(runner, x)
+    forest = model_io.load_xgboost_json(path)
+    for at in (0, 44000, rows - 2000):
+        np.testing.assert_allclose(got[at:at + 2000], cpu_oracle.predict(forest, x[at:at + 2000])[0], rtol=1e-5, atol=1e-6)

@@ -358,7 +358,9 @@ int32_t InferenceRunner::SplitBlocks(int64_t rows) const {
   const int64_t perCu = std::max<int64_t>(1, std::min<int64_t>(2048 / plan.ThreadsPerBlock(),
                                                                m_limits.ldsBytesPerBlock / (int64_t)(m_model.LdsBytes() + 512)));
   const int64_t places = perCu * m_limits.computeUnits; // blocks that run at once
-  if (blocks <= places || blocks % places == 0) return 0;
+  // (Whole rounds of blocks are no reason to keep the slices, which the plan may have chosen because the split serves them all
+  // alike: 90000 rows x 700 trees of 28 features 196 us in 33 rounds of 48 slices, 129 split; 45000 rows of six classes 95 and 55.)
+  if (blocks <= places) return 0;
   WalkShape shape;
   shape.rowBlocks = RowBlocks(rows);
   shape.rowsPerBlock = plan.rowsPerBlock;
