@@ -380,6 +380,14 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     int64_t perSlice = std::max<int64_t>((totalBytes + slices - 1) / slices + 4096, need);
     if (perSlice < plan.groupBytes) plan.groupBytes = (int32_t)((perSlice + 15) & ~15);
   }
+  // Four trees side by side hide more latency than two, but where a group holds fewer trees than the tree threads could take
+  // that way, threads without a bundle wait for the others.  262144 rows, 200 to 300 trees, two and four trees a lane: four tree
+  // threads 54 features 16.2 trees a group 132 and 122 us, 14.0 146 and 142, 12.1 106 and 120; eight 27.9 136 and 126, 22.8 147
+  // and 148, 19.5 158 and 171, 8.0 207 and 246; sixteen 47 147 and 141, 40 161 and 161, 31 183 and 189, 12 242 and 282; 40000
+  // rows alike.  (One tree a lane is never faster.)
+  if (!(ov && ov->treeWalkInterleaveFactor > 0) &&
+      (double)plan.groupBytes * (double)forest.trees.size() < (2.4 * plan.treeThreads + 3.4) * (double)totalBytes)
+    plan.interleave = 2;
   plan.treeSlices = (int32_t)std::max<int64_t>(1, slices);
   return plan;
 }
