@@ -639,8 +639,6 @@ hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
     for (int c = 0; c < Cn; ++c) {
       sums[(size_t)c] = p.initialValue;
       for (int s = 0; s < parts; ++s) sums[(size_t)c] += p.partial[((int64_t)s * p.rows + row) * Cn + c];
-      // (the wide form leaves class sums in a spare slot behind the last one)
-      if (C > 0 && p.treeSlices >= kWideFinalizeSlices) p.partial[((int64_t)p.treeSlices * p.rows + row) * Cn + c] = sums[(size_t)c];
     }
     if (C == 0) p.out[row] = FinishMargin(sums[0], p.transform);
     else FinishRow(sums.data(), C, row, p.out, p.classOut, p.margins, p.probabilities);

@@ -1290,11 +1290,14 @@ def test_rows_too_wide_for_lds_walk_from_global_memory(tmp_path, features, rows)
     check_against_oracle(runner, forest, x)
 
 
-@pytest.mark.parametrize("slices", [15, 16, 17, 31])
+@pytest.mark.parametrize("slices", [3, 4, 5, 15, 16, 17, 31])
 @pytest.mark.parametrize("rows", [1, 63, 65, 2048, 2049])
 def test_finalize_of_many_slices(synth_model, rows, slices):
-    """Class sums of a few rows over many tree slices, either side of the number of slices and of sums (2048 x 8) at which 64
-    sums a block take over."""
+    """Class sums and plain sums over several tree slices, either side of the numbers from which groups of lanes share the slices."""
+    regressor = make_runner(synth_model(2), rows)
+    regressor.set_plan(64, 2, 2, 8192, slices)
+    assert "treeSlices=%d " % slices in regressor.describe_plan()
+    check_against_oracle(regressor, model_io.load_xgboost_json(synth_model(2)), synth.CONFIGS[2].batch_rows(rows, seed_offset=9))
     x = synth.CONFIGS[3].batch_rows(rows, seed_offset=9)
     runner = make_runner(synth_model(3), rows)
     runner.set_plan(64, 2, 2, 8192, slices)

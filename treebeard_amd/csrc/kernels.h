@@ -64,10 +64,6 @@ struct WalkParams {
   int32_t splitBlocks = 0;
 };
 
-// From this many tree slices on, small batches are finalized by a wave per (row, class); classifiers then need
-// one spare slot of [rows][classes] doubles behind the last slice of the partial sums.
-constexpr int kWideFinalizeSlices = 16;
-
 // Row blocks x tree groups as one line of units, cut into equal parts for `blocks` <= units blocks.
 struct SplitLine {
   int64_t units;
@@ -89,7 +85,7 @@ struct SplitLine {
 };
 
 struct FinalizeParams {
-  double *partial = nullptr;   // [slices (+ 1 spare, see kWideFinalizeSlices)][rows][max(1, classes)]
+  double *partial = nullptr;   // [slices][rows][max(1, classes)]
   int64_t rows = 0;
   int32_t numClasses = 0;
   int32_t treeSlices = 1;      // number of partial sums per (row, class)

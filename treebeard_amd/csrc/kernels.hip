@@ -1411,28 +1411,45 @@ __global__ void __launch_bounds__(256) FinalizeKernel(const FinalizeParams p) {
 
 // Classifiers: the block's rows x classes are read as they lie (coalesced; a lane per row read a line per class and all
 // of them three times: 13 us for 65537 rows x 8 classes x 2 slices), meet in LDS, and the rows are finished there.  A sum per
-// lane: blocks of 128 rows, whose lanes wait for memory four times in a row, took 4.7 us longer with sums and softmax.
+// lane: blocks of 128 rows, whose lanes wait for memory four times in a row, took 4.7 us longer with sums and softmax.  With
+// four parts and more to add, two groups of 256 lanes take every second of them: calls of 1700 rows x 8 classes with sums and
+// softmax 29.4 us with one group, 27.5 with two, 28.0 with four; 9000 rows 39.7, 39.8, 41.5.
 constexpr int kFinalizeLds = 4096; // doubles of sums a block holds
 
-__global__ void __launch_bounds__(256) FinalizeClassesKernel(const FinalizeParams p, int rowsPerBlock) {
+__global__ void __launch_bounds__(1024) FinalizeClassesKernel(const FinalizeParams p, int rowsPerBlock) {
   extern __shared__ __align__(16) unsigned char lds[];
   double *sums = reinterpret_cast<double *>(lds); // [row][class], rows an odd number of doubles apart
   const int C = p.numClasses, stride = C | 1;
-  double *rowMax = sums + rowsPerBlock * stride, *rowZ = rowMax + rowsPerBlock;
+  double *rowMax = sums + rowsPerBlock * stride, *rowZ = rowMax + rowsPerBlock, *others = rowZ + rowsPerBlock;
   const int64_t row0 = (int64_t)blockIdx.x * rowsPerBlock;
   const int valid = p.rows - row0 < rowsPerBlock ? (int)(p.rows - row0) : rowsPerBlock;
   const int tid = threadIdx.x, threads = blockDim.x;
-  for (int e = tid; e < valid * C; e += threads) {
+  const int groups = threads >> 8, group = __builtin_amdgcn_readfirstlane(tid >> 8);
+  const int64_t slot = p.rows * C;
+  double *mine = group == 0 ? sums : others + (group - 1) * (rowsPerBlock * stride);
+  for (int e = tid & 255; e < valid * C; e += 256) {
     const int r = e / C, c = e - r * C;
-    // (the first two parts are on their way while the divisions that count the parts run; a slot is there, filled or not)
+    // (a group's first two parts are on their way while the divisions that count the parts run; a slot is there, filled or not)
     const double *at = p.partial + row0 * C + e;
-    const double first = at[0], second = p.treeSlices > 1 ? at[p.rows * C] : 0.0;
+    const double first = at[group * slot], second = group + groups < p.treeSlices ? at[(group + groups) * slot] : 0.0;
     const int parts = PartsOfRow(p, row0 + r);
-    double margin = p.initialValue + first;
-    if (parts > 1) margin += second;
-    for (int s = 2; s < parts; ++s) margin += at[(int64_t)s * p.rows * C];
-    sums[r * stride + c] = margin;
-    if (p.margins) p.margins[row0 * C + e] = (float)margin;
+    double sum = group == 0 ? p.initialValue : 0.0;
+    if (group < parts) sum += first;
+    if (group + groups < parts) sum += second;
+#pragma unroll 4
+    for (int s = group + 2 * groups; s < parts; s += groups) sum += at[s * slot];
+    mine[r * stride + c] = sum;
+    if (groups == 1 && p.margins) p.margins[row0 * C + e] = (float)sum;
+  }
+  if (groups > 1) {
+    __syncthreads();
+    for (int e = tid; e < valid * C; e += threads) {
+      const int r = e / C, c = e - r * C;
+      double sum = sums[r * stride + c];
+      for (int g = 1; g < groups; ++g) sum += others[(g - 1) * (rowsPerBlock * stride) + r * stride + c];
+      sums[r * stride + c] = sum;
+      if (p.margins) p.margins[row0 * C + e] = (float)sum;
+    }
   }
   __syncthreads();
   for (int r = tid; r < valid; r += threads) {
@@ -1482,37 +1499,31 @@ __global__ void __launch_bounds__(256) FinalizeManyClassesKernel(const FinalizeP
       p.numClasses, row, p.out, p.classOut, p.margins, p.probabilities);
 }
 
-// Small batches split over many tree slices (kWideFinalizeSlices or more): 64 (row, class) sums a block, a lane each, and its
-// waves share the slices, so that a lane waits for few loads and a wave reads 512 contiguous bytes.  (A wave per sum, lanes
-// along the slices, read a 64-byte piece of memory for each of its 8 bytes: 4096 rows x 32 slices 3.0 us, 2.5 here; the call 15.1 and 13.9.)  Each wave
-// adds its slices in slice order, the waves are added in order: the order of additions depends on the number of slices alone.
-constexpr int64_t kWideFinalizeItems = 16384; // (a call of 2048 rows x 8 classes 33.3 us without, 31.5 with; 64000 sums 38.5 and 39.9)
-constexpr int kWideFinalizeWaves = 8;
+// Small batches split over several tree slices: 64 rows a block, a lane each, and its waves share the slices, so that a lane
+// waits for few loads and a wave reads 512 contiguous bytes.  (A wave per sum, lanes along the slices, read a 64-byte piece of
+// memory for each of its 8 bytes: 4096 rows x 32 slices 3.0 us, 2.5 here; the call 15.1 and 13.9.)  Each wave adds its slices
+// in slice order, the waves are added in order: the order of additions depends on the number of slices alone.
+constexpr int kWideFinalizeSlices = 4;
+constexpr int64_t kWideFinalizeRows = 65536;
 
-__global__ void __launch_bounds__(kWideFinalizeWaves * 64) FinalizeWideKernel(const FinalizeParams p) {
-  __shared__ double meet[kWideFinalizeWaves][64];
+template <int kWaves> // 4, or 8 from so many slices on
+__global__ void __launch_bounds__(kWaves * 64) FinalizeWideKernel(const FinalizeParams p) {
+  __shared__ double meet[kWaves][64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t items = p.rows * (p.numClasses > 0 ? p.numClasses : 1);
-  const int64_t item = (int64_t)blockIdx.x * 64 + lane;
-  if (item < items) {
-    const int parts = PartsOfRow(p, p.numClasses > 0 ? item / p.numClasses : item);
+  const int64_t row = (int64_t)blockIdx.x * 64 + lane;
+  if (row < p.rows) {
+    const int parts = PartsOfRow(p, row);
     double sum = 0.0;
 #pragma unroll 4
-    for (int s = wave; s < parts; s += kWideFinalizeWaves) sum += p.partial[(int64_t)s * items + item];
+    for (int s = wave; s < parts; s += kWaves) sum += p.partial[(int64_t)s * p.rows + row];
     meet[wave][lane] = sum;
   }
   __syncthreads();
-  if (wave != 0 || item >= items) return;
+  if (wave != 0 || row >= p.rows) return;
   double sum = meet[0][lane];
-  for (int w = 1; w < kWideFinalizeWaves; ++w) sum += meet[w][lane];
+  for (int w = 1; w < kWaves; ++w) sum += meet[w][lane];
   const double margin = p.initialValue + sum;
-  if (p.numClasses == 0) {
-    p.out[item] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
-    return;
-  }
-  // classifiers: the class sum goes into the spare slot behind the last slice; FinalizeClassesKernel (1 slice, reading
-  // that slot) does the rest.  The slices themselves stay as they are, so the launch can be repeated.
-  p.partial[(int64_t)p.treeSlices * items + item] = margin - p.initialValue;
+  p.out[row] = (float)(p.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
 }
 
 // ---------------------------------------------------------------------------
@@ -2120,28 +2131,23 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
 
 hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
-  const int Cn = p.numClasses > 0 ? p.numClasses : 1;
-  FinalizeParams q = p;
-  if (p.treeSlices >= kWideFinalizeSlices && p.rows * Cn <= kWideFinalizeItems) { // few rows, many slices
-    hipError_t e = StartKernel(&FinalizeWideKernel, dim3((unsigned)((p.rows * Cn + 63) / 64)), dim3(kWideFinalizeWaves * 64), 0, stream,
-                               p.numClasses == 0 ? p.done : nullptr, p);
-    if (e != hipSuccess || p.numClasses == 0) return e;
-    q.partial = p.partial + (int64_t)p.treeSlices * p.rows * Cn; // the class sums now sit in the spare slot
-    q.treeSlices = 1;
-    q.splitBlocks = 0;
-  }
-  if (q.numClasses > 0) {
-    // (rows of a block: as many as LDS holds, fewer where that leaves compute units without a block)
-    const int64_t perBlock = std::max<int64_t>(1, std::min<int64_t>({256, kFinalizeLds / (q.numClasses | 1), std::max<int64_t>(8, 256 / q.numClasses)}));
-    const int64_t blocks = (q.rows + perBlock - 1) / perBlock;
-    const size_t ldsBytes = (size_t)perBlock * ((size_t)(q.numClasses | 1) + 2) * sizeof(double);
+  if (p.numClasses > 0) {
+    // (a sum per lane; fewer rows where LDS does not hold their sums)
+    const int64_t perBlock = std::max<int64_t>(1, std::min<int64_t>({256, kFinalizeLds / (p.numClasses | 1), std::max<int64_t>(8, 256 / p.numClasses)}));
+    const int64_t blocks = (p.rows + perBlock - 1) / perBlock;
+    const size_t sumBytes = (size_t)perBlock * (size_t)(p.numClasses | 1) * sizeof(double), rowBytes = (size_t)perBlock * 2 * sizeof(double);
     if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
-    if (ldsBytes > 64 * 1024)
-      return StartKernel(&FinalizeManyClassesKernel, dim3((unsigned)((q.rows + 255) / 256)), dim3(256), 0, stream, q.done, q);
-    return StartKernel(&FinalizeClassesKernel, dim3((unsigned)blocks), dim3(256), ldsBytes, stream, q.done, q, (int)perBlock);
+    if (sumBytes + rowBytes > 64 * 1024)
+      return StartKernel(&FinalizeManyClassesKernel, dim3((unsigned)((p.rows + 255) / 256)), dim3(256), 0, stream, p.done, p);
+    const int groups = p.treeSlices >= 4 && sumBytes * 2 + rowBytes <= 64 * 1024 ? 2 : 1;
+    return StartKernel(&FinalizeClassesKernel, dim3((unsigned)blocks), dim3((unsigned)(256 * groups)), sumBytes * groups + rowBytes, stream,
+                       p.done, p, (int)perBlock);
   }
-  const int64_t blocks = (q.rows + 255) / 256;
-  return StartKernel(&FinalizeKernel, dim3((unsigned)blocks), dim3(256), 0, stream, q.done, q);
+  if (p.treeSlices >= kWideFinalizeSlices && p.rows <= kWideFinalizeRows)
+    return StartKernel(p.treeSlices < 8 ? &FinalizeWideKernel<4> : &FinalizeWideKernel<8>, dim3((unsigned)((p.rows + 63) / 64)),
+                       dim3(p.treeSlices < 8 ? 256 : 512), 0, stream, p.done, p);
+  const int64_t blocks = (p.rows + 255) / 256;
+  return StartKernel(&FinalizeKernel, dim3((unsigned)blocks), dim3(256), 0, stream, p.done, p);
 }
 
 } // namespace tbamd

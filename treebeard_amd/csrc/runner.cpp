@@ -332,9 +332,7 @@ size_t InferenceRunner::PartialBytes(int64_t rows, bool split) const {
   }
   const int32_t splitBlocks = split ? SplitBlocks(rows) : 0;
   if (split ? splitBlocks == 0 : !NeedsFinalize()) return 0;
-  size_t slots = split ? (size_t)SplitLine::Slots(splitBlocks, RowBlocks(rows)) : (size_t)m_model.PartialCount();
-  // (+ the spare slot the wide finalize of a classifier leaves its class sums in)
-  if (m_forest.numClasses > 0 && slots >= (size_t)kWideFinalizeSlices) ++slots;
+  const size_t slots = split ? (size_t)SplitLine::Slots(splitBlocks, RowBlocks(rows)) : (size_t)m_model.PartialCount();
   return slots * (size_t)rows * (size_t)std::max(1, m_forest.numClasses) * sizeof(double);
 }
 
