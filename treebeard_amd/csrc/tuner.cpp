@@ -376,6 +376,22 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
       if (s == 1 || us < best) best = us, slices = s;
     }
   }
+  // Smaller row blocks than two blocks per compute unit leave room for:
+  //  * fewer than a block of 256 rows for each compute unit, and too few trees to slice: 128 rows x 8 tree threads.  33126 rows x
+  //    275 trees of depth 4 17.6 -> 15.5 us, 31046 x 182 12.8 -> 9.4, 20909 x 120 of depth 5 11.1 -> 9.5, 50001 x 100 of depth 8
+  //    18.9 -> 17.2;
+  //  * forests of up to 24 KB, whose rows take as long to stage as to walk: 128 x 4, of which three and more to a unit take
+  //    turns.  2^20 rows x 60 trees of depth 5 69.6 -> 58.0 us, 210411 x 62 19.6 -> 17.2, 402162 x 51 of depth 4 30.0 -> 26.0
+  //    (29 KB: 37.7 and 38.5).
+  if (forest.numClasses == 0 && slices == 1 && rb == 256 && budget == halfLds && !(ov && (ov->numRowsPerTB > 0 || ov->numTreeThreads > 0))) {
+    const bool idle = rowBlocks <= limits.computeUnits, fewTrees = totalBytes <= 24 * 1024;
+    if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits)) {
+      rb = plan.rowsPerBlock = 128;
+      plan.treeThreads = fewTrees ? 4 : 8;
+      plan.groupBytes = (int32_t)(std::min<int64_t>({65536, roomFor(rb, halfLds), 256LL * plan.ThreadsPerBlock()}) & ~15);
+      if (fewTrees) plan.groupBytes = std::min<int32_t>(plan.groupBytes, (int32_t)((totalBytes + 1024) & ~15));
+    }
+  }
   if (slices > groups) { // more, smaller groups so that every slice has one
     int64_t perSlice = std::max<int64_t>((totalBytes + slices - 1) / slices + 4096, need);
     if (perSlice < plan.groupBytes) plan.groupBytes = (int32_t)((perSlice + 15) & ~15);
