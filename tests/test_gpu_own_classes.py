@@ -1,4 +1,4 @@
-"""Classifiers whose classes are each one tree thread's: numbers of classes around the tree threads', classes without trees or with
+"""Classifiers whose classes are each one tree thread's: numbers of classes below, around and above the tree threads', classes without trees or with
 more than others, equal sums (the larger class id), every output, slices, even splits, groups of one and several rounds."""
 import numpy as np
 import pytest
@@ -45,7 +45,7 @@ def check(runner, path, x):
     np.testing.assert_allclose(margins.cpu().numpy(), sums, rtol=RTOL_SUM, atol=1e-7)
 
 
-@pytest.mark.parametrize("classes,threads", [(2, 2), (4, 4), (5, 4), (7, 4), (8, 4), (9, 8), (12, 2), (16, 16), (40, 16)])
+@pytest.mark.parametrize("classes,threads", [(2, 2), (2, 8), (3, 4), (4, 4), (5, 4), (7, 4), (8, 4), (9, 8), (12, 2), (12, 16), (16, 16), (40, 16)])
 @pytest.mark.parametrize("group,slices", [(16384, 1), (65536, 1), (16384, 3)])
 def test_own_classes_match_the_oracle(tmp_path, classes, threads, group, slices):
     path = class_model(tmp_path / "m.json", [t % classes for t in range(5 * classes + 1)], classes)
@@ -59,7 +59,7 @@ def test_classes_without_trees_and_unequal_classes(tmp_path):
     info = [0] * 3 + [3] * 9 + [4] * 2 + [5] * 7 + [8]     # 1, 2, 6, 7 and 9 have none
     path = class_model(tmp_path / "m.json", info, 10)
     runner = make_runner(path, 500)
-    for threads in (2, 4, 8):
+    for threads in (2, 4, 8):                 
         runner.set_plan(128, threads, 4, 32768, 1)
         check(runner, path, np.random.Generator(np.random.PCG64(4)).normal(size=(500, FEATURES)).astype(np.float32))
 

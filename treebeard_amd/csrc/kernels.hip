@@ -340,11 +340,11 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
   {                                                                                                                    \
     if (kFuse) {                                                                                                       \
       const float m = (float)(s.initialValue + acc);                                                                   \
-      if (!(best > m)) { best = m; bestClass = curClass; }                                                             \
+      if (curClass < C && !(best > m)) { best = m; bestClass = curClass; }                                             \
       const float m0 = (float)s.initialValue;                                                                          \
       for (int c = curClass + TT; c < (UPTO); c += TT)                                                                 \
         if (!(best > m0)) { best = m0; bestClass = c; }                                                                \
-    } else if (lane < valid) {                                                                                         \
+    } else if (curClass < C && lane < valid) { /* (more tree threads than classes: some have none) */                  \
       partialRow[curClass] = acc;                                                                                      \
       for (int c = curClass + TT; c < (UPTO); c += TT) partialRow[c] = 0.0;                                            \
     }                                                                                                                  \

@@ -976,17 +976,22 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     }
   };
 
-  // Classes of the tree threads' own: rounds of a bundle for every tree thread, class c's on thread c % treeThreads.  Taken where
-  // the threads that wait for the others' classes lose less than the meetings: 2^20 rows x 54 features, 800 trees of depth 6,
-  // four tree threads: 8 classes 916 -> 847 us, 12 969 -> 862 (no levels of a tree thread idle), 11 955 -> 894 (13 a class), 7
-  // 917 -> 910 (27), 10 862 -> 890 (24), 9 941 -> 957 (48), 5 853 -> 1015 (144); 700 trees of depth 5, 7 classes 651 -> 615 (18).
+  // Classes of the tree threads' own: rounds of a bundle for every tree thread, class c's on thread c % treeThreads.  Against them
+  // stand the classes one after the other, each dealt over all tree threads, which meet at its end: that costs as much as about
+  // 20 levels of a tree thread.  2^20 rows x 54 features, 800 trees of depth 6, four tree threads, levels of a tree thread that way
+  // and this, and what was measured: 8 classes 1504 and 1200, 916 and 847 us; 12 1680 and 1224, 969 and 862; 11 1540 and 1368,
+  // 955 and 894; 7 1484 and 1392, 917 and 910; 10 1400 and 1440, 862 and 890; 9 1476 and 1656, 941 and 957; 6 1416 and 1632, 898
+  // and 949; 5 1300 and 1920, 853 and 1015.
   std::vector<std::vector<int32_t>> rounds; // treeThreads * K trees each, -1: none
-  if (forest.numClasses >= plan.treeThreads && plan.treeThreads > 1 && T == 1 && plan.kernel == LaunchPlan::Kernel::kRowParallelLds) {
+  if (forest.numClasses > 1 && plan.treeThreads > 1 && T == 1 && plan.kernel == LaunchPlan::Kernel::kRowParallelLds) {
     const size_t TT = (size_t)plan.treeThreads, C = (size_t)forest.numClasses;
     std::vector<std::vector<int32_t>> ofClass(C);
     for (int32_t t : order) ofClass[(size_t)forest.trees[(size_t)t].classId].push_back(t);
-    double levels = 0.0, idle = 0.0;
+    double levels = 0.0;
     for (int32_t d : depth) levels += d;
+    const double bundleLevels = K * levels / (double)std::max<size_t>(1, numTrees);
+    double meeting = 0.0;
+    for (auto &trees : ofClass) meeting += (double)((trees.size() + TT * K - 1) / (TT * K)) * bundleLevels + 20.0;
     bool fits = true;
     for (size_t c0 = 0; c0 < C; c0 += TT) {
       size_t most = 0;
@@ -1000,12 +1005,11 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
             round[(c - c0) * K + k] = t;
             need += units[(size_t)t];
           }
-        for (int32_t t : round) idle += t < 0 ? levels / (double)numTrees : 0.0;
         fits = fits && need + 2 <= groupCapacity - 1;
         rounds.push_back(std::move(round));
       }
     }
-    pm.ownClasses = fits && !order.empty() && idle / (double)TT <= 20.0 * (double)C;
+    pm.ownClasses = fits && !order.empty() && (double)rounds.size() * bundleLevels < meeting;
   }
   if (pm.ownClasses) {
     const size_t TT = (size_t)plan.treeThreads;
@@ -1029,7 +1033,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
             emitTree(t, base);
           }
           const int32_t any = rounds[next][thread * K];
-          // (a bundle without trees keeps its thread's class; every thread has one in the first round of its first classes)
+          // (a bundle without trees keeps its thread's class, the first one's if it had none yet)
           b.classId = any >= 0 ? (uint16_t)forest.trees[(size_t)any].classId
                       : pm.bundles.size() >= TT ? pm.bundles[pm.bundles.size() - TT].classId : (uint16_t)thread;
           for (int k = 0; k < K; ++k) pm.bundleRoots.push_back(pm.nodes[g.nodeBegin + b.root[k] / kNodeBytes]);

@@ -404,6 +404,17 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   if (!(ov && ov->treeWalkInterleaveFactor > 0) &&
       (double)plan.groupBytes * (double)forest.trees.size() < (2.4 * plan.treeThreads + 3.4) * (double)totalBytes)
     plan.interleave = 2;
+  // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
+  // not fit and that way costs less (the packer's costs).
+  if (forest.numClasses > 1 && plan.treeThreads > 1 && plan.interleave == 4 && !(ov && ov->treeWalkInterleaveFactor > 0) &&
+      (double)plan.groupBytes * (double)forest.trees.size() < (4.0 * std::min(plan.treeThreads, forest.numClasses) + 0.3) * (double)totalBytes) {
+    double levels = 0.0;
+    for (const Tree &tree : forest.trees) levels += tree.Depth();
+    levels /= (double)forest.trees.size();
+    const double ofClass = (double)forest.trees.size() / forest.numClasses, threads = plan.treeThreads;
+    const double own = std::ceil(forest.numClasses / threads) * std::ceil(ofClass / 2) * 2 * levels;
+    if (own < forest.numClasses * (std::ceil(ofClass / (4 * threads)) * 4 * levels + 20.0)) plan.interleave = 2;
+  }
   plan.treeSlices = (int32_t)std::max<int64_t>(1, slices);
   return plan;
 }
