@@ -299,6 +299,11 @@ void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64
           continue;
         }
         const int cls = p.s.numClasses > 0 ? (int)bd.classId : 0;
+        if (p.s.numClasses > 0 && cls >= p.s.numClasses) { // a tree thread without a class: bundles without trees, no sum
+          if (!p.s.ownClasses || cls >= p.s.treeThreads || nodes[grp.nodeBegin + addr / kNodeBytes].value != 0.0f) std::abort();
+          if (p.leafIds && p.slotTree[bd.firstSlot + k] >= 0) std::abort();
+          continue;
+        }
         classSums[cls] += (double)nodes[grp.nodeBegin + addr / kNodeBytes].value;
         classSeen[cls] = true;
         if (p.leafIds) {
