@@ -383,7 +383,9 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   //  * forests of up to 24 KB, whose rows take as long to stage as to walk: 128 x 4, of which three and more to a unit take
   //    turns.  2^20 rows x 60 trees of depth 5 69.6 -> 58.0 us, 210411 x 62 19.6 -> 17.2, 402162 x 51 of depth 4 30.0 -> 26.0
   //    (29 KB: 37.7 and 38.5).
-  if (forest.numClasses == 0 && slices == 1 && rb == 256 && budget == halfLds && !(ov && (ov->numRowsPerTB > 0 || ov->numTreeThreads > 0))) {
+  // (Not where the biggest tree asks for more than the group beside them: the blocks of 256 rows may have taken the whole LDS for it.)
+  if (forest.numClasses == 0 && slices == 1 && rb == 256 && budget == halfLds && roomFor(128, halfLds) >= need &&
+      !(ov && (ov->numRowsPerTB > 0 || ov->numTreeThreads > 0))) {
     const bool idle = rowBlocks <= limits.computeUnits, fewTrees = totalBytes <= 24 * 1024;
     if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits)) {
       rb = plan.rowsPerBlock = 128;
