@@ -55,9 +55,33 @@ static void BigTrees() {
   std::printf("big trees: %ld\n", packed);
 }
 
+// Deep forests with as many nodes below the cuts as the tail array has places, and with one tree more.
+static void TailLimit() {
+  const DeviceLimits limits;
+  LaunchPlan plan;
+  std::vector<int32_t> cuts;
+  const struct { int32_t features, nodes; } shapes[] = {{28, 16383}, {28, 21391}, {10, 9665}, {10, 210345}, {200, 9001}};
+  for (auto shape : shapes) {
+    Forest forest = ForestOf(shape.features, 1, shape.nodes);
+    EXPECT(ChooseDeepWalk(forest, limits, &plan, &cuts), "%d features, %d nodes", shape.features, shape.nodes);
+    const size_t perTree = PackWithCuts(forest, plan, cuts).tailNodes.size() - 1, most = (kMaxTailNodes - 1) / perTree;
+    forest = ForestOf(shape.features, (int32_t)most, shape.nodes);
+    EXPECT(ChooseDeepWalk(forest, limits, &plan, &cuts), "%zu trees of %d nodes, %d features", most, shape.nodes, shape.features);
+    try {
+      const PackedModel pm = PackWithCuts(forest, plan, cuts);
+      EXPECT(pm.tailNodes.size() == most * perTree + 1, "%zu trees of %d nodes, %d features: %zu", most, shape.nodes, shape.features, pm.tailNodes.size());
+    } catch (const Error &e) {
+      EXPECT(false, "%zu trees of %d nodes, %d features: %s", most, shape.nodes, shape.features, e.what());
+    }
+    forest.trees.push_back(forest.trees[0]);
+    EXPECT(!ChooseDeepWalk(forest, limits, &plan, &cuts), "%zu trees of %d nodes, %d features", most + 1, shape.nodes, shape.features);
+  }
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
+  if (asked("tail_limit")) TailLimit();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

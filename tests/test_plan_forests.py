@@ -30,3 +30,7 @@ def run(driver, name):
 
 def test_big_trees_open_with_every_batch(driver):
     run(driver, "big_trees")
+
+
+def test_deep_forests_up_to_the_last_tail_node(driver):
+    run(driver, "tail_limit")

@@ -792,11 +792,14 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     if (cut < depth[t]) {
       bool nanLeaf = false; // (a NaN is what marks a stub)
       for (size_t i = 0; i < tree.NumNodes(); ++i) nanLeaf = nanLeaf || (tree.IsLeaf((int32_t)i) && tree.value[i] != tree.value[i]);
-      if (cut < depth[t] && tailBudget > 0 && !nanLeaf) {
-        uint32_t above = 0;
-        for (size_t i = 0; i < tree.NumNodes(); ++i)
-          if (nodeLevel[i] <= cut) ++above; // the top of the tree, the cut level's internal nodes as stubs
-        tailBudget -= (int64_t)(tree.NumNodes() - above) + 64;
+      uint32_t above = 0; // the top of the tree, the cut level's internal nodes as stubs
+      int64_t tails = 0;  // those internal nodes again, and all below them
+      for (size_t i = 0; i < tree.NumNodes(); ++i) {
+        if (nodeLevel[i] <= cut) ++above;
+        if (nodeLevel[i] > cut || (nodeLevel[i] == cut && !tree.IsLeaf((int32_t)i))) ++tails;
+      }
+      if (tails <= tailBudget && !nanLeaf) {
+        tailBudget -= tails;
         units[t] = above;
         depth[t] = cut;
         peel[t] = cut;

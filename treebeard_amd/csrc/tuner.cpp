@@ -155,15 +155,18 @@ bool ChooseDeepWalk(const Forest &forest, const DeviceLimits &limits, LaunchPlan
   const int64_t bundles = (int64_t)plan->treeThreads * plan->interleave;
   const int64_t mostTop = std::min(room * 5 / 4 / bundles, room) / kNodeBytes - 4;
   if (mostTop < 31) return false;
-  int64_t tails = 0; // nodes below the cuts
+  int64_t tails = 1; // places of the tail array: the null leaf, the cut levels' internal nodes and all below them
   cuts->clear();
   for (const Tree &tree : forest.trees) {
     int64_t top = 0;
     int32_t depth = 0, cut = -1;
     std::vector<int32_t> level{0}, below;
     for (; !level.empty(); ++depth) {
-      if (cut < 0 && top + (int64_t)level.size() > mostTop) cut = depth - 1;
-      if (cut < 0) top += (int64_t)level.size();
+      if (cut < 0 && top + (int64_t)level.size() > mostTop) {
+        cut = depth - 1;
+        tails += (int64_t)level.size() / 2; // (the parents of this level)
+      }
+      (cut < 0 ? top : tails) += (int64_t)level.size();
       below.clear();
       for (int32_t n : level) {
         if (tree.IsLeaf(n)) continue;
@@ -173,9 +176,8 @@ bool ChooseDeepWalk(const Forest &forest, const DeviceLimits &limits, LaunchPlan
       level.swap(below);
     }
     cuts->push_back(cut < 0 ? depth - 1 : cut);
-    tails += (int64_t)tree.NumNodes() - top + 64;
   }
-  if (tails >= kMaxTailNodes) return false;
+  if (tails > kMaxTailNodes) return false;
   plan->groupBytes = (int32_t)(std::min<int64_t>(room, std::max<int64_t>((bundles * mostTop + 4) * kNodeBytes, 1024)) & ~15);
   return true;
 }
