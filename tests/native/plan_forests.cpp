@@ -78,10 +78,74 @@ static void TailLimit() {
   }
 }
 
+// Nodes that no walk reaches (pruned models keep them) behind those of a tree: they take no place in any form.
+static Tree WithUnreachable(Tree tree, int32_t count) {
+  tree.value.insert(tree.value.end(), (size_t)count, 3.0f);
+  tree.feature.insert(tree.feature.end(), (size_t)count, 0);
+  tree.left.insert(tree.left.end(), (size_t)count, -1);
+  tree.right.insert(tree.right.end(), (size_t)count, -1);
+  return tree;
+}
+
+static void UnreachableNodes() {
+  const DeviceLimits limits;
+  for (int32_t features : {12, 120})
+    for (int32_t count : {1, 2, 700, 9000}) {
+      Forest forest, whole;
+      forest.numFeatures = whole.numFeatures = features;
+      for (int32_t nodes : {16383, 8191, 31, 1, 9001, 301}) { // (cut, and small enough to stay whole)
+        whole.trees.push_back(FullTree(nodes, features));
+        forest.trees.push_back(WithUnreachable(whole.trees.back(), count));
+      }
+      forest.Validate();
+      LaunchPlan plan, planOfWhole;
+      std::vector<int32_t> cuts, cutsOfWhole;
+      EXPECT(ChooseDeepWalk(forest, limits, &plan, &cuts) && ChooseDeepWalk(whole, limits, &planOfWhole, &cutsOfWhole) && cuts == cutsOfWhole,
+             "%d features, %d nodes", features, count);
+      try {
+        const PackedModel pm = PackWithCuts(forest, plan, cuts), pmOfWhole = PackWithCuts(whole, planOfWhole, cutsOfWhole);
+        EXPECT(pm.groups.size() == pmOfWhole.groups.size() && pm.tailNodes.size() == pmOfWhole.tailNodes.size() && pm.treesDeferred == pmOfWhole.treesDeferred,
+               "%d features, %d nodes: %zu groups and %zu tail nodes, %zu and %zu without", features, count, pm.groups.size(), pm.tailNodes.size(),
+               pmOfWhole.groups.size(), pmOfWhole.tailNodes.size());
+        for (size_t t = 0; t < whole.trees.size(); ++t) {
+          const Tree tree = UnpackTree(pm, (int32_t)t);
+          EXPECT(tree.value == whole.trees[t].value && tree.left == whole.trees[t].left && tree.right == whole.trees[t].right, "%d features, %d nodes, tree %zu",
+                 features, count, t);
+        }
+      } catch (const Error &e) {
+        EXPECT(false, "%d features, %d nodes: %s", features, count, e.what());
+      }
+      // deferred tails by a profile, of a tree that a tree group holds and that all rows leave at its first leaf
+      Tree tree{{0.5f, 0.1f}, {0, 0}, {1, -1}, {2, -1}, 0};
+      const Tree rest = FullTree(2047, features);
+      for (size_t n = 0; n < rest.NumNodes(); ++n) {
+        tree.value.push_back(rest.value[n]);
+        tree.feature.push_back(rest.feature[n]);
+        tree.left.push_back(rest.left[n] < 0 ? -1 : rest.left[n] + 2);
+        tree.right.push_back(rest.right[n] < 0 ? -1 : rest.right[n] + 2);
+      }
+      forest.trees = {WithUnreachable(tree, count % 2000)};
+      HitCountProfile profile;
+      profile.numRows = 100;
+      profile.hits.assign(1, std::vector<int64_t>(forest.trees[0].NumNodes(), 0));
+      profile.hits[0][0] = profile.hits[0][1] = 100;
+      WalkOptions walk;
+      walk.peelWalks = true;
+      try {
+        const LaunchPlan peeled = ChoosePlan(forest, 100000, nullptr, limits, walk);
+        EXPECT(peeled.deferTails, "%d features, %d nodes", features, count);
+        EXPECT(PackForest(forest, peeled, &profile).treesDeferred == 1, "%d features, %d nodes", features, count);
+      } catch (const Error &e) {
+        EXPECT(false, "%d features, %d nodes, by a profile: %s", features, count, e.what());
+      }
+    }
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
   if (asked("tail_limit")) TailLimit();
+  if (asked("unreachable_nodes")) UnreachableNodes();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

@@ -34,3 +34,7 @@ def test_big_trees_open_with_every_batch(driver):
 
 def test_deep_forests_up_to_the_last_tail_node(driver):
     run(driver, "tail_limit")
+
+
+def test_deep_trees_with_nodes_no_walk_reaches(driver):
+    run(driver, "unreachable_nodes")

@@ -740,12 +740,13 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
         if (tile.count == 0) leafLevel[tile.leafNode] = tile.level;
     } else {
       depth[t] = tree.Depth();
-      units[t] = (uint32_t)tree.NumNodes();
+      units[t] = 0; // (of the nodes that walks reach: pruned models keep others)
       std::vector<int32_t> stack{0};
       leafLevel[0] = 0;
       while (!stack.empty()) { // (the level of every node; only the leaves' entries are used)
         const int32_t n = stack.back();
         stack.pop_back();
+        ++units[t];
         if (tree.IsLeaf(n)) continue;
         leafLevel[tree.left[n]] = leafLevel[tree.right[n]] = leafLevel[n] + 1;
         stack.push_back(tree.left[n]);
@@ -795,7 +796,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
       uint32_t above = 0; // the top of the tree, the cut level's internal nodes as stubs
       int64_t tails = 0;  // those internal nodes again, and all below them
       for (size_t i = 0; i < tree.NumNodes(); ++i) {
-        if (nodeLevel[i] <= cut) ++above;
+        if (nodeLevel[i] >= 0 && nodeLevel[i] <= cut) ++above;
         if (nodeLevel[i] > cut || (nodeLevel[i] == cut && !tree.IsLeaf((int32_t)i))) ++tails;
       }
       if (tails <= tailBudget && !nanLeaf) {
