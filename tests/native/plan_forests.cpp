@@ -4,6 +4,7 @@
 
 #include <cstdio>
 #include <cstring>
+#include <limits>
 
 using namespace tbamd;
 
@@ -141,11 +142,39 @@ static void UnreachableNodes() {
     }
 }
 
+// Splits that no walk reaches may name any feature and compare with anything: they are no thresholds of the rows' ranks.
+static void UnreachableSplits() {
+  const DeviceLimits limits;
+  for (int32_t features : {12, 700}) {
+    Forest forest = ForestOf(features, 3, 255);
+    const int32_t most = MaxThresholdsPerFeature(forest);
+    for (Tree &tree : forest.trees)
+      for (int32_t n = 0; n < 400; ++n) {
+        tree.value.push_back(n % 3 ? 1000.0f + (float)n : std::numeric_limits<float>::quiet_NaN());
+        tree.feature.push_back(n % 2 ? 0 : 1 << 24);
+        tree.left.push_back(1);
+        tree.right.push_back(2);
+      }
+    forest.Validate();
+    EXPECT(MaxThresholdsPerFeature(forest) == most, "%d features: %d and %d", features, (int)MaxThresholdsPerFeature(forest), (int)most);
+    for (int64_t batch : {1, 1000, 1 << 20}) {
+      LaunchPlan plan = ChoosePlan(forest, batch, nullptr, limits);
+      (void)PackForest(forest, plan);
+      if (features > 100 || plan.kernel != LaunchPlan::Kernel::kRowParallelLds) continue;
+      plan.rankRows16 = true;
+      (void)PackForest(forest, plan);
+    }
+    (void)PackRankStream(forest);
+    (void)PackFewRows(forest);
+  }
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
   if (asked("tail_limit")) TailLimit();
   if (asked("unreachable_nodes")) UnreachableNodes();
+  if (asked("unreachable_splits")) UnreachableSplits();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

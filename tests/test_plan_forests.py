@@ -38,3 +38,7 @@ def test_deep_forests_up_to_the_last_tail_node(driver):
 
 def test_deep_trees_with_nodes_no_walk_reaches(driver):
     run(driver, "unreachable_nodes")
+
+
+def test_splits_no_walk_reaches_are_no_thresholds(driver):
+    run(driver, "unreachable_splits")

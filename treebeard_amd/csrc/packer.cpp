@@ -56,9 +56,17 @@ namespace {
 // Sorted distinct thresholds per feature of a forest already normalised to "x < t".
 std::vector<std::vector<float>> ThresholdsPerFeature(const Forest &forest) {
   std::vector<std::vector<float>> out((size_t)forest.numFeatures);
-  for (auto &tree : forest.trees)
-    for (size_t i = 0; i < tree.NumNodes(); ++i)
-      if (!tree.IsLeaf((int32_t)i)) out[(size_t)tree.feature[i]].push_back(tree.value[i]);
+  for (auto &tree : forest.trees) { // (of the splits that walks reach: nothing is known of others)
+    std::vector<int32_t> stack{0};
+    while (!stack.empty()) {
+      const int32_t n = stack.back();
+      stack.pop_back();
+      if (tree.IsLeaf(n)) continue;
+      out[(size_t)tree.feature[n]].push_back(tree.value[n]);
+      stack.push_back(tree.left[n]);
+      stack.push_back(tree.right[n]);
+    }
+  }
   for (auto &v : out) {
     std::sort(v.begin(), v.end());
     v.erase(std::unique(v.begin(), v.end()), v.end());
