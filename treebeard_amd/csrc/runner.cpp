@@ -258,9 +258,14 @@ void InferenceRunner::UploadDeep() {
   if (m_deep.packed) return; // (the forest's, whatever the launch plan)
   LaunchPlan plan;
   std::vector<int32_t> cuts;
-  if (ChooseDeepWalk(m_forest, m_limits, &plan, &cuts)) {
+  bool fits = ChooseDeepWalk(m_forest, m_limits, &plan, &cuts);
+  try {
+    if (fits) m_deep.model = PackWithCuts(m_forest, plan, cuts);
+  } catch (const Error &) { // (a form beside the plan: a forest that it cannot hold keeps the plan's kernel)
+    fits = false;
+  }
+  if (fits) {
     try {
-      m_deep.model = PackWithCuts(m_forest, plan, cuts);
       m_deep.nodes = Upload(m_deep.model.nodes, "upload nodes");
       m_deep.bundles = Upload(m_deep.model.bundles, "upload bundles");
       m_deep.bundleRoots = Upload(m_deep.model.bundleRoots, "upload bundle roots");
