@@ -2,6 +2,7 @@
 #include "packer.h"
 #include "tuner.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstring>
 #include <limits>
@@ -169,12 +170,38 @@ static void UnreachableSplits() {
   }
 }
 
+// Small forests with peeled walks have deferred tails whatever block shape the batch asks for, and stay in one tree group.
+static void SmallPeeled() {
+  const DeviceLimits limits;
+  WalkOptions walk;
+  walk.peelWalks = true;
+  for (int32_t features : {5, 20, 35})
+    for (int32_t nodes : {31, 127, 1023, 2047}) {
+      const Forest forest = ForestOf(features, std::max(1, 2900 / nodes), nodes);
+      HitCountProfile profile;
+      profile.numRows = 1;
+      for (const Tree &tree : forest.trees) profile.hits.emplace_back(tree.NumNodes(), 1);
+      for (int64_t batch : {20000, 60000, 100000, 200000, 1 << 20}) {
+        for (bool later : {false, true}) { // (with the model, or asked for when the runner is there)
+          LaunchPlan plan = ChoosePlan(forest, batch, nullptr, limits, later ? WalkOptions() : walk);
+          if (later) plan.peelWalks = true, plan.deferTails = DeferTailsFit(forest, &plan);
+          EXPECT(plan.deferTails, "%d features, %zu trees of %d nodes, %lld rows: %d x %d, groups of %d bytes", features, forest.trees.size(), nodes,
+                 (long long)batch, plan.rowsPerBlock, plan.treeThreads, plan.groupBytes);
+          const PackedModel pm = PackForest(forest, plan, &profile);
+          EXPECT(pm.groups.size() == 1 && pm.LdsBytes() <= (size_t)limits.ldsBytesPerBlock / 2, "%d features, %zu trees of %d nodes, %lld rows: %zu groups",
+                 features, forest.trees.size(), nodes, (long long)batch, pm.groups.size());
+        }
+      }
+    }
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
   if (asked("tail_limit")) TailLimit();
   if (asked("unreachable_nodes")) UnreachableNodes();
   if (asked("unreachable_splits")) UnreachableSplits();
+  if (asked("small_peeled")) SmallPeeled();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

@@ -42,3 +42,7 @@ def test_deep_trees_with_nodes_no_walk_reaches(driver):
 
 def test_splits_no_walk_reaches_are_no_thresholds(driver):
     run(driver, "unreachable_splits")
+
+
+def test_small_forests_keep_deferred_tails(driver):
+    run(driver, "small_peeled")

@@ -386,6 +386,7 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   //    turns.  2^20 rows x 60 trees of depth 5 69.6 -> 58.0 us, 210411 x 62 19.6 -> 17.2, 402162 x 51 of depth 4 30.0 -> 26.0
   //    (29 KB: 37.7 and 38.5).
   // (Not where the biggest tree asks for more than the group beside them: the blocks of 256 rows may have taken the whole LDS for it.)
+  int64_t held = plan.groupBytes; // of trees in a group, for the rule on the trees side by side
   if (forest.numClasses == 0 && slices == 1 && rb == 256 && budget == halfLds && roomFor(128, halfLds) >= need &&
       !(ov && (ov->numRowsPerTB > 0 || ov->numTreeThreads > 0))) {
     const bool idle = rowBlocks <= limits.computeUnits, fewTrees = totalBytes <= 24 * 1024;
@@ -393,12 +394,12 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
       rb = plan.rowsPerBlock = 128;
       plan.treeThreads = fewTrees ? 4 : 8;
       plan.groupBytes = (int32_t)(std::min<int64_t>({65536, roomFor(rb, halfLds), 256LL * plan.ThreadsPerBlock()}) & ~15);
-      if (fewTrees) plan.groupBytes = std::min<int32_t>(plan.groupBytes, (int32_t)((totalBytes + 1024) & ~15));
+      held = fewTrees ? std::min<int64_t>(plan.groupBytes, totalBytes + 1024) : plan.groupBytes;
     }
   }
   if (slices > groups) { // more, smaller groups so that every slice has one
     int64_t perSlice = std::max<int64_t>((totalBytes + slices - 1) / slices + 4096, need);
-    if (perSlice < plan.groupBytes) plan.groupBytes = (int32_t)((perSlice + 15) & ~15);
+    if (perSlice < plan.groupBytes) held = plan.groupBytes = (int32_t)((perSlice + 15) & ~15);
   }
   // Four trees side by side hide more latency than two, but where a group holds fewer trees than the tree threads could take
   // that way, threads without a bundle wait for the others.  262144 rows, 200 to 300 trees, two and four trees a lane: four tree
@@ -406,7 +407,7 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // and 148, 19.5 158 and 171, 8.0 207 and 246; sixteen 47 147 and 141, 40 161 and 161, 31 183 and 189, 12 242 and 282; 40000
   // rows alike.  (One tree a lane is never faster.)
   if (!(ov && ov->treeWalkInterleaveFactor > 0) &&
-      (double)plan.groupBytes * (double)forest.trees.size() < (2.4 * plan.treeThreads + 3.4) * (double)totalBytes)
+      (double)held * (double)forest.trees.size() < (2.4 * plan.treeThreads + 3.4) * (double)totalBytes)
     plan.interleave = 2;
   // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
   // not fit and that way costs less (the packer's costs).  200000 rows, four and two side by side: 100 trees of depth 7, 90
