@@ -195,6 +195,24 @@ static void SmallPeeled() {
     }
 }
 
+// The block shape of batches of up to a block of 256 rows for each compute unit, either side of its rule's lines.
+static void SmallBatches() {
+  const DeviceLimits limits;
+  const struct { int64_t batch; int32_t trees, nodes, features, rows, threads; } shapes[] = {
+      {32768, 30, 255, 20, 128, 8},  {32769, 30, 255, 20, 256, 4},                                // half of the units have a block, and more
+      {40000, 123, 31, 20, 256, 4},  {40000, 124, 31, 20, 128, 8},                                // 492 and 496 levels, one group
+      {40000, 93, 127, 20, 256, 4},  {40000, 94, 127, 20, 128, 8},                                // 558 and 564, two groups
+      {40000, 48, 127, 50, 256, 4},  {40000, 49, 127, 50, 128, 8},                                // 288 and 294, two groups beside 256 rows and one beside 128
+      {65536, 99, 255, 20, 256, 4},  {65536, 100, 255, 20, 128, 8}, {65537, 100, 255, 20, 256, 4}}; // 693 and 700, four groups
+  for (auto s : shapes) {
+    const Forest forest = ForestOf(s.features, s.trees, s.nodes);
+    const LaunchPlan plan = ChoosePlan(forest, s.batch, nullptr, limits);
+    EXPECT(plan.treeSlices > 1 || (plan.rowsPerBlock == s.rows && plan.treeThreads == s.threads), "%lld rows, %d trees of %d nodes: %d x %d",
+           (long long)s.batch, s.trees, s.nodes, plan.rowsPerBlock, plan.treeThreads);
+    EXPECT(plan.treeSlices == 1, "%lld rows, %d trees of %d nodes: %d slices", (long long)s.batch, s.trees, s.nodes, plan.treeSlices);
+  }
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
@@ -202,6 +220,7 @@ int main(int argc, char **argv) {
   if (asked("unreachable_nodes")) UnreachableNodes();
   if (asked("unreachable_splits")) UnreachableSplits();
   if (asked("small_peeled")) SmallPeeled();
+  if (asked("small_batches")) SmallBatches();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

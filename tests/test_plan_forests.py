@@ -46,3 +46,7 @@ def test_splits_no_walk_reaches_are_no_thresholds(driver):
 
 def test_small_forests_keep_deferred_tails(driver):
     run(driver, "small_peeled")
+
+
+def test_block_shapes_of_small_batches(driver):
+    run(driver, "small_batches")

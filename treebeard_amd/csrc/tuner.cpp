@@ -379,9 +379,14 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     }
   }
   // Smaller row blocks than two blocks per compute unit leave room for:
-  //  * fewer than a block of 256 rows for each compute unit, and too few trees to slice: 128 rows x 8 tree threads.  33126 rows x
-  //    275 trees of depth 4 17.6 -> 15.5 us, 31046 x 182 12.8 -> 9.4, 20909 x 120 of depth 5 11.1 -> 9.5, 50001 x 100 of depth 8
-  //    18.9 -> 17.2;
+  //  * up to a block of 256 rows for each compute unit, and too few trees to slice: 128 rows x 8 tree threads, two of which share a
+  //    unit once every other unit would have a block of 256.  Up to there they always win or tie (20761 rows x 266 trees of depth
+  //    6 21.0 -> 13.4 us, 8017 x 61 7.5 -> 7.0, 20755 x 79 of depth 3 7.0 and 7.1).  Beyond, twice the blocks stage every group:
+  //    that pays where the rows' walk is long for the groups there are, or where the smaller row tile saves groups.  125 forests of
+  //    30 to 320 trees on 32800 to 65536 rows, levels of a walk, groups beside 256 rows and beside 128: 541 levels 1 and 1 groups
+  //    10.5 -> 9.6 us, 472 1 1 9.5 and 9.3, 340 1 1 7.9 and 8.4, 258 1 1 7.4 -> 8.1; 669 2 2 13.8 -> 12.4, 561 2 2 11.3 -> 12.0;
+  //    778 3 3 15.0 and 14.6, 650 3 3 12.8 and 13.1; 700 4 4 15.5 -> 14.8; 397 2 1 9.7 -> 8.9.  Taken of them: none that loses
+  //    more than 3 %, left: none that would gain more than 0.4 us;
   //  * forests of up to 24 KB, whose rows take as long to stage as to walk: 128 x 4, of which three and more to a unit take
   //    turns.  2^20 rows x 60 trees of depth 5 69.6 -> 58.0 us, 210411 x 62 19.6 -> 17.2, 402162 x 51 of depth 4 30.0 -> 26.0
   //    (29 KB: 37.7 and 38.5).
@@ -389,12 +394,18 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   int64_t held = plan.groupBytes; // of trees in a group, for the rule on the trees side by side
   if (forest.numClasses == 0 && slices == 1 && rb == 256 && budget == halfLds && roomFor(128, halfLds) >= need &&
       !(ov && (ov->numRowsPerTB > 0 || ov->numTreeThreads > 0))) {
-    const bool idle = rowBlocks <= limits.computeUnits, fewTrees = totalBytes <= 24 * 1024;
+    const int64_t smaller = std::min<int64_t>(65536, roomFor(128, halfLds)) & ~15LL;
+    const int64_t smallerGroups = std::max<int64_t>(1, (totalBytes + smaller - 1) / smaller);
+    int64_t levels = 0;
+    for (const Tree &tree : forest.trees) levels += tree.Depth();
+    const bool fewTrees = totalBytes <= 24 * 1024;
+    const bool idle = rowBlocks * 2 <= limits.computeUnits ||
+                      (rowBlocks <= limits.computeUnits && (fewTrees || levels >= 424 + 69 * smallerGroups - 200 * (groups - smallerGroups)));
     if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits)) {
       rb = plan.rowsPerBlock = 128;
       plan.treeThreads = fewTrees ? 4 : 8;
-      plan.groupBytes = (int32_t)(std::min<int64_t>({65536, roomFor(rb, halfLds), 256LL * plan.ThreadsPerBlock()}) & ~15);
-      held = fewTrees ? std::min<int64_t>(plan.groupBytes, totalBytes + 1024) : plan.groupBytes;
+      plan.groupBytes = (int32_t)smaller;
+      held = fewTrees ? std::min<int64_t>(smaller, totalBytes + 1024) : smaller;
     }
   }
   if (slices > groups) { // more, smaller groups so that every slice has one
