@@ -1626,7 +1626,9 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
 // here, and the whole call 1.308 -> 1.223; 20000 rows 126 -> 120 us.  A level takes 0.067 ms (a wave's eight LDS reads and 20
 // VALU instructions in 34 cycles of its compute unit: LDS pipes 70 %, VALUs 60 % busy), the leaf values 0.065, the rest 0.16.
 // ---------------------------------------------------------------------------
-template <int K> // chains
+// kStays: workgroups go on with other rows.  Where none does, what that takes (76 VGPRs and 1700 bytes of code) is left out: 3644
+// rows x 167 trees of 896 features 16.8 -> 16.2 us, 5504 x 92 of 1401 21.7 -> 21.2, 7713 x 46 of 672 15.2 -> 14.5.
+template <int K, bool kStays> // chains
 __global__ void __launch_bounds__(kStreamMaxWaves * 64)
 RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__ words, const float *__restrict__ values,
                  const uint32_t *__restrict__ bundles, int64_t rows, int F, int numBundles, int slices, int transform,
@@ -1639,7 +1641,7 @@ RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__
   const auto blockOf = [](uint32_t linear) { return (int64_t)(linear >> 4) * 16 + (int64_t)((linear & 7u) * 2u + ((linear >> 3) & 1u)); };
   const uint32_t padded = (uint32_t)((rows + 16 * kStreamRows - 1) / (16 * kStreamRows)) * 16u;
   const auto blockFrom = [&](uint32_t linear) { // the first that has rows, of those this workgroup takes
-    while (linear < padded && blockOf(linear) * kStreamRows >= rows) linear += gridDim.x;
+    while (linear < padded && blockOf(linear) * kStreamRows >= rows) linear = kStays ? linear + gridDim.x : padded;
     return linear;
   };
   uint32_t linear = blockFrom(blockIdx.x);
@@ -1683,7 +1685,7 @@ RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__
   }
   // Bundles of wave w, per row block.  (One division, while the copies are on their way: one for every wave's sum, when a row
   // block ends, took 0.4 to 0.8 us of each: 217490 rows x 107 trees of 673 features 274 -> 254 us.)
-  const int everyWave = (last - first) / waves, waveMore = (last - first) - everyWave * waves;
+  const int everyWave = kStays ? (last - first) / waves : 0, waveMore = (last - first) - everyWave * waves;
   const auto bundlesOf = [&](int w) { return everyWave + (w < waveMore ? 1 : 0); };
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __syncthreads(); // the rows are there; until they are through, the waves run on their own
@@ -1692,8 +1694,8 @@ RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__
   const bool upper = lane >= 32;
   uint32_t buffer = mine;
   for (uint32_t pass = 0;; ++pass) {
-    const uint32_t nextLinear = blockFrom(linear + gridDim.x);
-    const bool more = nextLinear < padded;
+    const uint32_t nextLinear = kStays ? blockFrom(linear + gridDim.x) : padded;
+    const bool more = kStays && nextLinear < padded;
     U32x4 nextRanks[kStreamTilePieces];
 #define TBAMD_STREAM_NEXT_ROWS                                                                                         \
   _Pragma("unroll") for (int i = 0; i < kStreamTilePieces; ++i) {                                                      \
@@ -1760,9 +1762,10 @@ RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__
 #pragma unroll
     for (int k = 0; k < K; ++k) acc += (double)values[at[k]];
     acc += ShuffleXor(acc, 32);
-    // A wave's sums go where its last bundle was: its other buffer may hold the first one for the next rows.
+    // A wave's sums go where its last bundle was: its other buffer may hold the first one for the next rows.  (Of a workgroup
+    // that does not stay no copy is on its way any more: either buffer.)
     const auto meetOf = [&](int w) {
-      const uint32_t walked = (uint32_t)bundlesOf(w) * (pass + 1u);
+      const uint32_t walked = kStays ? (uint32_t)bundlesOf(w) * (pass + 1u) : 0u;
       return reinterpret_cast<double *>(lds + tileBytes + (uint32_t)w * (2u * kStreamBundleBytes) + (walked & 1u ? 0u : kStreamBundleBytes));
     };
     if (lane < kStreamRows) meetOf(wave)[lane] = acc;
@@ -2128,10 +2131,13 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
   // (a workgroup has a compute unit's LDS to itself and goes on with other rows; multiples of 16 keep the XCDs' row blocks)
   const int64_t groups = std::min<int64_t>(blocks, std::max(16, p.computeUnits / 16 * 16));
   const dim3 grid((unsigned)groups, (unsigned)p.slices), block((unsigned)waves * 64);
-  hipError_t e = p.chains == 4 ? AllowFullLds<&RankStreamKernel<4>>() : AllowFullLds<&RankStreamKernel<2>>();
+  const bool stays = groups < blocks, four = p.chains == 4;
+  hipError_t e = stays ? (four ? AllowFullLds<&RankStreamKernel<4, true>>() : AllowFullLds<&RankStreamKernel<2, true>>())
+                       : (four ? AllowFullLds<&RankStreamKernel<4, false>>() : AllowFullLds<&RankStreamKernel<2, false>>());
   if (e != hipSuccess) return e;
-  return StartKernel(p.chains == 4 ? &RankStreamKernel<4> : &RankStreamKernel<2>, grid, block, ldsBytes, stream, p.done, p.ranks, p.words,
-                     p.values, p.bundles, p.rows, p.numFeatures, p.numBundles, p.slices, p.transform, p.initialValue,
+  return StartKernel(stays ? (four ? &RankStreamKernel<4, true> : &RankStreamKernel<2, true>)
+                           : (four ? &RankStreamKernel<4, false> : &RankStreamKernel<2, false>),
+                     grid, block, ldsBytes, stream, p.done, p.ranks, p.words, p.values, p.bundles, p.rows, p.numFeatures, p.numBundles, p.slices, p.transform, p.initialValue,
                      p.slices > 1 ? nullptr : p.out, p.slices > 1 ? p.partial : nullptr);
 }
 
