@@ -213,6 +213,33 @@ static void SmallBatches() {
   }
 }
 
+// Classifiers walk two trees side by side for classes of the tree threads' own only where they are packed so, or where groups hold
+// few trees.
+static void TwoTreesOfClasses() {
+  const DeviceLimits limits;
+  long own = 0, few = 0;
+  for (int32_t features : {12, 33, 54, 78, 113})
+    for (int32_t classes : {3, 5, 7, 10, 13, 16})
+      for (int32_t trees : {61, 160, 321, 607}) {
+        Forest forest = ForestOf(features, trees, trees % 2 ? 127 : 255);
+        forest.numClasses = classes;
+        for (int32_t t = 0; t < trees; ++t) forest.trees[(size_t)t].classId = t % classes;
+        for (int64_t batch : {2600, 30000, 190000}) {
+          const LaunchPlan plan = ChoosePlan(forest, batch, nullptr, limits);
+          if (plan.interleave != 2 || plan.kernel != LaunchPlan::Kernel::kRowParallelLds) continue;
+          const double held = (double)plan.groupBytes / (double)(forest.trees[0].NumNodes() * kNodeBytes);
+          if (held < std::min(24.0, 2.4 * plan.treeThreads + 3.4)) {
+            ++few;
+            continue;
+          }
+          ++own;
+          EXPECT(PacksOwnClasses(forest, plan) && PackForest(forest, plan).ownClasses, "%d features, %d classes, %d trees, %lld rows: groups of %.1f trees",
+                 features, classes, trees, (long long)batch, held);
+        }
+      }
+  EXPECT(own > 0 && few > 0, "%ld, %ld", own, few);
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
@@ -221,6 +248,7 @@ int main(int argc, char **argv) {
   if (asked("unreachable_splits")) UnreachableSplits();
   if (asked("small_peeled")) SmallPeeled();
   if (asked("small_batches")) SmallBatches();
+  if (asked("two_trees_of_classes")) TwoTreesOfClasses();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

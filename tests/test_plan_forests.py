@@ -50,3 +50,7 @@ def test_small_forests_keep_deferred_tails(driver):
 
 def test_block_shapes_of_small_batches(driver):
     run(driver, "small_batches")
+
+
+def test_two_trees_side_by_side_of_classifiers(driver):
+    run(driver, "two_trees_of_classes")

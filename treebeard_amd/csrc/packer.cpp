@@ -575,6 +575,24 @@ FewRowsModel PackFewRows(const Forest &input) {
 
 namespace {
 PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile, const std::vector<int32_t> *cuts);
+bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth, const std::vector<uint32_t> &units,
+                    const std::vector<int32_t> &order, std::vector<std::vector<int32_t>> *rounds);
+}
+
+bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan) {
+  std::vector<int32_t> depth(forest.trees.size()), order(forest.trees.size());
+  std::vector<uint32_t> units(forest.trees.size());
+  for (size_t t = 0; t < forest.trees.size(); ++t) {
+    depth[t] = forest.trees[t].Depth();
+    units[t] = (uint32_t)MakeLevelOrder(forest.trees[t]).order.size();
+  }
+  std::iota(order.begin(), order.end(), 0);
+  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+    const int32_t ca = forest.trees[(size_t)a].classId, cb = forest.trees[(size_t)b].classId;
+    return ca != cb ? ca < cb : depth[(size_t)a] < depth[(size_t)b];
+  });
+  std::vector<std::vector<int32_t>> rounds;
+  return OwnClassRounds(forest, plan, depth, units, order, &rounds);
 }
 
 PackedModel PackForest(const Forest &forest, const LaunchPlan &plan, const HitCountProfile *profile) {
@@ -587,6 +605,52 @@ PackedModel PackWithCuts(const Forest &forest, const LaunchPlan &plan, const std
 }
 
 namespace {
+// Classes of the tree threads' own: rounds of a bundle for every tree thread, class c's on thread c % treeThreads.  Against them
+// stand the classes one after the other, each dealt over all tree threads, which meet at its end: that costs as much as about
+// 20 levels of a tree thread.  2^20 rows x 54 features, 800 trees of depth 6, four tree threads, levels of a tree thread that way
+// and this, and what was measured: 8 classes 1504 and 1200, 916 and 847 us; 12 1680 and 1224, 969 and 862; 11 1540 and 1368,
+// 955 and 894; 7 1484 and 1392, 917 and 910; 10 1400 and 1440, 862 and 890; 9 1476 and 1656, 941 and 957; 6 1416 and 1632, 898
+// and 949; 5 1300 and 1920, 853 and 1015.  `order`: by class.  False: the classes meet.
+bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth, const std::vector<uint32_t> &units,
+                    const std::vector<int32_t> &order, std::vector<std::vector<int32_t>> *rounds) {
+  if (forest.numClasses < 2 || plan.treeThreads < 2 || plan.kernel != LaunchPlan::Kernel::kRowParallelLds || order.empty()) return false;
+  const size_t TT = (size_t)plan.treeThreads, C = (size_t)forest.numClasses;
+  const int K = plan.interleave;
+  const uint32_t groupCapacity = (uint32_t)plan.groupBytes / kNodeBytes;
+  std::vector<std::vector<int32_t>> ofClass(C);
+  for (int32_t t : order) ofClass[(size_t)forest.trees[(size_t)t].classId].push_back(t);
+  double levels = 0.0;
+  for (int32_t d : depth) levels += d;
+  const double bundleLevels = K * levels / (double)forest.trees.size();
+  double meeting = 0.0;
+  size_t largest = 0;
+  for (auto &trees : ofClass) {
+    meeting += (double)((trees.size() + TT * K - 1) / (TT * K)) * bundleLevels + 20.0;
+    largest = std::max(largest, trees.size());
+  }
+  for (size_t c0 = 0; c0 < C; c0 += TT) {
+    size_t most = 0;
+    for (size_t c = c0; c < std::min(C, c0 + TT); ++c) most = std::max(most, (ofClass[c].size() + K - 1) / K);
+    for (size_t i = 0; i < most; ++i) {
+      std::vector<int32_t> round(TT * K, -1);
+      uint32_t need = 0;
+      for (size_t c = c0; c < std::min(C, c0 + TT); ++c)
+        for (size_t k = 0; k < (size_t)K && i * K + k < ofClass[c].size(); ++k) {
+          const int32_t t = ofClass[c][i * K + k];
+          round[(c - c0) * K + k] = t;
+          need += units[(size_t)t];
+        }
+      if (need + 2 > groupCapacity - 1) return false;
+      rounds->push_back(std::move(round));
+    }
+  }
+  // Near a tie the threads that wait can lose, with tree slices most.  230 forests of 2 to 16 classes, both ways: without slices
+  // 0.34 to 0.98 of the time up to 0.95 of the cost, but 1.04 at 0.92 where all of a class is one round of bundles (74 trees, five
+  // classes); with slices up to 1.01 below 0.81 of the cost, 1.10 at 0.84.
+  const double share = plan.treeSlices > 1 ? 0.81 : largest <= TT * K ? 0.9 : 0.95;
+  return (double)rounds->size() * bundleLevels < meeting * share;
+}
+
 constexpr uint32_t kPeeledTailNodes = 1u << 20; // below the cuts of a plan with a profile (8 MB: they stay in the caches)
 
 PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile, const std::vector<int32_t> *cuts) {
@@ -988,43 +1052,8 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     }
   };
 
-  // Classes of the tree threads' own: rounds of a bundle for every tree thread, class c's on thread c % treeThreads.  Against them
-  // stand the classes one after the other, each dealt over all tree threads, which meet at its end: that costs as much as about
-  // 20 levels of a tree thread.  2^20 rows x 54 features, 800 trees of depth 6, four tree threads, levels of a tree thread that way
-  // and this, and what was measured: 8 classes 1504 and 1200, 916 and 847 us; 12 1680 and 1224, 969 and 862; 11 1540 and 1368,
-  // 955 and 894; 7 1484 and 1392, 917 and 910; 10 1400 and 1440, 862 and 890; 9 1476 and 1656, 941 and 957; 6 1416 and 1632, 898
-  // and 949; 5 1300 and 1920, 853 and 1015.
-  std::vector<std::vector<int32_t>> rounds; // treeThreads * K trees each, -1: none
-  if (forest.numClasses > 1 && plan.treeThreads > 1 && T == 1 && plan.kernel == LaunchPlan::Kernel::kRowParallelLds) {
-    const size_t TT = (size_t)plan.treeThreads, C = (size_t)forest.numClasses;
-    std::vector<std::vector<int32_t>> ofClass(C);
-    for (int32_t t : order) ofClass[(size_t)forest.trees[(size_t)t].classId].push_back(t);
-    double levels = 0.0;
-    for (int32_t d : depth) levels += d;
-    const double bundleLevels = K * levels / (double)std::max<size_t>(1, numTrees);
-    double meeting = 0.0;
-    for (auto &trees : ofClass) meeting += (double)((trees.size() + TT * K - 1) / (TT * K)) * bundleLevels + 20.0;
-    bool fits = true;
-    for (size_t c0 = 0; c0 < C; c0 += TT) {
-      size_t most = 0;
-      for (size_t c = c0; c < std::min(C, c0 + TT); ++c) most = std::max(most, (ofClass[c].size() + K - 1) / K);
-      for (size_t i = 0; i < most; ++i) {
-        std::vector<int32_t> round(TT * K, -1);
-        uint32_t need = 0;
-        for (size_t c = c0; c < std::min(C, c0 + TT); ++c)
-          for (size_t k = 0; k < (size_t)K && i * K + k < ofClass[c].size(); ++k) {
-            const int32_t t = ofClass[c][i * K + k];
-            round[(c - c0) * K + k] = t;
-            need += units[(size_t)t];
-          }
-        fits = fits && need + 2 <= groupCapacity - 1;
-        rounds.push_back(std::move(round));
-      }
-    }
-    // (Near a tie the threads that wait lose, more so where blocks of few rounds share a row block: 8643 rows, 474 trees of depth
-    // 8, nine classes, seven slices, 1.00 of the cost, 38.0 -> 41.3 us; 50973 rows, 121 trees, two slices, 0.82 of it, 45.1 -> 46.3.)
-    pm.ownClasses = fits && !order.empty() && (double)rounds.size() * bundleLevels < meeting * (plan.treeSlices > 1 ? 0.81 : 0.95);
-  }
+  std::vector<std::vector<int32_t>> rounds; // classes of the tree threads' own: treeThreads * K trees each, -1: none
+  if (T == 1) pm.ownClasses = OwnClassRounds(forest, plan, depth, units, order, &rounds);
   if (pm.ownClasses) {
     const size_t TT = (size_t)plan.treeThreads;
     for (size_t next = 0; next < rounds.size();) {

@@ -183,6 +183,9 @@ PackedModel PackForest(const Forest &forest, const LaunchPlan &plan, const HitCo
 // weighed on a profile.
 PackedModel PackWithCuts(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &cuts);
 
+// Whether PackForest gives every class of a forest to one tree thread under a scalar row-parallel plan (PackedModel::ownClasses).
+bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan);
+
 // Inverse of PackForest for tests: rebuilds (value, feature, left, right) of
 // original tree `tree` from the packed arrays.
 Tree UnpackTree(const PackedModel &model, int32_t tree);

@@ -416,12 +416,14 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // that way, threads without a bundle wait for the others.  262144 rows, 200 to 300 trees, two and four trees a lane: four tree
   // threads 54 features 16.2 trees a group 132 and 122 us, 14.0 146 and 142, 12.1 106 and 120; eight 27.9 136 and 126, 22.8 147
   // and 148, 19.5 158 and 171, 8.0 207 and 246; sixteen 47 147 and 141, 40 161 and 161, 31 183 and 189, 12 242 and 282; 40000
-  // rows alike.  (One tree a lane is never faster.)
-  if (!(ov && ov->treeWalkInterleaveFactor > 0) &&
-      (double)held * (double)forest.trees.size() < (2.4 * plan.treeThreads + 3.4) * (double)totalBytes)
+  // rows alike.  (One tree a lane is never faster.)  Classifiers alike, but sixteen tree threads 16.9 298 and 279, 20.1 2396 and
+  // 2268, 23.2 105 and 105, 25.4 133 and 138, 80 and 83: a group holds few classes at a time.
+  const double fewInGroup = forest.numClasses > 0 ? std::min(24.0, 2.4 * plan.treeThreads + 3.4) : 2.4 * plan.treeThreads + 3.4;
+  if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)held * (double)forest.trees.size() < fewInGroup * (double)totalBytes)
     plan.interleave = 2;
   // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
-  // not fit and that way costs less (the packer's costs).  200000 rows, four and two side by side: 100 trees of depth 7, 90
+  // not fit, that way costs less (the packer's costs), and the packer will take it: where it does not, two side by side lose (607
+  // trees, 13 classes, 189139 rows 235 and 247 us, 321 trees, 7 classes, 2642 rows 27.2 and 29.2).  200000 rows, four and two side by side: 100 trees of depth 7, 90
   // features, 10 classes 103.7 and 60.7 us; 300 of depth 8, 54 features, 12 classes 177.1 and 137.8; 200 of depth 8, 70
   // features, 6 classes 132.8 and 105.9; 400 of depth 7, 90 features, 8 classes 195.4 and 152.3.
   if (forest.numClasses > 1 && plan.treeThreads > 1 && plan.interleave == 4 && !(ov && ov->treeWalkInterleaveFactor > 0) &&
@@ -431,7 +433,10 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     levels /= (double)forest.trees.size();
     const double ofClass = (double)forest.trees.size() / forest.numClasses, threads = plan.treeThreads;
     const double own = std::ceil(forest.numClasses / threads) * std::ceil(ofClass / 2) * 2 * levels;
-    if (own < forest.numClasses * (std::ceil(ofClass / (4 * threads)) * 4 * levels + 20.0)) plan.interleave = 2;
+    LaunchPlan two = plan;
+    two.interleave = 2;
+    two.treeSlices = (int32_t)std::max<int64_t>(1, slices);
+    if (own < forest.numClasses * (std::ceil(ofClass / (4 * threads)) * 4 * levels + 20.0) && PacksOwnClasses(forest, two)) plan.interleave = 2;
   }
   plan.treeSlices = (int32_t)std::max<int64_t>(1, slices);
   return plan;
