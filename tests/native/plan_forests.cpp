@@ -170,7 +170,7 @@ static void UnreachableSplits() {
   }
 }
 
-// Small forests with peeled walks have deferred tails whatever block shape the batch asks for, and stay in one tree group.
+// Small forests with peeled walks: no deferred tails in the blocks of their own, in others as before; one tree group either way.
 static void SmallPeeled() {
   const DeviceLimits limits;
   WalkOptions walk;
@@ -185,7 +185,9 @@ static void SmallPeeled() {
         for (bool later : {false, true}) { // (with the model, or asked for when the runner is there)
           LaunchPlan plan = ChoosePlan(forest, batch, nullptr, limits, later ? WalkOptions() : walk);
           if (later) plan.peelWalks = true, plan.deferTails = DeferTailsFit(forest, &plan);
-          EXPECT(plan.deferTails, "%d features, %zu trees of %d nodes, %lld rows: %d x %d, groups of %d bytes", features, forest.trees.size(), nodes,
+          EXPECT((plan.rowsPerBlock == 128 && plan.treeThreads == 4) == (batch != 100000), "%lld rows: %d x %d", (long long)batch, plan.rowsPerBlock,
+                 plan.treeThreads);
+          EXPECT(plan.deferTails == (batch == 100000) && plan.peelWalks, "%d features, %zu trees of %d nodes, %lld rows: %d x %d, groups of %d bytes", features, forest.trees.size(), nodes,
                  (long long)batch, plan.rowsPerBlock, plan.treeThreads, plan.groupBytes);
           const PackedModel pm = PackForest(forest, plan, &profile);
           EXPECT(pm.groups.size() == 1 && pm.LdsBytes() <= (size_t)limits.ldsBytesPerBlock / 2, "%d features, %zu trees of %d nodes, %lld rows: %zu groups",

@@ -44,7 +44,7 @@ def test_splits_no_walk_reaches_are_no_thresholds(driver):
     run(driver, "unreachable_splits")
 
 
-def test_small_forests_keep_deferred_tails(driver):
+def test_small_forests_with_peeled_walks(driver):
     run(driver, "small_peeled")
 
 

@@ -1097,6 +1097,7 @@ std::string InferenceRunner::DescribePlan() const {
     else if (m_forest.numClasses > 0) peel = "ignored(classes)";
     else if (p.quantizedRows || p.rankRows16) peel = "ignored(ranks)";
     else if (p.featureOffsetInWords) peel = "ignored(words)";
+    else if (SmallForestBlocks(m_forest, p)) peel = "ignored(small)";
     else peel = "ignored(lds)"; // the stub column and the queues do not fit beside this plan's tree groups
   }
   os << "kernel="

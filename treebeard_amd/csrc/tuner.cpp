@@ -114,6 +114,10 @@ double SplitWalkMicros(const WalkShape &w) {
   return BlockMicros(w, rounded * 1.03, w.blocksPerUnit) + std::ceil(share) * BlockMicros(w, 0.0, w.blocksPerUnit) + kFinalizeMicros;
 }
 
+namespace {
+constexpr int64_t kSmallForestBytes = 24 * 1024;
+}
+
 LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoScheduleOptions *ov,
                       const DeviceLimits &limits, const WalkOptions &walk) {
   if (walk.tileSize < 1 || walk.tileSize > kMaxTileSize)
@@ -187,10 +191,18 @@ int32_t DeepWalkSlices(int64_t rowBlocks, int64_t groups, const DeviceLimits &li
   return (int32_t)std::max<int64_t>(1, std::min<int64_t>(2LL * limits.computeUnits / std::max<int64_t>(1, rowBlocks), groups));
 }
 
+bool SmallForestBlocks(const Forest &forest, const LaunchPlan &plan) {
+  return plan.rowsPerBlock == 128 && plan.treeThreads == 4 && (int64_t)forest.NumNodes() * kNodeBytes <= kSmallForestBytes;
+}
+
 bool DeferTailsFit(const Forest &forest, LaunchPlan *plan) {
   if (plan->kernel != LaunchPlan::Kernel::kRowParallelLds || plan->WalkTile() != 1 || plan->quantizedRows || plan->rankRows16 ||
       plan->featureOffsetInWords || forest.numClasses > 0)
     return false;
+  // Blocks of small forests walk whole trees faster: 45 skewed forests of 2 to 24 KB, rows along the spines, 12000 to 950000 rows,
+  // 4 % (30 trees of depth 9) to 20 % (17 trees of depth 8, 610597 rows 32.3 -> 25.8 us) in 128 x 4, and all of them than with
+  // deferred tails in 256 x 4.
+  if (SmallForestBlocks(forest, *plan)) return false;
   // every wave's queue comes out of the tree group's share of LDS
   const int64_t extra = (int64_t)(plan->ThreadsPerBlock() / 64) * kDeferBytesPerWave + 32;
   if (forest.numFeatures + 1 >= (1 << kTailFeatureBits)) return false;
@@ -391,26 +403,24 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   //    turns.  2^20 rows x 60 trees of depth 5 69.6 -> 58.0 us, 210411 x 62 19.6 -> 17.2, 402162 x 51 of depth 4 30.0 -> 26.0
   //    (29 KB: 37.7 and 38.5).
   // (Not where the biggest tree asks for more than the group beside them: the blocks of 256 rows may have taken the whole LDS for it.)
-  int64_t held = plan.groupBytes; // of trees in a group, for the rule on the trees side by side
   if (forest.numClasses == 0 && slices == 1 && rb == 256 && budget == halfLds && roomFor(128, halfLds) >= need &&
       !(ov && (ov->numRowsPerTB > 0 || ov->numTreeThreads > 0))) {
     const int64_t smaller = std::min<int64_t>(65536, roomFor(128, halfLds)) & ~15LL;
     const int64_t smallerGroups = std::max<int64_t>(1, (totalBytes + smaller - 1) / smaller);
     int64_t levels = 0;
     for (const Tree &tree : forest.trees) levels += tree.Depth();
-    const bool fewTrees = totalBytes <= 24 * 1024;
+    const bool fewTrees = totalBytes <= kSmallForestBytes;
     const bool idle = rowBlocks * 2 <= limits.computeUnits ||
                       (rowBlocks <= limits.computeUnits && (fewTrees || levels >= 424 + 69 * smallerGroups - 200 * (groups - smallerGroups)));
     if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits)) {
       rb = plan.rowsPerBlock = 128;
       plan.treeThreads = fewTrees ? 4 : 8;
-      plan.groupBytes = (int32_t)smaller;
-      held = fewTrees ? std::min<int64_t>(smaller, totalBytes + 1024) : smaller;
+      plan.groupBytes = (int32_t)(fewTrees ? std::min<int64_t>(smaller, totalBytes + 1024) & ~15LL : smaller);
     }
   }
   if (slices > groups) { // more, smaller groups so that every slice has one
     int64_t perSlice = std::max<int64_t>((totalBytes + slices - 1) / slices + 4096, need);
-    if (perSlice < plan.groupBytes) held = plan.groupBytes = (int32_t)((perSlice + 15) & ~15);
+    if (perSlice < plan.groupBytes) plan.groupBytes = (int32_t)((perSlice + 15) & ~15);
   }
   // Four trees side by side hide more latency than two, but where a group holds fewer trees than the tree threads could take
   // that way, threads without a bundle wait for the others.  262144 rows, 200 to 300 trees, two and four trees a lane: four tree
@@ -419,7 +429,7 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // rows alike.  (One tree a lane is never faster.)  Classifiers alike, but sixteen tree threads 16.9 298 and 279, 20.1 2396 and
   // 2268, 23.2 105 and 105, 25.4 133 and 138, 80 and 83: a group holds few classes at a time.
   const double fewInGroup = forest.numClasses > 0 ? std::min(24.0, 2.4 * plan.treeThreads + 3.4) : 2.4 * plan.treeThreads + 3.4;
-  if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)held * (double)forest.trees.size() < fewInGroup * (double)totalBytes)
+  if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)plan.groupBytes * (double)forest.trees.size() < fewInGroup * (double)totalBytes)
     plan.interleave = 2;
   // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
   // not fit, that way costs less (the packer's costs), and the packer will take it: where it does not, two side by side lose (607

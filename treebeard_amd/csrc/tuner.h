@@ -50,6 +50,8 @@ LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoSche
 // tile with byte offsets, a model without classes); when it can, the plan's tree groups give up the LDS the stub
 // feature's column and the waves' queues take.  The caller sets the flag.
 bool DeferTailsFit(const Forest &forest, LaunchPlan *plan);
+// The block shape of forests of a few KB (ChoosePlan), which has no deferred tails.
+bool SmallForestBlocks(const Forest &forest, const LaunchPlan &plan);
 
 // A forest with a tree too big for an LDS tree group (LaunchPlan::Kernel::kGlobalWalk), walked with deferred tails instead of
 // node by node from global memory: the tops of its trees fit.  Sets a plan for PackWithCuts and the level every tree is cut
