@@ -175,7 +175,7 @@ static void SmallPeeled() {
   const DeviceLimits limits;
   WalkOptions walk;
   walk.peelWalks = true;
-  for (int32_t features : {5, 20, 35})
+  for (int32_t features : {5, 20, 30})
     for (int32_t nodes : {31, 127, 1023, 2047}) {
       const Forest forest = ForestOf(features, std::max(1, 2900 / nodes), nodes);
       HitCountProfile profile;
@@ -197,7 +197,7 @@ static void SmallPeeled() {
     }
 }
 
-// The block shape of batches of up to a block of 256 rows for each compute unit, either side of its rule's lines.
+// The block shapes of batches of up to a block of 256 rows for each compute unit, and of small forests, either side of their rules' lines.
 static void SmallBatches() {
   const DeviceLimits limits;
   const struct { int64_t batch; int32_t trees, nodes, features, rows, threads; } shapes[] = {
@@ -205,7 +205,10 @@ static void SmallBatches() {
       {40000, 123, 31, 20, 256, 4},  {40000, 124, 31, 20, 128, 8},                                // 492 and 496 levels, one group
       {40000, 93, 127, 20, 256, 4},  {40000, 94, 127, 20, 128, 8},                                // 558 and 564, two groups
       {40000, 48, 127, 50, 256, 4},  {40000, 49, 127, 50, 128, 8},                                // 288 and 294, two groups beside 256 rows and one beside 128
-      {65536, 99, 255, 20, 256, 4},  {65536, 100, 255, 20, 128, 8}, {65537, 100, 255, 20, 256, 4}}; // 693 and 700, four groups
+      {65536, 99, 255, 20, 256, 4},  {65536, 100, 255, 20, 128, 8}, {65537, 100, 255, 20, 256, 4}, // 693 and 700, four groups
+      {131072, 59, 31, 50, 256, 4},  {131073, 59, 31, 50, 128, 4},                                // a round of blocks of 256 rows, and more
+      {300000, 59, 31, 50, 128, 4},  {300000, 60, 31, 50, 256, 4},                                // four fit a unit's LDS, and three
+      {163840, 60, 31, 50, 128, 4},  {163841, 60, 31, 50, 256, 4}};                               // three, of a round and a quarter
   for (auto s : shapes) {
     const Forest forest = ForestOf(s.features, s.trees, s.nodes);
     const LaunchPlan plan = ChoosePlan(forest, s.batch, nullptr, limits);

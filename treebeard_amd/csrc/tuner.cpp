@@ -401,7 +401,9 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   //    more than 3 %, left: none that would gain more than 0.4 us;
   //  * forests of up to 24 KB, whose rows take as long to stage as to walk: 128 x 4, of which three and more to a unit take
   //    turns.  2^20 rows x 60 trees of depth 5 69.6 -> 58.0 us, 210411 x 62 19.6 -> 17.2, 402162 x 51 of depth 4 30.0 -> 26.0
-  //    (29 KB: 37.7 and 38.5).
+  //    (29 KB: 37.7 and 38.5).  Four to a unit, that is: of 89 forests of 2 to 24 KB on 131100 to 2^20 rows they win by 0 to 16 %
+  //    where four fit its LDS (but for one, 1 %), and where three do lose 2 to 9 % (388783 rows x 60 trees of 58 features 31.9 ->
+  //    34.7 us, 311105 x 17 of 51 25.0 -> 27.7) unless one round of either is enough (157757 rows 12.8 -> 12.3, 199341 29.9 -> 29.2).
   // (Not where the biggest tree asks for more than the group beside them: the blocks of 256 rows may have taken the whole LDS for it.)
   if (forest.numClasses == 0 && slices == 1 && rb == 256 && budget == halfLds && roomFor(128, halfLds) >= need &&
       !(ov && (ov->numRowsPerTB > 0 || ov->numTreeThreads > 0))) {
@@ -412,7 +414,8 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     const bool fewTrees = totalBytes <= kSmallForestBytes;
     const bool idle = rowBlocks * 2 <= limits.computeUnits ||
                       (rowBlocks <= limits.computeUnits && (fewTrees || levels >= 424 + 69 * smallerGroups - 200 * (groups - smallerGroups)));
-    if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits)) {
+    const bool fourFit = (int64_t)(forest.numFeatures + 1) * 128 * 4 + totalBytes + 32 <= limits.ldsBytesPerBlock / 4;
+    if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits && (fourFit || rowBlocks <= 5LL * limits.computeUnits / 2))) {
       rb = plan.rowsPerBlock = 128;
       plan.treeThreads = fewTrees ? 4 : 8;
       plan.groupBytes = (int32_t)(fewTrees ? std::min<int64_t>(smaller, totalBytes + 1024) & ~15LL : smaller);
