@@ -90,3 +90,18 @@ def test_even_split_of_own_classes(tmp_path):
     pred, sums = cpu_oracle.predict(forest, x)
     np.testing.assert_array_equal(ids.cpu().numpy().astype(np.float32), pred)
     np.testing.assert_allclose(margins.cpu().numpy(), sums, rtol=RTOL_SUM, atol=1e-7)
+
+
+def test_a_base_score_that_is_no_number(tmp_path):
+    """Every sum is NaN: the class the running rule ends with is the last one, as without classes of the tree threads' own."""
+    path = class_model(tmp_path / "m.json", [t % 7 for t in range(35)], 7)
+    text = open(path).read()
+    assert text.count('"base_score"') == 1
+    start = text.index('"', text.index(":", text.index('"base_score"'))) + 1
+    open(path, "w").write(text[:start] + "nan" + text[text.index('"', start):])
+    x = np.random.Generator(np.random.PCG64(8)).normal(size=(500, FEATURES)).astype(np.float32)
+    for threads, own in ((1, 0), (4, 1), (2, 1)):
+        runner = make_runner(path, 500)
+        runner.set_plan(128, threads, 2, 32768, 1)
+        assert " ownClasses=%d" % own in runner.describe_plan()
+        np.testing.assert_array_equal(gpu_predict(runner, x), np.full(500, 6))

@@ -532,6 +532,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
     TBAMD_FLUSH_OWN_CLASS(C)
     if (!kFuse) return;
     // each tree thread has the best of its own classes: the larger sum, or the larger class id of equal ones, as the running rule
+    // (and of sums that are no numbers, by a base score that is none; a thread without a class has -inf and class 0)
     __syncthreads();
     float *bests = reinterpret_cast<float *>(lds);
     int *classes = reinterpret_cast<int *>(lds) + threads;
@@ -542,7 +543,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
     for (int t = 1; t < TT; ++t) {
       const float m = bests[t * RB + lane];
       const int c = classes[t * RB + lane];
-      if (m > best || (m == best && c > bestClass)) { best = m; bestClass = c; }
+      if (m > best || (!(best > m) && c > bestClass)) { best = m; bestClass = c; }
     }
     if (classOut) classOut[row] = (int8_t)bestClass;
     else out[row] = (float)bestClass;
