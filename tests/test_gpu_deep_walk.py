@@ -1,5 +1,7 @@
 """Forests whose trees do not fit LDS whole, walked with deferred tails: leaf for leaf the global-memory walk's predictions, over
 the three block shapes, odd batches, rows of infinities and NaN, the four comparisons."""
+import json
+
 import numpy as np
 import pytest
 
@@ -12,6 +14,7 @@ from treebeard_amd import synth  # noqa: E402
 
 from onnx_writer import write_onnx  # noqa: E402
 from test_gpu_parity import RTOL_SUM, gpu_predict, make_runner  # noqa: E402
+from test_gpu_plan_shapes import full_tree  # noqa: E402
 
 
 def deep_model(path, features, trees=9, leaf=lambda rng: rng.normal(0.0, 0.1), depth=13, **kind):
@@ -85,3 +88,44 @@ def test_plan_search_of_a_deep_forest(tmp_path):
     runner.autotune(dx.data_ptr(), rows)
     assert "batchKernel=deep_walk" in runner.describe_plan()
     np.testing.assert_allclose(gpu_predict(runner, x), cpu_oracle.predict(forest, x)[0], rtol=0, atol=1e-6)
+
+
+def test_nodes_that_no_walk_reaches(tmp_path):
+    """Leaves behind those of the trees, as pruning leaves them, in trees that are cut and in trees that stay whole."""
+    rng = np.random.Generator(np.random.PCG64(11))
+    trees = [full_tree(rng, nodes, 12) for nodes in (16383, 9001, 31, 1, 301)]
+    for tree, more in zip(trees, (2, 700, 9000, 1, 1)):
+        tree.left += [-1] * more
+        tree.right += [-1] * more
+        tree.parent += [0] * more
+        tree.feature += [0] * more
+        tree.value += [100.0] * more
+    path = str(tmp_path / "pruned.json")
+    synth.write_xgboost_json(path, trees, 12)
+    rows = batch_of(make_runner(path, 100), 2000)
+    runner = make_runner(path, rows)
+    assert "batchKernel=deep_walk " in runner.describe_plan()
+    x = rng.standard_normal((rows, 12), dtype=np.float32)
+    np.testing.assert_allclose(gpu_predict(runner, x), cpu_oracle.predict(model_io.load_xgboost_json(path), x)[0], rtol=RTOL_SUM, atol=1e-7)
+
+
+# 260 trees of 16128 tail nodes each are the most the tail array holds; 263 were the fewest that an estimate let through
+@pytest.mark.parametrize("trees,kernel", [(260, "deep_walk"), (263, "global_walk")])
+def test_as_many_tail_nodes_as_there_are_places(tmp_path, trees, kernel):
+    """The same tree over and over: the sum is so many times one tree's leaf."""
+    rng = np.random.Generator(np.random.PCG64(12))
+    one, many = str(tmp_path / "one.json"), str(tmp_path / "many.json")
+    synth.write_xgboost_json(one, [full_tree(rng, 16383, 28)], 28)
+    doc = json.load(open(one))
+    model = doc["learner"]["gradient_booster"]["model"]
+    tree = json.dumps({k: v for k, v in model["trees"][0].items()
+                       if k in ("left_children", "right_children", "split_conditions", "split_indices", "tree_param")})
+    model["gbtree_model_param"]["num_trees"], model["tree_info"], model["trees"] = str(trees), [0] * trees, ["TREES"]
+    with open(many, "w") as out:
+        out.write(json.dumps(doc).replace('"TREES"', ",".join([tree] * trees)))
+    runner = make_runner(many, 5000)
+    assert "batchKernel=%s " % kernel in runner.describe_plan(), runner.describe_plan()
+    x = rng.standard_normal((5000, 28), dtype=np.float32)
+    leaf = cpu_oracle.predict(model_io.load_xgboost_json(one), x)[0].astype(np.float64) - 0.5
+    # (one tree's prediction is rounded to 32 bits next to 0.5, half a unit in the last place 3e-8, and taken `trees` times)
+    np.testing.assert_allclose(gpu_predict(runner, x), 0.5 + trees * leaf, rtol=RTOL_SUM, atol=trees * 6e-8)
