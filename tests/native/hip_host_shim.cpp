@@ -719,12 +719,14 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
     for (int64_t row = 0; row < p.rows; ++row) {
       double sum = 0.0;
       for (int b = first; b < last; ++b) {
-        const uint32_t begin = p.bundles[b], words = kStreamBundleBytes / 4;
+        const uint32_t begin = p.bundles[b];
         if (begin % 4) std::abort();
         DeviceStreamHead heads[2];
         std::memcpy(heads, p.words + begin, sizeof(heads));
-        const uint32_t depth = heads[0].depth;
-        if (heads[1].depth != depth || p.words[begin + words - 1] == 0xFFFFFFFFu) std::abort(); // (the copy reads that far)
+        const uint32_t depth = heads[0].depth, words = heads[0].words;
+        if (heads[1].depth != depth || heads[1].words != words || words * 4 > kStreamBundleBytes) std::abort();
+        if (b + 1 < p.numBundles && p.bundles[b + 1] != begin + words) std::abort();
+        if (p.words[begin + kStreamBundleBytes / 4 - 1] == 0xFFFFFFFFu) std::abort(); // (the copy reads that far)
         for (int k = 0; k < 2 * p.chains; ++k) {
           const uint32_t root = heads[k & 1].roots[k / 2] / 4u;
           if (root % 2) std::abort(); // (children are read two words at a time)

@@ -159,7 +159,7 @@ constexpr uint32_t kFewRowsLeaf = 0xFFFFu;
 struct alignas(16) DeviceStreamHead {
   uint16_t roots[4];      // byte offsets of the half's trees in the image
   uint32_t depth;         // of the deepest tree of the bundle
-  uint32_t reserved;
+  uint32_t words;         // of the image (what reads it on the host checks against)
   uint32_t valueBegin[4]; // of every tree, in the array of predictions (entry 0 is 0.0: the empty places')
 };
 static_assert(sizeof(DeviceStreamHead) == 32, "two 16-byte LDS reads");

@@ -513,6 +513,7 @@ RankStreamModel PackRankStream(const Forest &input) {
         }
       }
       while (sm.words.size() % 4) sm.words.push_back(0u);
+      for (DeviceStreamHead &head : heads) head.words = (uint32_t)sm.words.size() - begin;
       std::memcpy(sm.words.data() + begin, heads, sizeof(heads));
       if (sm.words.size() > 0x7FFFFFF0u) throw Error("forest has too many nodes");
       sm.bundles.push_back(begin);
