@@ -63,20 +63,19 @@ def test_wide_rows_split_on_rank_tiles(synth_model):
                 close(forest, gpu_predict(runner, x[:rows]), expected[:rows])
 
 
-def test_whole_rounds_of_many_slices_are_split_too(tmp_path):
-    """352 row blocks, for which the plan takes 48 slices (any number serves the split alike): 33 whole rounds of blocks."""
+@pytest.mark.parametrize("rows,group,slices", [(90000, 38912, 48), (131072, 51712, 20)])
+def test_whole_rounds_of_many_slices_are_split_too(tmp_path, rows, group, slices):
+    """352 row blocks x 48 slices make 33 whole rounds of 512 blocks, 512 x 20 make 20."""
     rng = np.random.Generator(np.random.PCG64(12))
     trees = [synth._grow_tree(rng, 9, lambda d, s: 0.9, lambda: (rng.integers(0, 20), rng.normal()), rng.normal) for _ in range(500)]
     path = str(tmp_path / "m.json")
     synth.write_xgboost_json(path, trees, 20)
-    rows = 90000
     runner = make_runner(path, rows)
-    plan = runner.describe_plan()
-    slices = int(plan.split("treeSlices=")[1].split()[0])
-    runner.set_plan(256, 4, 4, 51712, 48)
-    pinned = runner.describe_plan()
-    assert "batchKernel=rows_lds_split" in plan, plan
-    assert "treeSlices=48" not in pinned or "batchKernel=rows_lds_split" in pinned, (slices, pinned)
+    runner.set_plan(256, 4, 4, group, slices)
+    plan = dict(item.split("=", 1) for item in runner.describe_plan().split() if "=" in item)
+    places = 256 * min(2, 163840 // (int(plan["ldsBytes"]) + 512))
+    assert int(plan["treeSlices"]) == slices and (rows + 255) // 256 * slices % places == 0, plan
+    assert plan["batchKernel"] == "rows_lds_split", plan
     x = rng.standard_normal((rows, 20), dtype=np.float32)
     got = gpu_predict(runner, x)
     forest = model_io.load_xgboost_json(path)
