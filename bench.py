@@ -204,7 +204,7 @@ def main():
         per_level = 8.0 / (lds_measured["b64"] * 1e9) + 4.0 / (lds_measured["b32"] * 1e9)
         per_leaf = 4.0 / (lds_measured["b32"] * 1e9)
         # (peeled walks stop trees early: the plan says how many levels its lock-step walk takes per row)
-        depth_sum = float(plan_fields.get("lockStepSteps") or sum(forest.depth(t) for t in range(forest.num_trees)))
+        depth_sum = float(plan_fields.get("deepLockStepSteps") or plan_fields.get("lockStepSteps") or sum(forest.depth(t) for t in range(forest.num_trees)))
         visited_ms = rows * (steps_per_row * per_level + forest.num_trees * per_leaf) * 1e3
         lockstep_ms = rows * (depth_sum * per_level + forest.num_trees * per_leaf) * 1e3
         lds_floor = {"visited_nodes_ms": visited_ms, "frac_of_visited_floor": visited_ms / walk_ms,

@@ -129,3 +129,14 @@ def test_as_many_tail_nodes_as_there_are_places(tmp_path, trees, kernel):
     leaf = cpu_oracle.predict(model_io.load_xgboost_json(one), x)[0].astype(np.float64) - 0.5
     # (one tree's prediction is rounded to 32 bits next to 0.5, half a unit in the last place 3e-8, and taken `trees` times)
     np.testing.assert_allclose(gpu_predict(runner, x), 0.5 + trees * leaf, rtol=RTOL_SUM, atol=trees * 6e-8)
+
+
+def test_plan_description_has_the_shape_of_the_deep_walk(tmp_path):
+    runner = make_runner(deep_model(tmp_path / "deep.json", 20), 60000)
+    fields = dict(item.split("=", 1) for item in runner.describe_plan().split() if "=" in item)
+    assert fields["batchKernel"] == "deep_walk" and fields["kernel"] == "global_walk"
+    assert fields["deepRowsPerBlock"] == "256" and fields["deepTreeThreads"] == "4" and fields["deepInterleave"] == "2"
+    assert int(fields["deepTreesDeferred"]) > 0 and int(fields["deepTreeSlices"]) in (1, 2)
+    assert 0 < int(fields["deepLockStepSteps"]) < 9 * 14 and 0 < int(fields["deepLdsBytes"]) <= 80 * 1024
+    runner.set_global_walk_plan(256, 4, 1)
+    assert "deepRowsPerBlock" not in runner.describe_plan()

@@ -1117,6 +1117,13 @@ std::string InferenceRunner::DescribePlan() const {
      << " batchKernel=" << KernelOfBatch() << " fewRowsLimit=" << m_fewRowsLimit
      << " treesDeferred=" << m_model.treesDeferred << " deferredEntriesPerRow=" << m_model.deferredEntriesPerRow
      << " ownClasses=" << (m_model.ownClasses ? 1 : 0);
+  if (WalksDeep()) { // the fields above are the launch plan's: what calls run in its place has a shape of its own
+    const LaunchPlan &d = m_deep.model.plan;
+    os << " deepRowsPerBlock=" << d.rowsPerBlock << " deepTreeThreads=" << d.treeThreads << " deepInterleave=" << d.interleave
+       << " deepTreeSlices=" << DeepSlices(m_options.batchSize) << " deepGroups=" << m_deep.model.groups.size()
+       << " deepLdsBytes=" << m_deep.model.LdsBytes() << " deepTreesDeferred=" << m_deep.model.treesDeferred
+       << " deepLockStepSteps=" << m_deep.model.lockStepSteps;
+  }
   return os.str();
 }
 
