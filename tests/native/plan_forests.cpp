@@ -245,6 +245,30 @@ static void TwoTreesOfClasses() {
   EXPECT(own > 0 && few > 0, "%ld, %ld", own, few);
 }
 
+// Two trees side by side leave no slice a second group where four leave it one.
+static void TwoTreesOfSlices() {
+  const DeviceLimits limits;
+  long two = 0, kept = 0;
+  for (int32_t features : {8, 26, 33, 60, 90, 130})
+    for (int32_t trees : {61, 72, 89, 161, 300})
+      for (int32_t nodes : {127, 255, 511})
+        for (int64_t batch : {4000, 7414, 12708, 16925, 30000}) {
+          const Forest forest = ForestOf(features, trees, nodes);
+          LaunchPlan plan = ChoosePlan(forest, batch, nullptr, limits);
+          if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.treeSlices == 1) continue;
+          const size_t slices = (size_t)plan.treeSlices;
+          const bool chosen = plan.interleave == 2;
+          plan.interleave = 4;
+          if (PackForest(forest, plan).groups.size() > slices) continue;
+          plan.interleave = 2;
+          const size_t groups = PackForest(forest, plan).groups.size();
+          EXPECT(!chosen || groups <= slices, "%d features, %d trees of %d nodes, %lld rows: %zu groups, %zu slices", features, trees, nodes,
+                 (long long)batch, groups, slices);
+          ++(chosen ? two : kept);
+        }
+  EXPECT(two > 0 && kept > 0, "%ld, %ld", two, kept);
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
@@ -254,6 +278,7 @@ int main(int argc, char **argv) {
   if (asked("small_peeled")) SmallPeeled();
   if (asked("small_batches")) SmallBatches();
   if (asked("two_trees_of_classes")) TwoTreesOfClasses();
+  if (asked("two_trees_of_slices")) TwoTreesOfSlices();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

@@ -54,3 +54,7 @@ def test_block_shapes_of_small_batches(driver):
 
 def test_two_trees_side_by_side_of_classifiers(driver):
     run(driver, "two_trees_of_classes")
+
+
+def test_two_trees_side_by_side_of_sliced_forests(driver):
+    run(driver, "two_trees_of_slices")

@@ -432,8 +432,12 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // rows alike.  (One tree a lane is never faster.)  Classifiers alike, but sixteen tree threads 16.9 298 and 279, 20.1 2396 and
   // 2268, 23.2 105 and 105, 25.4 133 and 138, 80 and 83: a group holds few classes at a time.
   const double fewInGroup = forest.numClasses > 0 ? std::min(24.0, 2.4 * plan.treeThreads + 3.4) : 2.4 * plan.treeThreads + 3.4;
-  if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)plan.groupBytes * (double)forest.trees.size() < fewInGroup * (double)totalBytes)
-    plan.interleave = 2;
+  // (Not where every slice has one group and, as groups end on whole rounds of the tree threads, two a lane would leave some slices a
+  // second one: 16925 rows x 72 trees, seven slices 10.8 -> 11.5 us, 12708 x 89, ten 10.8 -> 11.9, 7414 x 161, sixteen 10.4 -> 11.8.)
+  const double trees = (double)forest.trees.size(), held = totalBytes > 0 ? (double)plan.groupBytes * trees / (double)totalBytes : 1e9;
+  const double round = 2.0 * plan.treeThreads, heldInRounds = held < round ? held : std::floor(held / round) * round;
+  const bool secondGroup = slices > 1 && held * (double)slices >= trees && heldInRounds * (double)slices < trees;
+  if (!(ov && ov->treeWalkInterleaveFactor > 0) && held < fewInGroup && !secondGroup) plan.interleave = 2;
   // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
   // not fit, that way costs less (the packer's costs), and the packer will take it: where it does not, two side by side lose (607
   // trees, 13 classes, 189139 rows 235 and 247 us, 321 trees, 7 classes, 2642 rows 27.2 and 29.2).  200000 rows, four and two side by side: 100 trees of depth 7, 90
