@@ -13,9 +13,9 @@ from test_gpu_own_classes import FEATURES, class_model  # noqa: E402
 from test_gpu_parity import RTOL_SUM, make_runner  # noqa: E402
 
 
-# rows / 1024 below, at and above 256 / classes; the largest blocks (256 rows, 2048 sums); more classes than a wave has lanes
-@pytest.mark.parametrize("classes,rows", [(2, 131071), (2, 132096), (2, 262145), (5, 53000), (5, 54273), (5, 300001), (12, 22527), (12, 200003),
-                                          (16, 131073), (100, 20481)])
+# blocks of a sum per lane and of twice as many rows, either side of the line; the largest (256 rows, 2048 sums); blocks of 8 rows and more
+@pytest.mark.parametrize("classes,rows", [(2, 131071), (2, 196607), (2, 196608), (2, 262145), (5, 78847), (5, 78848), (5, 300001), (12, 32767), (12, 32768),
+                                          (12, 200003), (16, 131073), (100, 11000), (100, 20481)])
 def test_blocks_of_more_rows_than_a_sum_per_lane(tmp_path, classes, rows):
     path = class_model(tmp_path / "m.json", [t % classes for t in range(2 * classes + 1)], classes, depth=3)
     runner = make_runner(path, rows)

@@ -2145,13 +2145,16 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
 hipError_t LaunchFinalize(const FinalizeParams &p, hipStream_t stream) {
   if (p.rows <= 0) return hipSuccess;
   if (p.numClasses > 0) {
-    // A sum per lane, and 8 rows at least; more rows from 1024 such blocks on, where the chip is full and a block in which few
-    // lanes finish a row costs more than the wait of one that takes several sums a lane.  Calls with sums and softmax of 40 trees, a
-    // sum per lane, 64, 128 and 256 rows: 5 classes 65537 rows 24.7, 24.8, 25.0 and 25.3 us, 150000 34.0, 33.7, 32.3, 31.0, 700000
-    // 75.4, 74.1, 68.7, 67.1; 12 classes 25000 rows 23.8, 24.3, 25.9, 27.6, 65537 30.5, 28.6, 30.3, 31.0, 300000 67.4, 58.2, 58.5,
-    // 57.2; 16 classes 700000 rows 152.5, 120.6, 118.9 and (240 rows) 126.0.
-    const int64_t stride = p.numClasses | 1, most = std::min<int64_t>(256, kFinalizeLds / 2 / stride);
-    const int64_t perBlock = std::min<int64_t>(kFinalizeLds / stride, std::max<int64_t>({8, 256 / p.numClasses, std::min<int64_t>(most, p.rows / 1024)}));
+    // A sum per lane, and 8 rows at least; about rows / 1024 of a batch that has more than 1024 such blocks: the chip is full then,
+    // and a block in which few lanes finish a row costs more than the wait of one that takes several sums a lane.  (As many as make
+    // whole rounds of the lanes: 30 rows instead of 28 of nine classes took 31377 rows 0.8 us longer.)  Calls with sums and softmax
+    // of 40 trees, a sum per lane, 64, 128 and 256 rows: 5 classes 65537 rows 24.7, 24.8, 25.0 and 25.3 us, 150000 34.0, 33.7, 32.3,
+    // 31.0, 700000 75.4, 74.1, 68.7, 67.1; 12 classes 25000 rows 23.8, 24.3, 25.9, 27.6, 65537 30.5, 28.6, 30.3, 31.0, 300000 67.4,
+    // 58.2, 58.5, 57.2; 16 classes 700000 rows 152.5, 120.6, 118.9 and (240 rows) 126.0.
+    const int64_t stride = p.numClasses | 1, perLane = std::max(8, 256 / p.numClasses);
+    const int64_t most = std::max<int64_t>(perLane, std::min<int64_t>(256, kFinalizeLds / 2 / stride));
+    const int64_t wanted = std::max<int64_t>(1, (p.rows / 1024 + perLane / 2) / perLane) * perLane;
+    const int64_t perBlock = std::min<int64_t>(kFinalizeLds / stride, std::min(most, wanted));
     const int64_t blocks = (p.rows + perBlock - 1) / perBlock;
     const size_t sumBytes = (size_t)perBlock * (size_t)(p.numClasses | 1) * sizeof(double), rowBytes = (size_t)perBlock * 2 * sizeof(double);
     if (blocks > 0x7FFFFFFF) return hipErrorInvalidValue;
