@@ -8,9 +8,10 @@ pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
 
 from oracle import cpu_oracle, model_io  # noqa: E402
+from treebeard_amd import synth  # noqa: E402
 
 from test_gpu_own_classes import FEATURES, class_model  # noqa: E402
-from test_gpu_parity import RTOL_SUM, make_runner  # noqa: E402
+from test_gpu_parity import RTOL_SUM, check_against_oracle, make_runner  # noqa: E402
 
 
 # blocks of a sum per lane and of twice as many rows, either side of the line; the largest (256 rows, 2048 sums); blocks of 8 rows and more
@@ -34,3 +35,13 @@ def test_blocks_of_more_rows_than_a_sum_per_lane(tmp_path, classes, rows):
     wide = np.exp(wide - wide.max(axis=1, keepdims=True))
     # (the sums are rounded to 32 bits in `got`, half a unit in the last place of values below 2: 1.2e-7 in the exponent)
     np.testing.assert_allclose(probabilities.cpu().numpy(), wide / wide.sum(axis=1, keepdims=True), rtol=1e-6, atol=1e-9)
+
+
+@pytest.mark.parametrize("slices", [5, 6, 7, 8, 9])
+def test_plain_sums_of_several_slices(synth_model, slices):
+    """A lane per row, four waves that share the slices, eight."""
+    for rows in (1, 64, 2047, 65537):
+        runner = make_runner(synth_model(2), rows)
+        runner.set_plan(64, 2, 2, 8192, slices)
+        assert " treeSlices=%d " % slices in runner.describe_plan()
+        check_against_oracle(runner, model_io.load_xgboost_json(synth_model(2)), synth.CONFIGS[2].batch_rows(rows, seed_offset=3))

@@ -1506,8 +1506,10 @@ __global__ void __launch_bounds__(256) FinalizeManyClassesKernel(const FinalizeP
 // Small batches split over several tree slices: 64 rows a block, a lane each, and its waves share the slices, so that a lane
 // waits for few loads and a wave reads 512 contiguous bytes.  (A wave per sum, lanes along the slices, read a 64-byte piece of
 // memory for each of its 8 bytes: 4096 rows x 32 slices 3.0 us, 2.5 here; the call 15.1 and 13.9.)  Each wave adds its slices
-// in slice order, the waves are added in order: the order of additions depends on the number of slices alone.
-constexpr int kWideFinalizeSlices = 4;
+// in slice order, the waves are added in order: the order of additions depends on the number of slices alone.  Calls that way and
+// with a lane per row, 2000 to 66000 rows: two to five slices the same within 4 % either way (13744 rows in four 10.4 and 10.2 us,
+// 26518 17.5 and 16.8), six 2 % less (10042 rows 10.2 and 10.4), ten 6 to 8 % (6233 12.5 and 13.6), twenty 6 to 13 %.
+constexpr int kWideFinalizeSlices = 6;
 constexpr int64_t kWideFinalizeRows = 65536;
 
 template <int kWaves> // 4, or 8 from so many slices on
