@@ -396,7 +396,7 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   //    6 21.0 -> 13.4 us, 8017 x 61 7.5 -> 7.0, 20755 x 79 of depth 3 7.0 and 7.1).  Beyond, twice the blocks stage every group:
   //    that pays where the rows' walk is long for the groups there are, or where the smaller row tile saves groups.  125 forests of
   //    30 to 320 trees on 32800 to 65536 rows, levels of a walk, groups beside 256 rows and beside 128: 541 levels 1 and 1 groups
-  //    10.5 -> 9.6 us, 472 1 1 9.5 and 9.3, 340 1 1 7.9 and 8.4, 258 1 1 7.4 -> 8.1; 669 2 2 13.8 -> 12.4, 561 2 2 11.3 -> 12.0;
+  //    10.5 -> 9.6 us, 481 1 1 9.8 -> 9.3, 403 1 1 8.9 and 8.6, 340 1 1 7.9 and 8.4, 258 1 1 7.4 -> 8.1; 669 2 2 13.8 -> 12.4, 561 2 2 11.3 -> 12.0;
   //    778 3 3 15.0 and 14.6, 650 3 3 12.8 and 13.1; 700 4 4 15.5 -> 14.8; 397 2 1 9.7 -> 8.9.  Taken of them: none that loses
   //    more than 3 %, left: none that would gain more than 0.4 us;
   //  * forests of up to 24 KB, whose rows take as long to stage as to walk: 128 x 4, of which three and more to a unit take
@@ -412,8 +412,8 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     int64_t levels = 0;
     for (const Tree &tree : forest.trees) levels += tree.Depth();
     const bool fewTrees = totalBytes <= kSmallForestBytes;
-    const bool idle = rowBlocks * 2 <= limits.computeUnits ||
-                      (rowBlocks <= limits.computeUnits && (fewTrees || levels >= 424 + 69 * smallerGroups - 200 * (groups - smallerGroups)));
+    const int64_t enough = groups == 1 ? 390 : 424 + 69 * smallerGroups - 200 * (groups - smallerGroups);
+    const bool idle = rowBlocks * 2 <= limits.computeUnits || (rowBlocks <= limits.computeUnits && (fewTrees || levels >= enough));
     const bool fourFit = (int64_t)(forest.numFeatures + 1) * 128 * 4 + totalBytes + 32 <= limits.ldsBytesPerBlock / 4;
     if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits && (fourFit || rowBlocks <= 5LL * limits.computeUnits / 2))) {
       rb = plan.rowsPerBlock = 128;
