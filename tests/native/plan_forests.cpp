@@ -245,25 +245,29 @@ static void TwoTreesOfClasses() {
   EXPECT(own > 0 && few > 0, "%ld, %ld", own, few);
 }
 
-// Two trees side by side leave no slice a second group where four leave it one.
+// Two trees side by side give no slice half as many groups again as four do; the planner counts the groups that are packed.
 static void TwoTreesOfSlices() {
   const DeviceLimits limits;
   long two = 0, kept = 0;
-  for (int32_t features : {8, 26, 33, 60, 90, 130})
-    for (int32_t trees : {61, 72, 89, 161, 300})
+  for (int32_t features : {8, 26, 33, 57, 90, 130})
+    for (int32_t trees : {61, 80, 89, 161, 300})
       for (int32_t nodes : {127, 255, 511})
         for (int64_t batch : {4000, 7414, 12708, 16925, 30000}) {
-          const Forest forest = ForestOf(features, trees, nodes);
+          Forest forest = ForestOf(features, trees, nodes);
+          for (size_t t = 0; t < forest.trees.size(); t += 3) forest.trees[t] = FullTree(nodes / 4 * 2 + 1, features);
           LaunchPlan plan = ChoosePlan(forest, batch, nullptr, limits);
           if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.treeSlices == 1) continue;
-          const size_t slices = (size_t)plan.treeSlices;
           const bool chosen = plan.interleave == 2;
-          plan.interleave = 4;
-          if (PackForest(forest, plan).groups.size() > slices) continue;
-          plan.interleave = 2;
-          const size_t groups = PackForest(forest, plan).groups.size();
-          EXPECT(!chosen || groups <= slices, "%d features, %d trees of %d nodes, %lld rows: %zu groups, %zu slices", features, trees, nodes,
-                 (long long)batch, groups, slices);
+          size_t turns[2];
+          for (int32_t k : {2, 4}) {
+            plan.interleave = k;
+            const size_t groups = PackForest(forest, plan).groups.size();
+            EXPECT(groups == (size_t)CountTreeGroups(forest, plan), "%d features, %d trees of %d nodes, %lld rows: %zu and %d groups", features, trees, nodes,
+                   (long long)batch, groups, CountTreeGroups(forest, plan));
+            turns[k / 4] = (groups + (size_t)plan.treeSlices - 1) / (size_t)plan.treeSlices;
+          }
+          EXPECT(!chosen || turns[0] * 2 < turns[1] * 3, "%d features, %d trees of %d nodes, %lld rows: %zu and %zu groups a slice", features, trees, nodes,
+                 (long long)batch, turns[0], turns[1]);
           ++(chosen ? two : kept);
         }
   EXPECT(two > 0 && kept > 0, "%ld, %ld", two, kept);

@@ -578,22 +578,45 @@ namespace {
 PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile, const std::vector<int32_t> *cuts);
 bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth, const std::vector<uint32_t> &units,
                     const std::vector<int32_t> &order, std::vector<std::vector<int32_t>> *rounds);
+// Trees order[first], ..., order[first + count - 1] are a bundle of tree group `group`.
+struct BundleTrees {
+  int32_t group;
+  size_t first;
+  int32_t count;
+};
+std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &plan, const std::vector<uint32_t> &units, uint32_t tileUnits,
+                                      const std::vector<int32_t> &order);
 }
 
-bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan) {
-  std::vector<int32_t> depth(forest.trees.size()), order(forest.trees.size());
-  std::vector<uint32_t> units(forest.trees.size());
-  for (size_t t = 0; t < forest.trees.size(); ++t) {
-    depth[t] = forest.trees[t].Depth();
-    units[t] = (uint32_t)MakeLevelOrder(forest.trees[t]).order.size();
+namespace {
+// What PackForest goes by of a scalar plan without a profile: the trees' depths and sizes, in its order.
+struct PlainTrees {
+  std::vector<int32_t> depth, order;
+  std::vector<uint32_t> units;
+  explicit PlainTrees(const Forest &forest) : depth(forest.trees.size()), order(forest.trees.size()), units(forest.trees.size()) {
+    for (size_t t = 0; t < forest.trees.size(); ++t) {
+      depth[t] = forest.trees[t].Depth();
+      units[t] = (uint32_t)MakeLevelOrder(forest.trees[t]).order.size();
+    }
+    std::iota(order.begin(), order.end(), 0);
+    std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
+      const int32_t ca = forest.numClasses > 0 ? forest.trees[(size_t)a].classId : 0, cb = forest.numClasses > 0 ? forest.trees[(size_t)b].classId : 0;
+      return ca != cb ? ca < cb : depth[(size_t)a] < depth[(size_t)b];
+    });
   }
-  std::iota(order.begin(), order.end(), 0);
-  std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
-    const int32_t ca = forest.trees[(size_t)a].classId, cb = forest.trees[(size_t)b].classId;
-    return ca != cb ? ca < cb : depth[(size_t)a] < depth[(size_t)b];
-  });
+};
+} // namespace
+
+bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan) {
+  const PlainTrees trees(forest);
   std::vector<std::vector<int32_t>> rounds;
-  return OwnClassRounds(forest, plan, depth, units, order, &rounds);
+  return OwnClassRounds(forest, plan, trees.depth, trees.units, trees.order, &rounds);
+}
+
+int32_t CountTreeGroups(const Forest &forest, const LaunchPlan &plan) {
+  const PlainTrees trees(forest);
+  const std::vector<BundleTrees> bundles = LayOutGroups(forest, plan, trees.units, 1, trees.order);
+  return bundles.empty() ? 1 : bundles.back().group + 1;
 }
 
 PackedModel PackForest(const Forest &forest, const LaunchPlan &plan, const HitCountProfile *profile) {
@@ -650,6 +673,46 @@ bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vec
   // classes); with slices up to 1.01 below 0.81 of the cost, 1.10 at 0.84.
   const double share = plan.treeSlices > 1 ? 0.81 : largest <= TT * K ? 0.9 : 0.95;
   return (double)rounds->size() * bundleLevels < meeting * share;
+}
+
+// Bundles of up to K consecutive trees of one class, in groups of what fits the plan's group size.  Tree threads take bundles
+// round-robin: when more trees follow, a group ends on a multiple of treeThreads bundles so that no thread idles through a last
+// partial round.
+std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &plan, const std::vector<uint32_t> &units, uint32_t tileUnits,
+                                      const std::vector<int32_t> &order) {
+  const uint32_t groupCapacity = (uint32_t)plan.groupBytes / kNodeBytes;
+  const size_t multiple = plan.kernel == LaunchPlan::Kernel::kRowParallelLds ? (size_t)plan.treeThreads : 1;
+  std::vector<BundleTrees> out;
+  size_t next = 0;
+  for (int32_t group = 0; next < order.size(); ++group) {
+    const size_t begin = out.size();
+    uint32_t used = tileUnits; // the null leaf
+    while (next < order.size()) {
+      const int32_t cls = forest.numClasses > 0 ? forest.trees[order[next]].classId : 0;
+      int32_t count = 0;
+      while (count < plan.interleave && next + count < order.size()) {
+        const int32_t t = order[next + count];
+        const int32_t c = forest.numClasses > 0 ? forest.trees[t].classId : 0;
+        if (c != cls) break;
+        if (units[t] + 2 * tileUnits > groupCapacity)
+          throw Error("a tree of " + std::to_string(forest.trees[t].NumNodes()) + " nodes does not fit one LDS tree group");
+        if (used + units[t] > groupCapacity - 1) break; // (one spare unit keeps room for the alignment pad)
+        used += units[t];
+        ++count;
+      }
+      if (count == 0) break; // group full
+      out.push_back(BundleTrees{group, next, count});
+      next += (size_t)count;
+    }
+    if (out.size() == begin) throw Error("internal error: empty tree group");
+    const size_t bundles = out.size() - begin;
+    if (next < order.size() && multiple > 1 && bundles > multiple && bundles % multiple != 0) {
+      const size_t keep = begin + bundles - bundles % multiple;
+      next = out[keep].first;
+      out.resize(keep);
+    }
+  }
+  return out;
 }
 
 constexpr uint32_t kPeeledTailNodes = 1u << 20; // below the cuts of a plan with a profile (8 MB: they stay in the caches)
@@ -1088,43 +1151,21 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     }
   }
 
-  size_t next = pm.ownClasses ? order.size() : 0;
-  while (next < order.size()) {
+  const std::vector<BundleTrees> laidOut = pm.ownClasses ? std::vector<BundleTrees>() : LayOutGroups(forest, plan, units, tileUnits, order);
+  for (size_t at = 0; at < laidOut.size();) {
     openGroup();
     DeviceGroup &g = pm.groups.back();
-    // one spare unit keeps room for the alignment pad
-    auto freeNodes = [&]() { return groupCapacity - 1 - ((uint32_t)pm.nodes.size() - g.nodeBegin); };
-    bool any = false;
-    struct Mark { size_t nodes, slots, next, tail; };
-    std::vector<Mark> marks; // state before each bundle of this group
-    const size_t multiple = plan.kernel == LaunchPlan::Kernel::kRowParallelLds ? (size_t)plan.treeThreads : 1;
-    while (next < order.size()) {
-      // gather up to K consecutive trees of one class that still fit
+    for (const int32_t group = laidOut[at].group; at < laidOut.size() && laidOut[at].group == group; ++at) {
       DeviceBundle b{};
-      const int32_t cls = forest.numClasses > 0 ? forest.trees[order[next]].classId : 0;
-      uint32_t need = 0;
-      int count = 0;
-      while (count < K && next + count < order.size()) {
-        const int32_t t = order[next + count];
-        const int32_t c = forest.numClasses > 0 ? forest.trees[t].classId : 0;
-        if (c != cls) break;
-        if (units[t] + 2 * tileUnits > groupCapacity)
-          throw Error("a tree of " + std::to_string(forest.trees[t].NumNodes()) + " nodes does not fit one LDS tree group");
-        if (need + units[t] > freeNodes()) break;
-        need += units[t];
-        ++count;
-      }
-      if (count == 0) break; // group full
-      marks.push_back(Mark{pm.nodes.size(), pm.slotTree.size(), next, pm.tailNodes.size()});
-      b.classId = (uint16_t)cls;
+      b.classId = (uint16_t)(forest.numClasses > 0 ? forest.trees[order[laidOut[at].first]].classId : 0);
       b.firstSlot = (uint32_t)pm.slotTree.size();
       for (int k = 0; k < K; ++k) {
-        if (k >= count) {
+        if (k >= laidOut[at].count) {
           b.root[k] = 0; // null leaf
           pm.slotTree.push_back(-1);
           continue;
         }
-        const int32_t t = order[next + k];
+        const int32_t t = order[laidOut[at].first + k];
         const uint32_t base = (uint32_t)pm.nodes.size() - g.nodeBegin; // unit index inside the group
         b.root[k] = (uint16_t)(base * kNodeBytes);
         b.depth = std::max<uint32_t>(b.depth, (uint32_t)depth[t]);
@@ -1135,24 +1176,8 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
       }
       for (int k = 0; k < K; ++k) pm.bundleRoots.push_back(pm.nodes[g.nodeBegin + b.root[k] / kNodeBytes]);
       pm.bundles.push_back(b);
-      next += count;
-      any = true;
-    }
-    // Tree threads take bundles round-robin: when more trees follow, end the group on a
-    // multiple of treeThreads bundles so that no thread idles through a last partial round.
-    if (next < order.size() && multiple > 1 && marks.size() > multiple && marks.size() % multiple != 0) {
-      const size_t keep = marks.size() - marks.size() % multiple;
-      pm.nodes.resize(marks[keep].nodes);
-      pm.nodeOrigin.resize(marks[keep].nodes);
-      pm.slotTree.resize(marks[keep].slots);
-      pm.tailNodes.resize(marks[keep].tail);
-      pm.tailOrigin.resize(marks[keep].tail);
-      pm.bundles.resize(g.bundleBegin + keep);
-      pm.bundleRoots.resize((size_t)(g.bundleBegin + keep) * K);
-      next = marks[keep].next;
     }
     closeGroup();
-    if (!any) throw Error("internal error: empty tree group");
   }
   if (pm.groups.empty()) { // a forest without trees still needs one (empty) group
     openGroup();

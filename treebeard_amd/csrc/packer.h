@@ -185,6 +185,8 @@ PackedModel PackWithCuts(const Forest &forest, const LaunchPlan &plan, const std
 
 // Whether PackForest gives every class of a forest to one tree thread under a scalar row-parallel plan (PackedModel::ownClasses).
 bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan);
+// How many tree groups PackForest makes under a scalar plan, classes of the tree threads' own aside.
+int32_t CountTreeGroups(const Forest &forest, const LaunchPlan &plan);
 
 // Inverse of PackForest for tests: rebuilds (value, feature, left, right) of
 // original tree `tree` from the packed arrays.

@@ -432,12 +432,17 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // rows alike.  (One tree a lane is never faster.)  Classifiers alike, but sixteen tree threads 16.9 298 and 279, 20.1 2396 and
   // 2268, 23.2 105 and 105, 25.4 133 and 138, 80 and 83: a group holds few classes at a time.
   const double fewInGroup = forest.numClasses > 0 ? std::min(24.0, 2.4 * plan.treeThreads + 3.4) : 2.4 * plan.treeThreads + 3.4;
-  // (Not where every slice has one group and, as groups end on whole rounds of the tree threads, two a lane would leave some slices a
-  // second one: 16925 rows x 72 trees, seven slices 10.8 -> 11.5 us, 12708 x 89, ten 10.8 -> 11.9, 7414 x 161, sixteen 10.4 -> 11.8.)
-  const double trees = (double)forest.trees.size(), held = totalBytes > 0 ? (double)plan.groupBytes * trees / (double)totalBytes : 1e9;
-  const double round = 2.0 * plan.treeThreads, heldInRounds = held < round ? held : std::floor(held / round) * round;
-  const bool secondGroup = slices > 1 && held * (double)slices >= trees && heldInRounds * (double)slices < trees;
-  if (!(ov && ov->treeWalkInterleaveFactor > 0) && held < fewInGroup && !secondGroup) plan.interleave = 2;
+  // Groups end on whole rounds of the tree threads, so that bundles of two can take more of them.  Not where the slices then have half
+  // as many again to walk: one group and two 12708 rows x 89 trees in ten slices 10.8 -> 11.9 us, 16925 x 72 in seven 10.8 -> 11.5,
+  // two and three 4814 x 193 in five 10.2 -> 11.3, 15744 x 80 in four 10.6 -> 10.9; three and four 11.8 and 11.5, 14.8 and 15.0,
+  // five and six 19.8 -> 19.0, 14.9 -> 14.2, alike 13.2 -> 12.1.
+  if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)plan.groupBytes * (double)forest.trees.size() < fewInGroup * (double)totalBytes) {
+    LaunchPlan two = plan;
+    two.interleave = 2;
+    two.treeSlices = (int32_t)std::max<int64_t>(1, slices);
+    const auto turns = [&](const LaunchPlan &p) { return (CountTreeGroups(forest, p) + slices - 1) / slices; };
+    if (slices == 1 || PacksOwnClasses(forest, two) || turns(two) * 2 < turns(plan) * 3) plan.interleave = 2;
+  }
   // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
   // not fit, that way costs less (the packer's costs), and the packer will take it: where it does not, two side by side lose (607
   // trees, 13 classes, 189139 rows 235 and 247 us, 321 trees, 7 classes, 2642 rows 27.2 and 29.2).  200000 rows, four and two side by side: 100 trees of depth 7, 90
