@@ -1628,9 +1628,9 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
 // bundle's roots and depth stand in its image, its place comes through a vector load (a scalar load took its latency every
 // bundle); and a workgroup stays, with the next rows' ranks on their way to registers while its last bundle is walked (it
 // has its compute unit's LDS to itself: nothing else walks while it loads).  Walk of 262144 rows x 2000 features, 1000 trees
-// of depth 8, on the same ranks: 1.33 ms with tree groups, 0.84 with two trips a level and a workgroup per 32 rows, 0.76
-// here, and the whole call 1.308 -> 1.223; 20000 rows 126 -> 120 us.  A level takes 0.067 ms (a wave's eight LDS reads and 20
-// VALU instructions in 34 cycles of its compute unit: LDS pipes 70 %, VALUs 60 % busy), the leaf values 0.065, the rest 0.16.
+// of depth 8, on the same ranks, traced: 1.33 ms with tree groups, 0.80 with two trips a level and a workgroup per 32 rows, 0.73
+// here (LDS pipes 52 % busy, a quarter of that conflicts of the rank reads, VALUs 58 %), and the whole call 1.308 -> 1.223; 20000
+// rows 126 -> 120 us.
 // ---------------------------------------------------------------------------
 // kStays: workgroups go on with other rows.  Where none does, what that takes (76 VGPRs and 1700 bytes of code) is left out: 3644
 // rows x 167 trees of 896 features 16.8 -> 16.2 us, 5504 x 92 of 1401 21.7 -> 21.2, 7713 x 46 of 672 15.2 -> 14.5.

@@ -362,7 +362,7 @@ int32_t InferenceRunner::SplitBlocks(int64_t rows) const {
                                                                m_limits.ldsBytesPerBlock / (int64_t)(m_model.LdsBytes() + 512)));
   const int64_t places = perCu * m_limits.computeUnits; // blocks that run at once
   // (Whole rounds of blocks are no reason to keep the slices, which the plan may have chosen because the split serves them all
-  // alike: 90000 rows x 700 trees of 28 features 196 us in 33 rounds of 48 slices, 129 split; 45000 rows of six classes 95 and 55.)
+  // alike: 90000 rows x 700 trees of 20 features 196 us in 33 rounds of 48 slices, 129 split; 45000 rows of six classes 95 and 55.)
   if (blocks <= places) return 0;
   WalkShape shape;
   shape.rowBlocks = RowBlocks(rows);
