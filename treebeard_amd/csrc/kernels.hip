@@ -1413,12 +1413,12 @@ __global__ void __launch_bounds__(256) FinalizeKernel(const FinalizeParams p) {
 // Classifiers: the block's rows x classes are read as they lie (coalesced; a lane per row read a line per class and all
 // of them three times: 13 us for 65537 rows x 8 classes x 2 slices), meet in LDS, and the rows are finished there.  A sum per
 // lane (more in large batches): blocks of 128 rows, whose lanes wait for memory four times in a row, took 65537 rows x 8 classes
-// 4.7 us longer with sums and softmax.  With sixteen parts and more to add, two groups of 256 lanes take every second of them:
+// 4.7 us longer with sums and softmax.  With twelve parts and more to add, two groups of 256 lanes take every second of them:
 // class ids of 900 trees, 1400 rows x 5 classes in 40 parts 18.2 us with one group and 16.9 with two, 1800 x 8 in 23 15.0 and
-// 14.6, 4000 x 3 in 16 14.5 and 14.2; but 6000 x 3 in ten 15.0 and 15.6, 25000 x 9 in ten 41.5 and 43.9, 45000 x 6 in four 48.1
+// 14.6, 4380 x 8 in twelve 16.0 and 15.6; but 6000 x 3 in ten 15.0 and 15.6, 25000 x 9 in ten 41.5 and 43.9, 45000 x 6 in four 48.1
 // and 50.1, 80000 x 13 in up to five 94.6 and 99.9.
 constexpr int kFinalizeLds = 4096; // doubles of sums a block holds
-constexpr int kClassPartsShared = 16;
+constexpr int kClassPartsShared = 12;
 
 __global__ void __launch_bounds__(1024) FinalizeClassesKernel(const FinalizeParams p, int rowsPerBlock) {
   extern __shared__ __align__(16) unsigned char lds[];
