@@ -203,9 +203,9 @@ static void SmallBatches() {
   const struct { int64_t batch; int32_t trees, nodes, features, rows, threads; } shapes[] = {
       {32768, 30, 255, 20, 128, 8},  {32769, 30, 255, 20, 256, 4},                                // half of the units have a block, and more
       {40000, 77, 63, 20, 256, 4},   {40000, 78, 63, 20, 128, 8},                                 // 385 and 390 levels, one group
-      {40000, 93, 127, 20, 256, 4},  {40000, 94, 127, 20, 128, 8},                                // 558 and 564, two groups
-      {40000, 48, 127, 50, 256, 4},  {40000, 49, 127, 50, 128, 8},                                // 288 and 294, two groups beside 256 rows and one beside 128
-      {65536, 99, 255, 20, 256, 4},  {65536, 100, 255, 20, 128, 8}, {65537, 100, 255, 20, 256, 4}, // 693 and 700, four groups
+      {40000, 107, 127, 20, 256, 4}, {40000, 108, 127, 20, 128, 8},                               // 642 and 648, two groups
+      {40000, 73, 63, 50, 256, 4},   {40000, 74, 63, 50, 128, 8},                                 // 365 and 370, two groups beside 256 rows and one beside 128
+      {65536, 100, 255, 20, 128, 8}, {65537, 100, 255, 20, 256, 4},                               // four groups
       {131072, 59, 31, 50, 256, 4},  {131073, 59, 31, 50, 128, 4},                                // a round of blocks of 256 rows, and more
       {300000, 59, 31, 50, 128, 4},  {300000, 60, 31, 50, 256, 4},                                // four fit a unit's LDS, and three
       {163840, 60, 31, 50, 128, 4},  {163841, 60, 31, 50, 256, 4}};                               // three, of a round and a quarter

@@ -33,7 +33,7 @@ def test_interleave_follows_the_trees_a_group_holds(tmp_path, features, depth, e
     (30000, 40, 4, 20, (128, 4)), (65536, 40, 4, 20, (128, 4)),        # few trees as well
     (131072, 40, 4, 20, (256, 4)), (131073, 40, 4, 20, (128, 4)),      # few trees, at most and more than a round of blocks
     (131073, 90, 5, 20, (256, 4)),                                     # more than 24 KB
-    (40000, 48, 6, 50, (256, 4)), (40000, 49, 6, 50, (128, 8)),        # levels for two groups beside 256 rows and one beside 128
+    (40000, 73, 5, 50, (256, 4)), (40000, 74, 5, 50, (128, 8)),        # levels for two groups beside 256 rows and one beside 128
     (163840, 60, 4, 50, (128, 4)), (163841, 60, 4, 50, (256, 4)),      # three blocks to a unit: a round and a quarter, and more
     (300000, 59, 4, 50, (128, 4))])                                    # four
 def test_block_shapes_of_small_forests_and_batches(tmp_path, rows, trees, depth, features, shape):

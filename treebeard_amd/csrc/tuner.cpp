@@ -396,9 +396,9 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   //    6 21.0 -> 13.4 us, 8017 x 61 7.5 -> 7.0, 20755 x 79 of depth 3 7.0 and 7.1).  Beyond, twice the blocks stage every group:
   //    that pays where the rows' walk is long for the groups there are, or where the smaller row tile saves groups.  125 forests of
   //    30 to 320 trees on 32800 to 65536 rows, levels of a walk, groups beside 256 rows and beside 128: 541 levels 1 and 1 groups
-  //    10.5 -> 9.6 us, 481 1 1 9.8 -> 9.3, 403 1 1 8.9 and 8.6, 340 1 1 7.9 and 8.4, 258 1 1 7.4 -> 8.1; 669 2 2 13.8 -> 12.4, 561 2 2 11.3 -> 12.0;
-  //    778 3 3 15.0 and 14.6, 650 3 3 12.8 and 13.1; 700 4 4 15.5 -> 14.8; 397 2 1 9.7 -> 8.9.  Taken of them: none that loses
-  //    more than 3 %, left: none that would gain more than 0.4 us;
+  //    10.5 -> 9.6 us, 481 1 1 9.8 -> 9.3, 403 1 1 8.9 and 8.6, 340 1 1 7.9 and 8.4, 258 1 1 7.4 -> 8.1; 700 2 2 12.6 -> 12.1, 572 2 2
+  //    12.4 and 12.8, 561 2 2 11.3 -> 12.0; 632 3 3 (of 33 features) 14.4 -> 13.5, 650 3 3 (of 6) 12.8 and 13.1; 700 4 4 15.5 ->
+  //    14.8; 397 2 1 9.7 -> 8.9.  Taken of them: none that loses, left: none that would gain more than 0.4 us;
   //  * forests of up to 24 KB, whose rows take as long to stage as to walk: 128 x 4, of which three and more to a unit take
   //    turns.  2^20 rows x 60 trees of depth 5 69.6 -> 58.0 us, 210411 x 62 19.6 -> 17.2, 402162 x 51 of depth 4 30.0 -> 26.0
   //    (29 KB: 37.7 and 38.5).  Four to a unit, that is: of 89 forests of 2 to 24 KB on 131100 to 2^20 rows they win by 0 to 16 %
@@ -412,7 +412,7 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     int64_t levels = 0;
     for (const Tree &tree : forest.trees) levels += tree.Depth();
     const bool fewTrees = totalBytes <= kSmallForestBytes;
-    const int64_t enough = groups == 1 ? 390 : 424 + 69 * smallerGroups - 200 * (groups - smallerGroups);
+    const int64_t enough = groups == 1 ? 390 : 670 - forest.numFeatures * 6 / 5 - 240 * (groups - smallerGroups);
     const bool idle = rowBlocks * 2 <= limits.computeUnits || (rowBlocks <= limits.computeUnits && (fewTrees || levels >= enough));
     const bool fourFit = (int64_t)(forest.numFeatures + 1) * 128 * 4 + totalBytes + 32 <= limits.ldsBytesPerBlock / 4;
     if (idle || (fewTrees && rowBlocks > 2LL * limits.computeUnits && (fourFit || rowBlocks <= 5LL * limits.computeUnits / 2))) {
@@ -441,7 +441,7 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     two.interleave = 2;
     two.treeSlices = (int32_t)std::max<int64_t>(1, slices);
     const auto turns = [&](const LaunchPlan &p) { return (CountTreeGroups(forest, p) + slices - 1) / slices; };
-    if (slices == 1 || PacksOwnClasses(forest, two) || turns(two) * 2 < turns(plan) * 3) plan.interleave = 2;
+    if (slices == 1 || (forest.numClasses > 1 && PacksOwnClasses(forest, two)) || turns(two) * 2 < turns(plan) * 3) plan.interleave = 2;
   }
   // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
   // not fit, that way costs less (the packer's costs), and the packer will take it: where it does not, two side by side lose (607
