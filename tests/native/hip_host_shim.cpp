@@ -232,7 +232,7 @@ hipError_t Launched(hipEvent_t done, hipStream_t stream) { return done ? hipEven
 // rankRows: 0 f32 rows, 1 one-byte ranks, 2 two-byte ranks ([row block][feature pair][row][2], `stride` = bytes of
 // one feature pair's column = rows per block x 4)
 void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64_t row, int gBegin, int gEnd, double *classSums,
-                bool *classSeen) {
+                bool *classSeen, bool leavesOutside) {
   const DeviceNode *nodes = reinterpret_cast<const DeviceNode *>(p.nodes16);
   const int F = p.s.numFeatures;
   for (int g = gBegin; g < gEnd; ++g) {
@@ -244,7 +244,7 @@ void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64
         for (uint32_t d = 0; d < bd.depth; ++d) {
           if (addr % kNodeBytes != 0 || addr / kNodeBytes >= grp.nodeCount) std::abort(); // pointer outside the group
           const DeviceNode node = nodes[grp.nodeBegin + addr / kNodeBytes];
-          const uint32_t offset = node.meta & 0xFFFFu;
+          const uint32_t offset = MetaFeature(node.meta);
           const uint32_t f = rankRows == 2 ? offset / stride * 2u + ((offset >> 1) & 1u) : offset / stride;
           if ((rankRows == 2 ? (offset % stride) & ~2u : offset % stride) != 0 || (int)f > F) std::abort(); // offset outside the row tile
           bool left;
@@ -261,9 +261,11 @@ void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64
             const float x = (int)f >= F ? -INFINITY : p.x[row * F + f]; // (the pad feature and the stub feature hold -inf)
             left = x < node.value;
           }
-          addr = (node.meta >> 16) + (left ? 0u : kNodeBytes);
+          addr = MetaChild(node.meta) + (left ? 0u : leavesOutside && d + 1 == bd.depth ? 4u : kNodeBytes); // (the last level: leaves of 4 bytes)
         }
-        if (addr / kNodeBytes >= grp.nodeCount) std::abort();
+        if (addr % 4 != 0 || (addr < grp.nodeCount * kNodeBytes ? addr % kNodeBytes != 0 : !leavesOutside || addr / kNodeBytes >= grp.imageCount)) std::abort();
+        float leafValue; // (of the group's image, in LDS or not)
+        std::memcpy(&leafValue, reinterpret_cast<const char *>(nodes + grp.nodeBegin) + addr, sizeof(leafValue));
         bool inTail = false;
         uint32_t at = 0;
         if (p.s.deferTails) {
@@ -272,7 +274,7 @@ void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64
           const DeviceNode stop = nodes[grp.nodeBegin + addr / kNodeBytes];
           if (rankRows != 0 || stride == 0) std::abort();
           if (stop.value != stop.value) { // a NaN marks a stub; its payload is the tail index
-            if (!bd.hasStubs || (stop.meta >> 16) + kNodeBytes != addr || (Bits(stop.value) & ~kStubIndexMask) != kStubValueBits ||
+            if (!bd.hasStubs || MetaChild(stop.meta) + kNodeBytes != addr || (Bits(stop.value) & ~kStubIndexMask) != kStubValueBits ||
                 !p.tailNodes || (p.leafIds && !p.tailOrigin))
               std::abort();
             inTail = true;
@@ -300,15 +302,15 @@ void WalkRowLds(const WalkParams &p, int K, uint32_t stride, int rankRows, int64
         }
         const int cls = p.s.numClasses > 0 ? (int)bd.classId : 0;
         if (p.s.numClasses > 0 && cls >= p.s.numClasses) { // a tree thread without a class: bundles without trees, no sum
-          if (!p.s.ownClasses || cls >= p.s.treeThreads || nodes[grp.nodeBegin + addr / kNodeBytes].value != 0.0f) std::abort();
+          if (!p.s.ownClasses || cls >= p.s.treeThreads || leafValue != 0.0f) std::abort();
           if (p.leafIds && p.slotTree[bd.firstSlot + k] >= 0) std::abort();
           continue;
         }
-        classSums[cls] += (double)nodes[grp.nodeBegin + addr / kNodeBytes].value;
+        classSums[cls] += (double)leafValue;
         classSeen[cls] = true;
         if (p.leafIds) {
           const int tree = p.slotTree[bd.firstSlot + k];
-          if (tree >= 0) p.leafIds[row * p.s.numTrees + tree] = p.nodeOrigin[grp.nodeBegin + addr / kNodeBytes];
+          if (tree >= 0) p.leafIds[row * p.s.numTrees + tree] = p.nodeOrigin[grp.nodeBegin * 2 + addr / 4];
         }
       }
     }
@@ -344,7 +346,8 @@ void ClearPartial(const WalkParams &p, int64_t slots) {
   if (p.partial) std::fill_n(p.partial, slots * p.s.rows * std::max(1, p.s.numClasses), std::nan(""));
 }
 
-hipError_t WalkLds(const WalkParams &p, int K, uint32_t stride, int rankRows, hipStream_t stream) {
+// leavesOutside: the last level of a bundle's walk is leaves of 4 bytes, not in LDS
+hipError_t WalkLds(const WalkParams &p, int K, uint32_t stride, int rankRows, bool leavesOutside, hipStream_t stream) {
   if (K != 1 && K != 2 && K != 4 && K != 8) return hipErrorInvalidValue;
   if (p.s.treeSlices > 1 && !p.partial) std::abort(); // slices meet in the partial-sum buffer
   const int Cn = p.s.numClasses > 0 ? p.s.numClasses : 1;
@@ -353,7 +356,7 @@ hipError_t WalkLds(const WalkParams &p, int K, uint32_t stride, int rankRows, hi
   const auto walk = [&](int64_t firstRow, int64_t lastRow, int gBegin, int gEnd, int slot) {
     for (int64_t row = firstRow; row < lastRow; ++row) {
       std::fill(sums.begin(), sums.end(), 0.0);
-      WalkRowLds(p, K, stride, rankRows, row, gBegin, gEnd, sums.data(), reinterpret_cast<bool *>(seen.data()));
+      WalkRowLds(p, K, stride, rankRows, row, gBegin, gEnd, sums.data(), reinterpret_cast<bool *>(seen.data()), leavesOutside);
       StoreRow(p, row, slot, sums.data());
     }
   };
@@ -396,7 +399,7 @@ hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, 
   if (tileMode < 0 || tileMode > 3 || (tileMode == 3 && p.splitBlocks)) return hipErrorInvalidValue;
   if (tileMode == 3 && (int64_t)((p.s.numFeatures + 2) / 2) * RB * 4 > 0x10000) return hipErrorInvalidValue;
   const uint32_t stride = tileMode == 0 || tileMode == 3 ? (uint32_t)RB * 4u : tileMode == 1 ? (uint32_t)RB : (uint32_t)RB / 4u;
-  return WalkLds(p, interleave, stride, tileMode == 3 ? 2 : tileMode == 2 ? 1 : 0, stream);
+  return WalkLds(p, interleave, stride, tileMode == 3 ? 2 : tileMode == 2 ? 1 : 0, p.s.leavesOutside != 0, stream);
 }
 
 namespace {
@@ -495,7 +498,7 @@ hipError_t LaunchWalkRowsTiled(const WalkParams &p, int tileSize, int interleave
             sums[p.s.numClasses > 0 ? bd.classId : 0] += (double)value;
             if (p.leafIds) {
               const int tree = p.slotTree[bd.firstSlot + k];
-              if (tree >= 0) p.leafIds[row * p.s.numTrees + tree] = p.nodeOrigin[grp.nodeBegin + addr / kNodeBytes];
+              if (tree >= 0) p.leafIds[row * p.s.numTrees + tree] = p.nodeOrigin[grp.nodeBegin * 2 + addr / 4];
             }
           }
         }
@@ -514,7 +517,7 @@ hipError_t LaunchWalkTreeParallel(const WalkParams &p, int interleave, size_t ld
   if (threads > 1024 || threads % 64 != 0) return hipErrorInvalidValue;
   if (p.s.treeSlices < 1 || p.s.treeSlices > 65535) return hipErrorInvalidValue;
   if ((int)((p.s.groupRegionBytes / 16 + threads - 1) / threads) > 16) return hipErrorInvalidValue;
-  return WalkLds(p, interleave, 4u, 0, stream);
+  return WalkLds(p, interleave, 4u, 0, false, stream);
 }
 
 hipError_t LaunchWalkGlobal(const WalkParams &p, int interleave, hipStream_t stream) {

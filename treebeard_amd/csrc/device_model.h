@@ -19,6 +19,10 @@
 //    whose column holds -inf: `x < value` is then always true, the walk takes
 //    the "left" pointer and stays on the leaf.  A walk of `depth` steps thus
 //    needs no leaf test: it ends on the leaf for every row.
+//  * Leaves outside (PackedModel::leavesOutside): a walk's last step needs no node of the level it leads to, only which leaf it
+//    is.  The leaves on the last level of a bundle's walk can therefore stay in global memory: behind the nodes that are copied
+//    into LDS the group's image holds their values, 4 bytes each, siblings side by side (the last step adds 4 bytes for the right
+//    one), and the walk ends with one read of the image at the address it arrived at, wherever that leaf stands.
 //  * Deferred tails (LaunchPlan::deferTails; the reference's peeled walks for skewed trees,
 //    src/mlir/ProbabilityBasedTilingTransform.cpp:66-73, src/mlir/WalkDecisionTreeLoweringPass.cpp:231-315): the
 //    lock-step walk of a tree may stop at a level above its leaves.  The internal nodes of that level are then
@@ -96,6 +100,9 @@ struct DeviceNode {
   float value;
   uint32_t meta;
 };
+constexpr uint32_t NodeMeta(uint32_t child, uint32_t featureOffset) { return child << 16 | featureOffset; }
+constexpr uint32_t MetaChild(uint32_t meta) { return meta >> 16; }
+constexpr uint32_t MetaFeature(uint32_t meta) { return meta & 0xFFFFu; }
 
 struct alignas(32) DeviceBundle {
   uint16_t root[kMaxInterleave]; // byte address of each tree's root inside the group
@@ -175,7 +182,8 @@ struct DeviceGroup {
   uint32_t bundleBegin;
   uint32_t bundleCount;
   uint32_t uniformClass; // class id + 1 when every bundle of the group votes for one class, else 0
-  uint32_t reserved[3];
+  uint32_t imageCount;   // 8-byte units of the group's image: nodeCount of them in LDS, behind them the leaves that are not, 4 bytes each
+  uint32_t reserved[2];
 };
 static_assert(sizeof(DeviceGroup) == 32, "group descriptors are fetched with one 32-byte scalar load");
 

@@ -28,6 +28,8 @@ struct WalkScalars {
   // Row-parallel scalar walk of a classifier: bundle i of a group is tree thread i % treeThreads', and class c's trees are all
   // tree thread c % treeThreads' (PackedModel::ownClasses).
   int32_t ownClasses = 0;
+  // Scalar row-parallel walk: the leaves of a bundle's last level are not in LDS (PackedModel::leavesOutside).
+  int32_t leavesOutside = 0;
   // Scalar row-parallel walk on an f32 tile with byte offsets: trees may end in stubs (device_model.h); the row
   // tile then has a column for the stub feature and every wave a queue of deferred walks behind it.
   int32_t deferTails = 0;

@@ -166,7 +166,10 @@ __device__ __forceinline__ void StageRows(const float *__restrict__ src, int val
 // barriers of its round while the compute unit's other blocks walk (PF == 0).
 // A lane walks K trees at a time in lock step: all lanes take `depth` steps and
 // leaves hold the walk in place (see device_model.h), so the loop body has no
-// leaf test and no divergence.  `treeThreads` lanes (in different waves) share
+// leaf test and no divergence.  Where leaves stay out of the groups (kWalkOutside) their values are gathered from L2,
+// asked for when a bundle ends and added when the next one does: 16 address cycles per wave and tree on a path the walk
+// leaves idle, for two cycles of the LDS pipe and 15 to 50 % of a group's room (2^20 rows x 28 features, 1000 trees of
+// depth 8 1162 -> 1069 us: LDS pipes 83 -> 79 % busy, conflicts 0.30 -> 0.16 cycles a read).  `treeThreads` lanes (in different waves) share
 // one row and split each group's bundles between them, which buys occupancy
 // without growing the row tile; their sums meet in an LDS cross-wave pass.
 // Sums are kept in double; trees are added in packed order.
@@ -186,11 +189,14 @@ __device__ __forceinline__ void StageRows(const float *__restrict__ src, int val
 // is merely present): kWalkDump the leaf-id dump of the parity checks, kWalkDefer the deferred tails, kWalkFuse
 // the classifiers' running arg-max (WalkScalars::fuseArgmax), kWalkOwn and kWalkOwnFuse classes of the tree threads' own
 // (WalkScalars::ownClasses; as a run-time branch of the plain walk it cost 1000 trees without classes 40 %: SGPRs).
-enum WalkVariant : int { kWalkPlain = 0, kWalkDump = 1, kWalkDefer = 2, kWalkFuse = 3, kWalkOwn = 4, kWalkOwnFuse = 5 };
+// kWalkOutside is added to those (not to the dump, which looks where the leaves are, nor to deferred tails) where the leaves of a
+// bundle's last level stay in global memory (PackedModel::leavesOutside): the walk's last step leads to their place, their values
+// are asked for there and added a bundle later.  (As a run-time branch it cost 1000 trees on 2^20 rows 2 %.)
+enum WalkVariant : int { kWalkPlain = 0, kWalkDump = 1, kWalkDefer = 2, kWalkFuse = 3, kWalkOwn = 4, kWalkOwnFuse = 5, kWalkOutside = 8 };
 
 // Groups [gBegin, gEnd) of one row block: everything a block of the row-parallel walk does.  `slice` names the slot of
 // the partial sums this part fills.
-template <int K, int PF, int kMode, int kVariant>
+template <int K, int PF, int kMode, int kVariantBits>
 __device__ __forceinline__ void
 WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int slice,
              const float *__restrict__ x, const uint4 *__restrict__ nodes16,
@@ -199,7 +205,8 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
              const WalkScalars &s, float *__restrict__ out, int8_t *__restrict__ classOut,
              double *__restrict__ partial, int32_t *__restrict__ leafIds, const int32_t *__restrict__ nodeOrigin,
              const int32_t *__restrict__ slotTree, const U32x2 *__restrict__ tailNodes, const int32_t *__restrict__ tailOrigin) {
-  constexpr bool kDump = kVariant == kWalkDump, kDefer = kVariant == kWalkDefer;
+  constexpr int kVariant = kVariantBits & ~kWalkOutside;
+  constexpr bool kDump = kVariant == kWalkDump, kDefer = kVariant == kWalkDefer, kOutside = (kVariantBits & kWalkOutside) != 0;
   constexpr bool kFuse = kVariant == kWalkFuse || kVariant == kWalkOwnFuse;
   const bool own = kVariant == kWalkOwn || kVariant == kWalkOwnFuse || (kDump && s.ownClasses);
   // LDS: [tree group nodes | transposed row tile].  The group sits at LDS
@@ -290,6 +297,16 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
             : lds);
 
   double acc = 0.0;
+  float leaf[K]; // kOutside: the last bundle's leaf values, on their way
+#pragma unroll
+  for (int k = 0; k < K; ++k) leaf[k] = 0.0f;
+#define TBAMD_ADD_LEAVES                                                                                               \
+  if (kOutside) {                                                                                                      \
+    _Pragma("unroll") for (int k = 0; k < K; ++k) {                                                                    \
+      acc += (double)leaf[k];                                                                                          \
+      leaf[k] = 0.0f;                                                                                                  \
+    }                                                                                                                  \
+  }
   int curClass = own ? tt : 0;
   float best = -INFINITY; // fuseArgmax: running maximum of the class sums and its class (tree thread 0)
   int bestClass = 0;
@@ -396,7 +413,12 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
 
   for (int g = gBegin; g < gEnd; ++g) {
     const DeviceGroup grp = groups[g];
-    if (PF > 0 || g > gBegin) __syncthreads(); // rows staged / previous group no longer read
+    if (PF > 0 || g > gBegin) { // rows staged / previous group no longer read
+      // (leaf values may still be on their way: only LDS accesses are waited for)
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
     if (PF > 0) {
       U32x4 *dst = reinterpret_cast<U32x4 *>(lds);
       const int pieces = (int)(grp.nodeCount >> 1);
@@ -407,7 +429,8 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
       }
     } else {
       if (g > gBegin) TBAMD_COPY_GROUP(grp)
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0x0F70);
+      asm volatile("" ::: "memory");
     }
     __syncthreads();
     if (PF > 0 && g + 1 < gEnd) TBAMD_PREFETCH_GROUP(groups[g + 1]) // in flight while this group is walked
@@ -423,6 +446,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
         // most groups vote for one class: the descriptor says so and no bundle has to be looked at
         const int cls = grp.uniformClass ? (int)grp.uniformClass - 1 : (int)bundles[grp.bundleBegin + b0].classId;
         if (cls != curClass) { // classes arrive in ascending order
+          TBAMD_ADD_LEAVES
           TBAMD_FLUSH_CLASS(cls)
           curClass = cls;
         }
@@ -434,6 +458,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
       for (uint32_t b = b0 + tt; b < b1; b += TT) {
         const DeviceBundle bd = bundles[grp.bundleBegin + b];
         if (own && (int)bd.classId != curClass) {
+          TBAMD_ADD_LEAVES
           TBAMD_FLUSH_OWN_CLASS((int)bd.classId)
           curClass = (int)bd.classId;
         }
@@ -444,30 +469,36 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
         // Level 0 of the f32 tiles: copies of the root nodes sit next to the bundles and arrive in scalar
         // registers, only the feature is read from LDS.  A root that is a leaf holds the walk in place like any other leaf, so the step is safe
         // for depth 0.  (On rank tiles, whose rounds are latency-bound, the extra scalar load did not pay.)
+        // (the last level's leaves stand 4 bytes apart)
+        const uint32_t lastRight = kOutside || (kDump && s.leavesOutside) ? 4u : kNodeBytes;
+        const uint32_t rootRight = (kOutside || kDump) && depth == 1 ? lastRight : kNodeBytes;
         if (kMode != kTileRankU8) {
           const DeviceNode *roots = bundleRoots + (size_t)(grp.bundleBegin + b) * K;
 #pragma unroll
           for (int k = 0; k < K; ++k) {
             const DeviceNode root = roots[k];
-            const uint32_t off = kMode == kTileF32Words ? (root.meta & 0xFFFFu) << 2 : (root.meta & 0xFFFFu);
+            const uint32_t off = kMode == kTileF32Words ? MetaFeature(root.meta) << 2 : MetaFeature(root.meta);
             bool left;
             if (kMode == kTileRankU16) left = RankGoesLeft<kMode>(column + off, __float_as_uint(root.value));
             else left = LdsLoadFloat(column + off) < root.value;
-            addr[k] = (root.meta >> 16) + (left ? 0u : kNodeBytes);
+            addr[k] = MetaChild(root.meta) + (left ? 0u : rootRight);
           }
         }
-#pragma unroll 2
-        for (int d = kMode != kTileRankU8 ? 1 : 0; d < depth; ++d) {
+        const auto step = [&](uint32_t right) {
 #pragma unroll
           for (int k = 0; k < K; ++k) {
             const U32x2 node = LdsLoadNode(addr[k]);
-            const uint32_t off = kMode == kTileF32Bytes || kMode == kTileRankU16 ? (node.y & 0xFFFFu) : (node.y & 0xFFFFu) << 2;
+            const uint32_t off = kMode == kTileF32Bytes || kMode == kTileRankU16 ? MetaFeature(node.y) : MetaFeature(node.y) << 2;
             bool left;
             if (IsRankTile(kMode)) left = RankGoesLeft<kMode>(column + off, node.x); // rank <= threshold index
             else left = LdsLoadFloat(column + off) < AsFloat(node.x);
-            addr[k] = (node.y >> 16) + (left ? 0u : kNodeBytes);
+            addr[k] = MetaChild(node.y) + (left ? 0u : right);
           }
-        }
+        };
+        constexpr int kFirstLevel = kMode != kTileRankU8 ? 1 : 0;
+#pragma unroll 2
+        for (int d = kFirstLevel; d < depth - (kOutside || kDump ? 1 : 0); ++d) step(kNodeBytes);
+        if ((kOutside || kDump) && depth > kFirstLevel) step(lastRight);
         if (kDefer && bd.hasStubs) {
           // rows on a stub are queued, the others add their leaf; the queue is walked on as soon as it holds a wave's worth
           float value[K];
@@ -507,8 +538,14 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
               }
             }
           }
+          const char *image = reinterpret_cast<const char *>(nodes16) + (size_t)grp.nodeBegin * kNodeBytes;
+          TBAMD_ADD_LEAVES
 #pragma unroll
-          for (int k = 0; k < K; ++k) acc += (double)LdsLoadFloat(addr[k]);
+          for (int k = 0; k < K; ++k) {
+            if (kOutside) leaf[k] = *reinterpret_cast<const float *>(image + addr[k]);
+            else if (kDump) acc += (double)*reinterpret_cast<const float *>(image + addr[k]);
+            else acc += (double)LdsLoadFloat(addr[k]);
+          }
         }
         if (kDump) {
           if (lane < valid) {
@@ -516,7 +553,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
             for (int k = 0; k < K; ++k) {
               const int tree = slotTree[bd.firstSlot + k];
               if (tree >= 0 && !(s.deferTails && addr[k] == 0u))
-                leafIds[row * s.numTrees + tree] = nodeOrigin[grp.nodeBegin + addr[k] / kNodeBytes];
+                leafIds[row * s.numTrees + tree] = nodeOrigin[grp.nodeBegin * 2u + addr[k] / 4u];
             }
           }
         }
@@ -528,6 +565,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
   if (kDefer) // what is still queued is walked on now
     while (queued > 0u) TBAMD_WALK_QUEUE
 
+  TBAMD_ADD_LEAVES
   if (own) {
     TBAMD_FLUSH_OWN_CLASS(C)
     if (!kFuse) return;
@@ -573,6 +611,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
     out[row] = (float)(s.transform == 1 ? 1.0 / (1.0 + exp(-margin)) : margin);
   }
 #undef TBAMD_COPY_GROUP
+#undef TBAMD_ADD_LEAVES
 #undef TBAMD_FLUSH_CLASS
 #undef TBAMD_FLUSH_OWN_CLASS
 #undef TBAMD_PREFETCH_GROUP
@@ -604,7 +643,7 @@ WalkRowsLdsKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes16
 // write-through stores, the ticket and the reads are three round trips to memory, 5 to 12 us where the finalize launch
 // takes 4.)
 // ---------------------------------------------------------------------------
-template <int K, int kMode, int kVariant> // kWalkPlain or kWalkOwn
+template <int K, int kMode, int kVariant> // kWalkPlain or kWalkOwn, their leaves in LDS or not
 // (80 SGPRs: with the 16 the trap handler takes, 8 waves per SIMD - two blocks of 16 waves - leave each wave 100; at 88 one
 // block per CU ran, 40 % slower)
 __global__ void __launch_bounds__(1024) __attribute__((amdgpu_num_sgpr(80)))
@@ -835,7 +874,7 @@ WalkRowsTiledKernel(const float *__restrict__ x, const uint4 *__restrict__ nodes
 #pragma unroll
             for (int k = 0; k < K; ++k) {
               const int tree = slotTree[bd.firstSlot + k];
-              if (tree >= 0) leafIds[row * s.numTrees + tree] = nodeOrigin[grp.nodeBegin + addr[k] / kNodeBytes];
+              if (tree >= 0) leafIds[row * s.numTrees + tree] = nodeOrigin[grp.nodeBegin * 2u + addr[k] / 4u];
             }
           }
         }
@@ -992,8 +1031,8 @@ WalkTreeParallelKernel(const float *__restrict__ x, const uint4 *__restrict__ no
 #pragma unroll
           for (int k = 0; k < K; ++k) {
             const U32x2 node = LdsLoadNode(addr[k]);
-            const float xv = LdsLoadFloat(rowBase + (node.y & 0xFFFFu));
-            addr[k] = (node.y >> 16) + (xv < AsFloat(node.x) ? 0u : kNodeBytes);
+            const float xv = LdsLoadFloat(rowBase + MetaFeature(node.y));
+            addr[k] = MetaChild(node.y) + (xv < AsFloat(node.x) ? 0u : kNodeBytes);
           }
         }
 #pragma unroll
@@ -1003,7 +1042,7 @@ WalkTreeParallelKernel(const float *__restrict__ x, const uint4 *__restrict__ no
 #pragma unroll
             for (int k = 0; k < K; ++k) {
               const int tree = slotTree[bd.firstSlot + k];
-              if (tree >= 0) leafIds[row * s.numTrees + tree] = nodeOrigin[grp.nodeBegin + addr[k] / kNodeBytes];
+              if (tree >= 0) leafIds[row * s.numTrees + tree] = nodeOrigin[grp.nodeBegin * 2u + addr[k] / 4u];
             }
           }
         }
@@ -1837,15 +1876,35 @@ hipError_t LaunchWalkVariant(const WalkParams &p, dim3 grid, dim3 block, size_t 
                      reinterpret_cast<const U32x2 *>(p.tailNodes), p.tailOrigin);
 }
 
+template <int K, int W, int V>
+hipError_t LaunchSplitVariant(const WalkParams &p, dim3 block, size_t ldsBytes, hipStream_t stream) {
+  hipError_t e = AllowFullLds<&WalkRowsSplitKernel<K, W, V>>();
+  if (e != hipSuccess) return e;
+  return StartKernel(&WalkRowsSplitKernel<K, W, V>, dim3((unsigned)p.splitBlocks), block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles,
+                     p.bundleRoots, p.groups, p.s, p.partial);
+}
+
 template <int K, int W>
 hipError_t LaunchSplit(const WalkParams &p, dim3 block, size_t ldsBytes, hipStream_t stream) {
   const int64_t rowBlocks = (p.s.rows + p.s.rowsPerBlock - 1) / p.s.rowsPerBlock;
   if (p.splitBlocks < 1 || p.splitBlocks > rowBlocks * p.s.numGroups || !p.partial || p.leafIds || p.s.deferTails || p.s.fuseArgmax)
     return hipErrorInvalidValue;
-  hipError_t e = p.s.ownClasses ? AllowFullLds<&WalkRowsSplitKernel<K, W, kWalkOwn>>() : AllowFullLds<&WalkRowsSplitKernel<K, W, kWalkPlain>>();
-  if (e != hipSuccess) return e;
-  return StartKernel(p.s.ownClasses ? &WalkRowsSplitKernel<K, W, kWalkOwn> : &WalkRowsSplitKernel<K, W, kWalkPlain>, dim3((unsigned)p.splitBlocks), block, ldsBytes, stream, p.done, p.x, p.nodes16, p.bundles,
-                     p.bundleRoots, p.groups, p.s, p.partial);
+  if (p.s.ownClasses)
+    return p.s.leavesOutside && !IsRankTile(W) ? LaunchSplitVariant<K, W, kWalkOwn | kWalkOutside>(p, block, ldsBytes, stream)
+                                               : LaunchSplitVariant<K, W, kWalkOwn>(p, block, ldsBytes, stream);
+  return p.s.leavesOutside && !IsRankTile(W) ? LaunchSplitVariant<K, W, kWalkPlain | kWalkOutside>(p, block, ldsBytes, stream)
+                                             : LaunchSplitVariant<K, W, kWalkPlain>(p, block, ldsBytes, stream);
+}
+
+// The variant for where the last level's leaves are (rank tiles: always in LDS).
+template <int K, int PF, int W, int V>
+hipError_t LaunchWalkLeaves(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream) {
+  if constexpr (IsRankTile(W)) {
+    return p.s.leavesOutside ? hipErrorInvalidValue : LaunchWalkVariant<K, PF, W, V>(p, grid, block, ldsBytes, stream);
+  } else {
+    return p.s.leavesOutside ? LaunchWalkVariant<K, PF, W, V | kWalkOutside>(p, grid, block, ldsBytes, stream)
+                             : LaunchWalkVariant<K, PF, W, V>(p, grid, block, ldsBytes, stream);
+  }
 }
 
 template <int K, int PF, int W>
@@ -1855,15 +1914,15 @@ hipError_t LaunchWalkKP(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBy
     return LaunchWalkVariant<K, PF, W, kWalkDump>(p, grid, block, ldsBytes, stream);
   }
   if (p.s.ownClasses)
-    return p.s.fuseArgmax ? LaunchWalkVariant<K, PF, W, kWalkOwnFuse>(p, grid, block, ldsBytes, stream)
-                          : LaunchWalkVariant<K, PF, W, kWalkOwn>(p, grid, block, ldsBytes, stream);
-  if (p.s.fuseArgmax) return LaunchWalkVariant<K, PF, W, kWalkFuse>(p, grid, block, ldsBytes, stream);
+    return p.s.fuseArgmax ? LaunchWalkLeaves<K, PF, W, kWalkOwnFuse>(p, grid, block, ldsBytes, stream)
+                          : LaunchWalkLeaves<K, PF, W, kWalkOwn>(p, grid, block, ldsBytes, stream);
+  if (p.s.fuseArgmax) return LaunchWalkLeaves<K, PF, W, kWalkFuse>(p, grid, block, ldsBytes, stream);
   // deferred tails are built for the f32 tile with byte offsets only (the packer makes stubs for no other plan)
   if (p.s.deferTails) {
-    if (W != kTileF32Bytes || p.s.numClasses > 0) return hipErrorInvalidValue;
+    if (W != kTileF32Bytes || p.s.numClasses > 0 || p.s.leavesOutside) return hipErrorInvalidValue;
     return LaunchWalkVariant<K, PF, kTileF32Bytes, kWalkDefer>(p, grid, block, ldsBytes, stream);
   }
-  return LaunchWalkVariant<K, PF, W, kWalkPlain>(p, grid, block, ldsBytes, stream);
+  return LaunchWalkLeaves<K, PF, W, kWalkPlain>(p, grid, block, ldsBytes, stream);
 }
 
 template <int K, int W>

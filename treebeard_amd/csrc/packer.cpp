@@ -575,8 +575,59 @@ FewRowsModel PackFewRows(const Forest &input) {
 }
 
 namespace {
+// A tree in a group's image, in units of 8 bytes.
+struct TreeUnits {
+  uint32_t whole = 0;
+  uint32_t lowest = 0; // of which the leaves of its last level, where the walk can take those from global memory
+};
+
+// How many nodes that walks reach a tree has on each level.
+std::vector<uint32_t> NodesPerLevel(const Tree &tree) {
+  std::vector<uint32_t> counts;
+  std::vector<int32_t> level{0}, below;
+  while (!level.empty()) {
+    counts.push_back((uint32_t)level.size());
+    below.clear();
+    for (int32_t n : level)
+      if (!tree.IsLeaf(n)) below.insert(below.end(), {tree.left[(size_t)n], tree.right[(size_t)n]});
+    level.swap(below);
+  }
+  return counts;
+}
+
+TreeUnits UnitsOfTree(const std::vector<uint32_t> &levels, bool leavesOutside) {
+  TreeUnits u;
+  for (uint32_t n : levels) u.whole += n;
+  if (leavesOutside && levels.size() > 1) u.lowest = levels.back();
+  return u;
+}
+
+// What a bundle of trees takes in LDS: of those as deep as its walk all but the last level.
+struct BundleUnits {
+  uint32_t lds = 0;
+  uint32_t outside = 0; // leaves that stay out of it
+};
+BundleUnits UnitsOfBundle(const int32_t *trees, size_t count, const std::vector<int32_t> &depth, const std::vector<TreeUnits> &units) {
+  int32_t deepest = 0;
+  for (size_t k = 0; k < count; ++k)
+    if (trees[k] >= 0) deepest = std::max(deepest, depth[(size_t)trees[k]]);
+  BundleUnits b;
+  for (size_t k = 0; k < count; ++k) {
+    if (trees[k] < 0) continue;
+    const TreeUnits &u = units[(size_t)trees[k]];
+    const uint32_t lowest = depth[(size_t)trees[k]] == deepest ? u.lowest : 0u;
+    b.lds += u.whole - lowest;
+    b.outside += lowest;
+  }
+  return b;
+}
+// Whether nodes in LDS and leaves outside (4 bytes each), whole 16-byte pieces of either, keep 16-bit addresses.
+bool AddressesFit(uint32_t ldsUnits, uint32_t outside) {
+  return ((ldsUnits * kNodeBytes + 15u) & ~15u) + ((outside * 4u + 15u) & ~15u) <= 0x10000u;
+}
+
 PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile, const std::vector<int32_t> *cuts);
-bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth, const std::vector<uint32_t> &units,
+bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth, const std::vector<TreeUnits> &units,
                     const std::vector<int32_t> &order, std::vector<std::vector<int32_t>> *rounds);
 // Trees order[first], ..., order[first + count - 1] are a bundle of tree group `group`.
 struct BundleTrees {
@@ -584,19 +635,21 @@ struct BundleTrees {
   size_t first;
   int32_t count;
 };
-std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &plan, const std::vector<uint32_t> &units, uint32_t tileUnits,
-                                      const std::vector<int32_t> &order);
+std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth,
+                                      const std::vector<TreeUnits> &units, uint32_t tileUnits, const std::vector<int32_t> &order);
 }
 
 namespace {
 // What PackForest goes by of a scalar plan without a profile: the trees' depths and sizes, in its order.
 struct PlainTrees {
   std::vector<int32_t> depth, order;
-  std::vector<uint32_t> units;
-  explicit PlainTrees(const Forest &forest) : depth(forest.trees.size()), order(forest.trees.size()), units(forest.trees.size()) {
+  std::vector<TreeUnits> units;
+  PlainTrees(const Forest &forest, const LaunchPlan &plan) : depth(forest.trees.size()), order(forest.trees.size()), units(forest.trees.size()) {
+    const bool outside = LeavesOutside(forest, plan);
     for (size_t t = 0; t < forest.trees.size(); ++t) {
-      depth[t] = forest.trees[t].Depth();
-      units[t] = (uint32_t)MakeLevelOrder(forest.trees[t]).order.size();
+      const std::vector<uint32_t> levels = NodesPerLevel(forest.trees[t]);
+      depth[t] = (int32_t)levels.size() - 1;
+      units[t] = UnitsOfTree(levels, outside);
     }
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(), [&](int32_t a, int32_t b) {
@@ -608,14 +661,37 @@ struct PlainTrees {
 } // namespace
 
 bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan) {
-  const PlainTrees trees(forest);
+  const PlainTrees trees(forest, plan);
   std::vector<std::vector<int32_t>> rounds;
   return OwnClassRounds(forest, plan, trees.depth, trees.units, trees.order, &rounds);
 }
 
+int64_t TreeBytesInLds(const Forest &forest, bool leavesOutside) {
+  int64_t total = 0;
+  for (const Tree &tree : forest.trees) {
+    const TreeUnits u = UnitsOfTree(NodesPerLevel(tree), leavesOutside);
+    total += u.whole - u.lowest;
+  }
+  return total * kNodeBytes;
+}
+
+// What stays out of LDS makes room for more trees between two barriers and takes the leaf reads off the LDS pipes, and costs a
+// gather from L2 per tree.  2^20 rows x 1000 trees of depth 8 (30 % of the nodes are such leaves) 27 groups and 16: 1162 -> 1069
+// us; 800 complete trees of depth 6 in 8 classes (half of the nodes) 50 and 25: 849 -> 790.  Not where no group is saved: one
+// group either way, 338838 rows x 52 trees of depth 5 22.3 and 22.9, 32 slices of a group, 4096 rows x 1000 trees 12.8 and 13.4;
+// nor for the few leaves of skewed trees: 800 of depth 12 in 20 groups and 17 1213 and 1239.
+bool LeavesOutside(const Forest &forest, const LaunchPlan &plan) {
+  if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.WalkTile() > 1 || plan.deferTails || plan.quantizedRows || plan.rankRows16)
+    return false;
+  const int64_t inside = TreeBytesInLds(forest, false), without = TreeBytesInLds(forest, true);
+  const auto groups = [&](int64_t bytes) { return std::max<int64_t>(1, (bytes + plan.groupBytes - 1) / plan.groupBytes); };
+  const auto turns = [&](int64_t bytes) { return (groups(bytes) + plan.treeSlices - 1) / plan.treeSlices; };
+  return without * 5 < inside * 4 && groups(without) >= plan.treeSlices && turns(without) < turns(inside);
+}
+
 int32_t CountTreeGroups(const Forest &forest, const LaunchPlan &plan) {
-  const PlainTrees trees(forest);
-  const std::vector<BundleTrees> bundles = LayOutGroups(forest, plan, trees.units, 1, trees.order);
+  const PlainTrees trees(forest, plan);
+  const std::vector<BundleTrees> bundles = LayOutGroups(forest, plan, trees.depth, trees.units, 1, trees.order);
   return bundles.empty() ? 1 : bundles.back().group + 1;
 }
 
@@ -635,7 +711,7 @@ namespace {
 // and this, and what was measured: 8 classes 1504 and 1200, 916 and 847 us; 12 1680 and 1224, 969 and 862; 11 1540 and 1368,
 // 955 and 894; 7 1484 and 1392, 917 and 910; 10 1400 and 1440, 862 and 890; 9 1476 and 1656, 941 and 957; 6 1416 and 1632, 898
 // and 949; 5 1300 and 1920, 853 and 1015.  `order`: by class.  False: the classes meet.
-bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth, const std::vector<uint32_t> &units,
+bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth, const std::vector<TreeUnits> &units,
                     const std::vector<int32_t> &order, std::vector<std::vector<int32_t>> *rounds) {
   if (forest.numClasses < 2 || plan.treeThreads < 2 || plan.kernel != LaunchPlan::Kernel::kRowParallelLds || order.empty()) return false;
   const size_t TT = (size_t)plan.treeThreads, C = (size_t)forest.numClasses;
@@ -657,14 +733,14 @@ bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vec
     for (size_t c = c0; c < std::min(C, c0 + TT); ++c) most = std::max(most, (ofClass[c].size() + K - 1) / K);
     for (size_t i = 0; i < most; ++i) {
       std::vector<int32_t> round(TT * K, -1);
-      uint32_t need = 0;
-      for (size_t c = c0; c < std::min(C, c0 + TT); ++c)
-        for (size_t k = 0; k < (size_t)K && i * K + k < ofClass[c].size(); ++k) {
-          const int32_t t = ofClass[c][i * K + k];
-          round[(c - c0) * K + k] = t;
-          need += units[(size_t)t];
-        }
-      if (need + 2 > groupCapacity - 1) return false;
+      BundleUnits need;
+      for (size_t c = c0; c < std::min(C, c0 + TT); ++c) {
+        for (size_t k = 0; k < (size_t)K && i * K + k < ofClass[c].size(); ++k) round[(c - c0) * K + k] = ofClass[c][i * K + k];
+        const BundleUnits bundle = UnitsOfBundle(&round[(c - c0) * K], (size_t)K, depth, units);
+        need.lds += bundle.lds;
+        need.outside += bundle.outside;
+      }
+      if (need.lds + 2 > groupCapacity - 1 || !AddressesFit(need.lds + 2, need.outside)) return false;
       rounds->push_back(std::move(round));
     }
   }
@@ -678,29 +754,33 @@ bool OwnClassRounds(const Forest &forest, const LaunchPlan &plan, const std::vec
 // Bundles of up to K consecutive trees of one class, in groups of what fits the plan's group size.  Tree threads take bundles
 // round-robin: when more trees follow, a group ends on a multiple of treeThreads bundles so that no thread idles through a last
 // partial round.
-std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &plan, const std::vector<uint32_t> &units, uint32_t tileUnits,
-                                      const std::vector<int32_t> &order) {
+std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &plan, const std::vector<int32_t> &depth,
+                                      const std::vector<TreeUnits> &units, uint32_t tileUnits, const std::vector<int32_t> &order) {
   const uint32_t groupCapacity = (uint32_t)plan.groupBytes / kNodeBytes;
   const size_t multiple = plan.kernel == LaunchPlan::Kernel::kRowParallelLds ? (size_t)plan.treeThreads : 1;
   std::vector<BundleTrees> out;
   size_t next = 0;
   for (int32_t group = 0; next < order.size(); ++group) {
     const size_t begin = out.size();
-    uint32_t used = tileUnits; // the null leaf
+    uint32_t used = tileUnits, usedOutside = 0; // the null leaf
     while (next < order.size()) {
       const int32_t cls = forest.numClasses > 0 ? forest.trees[order[next]].classId : 0;
       int32_t count = 0;
+      BundleUnits bundle;
       while (count < plan.interleave && next + count < order.size()) {
         const int32_t t = order[next + count];
         const int32_t c = forest.numClasses > 0 ? forest.trees[t].classId : 0;
         if (c != cls) break;
-        if (units[t] + 2 * tileUnits > groupCapacity)
+        if (units[t].whole + 2 * tileUnits > groupCapacity)
           throw Error("a tree of " + std::to_string(forest.trees[t].NumNodes()) + " nodes does not fit one LDS tree group");
-        if (used + units[t] > groupCapacity - 1) break; // (one spare unit keeps room for the alignment pad)
-        used += units[t];
+        const BundleUnits with = UnitsOfBundle(&order[next], (size_t)count + 1, depth, units);
+        if (used + with.lds > groupCapacity - 1 || !AddressesFit(used + with.lds, usedOutside + with.outside)) break; // (one spare unit keeps room for the alignment pad)
+        bundle = with;
         ++count;
       }
       if (count == 0) break; // group full
+      used += bundle.lds;
+      usedOutside += bundle.outside;
       out.push_back(BundleTrees{group, next, count});
       next += (size_t)count;
     }
@@ -771,6 +851,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
   pm.numFeatures = forest.numFeatures;
   pm.numClasses = forest.numClasses;
   pm.numTrees = (int32_t)forest.trees.size();
+  pm.leavesOutside = LeavesOutside(forest, plan);
   if (plan.deferTails) { // tail node 0: a leaf of value 0, what a lane without a queue entry walks
     pm.tailNodes.push_back(DeviceNode{0.0f, (0u << kTailFeatureBits) | (uint32_t)forest.numFeatures});
     pm.tailOrigin.push_back(-1);
@@ -860,7 +941,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
   std::vector<int32_t> depth(numTrees), peel(numTrees);
   std::vector<int32_t> fullDepth(numTrees, 0); // deferred tails: the tree's own depth (depth[] is then where its walk stops)
   int64_t tailBudget = plan.deferTails && forest.numFeatures + 1 < (1 << kTailFeatureBits) ? (int64_t)(cuts ? kMaxTailNodes : kPeeledTailNodes) - 1 : 0;
-  std::vector<uint32_t> units(numTrees);
+  std::vector<TreeUnits> units(numTrees);
   for (size_t t = 0; t < numTrees; ++t) {
     const Tree &tree = forest.trees[t];
     const std::vector<int64_t> *hits = profile ? &profile->hits[t] : nullptr;
@@ -869,20 +950,19 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     if (T > 1) {
       tiled[t] = TileTree(tree, T, plan.tiling, hits);
       depth[t] = tiled[t].depth;
-      units[t] = (uint32_t)tiled[t].tiles.size() * tileUnits;
+      units[t].whole = (uint32_t)tiled[t].tiles.size() * tileUnits;
       pm.treesTiledByProfile += tiled[t].byProfile ? 1 : 0;
       pm.maxTileHops = std::max(pm.maxTileHops, tiled[t].hops);
       for (const TileInfo &tile : tiled[t].tiles)
         if (tile.count == 0) leafLevel[tile.leafNode] = tile.level;
     } else {
       depth[t] = tree.Depth();
-      units[t] = 0; // (of the nodes that walks reach: pruned models keep others)
+      units[t] = UnitsOfTree(NodesPerLevel(tree), pm.leavesOutside); // (of the nodes that walks reach: pruned models keep others)
       std::vector<int32_t> stack{0};
       leafLevel[0] = 0;
       while (!stack.empty()) { // (the level of every node; only the leaves' entries are used)
         const int32_t n = stack.back();
         stack.pop_back();
-        ++units[t];
         if (tree.IsLeaf(n)) continue;
         leafLevel[tree.left[n]] = leafLevel[tree.right[n]] = leafLevel[n] + 1;
         stack.push_back(tree.left[n]);
@@ -937,7 +1017,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
       }
       if (tails <= tailBudget && !nanLeaf) {
         tailBudget -= tails;
-        units[t] = above;
+        units[t].whole = above;
         depth[t] = cut;
         peel[t] = cut;
         pm.treesDeferred += 1;
@@ -965,6 +1045,11 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     return peel[a] < peel[b];
   });
 
+  const auto pushUnit = [&](const DeviceNode &node, int32_t origin, int32_t second = -1) {
+    pm.nodes.push_back(node);
+    pm.nodeOrigin.push_back(origin);
+    pm.nodeOrigin.push_back(second);
+  };
   // The null leaf that padding trees of a bundle point at: a leaf of value 0 at address 0 of every group.
   auto pushNullLeaf = [&]() {
     if (T > 1) {
@@ -979,12 +1064,10 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
       for (uint32_t u = 0; u < tileUnits; ++u) {
         DeviceNode unit;
         std::memcpy(&unit, bytes.data() + u * kNodeBytes, kNodeBytes);
-        pm.nodes.push_back(unit);
-        pm.nodeOrigin.push_back(-1);
+        pushUnit(unit, -1);
       }
     } else {
-      pm.nodes.push_back(DeviceNode{0.0f, (0u << 16) | (uint32_t)padOffset});
-      pm.nodeOrigin.push_back(-1);
+      pushUnit(DeviceNode{0.0f, NodeMeta(0, (uint32_t)padOffset)}, -1);
     }
   };
   auto openGroup = [&]() {
@@ -994,14 +1077,37 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     pm.groups.push_back(g);
     pushNullLeaf();
   };
+  // Leaves of the group that stay out of LDS, and the nodes whose children they are (which count from the first of them until it
+  // is known where that lies).
+  std::vector<float> outside;
+  std::vector<int32_t> outsideOrigin;
+  std::vector<size_t> aboveOutside;
+  auto pad = [&]() { // whole 16-byte pieces
+    if ((pm.nodes.size() - pm.groups.back().nodeBegin) & 1) pushUnit(DeviceNode{0.0f, NodeMeta(0, (uint32_t)padOffset)}, -1);
+  };
   auto closeGroup = [&]() {
     DeviceGroup &g = pm.groups.back();
-    if ((pm.nodes.size() - g.nodeBegin) & 1) { // whole 16-byte pieces
-      pm.nodes.push_back(DeviceNode{0.0f, (0u << 16) | (uint32_t)padOffset});
-      pm.nodeOrigin.push_back(-1);
-    }
+    pad();
     g.nodeCount = (uint32_t)pm.nodes.size() - g.nodeBegin;
+    for (size_t n : aboveOutside) pm.nodes[n].meta = NodeMeta(MetaChild(pm.nodes[n].meta) + g.nodeCount * kNodeBytes, MetaFeature(pm.nodes[n].meta));
+    if (outside.size() & 1) {
+      outside.push_back(0.0f);
+      outsideOrigin.push_back(-1);
+    }
+    for (size_t i = 0; i < outside.size(); i += 2) {
+      DeviceNode two;
+      std::memcpy(&two, &outside[i], sizeof(two));
+      pushUnit(two, outsideOrigin[i], outsideOrigin[i + 1]);
+    }
+    outside.clear();
+    outsideOrigin.clear();
+    aboveOutside.clear();
+    pad();
+    g.imageCount = (uint32_t)pm.nodes.size() - g.nodeBegin;
+    if (g.imageCount * kNodeBytes > 0x10000u) throw Error("internal error: tree group beyond 16-bit addresses");
     g.bundleCount = (uint32_t)pm.bundles.size() - g.bundleBegin;
+    for (uint32_t b = g.bundleBegin; b < pm.bundles.size(); ++b)
+      for (int k = 0; k < K; ++k) pm.bundleRoots.push_back(pm.nodes[g.nodeBegin + pm.bundles[b].root[k] / kNodeBytes]);
     g.uniformClass = 0;
     if (g.bundleCount > 0) {
       const uint32_t first = pm.bundles[g.bundleBegin].classId;
@@ -1011,8 +1117,8 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     }
     pm.maxGroupNodes = std::max(pm.maxGroupNodes, g.nodeCount);
   };
-  // Writes tree t with its first unit at unit `base` of the current group.
-  auto emitTree = [&](int32_t t, uint32_t base) {
+  // Writes tree t with its first unit at unit `base` of the current group, to be walked for `steps` levels.
+  auto emitTree = [&](int32_t t, uint32_t base, int32_t steps) {
     const Tree &tree = forest.trees[t];
     if (T > 1) {
       std::vector<unsigned char> bytes(TileBytes(T));
@@ -1022,8 +1128,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
         for (uint32_t u = 0; u < tileUnits; ++u) {
           DeviceNode unit;
           std::memcpy(&unit, bytes.data() + u * kNodeBytes, kNodeBytes);
-          pm.nodes.push_back(unit);
-          pm.nodeOrigin.push_back(u == 0 ? (tile.count == 0 ? tile.leafNode : tile.members[0]) : -1);
+          pushUnit(unit, u == 0 ? (tile.count == 0 ? tile.leafNode : tile.members[0]) : -1);
         }
       }
       return;
@@ -1046,7 +1151,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
           queue.push_back({tree.right[n], level + 1});
         }
       }
-      if (top.size() != units[t]) throw Error("internal error: deferred tree size out of step");
+      if (top.size() != units[t].whole) throw Error("internal error: deferred tree size out of step");
       std::vector<uint32_t> tailIndex(tree.NumNodes(), 0);
       for (int32_t first : cutNodes) {
         std::vector<int32_t> queue{first};
@@ -1076,27 +1181,33 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
         DeviceNode dn;
         if (tree.IsLeaf(n)) {
           dn.value = tree.value[n];
-          dn.meta = (self << 16) | (uint32_t)padOffset;
+          dn.meta = NodeMeta(self, (uint32_t)padOffset);
         } else if (tailIndex[n] != 0) { // a stub: NaN compares false, so the walk takes the "right" child: the stub itself
           const uint32_t bits = kStubValueBits | tailIndex[n];
           std::memcpy(&dn.value, &bits, sizeof(bits));
-          dn.meta = ((self - kNodeBytes) << 16) | (uint32_t)padOffset;
+          dn.meta = NodeMeta(self - kNodeBytes, (uint32_t)padOffset);
         } else {
           dn.value = tree.value[n];
           if (where[tree.right[n]] != where[tree.left[n]] + 1) throw Error("internal error: siblings not adjacent");
-          dn.meta = (((base + (uint32_t)where[tree.left[n]]) * kNodeBytes) << 16) | plan.FeatureOffset((uint32_t)tree.feature[n]);
+          dn.meta = NodeMeta((base + (uint32_t)where[tree.left[n]]) * kNodeBytes, plan.FeatureOffset((uint32_t)tree.feature[n]));
         }
-        pm.nodes.push_back(dn);
-        pm.nodeOrigin.push_back(n);
+        pushUnit(dn, n);
       }
       pm.maxTailDepth = std::max<uint32_t>(pm.maxTailDepth, (uint32_t)(fullDepth[t] - cut));
       return;
     }
     const LevelOrder lo = MakeLevelOrder(tree);
+    const size_t inside = lo.order.size() - (depth[t] == steps ? units[t].lowest : 0u); // (level order: the last level comes last)
+    const size_t firstOutside = outside.size();
     for (size_t i = 0; i < lo.order.size(); ++i) {
       const int32_t n = lo.order[i];
       DeviceNode dn;
       dn.value = tree.value[n];
+      if (i >= inside) {
+        outside.push_back(tree.value[n]);
+        outsideOrigin.push_back(n);
+        continue;
+      }
       if ((plan.quantizedRows || plan.rankRows16) && !tree.IsLeaf(n)) {
         const auto &sorted = ranks[(size_t)tree.feature[n]];
         const uint32_t j = (uint32_t)(std::lower_bound(sorted.begin(), sorted.end(), tree.value[n]) - sorted.begin());
@@ -1104,15 +1215,16 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
         std::memcpy(&dn.value, &j, sizeof(j));
       }
       if (tree.IsLeaf(n)) {
-        dn.meta = (((base + (uint32_t)i) * kNodeBytes) << 16) | (uint32_t)padOffset;
+        dn.meta = NodeMeta((base + (uint32_t)i) * kNodeBytes, (uint32_t)padOffset);
       } else {
-        const uint32_t child = base + (uint32_t)lo.position[tree.left[n]];
+        const size_t left = (size_t)lo.position[tree.left[n]];
         if (lo.position[tree.right[n]] != lo.position[tree.left[n]] + 1)
           throw Error("internal error: siblings not adjacent");
-        dn.meta = ((child * kNodeBytes) << 16) | plan.FeatureOffset((uint32_t)tree.feature[n]);
+        const uint32_t child = (uint32_t)(left < inside ? (base + left) * kNodeBytes : (firstOutside + (left - inside)) * 4u);
+        if (left >= inside) aboveOutside.push_back(pm.nodes.size());
+        dn.meta = NodeMeta(child, plan.FeatureOffset((uint32_t)tree.feature[n]));
       }
-      pm.nodes.push_back(dn);
-      pm.nodeOrigin.push_back(n);
+      pushUnit(dn, n);
     }
   };
 
@@ -1124,26 +1236,33 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
       openGroup();
       DeviceGroup &g = pm.groups.back();
       for (; next < rounds.size(); ++next) {
-        uint32_t need = 0;
-        for (int32_t t : rounds[next]) need += t < 0 ? 0 : units[(size_t)t];
-        if (need > groupCapacity - 1 - ((uint32_t)pm.nodes.size() - g.nodeBegin)) break;
+        BundleUnits need;
+        for (size_t thread = 0; thread < TT; ++thread) {
+          const BundleUnits bundle = UnitsOfBundle(&rounds[next][thread * K], (size_t)K, depth, units);
+          need.lds += bundle.lds;
+          need.outside += bundle.outside;
+        }
+        const uint32_t used = (uint32_t)pm.nodes.size() - g.nodeBegin;
+        if (need.lds > groupCapacity - 1 - used || !AddressesFit(used + need.lds, (uint32_t)outside.size() + need.outside)) break;
         for (size_t thread = 0; thread < TT; ++thread) {
           DeviceBundle b{};
           b.firstSlot = (uint32_t)pm.slotTree.size();
           for (int k = 0; k < K; ++k) {
             const int32_t t = rounds[next][thread * K + (size_t)k];
             pm.slotTree.push_back(t);
+            if (t >= 0) b.depth = b.peelDepth = std::max<uint32_t>(b.depth, (uint32_t)depth[(size_t)t]);
+          }
+          for (int k = 0; k < K; ++k) {
+            const int32_t t = rounds[next][thread * K + (size_t)k];
             if (t < 0) continue; // (root 0: the null leaf)
             const uint32_t base = (uint32_t)pm.nodes.size() - g.nodeBegin;
             b.root[k] = (uint16_t)(base * kNodeBytes);
-            b.depth = b.peelDepth = std::max<uint32_t>(b.depth, (uint32_t)depth[(size_t)t]);
-            emitTree(t, base);
+            emitTree(t, base, (int32_t)b.depth);
           }
           const int32_t any = rounds[next][thread * K];
           // (a bundle without trees keeps its thread's class, the first one's if it had none yet)
           b.classId = any >= 0 ? (uint16_t)forest.trees[(size_t)any].classId
                       : pm.bundles.size() >= TT ? pm.bundles[pm.bundles.size() - TT].classId : (uint16_t)thread;
-          for (int k = 0; k < K; ++k) pm.bundleRoots.push_back(pm.nodes[g.nodeBegin + b.root[k] / kNodeBytes]);
           pm.bundles.push_back(b);
         }
       }
@@ -1151,7 +1270,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     }
   }
 
-  const std::vector<BundleTrees> laidOut = pm.ownClasses ? std::vector<BundleTrees>() : LayOutGroups(forest, plan, units, tileUnits, order);
+  const std::vector<BundleTrees> laidOut = pm.ownClasses ? std::vector<BundleTrees>() : LayOutGroups(forest, plan, depth, units, tileUnits, order);
   for (size_t at = 0; at < laidOut.size();) {
     openGroup();
     DeviceGroup &g = pm.groups.back();
@@ -1159,6 +1278,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
       DeviceBundle b{};
       b.classId = (uint16_t)(forest.numClasses > 0 ? forest.trees[order[laidOut[at].first]].classId : 0);
       b.firstSlot = (uint32_t)pm.slotTree.size();
+      for (int k = 0; k < laidOut[at].count; ++k) b.depth = std::max<uint32_t>(b.depth, (uint32_t)depth[order[laidOut[at].first + k]]);
       for (int k = 0; k < K; ++k) {
         if (k >= laidOut[at].count) {
           b.root[k] = 0; // null leaf
@@ -1168,13 +1288,11 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
         const int32_t t = order[laidOut[at].first + k];
         const uint32_t base = (uint32_t)pm.nodes.size() - g.nodeBegin; // unit index inside the group
         b.root[k] = (uint16_t)(base * kNodeBytes);
-        b.depth = std::max<uint32_t>(b.depth, (uint32_t)depth[t]);
         b.peelDepth = std::max<uint32_t>(b.peelDepth, (uint32_t)peel[t]);
         if (plan.deferTails && depth[t] < fullDepth[t]) b.hasStubs = 1;
         pm.slotTree.push_back(t);
-        emitTree(t, base);
+        emitTree(t, base, (int32_t)b.depth);
       }
-      for (int k = 0; k < K; ++k) pm.bundleRoots.push_back(pm.nodes[g.nodeBegin + b.root[k] / kNodeBytes]);
       pm.bundles.push_back(b);
     }
     closeGroup();
@@ -1226,39 +1344,49 @@ Tree UnpackTree(const PackedModel &pm, int32_t treeIndex) {
         if (pm.slotTree[pm.bundles[bi].firstSlot + k] != treeIndex) continue;
         // walk the packed tree breadth first, restoring original node ids (a stub stands for the node its value
         // field points at)
-        // (units of the group's image; a stub stands for a node of the tail array, noted as kTailBit | index)
+        // (words of the group's image, whose nodes take two and whose leaves outside LDS one; a stub stands for a node of the
+        // tail array, noted as kTailBit | index)
         constexpr uint32_t kTailBit = 0x80000000u;
-        auto resolve = [&](uint32_t unit) {
-          const DeviceNode &dn = pm.nodes[g.nodeBegin + unit];
+        auto resolve = [&](uint32_t word) {
+          if (word >= g.nodeCount * 2) return word;
+          const DeviceNode &dn = pm.nodes[g.nodeBegin + word / 2];
           uint32_t bits;
           std::memcpy(&bits, &dn.value, sizeof(bits));
-          const bool stub = pm.plan.deferTails && (dn.meta >> 16) / kNodeBytes + 1 == unit && (bits & ~kStubIndexMask) == kStubValueBits;
-          if (!stub) return unit;
+          const bool stub = pm.plan.deferTails && MetaChild(dn.meta) / kNodeBytes + 1 == word / 2 && (bits & ~kStubIndexMask) == kStubValueBits;
+          if (!stub) return word;
           return kTailBit | (bits & kStubIndexMask);
         };
-        auto nodeAt = [&](uint32_t q) -> const DeviceNode & { return q & kTailBit ? pm.tailNodes[q & ~kTailBit] : pm.nodes[g.nodeBegin + q]; };
-        auto originAt = [&](uint32_t q) { return q & kTailBit ? pm.tailOrigin[q & ~kTailBit] : pm.nodeOrigin[g.nodeBegin + q]; };
-        auto leftOf = [&](uint32_t q) -> uint32_t { // the left child (same notation), or q itself on a leaf
-          const DeviceNode &dn = nodeAt(q);
+        auto outsideLds = [&](uint32_t q) { return !(q & kTailBit) && q >= g.nodeCount * 2; };
+        auto nodeAt = [&](uint32_t q) {
+          if (q & kTailBit) return pm.tailNodes[q & ~kTailBit];
+          DeviceNode dn = pm.nodes[g.nodeBegin + q / 2];
+          if (outsideLds(q) && (q & 1)) std::memcpy(&dn.value, &dn.meta, sizeof(dn.value));
+          return dn;
+        };
+        auto originAt = [&](uint32_t q) { return q & kTailBit ? pm.tailOrigin[q & ~kTailBit] : pm.nodeOrigin[(size_t)g.nodeBegin * 2 + q]; };
+        auto isLeaf = [&](uint32_t q) {
+          if (outsideLds(q)) return true;
+          const DeviceNode dn = nodeAt(q);
+          return q & kTailBit ? (dn.meta >> kTailFeatureBits) == (q & ~kTailBit) : MetaChild(dn.meta) / 4 == q;
+        };
+        auto leftOf = [&](uint32_t q) -> uint32_t { // the left child (same notation) of a split
+          const DeviceNode dn = nodeAt(q);
           if (q & kTailBit) return kTailBit | (dn.meta >> kTailFeatureBits);
-          return resolve((dn.meta >> 16) / kNodeBytes);
+          return resolve(MetaChild(dn.meta) / 4);
         };
         auto rightOf = [&](uint32_t q) -> uint32_t {
-          const DeviceNode &dn = nodeAt(q);
+          const DeviceNode dn = nodeAt(q);
           if (q & kTailBit) return kTailBit | ((dn.meta >> kTailFeatureBits) + 1);
-          return resolve((dn.meta >> 16) / kNodeBytes + 1);
-        };
-        auto isLeaf = [&](uint32_t q) {
-          const DeviceNode &dn = nodeAt(q);
-          return q & kTailBit ? (dn.meta >> kTailFeatureBits) == (q & ~kTailBit) : (dn.meta >> 16) / kNodeBytes == q;
+          const uint32_t left = MetaChild(dn.meta) / 4;
+          return resolve(left + (left >= g.nodeCount * 2 ? 1 : 2));
         };
         auto featureOf = [&](uint32_t q) -> int32_t {
-          const DeviceNode &dn = nodeAt(q);
-          return q & kTailBit ? (int32_t)(dn.meta & ((1u << kTailFeatureBits) - 1u)) : (int32_t)pm.plan.FeatureOfOffset(dn.meta & 0xFFFFu);
+          const DeviceNode dn = nodeAt(q);
+          return q & kTailBit ? (int32_t)(dn.meta & ((1u << kTailFeatureBits) - 1u)) : (int32_t)pm.plan.FeatureOfOffset(MetaFeature(dn.meta));
         };
         Tree tree;
         tree.classId = pm.bundles[bi].classId;
-        std::vector<uint32_t> queue{resolve(pm.bundles[bi].root[k] / kNodeBytes)};
+        std::vector<uint32_t> queue{resolve(pm.bundles[bi].root[k] / 4)};
         size_t total = 0;
         for (size_t head = 0; head < queue.size(); ++head) {
           total = std::max<size_t>(total, (size_t)originAt(queue[head]) + 1);
@@ -1269,7 +1397,7 @@ Tree UnpackTree(const PackedModel &pm, int32_t treeIndex) {
         tree.left.assign(total, -1);
         tree.right.assign(total, -1);
         for (uint32_t q : queue) {
-          const DeviceNode &dn = nodeAt(q);
+          const DeviceNode dn = nodeAt(q);
           const int32_t me = originAt(q);
           tree.value[me] = dn.value;
           const bool leaf = isLeaf(q);

@@ -90,7 +90,7 @@ struct PackedModel {
   std::vector<DeviceBundle> bundles;
   std::vector<DeviceGroup> groups;
   // Parity/debug side tables (not touched by the timed kernels):
-  std::vector<int32_t> nodeOrigin; // per packed node: original node id inside its tree (-1: null leaf)
+  std::vector<int32_t> nodeOrigin; // per 4 bytes of the packed nodes: original node id inside its tree (-1: null leaf, second half of a node)
   std::vector<int32_t> slotTree;   // per bundle slot: original tree index, -1 for a padding tree
   // Copies of the root nodes, plan.interleave per bundle: every lane of a wave starts a tree at its root, so
   // the f32 row-parallel walk takes level 0 from scalar registers instead of an LDS node read.
@@ -99,6 +99,9 @@ struct PackedModel {
   // Classifiers on scalar row-parallel plans: every class is one tree thread's, so that class sums need no meeting of the tree
   // threads.  Groups are whole rounds of a bundle for every tree thread, bundles without trees among them.
   bool ownClasses = false;
+  // Scalar row-parallel plans: the leaves of the last level of a bundle's walk stay in global memory, in 4 bytes each behind the
+  // group's nodes (device_model.h).
+  bool leavesOutside = false;
   // Tiled plans: how many trees were tiled by visit counts (the others breadth first), and the tile steps
   // one row takes over the whole forest: lock-step (deepest leaf of every tree) and, when a profile was
   // given, what the profiled rows need on average.
@@ -185,6 +188,10 @@ PackedModel PackWithCuts(const Forest &forest, const LaunchPlan &plan, const std
 
 // Whether PackForest gives every class of a forest to one tree thread under a scalar row-parallel plan (PackedModel::ownClasses).
 bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan);
+// LDS bytes of all trees of a forest under a scalar row-parallel plan, with the leaves of the trees' last levels or without.
+int64_t TreeBytesInLds(const Forest &forest, bool leavesOutside);
+// Whether PackForest leaves those out (PackedModel::leavesOutside): where that saves tree groups.
+bool LeavesOutside(const Forest &forest, const LaunchPlan &plan);
 // How many tree groups PackForest makes under a scalar plan, classes of the tree threads' own aside.
 int32_t CountTreeGroups(const Forest &forest, const LaunchPlan &plan);
 

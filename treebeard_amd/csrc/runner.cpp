@@ -43,9 +43,9 @@ unsigned char *ScratchOfCurrentDevice() {
   return gScratchAddress[device];
 }
 
-template <typename T> T *Upload(const std::vector<T> &host, const char *what) {
+template <typename T> T *Upload(const std::vector<T> &host, const char *what, size_t spareBytes = 0) {
   T *ptr = nullptr;
-  const size_t bytes = std::max<size_t>(host.size(), 1) * sizeof(T);
+  const size_t bytes = std::max<size_t>(host.size(), 1) * sizeof(T) + spareBytes;
   Check(hipMalloc(reinterpret_cast<void **>(&ptr), bytes), what);
   if (!host.empty()) Check(hipMemcpy(ptr, host.data(), host.size() * sizeof(T), hipMemcpyHostToDevice), what);
   return ptr;
@@ -217,7 +217,8 @@ void InferenceRunner::UploadModel() {
   // treeSlices never exceeds the number of groups the packer produced
   m_model.plan.treeSlices = std::max(1, std::min<int32_t>(m_model.plan.treeSlices, (int32_t)m_model.groups.size()));
   if (m_model.LdsBytes() > (size_t)m_limits.ldsBytesPerBlock) throw Error("launch plan exceeds the LDS of one workgroup");
-  m_dNodes = Upload(m_model.nodes, "upload nodes");
+  // (the walk looks leaf values up at 16-bit addresses of a group's image: behind the last group's, any such address is the buffer's)
+  m_dNodes = Upload(m_model.nodes, "upload nodes", 0x10000 + 2 * kNodeBytes);
   m_dBundles = Upload(m_model.bundles, "upload bundles");
   m_dBundleRoots = Upload(m_model.bundleRoots, "upload bundle roots");
   m_dGroups = Upload(m_model.groups, "upload groups");
@@ -503,6 +504,7 @@ WalkParams InferenceRunner::MakeWalkParams(const float *deviceInputs, int64_t ro
   p.s.tailDepth = (int32_t)model.maxTailDepth;
   p.s.tileHops = model.maxTileHops;
   p.s.ownClasses = model.ownClasses ? 1 : 0;
+  p.s.leavesOutside = model.leavesOutside ? 1 : 0;
   p.tailNodes = m_dTailNodes;
   p.tailOrigin = m_dTailOrigin;
   p.directStaging = DirectStaging();
@@ -1116,7 +1118,7 @@ std::string InferenceRunner::DescribePlan() const {
      << " lockStepSteps=" << m_model.lockStepSteps << " profiledSteps=" << m_model.profiledSteps
      << " batchKernel=" << KernelOfBatch() << " fewRowsLimit=" << m_fewRowsLimit
      << " treesDeferred=" << m_model.treesDeferred << " deferredEntriesPerRow=" << m_model.deferredEntriesPerRow
-     << " ownClasses=" << (m_model.ownClasses ? 1 : 0);
+     << " ownClasses=" << (m_model.ownClasses ? 1 : 0) << " leavesOutside=" << (m_model.leavesOutside ? 1 : 0);
   if (WalksDeep()) { // the fields above are the launch plan's: what calls run in its place has a shape of its own
     const LaunchPlan &d = m_deep.model.plan;
     os << " deepRowsPerBlock=" << d.rowsPerBlock << " deepTreeThreads=" << d.treeThreads << " deepInterleave=" << d.interleave

@@ -88,7 +88,7 @@ LaunchPlan ChooseTreeParallelPlan(const Forest &forest, int64_t batchSize, const
 
 namespace {
 LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAutoScheduleOptions *ov,
-                            const DeviceLimits &limits, int tileSize);
+                            const DeviceLimits &limits, int tileSize, bool peelWalks);
 // LDS bytes a tree group must offer the biggest tree of a tiled forest (the null leaf tile and the alignment
 // pad of a group included).
 int64_t TiledGroupNeed(const Forest &forest, int tileSize) {
@@ -128,7 +128,7 @@ LaunchPlan ChoosePlan(const Forest &forest, int64_t batchSize, const GPUAutoSche
   LaunchPlan wanted;
   wanted.tileSize = walk.tileSize;
   wanted.tiling = walk.tiling;
-  LaunchPlan plan = ChooseScalarPlan(forest, batchSize, ov, limits, wanted.WalkTile());
+  LaunchPlan plan = ChooseScalarPlan(forest, batchSize, ov, limits, wanted.WalkTile(), walk.peelWalks);
   plan.tileSize = walk.tileSize;
   plan.tiling = walk.tiling;
   plan.peelWalks = walk.peelWalks;
@@ -218,7 +218,7 @@ namespace {
 // into a row tile below 64 KB), and groups are sized for tiles, which take three to eight times the bytes of
 // scalar nodes.
 LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAutoScheduleOptions *ov,
-                            const DeviceLimits &limits, int tileSize) {
+                            const DeviceLimits &limits, int tileSize, bool peelWalks) {
   if (tileSize > 1) {
     const int64_t need = TiledGroupNeed(forest, tileSize);
     if (need > 65536)
@@ -436,10 +436,11 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // as many again to walk: one group and two 12708 rows x 89 trees in ten slices 10.8 -> 11.9 us, 16925 x 72 in seven 10.8 -> 11.5,
   // two and three 4814 x 193 in five 10.2 -> 11.3, 15744 x 80 in four 10.6 -> 10.9; three and four 11.8 and 11.5, 14.8 and 15.0,
   // five and six 19.8 -> 19.0, 14.9 -> 14.2, alike 13.2 -> 12.1.
-  if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)plan.groupBytes * (double)forest.trees.size() < fewInGroup * (double)totalBytes) {
+  plan.treeSlices = (int32_t)std::max<int64_t>(1, slices);
+  const int64_t inLds = !peelWalks && LeavesOutside(forest, plan) ? TreeBytesInLds(forest, true) : totalBytes; // (peeled walks keep all in LDS)
+  if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)plan.groupBytes * (double)forest.trees.size() < fewInGroup * (double)inLds) {
     LaunchPlan two = plan;
     two.interleave = 2;
-    two.treeSlices = (int32_t)std::max<int64_t>(1, slices);
     const auto turns = [&](const LaunchPlan &p) { return (CountTreeGroups(forest, p) + slices - 1) / slices; };
     if (slices == 1 || (forest.numClasses > 1 && PacksOwnClasses(forest, two)) || turns(two) * 2 < turns(plan) * 3) plan.interleave = 2;
   }
@@ -449,7 +450,7 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // features, 10 classes 103.7 and 60.7 us; 300 of depth 8, 54 features, 12 classes 177.1 and 137.8; 200 of depth 8, 70
   // features, 6 classes 132.8 and 105.9; 400 of depth 7, 90 features, 8 classes 195.4 and 152.3.
   if (forest.numClasses > 1 && plan.treeThreads > 1 && plan.interleave == 4 && !(ov && ov->treeWalkInterleaveFactor > 0) &&
-      (double)plan.groupBytes * (double)forest.trees.size() < (4.0 * std::min(plan.treeThreads, forest.numClasses) + 0.3) * (double)totalBytes) {
+      (double)plan.groupBytes * (double)forest.trees.size() < (4.0 * std::min(plan.treeThreads, forest.numClasses) + 0.3) * (double)inLds) {
     double levels = 0.0;
     for (const Tree &tree : forest.trees) levels += tree.Depth();
     levels /= (double)forest.trees.size();
@@ -457,10 +458,8 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     const double own = std::ceil(forest.numClasses / threads) * std::ceil(ofClass / 2) * 2 * levels;
     LaunchPlan two = plan;
     two.interleave = 2;
-    two.treeSlices = (int32_t)std::max<int64_t>(1, slices);
     if (own < forest.numClasses * (std::ceil(ofClass / (4 * threads)) * 4 * levels + 20.0) && PacksOwnClasses(forest, two)) plan.interleave = 2;
   }
-  plan.treeSlices = (int32_t)std::max<int64_t>(1, slices);
   return plan;
 }
 
