@@ -10,8 +10,10 @@
 //    run of 8-byte nodes that is copied verbatim into LDS, so every pointer a
 //    node holds is a byte address relative to the start of its group.
 //  * Node = { f32 value; u32 meta }.  value is the split threshold or, on a
-//    leaf, the prediction.  meta = (left-child byte address << 16) | feature
-//    offset.  The right child always follows the left one (+8 bytes).
+//    leaf, the prediction.  meta = (feature offset << 16) | left-child byte
+//    address (that way round: a 16-bit addition to the low half is cheaper on
+//    the device than one that selects the high half).  The right child always
+//    follows the left one (+8 bytes).
 //  * The feature offset is pre-multiplied for the transposed row tile the
 //    kernel keeps in LDS (feature-major, one column per row of the block), so
 //    the address of the feature value is `featureOffset + 4*rowSlot`.
@@ -100,9 +102,9 @@ struct DeviceNode {
   float value;
   uint32_t meta;
 };
-constexpr uint32_t NodeMeta(uint32_t child, uint32_t featureOffset) { return child << 16 | featureOffset; }
-constexpr uint32_t MetaChild(uint32_t meta) { return meta >> 16; }
-constexpr uint32_t MetaFeature(uint32_t meta) { return meta & 0xFFFFu; }
+constexpr uint32_t NodeMeta(uint32_t child, uint32_t featureOffset) { return featureOffset << 16 | child; }
+constexpr uint32_t MetaChild(uint32_t meta) { return meta & 0xFFFFu; }
+constexpr uint32_t MetaFeature(uint32_t meta) { return meta >> 16; }
 
 struct alignas(32) DeviceBundle {
   uint16_t root[kMaxInterleave]; // byte address of each tree's root inside the group

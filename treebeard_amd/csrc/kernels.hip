@@ -34,6 +34,14 @@ __device__ __forceinline__ uint32_t LdsLoadByte(uint32_t address) { return *(Lds
 typedef const __attribute__((address_space(3))) uint16_t *LdsHalfPtr;
 __device__ __forceinline__ uint32_t LdsLoadHalf(uint32_t address) { return *(LdsHalfPtr)(uintptr_t)address; }
 
+// A node's child pointer (the low half of its meta word) plus `more`: a 16-bit addition leaves the upper half of the result zero and
+// takes 2.6 cycles of a SIMD where one that selects a half (SDWA), a compare or a conditional move takes 4.3.
+__device__ __forceinline__ uint32_t AddChild(uint32_t meta, uint32_t more) {
+  uint32_t address;
+  asm("v_add_u16_e32 %0, %1, %2" : "=v"(address) : "v"(meta), "v"(more));
+  return address;
+}
+
 // How a node's 16-bit feature offset addresses the row tile of the row-parallel kernel.
 enum RowTileMode : int {
   kTileF32Bytes = 0, // f32 tile, offset in bytes
@@ -492,7 +500,7 @@ WalkRowBlock(unsigned char *lds, int64_t rowBlock, int gBegin, int gEnd, int sli
             bool left;
             if (IsRankTile(kMode)) left = RankGoesLeft<kMode>(column + off, node.x); // rank <= threshold index
             else left = LdsLoadFloat(column + off) < AsFloat(node.x);
-            addr[k] = MetaChild(node.y) + (left ? 0u : right);
+            addr[k] = AddChild(node.y, left ? 0u : right);
           }
         };
         constexpr int kFirstLevel = kMode != kTileRankU8 ? 1 : 0;
@@ -1032,7 +1040,7 @@ WalkTreeParallelKernel(const float *__restrict__ x, const uint4 *__restrict__ no
           for (int k = 0; k < K; ++k) {
             const U32x2 node = LdsLoadNode(addr[k]);
             const float xv = LdsLoadFloat(rowBase + MetaFeature(node.y));
-            addr[k] = MetaChild(node.y) + (xv < AsFloat(node.x) ? 0u : kNodeBytes);
+            addr[k] = AddChild(node.y, xv < AsFloat(node.x) ? 0u : kNodeBytes);
           }
         }
 #pragma unroll
