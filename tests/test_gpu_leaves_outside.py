@@ -60,11 +60,13 @@ def test_by_the_groups_it_saves(tmp_path, depths, split, outside):
         check_against_oracle(runner, model_io.load_xgboost_json(path), rows_for(20, rows))
 
 
-@pytest.mark.parametrize("classes,trees,own", [(8, 200, True), (5, 451, False)])
-def test_classes(tmp_path, classes, trees, own):
+@pytest.mark.parametrize("classes,trees,own,room", [(8, 200, True, 25088), (5, 451, False, 16896)])
+def test_classes(tmp_path, classes, trees, own, room):
+    """Tree threads with classes of their own leave their meeting place, 8 KB, to the groups."""
     depths = [6, 6, 5, 6, 3, 6, 0][:7] * (trees // 7 + 1)
     path = write_model(tmp_path / "m.json", 54, depths[:trees], 1.0, classes)
     runner = make_runner(path, 1 << 20)
-    assert " leavesOutside=1" in runner.describe_plan() and " ownClasses=%d " % own in runner.describe_plan(), runner.describe_plan()
+    plan = runner.describe_plan()
+    assert " leavesOutside=1" in plan and " ownClasses=%d " % own in plan and " groupBytes=%d " % room in plan, plan
     for rows in (2000, 66000):
         check_against_oracle(runner, model_io.load_xgboost_json(path), rows_for(54, rows))

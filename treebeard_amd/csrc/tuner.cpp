@@ -460,6 +460,13 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     two.interleave = 2;
     if (own < forest.numClasses * (std::ceil(ofClass / (4 * threads)) * 4 * levels + 20.0) && PacksOwnClasses(forest, two)) plan.interleave = 2;
   }
+  // Tree threads with classes of their own never meet: their place behind the rows goes to the groups (2^20 rows x 54 features, 800
+  // trees of depth 6, 8 classes: 25 groups and 17, 778 -> 741 us; 65537 rows with sums 81.6 -> 79.7).
+  if (meet > 0 && plan.groupBytes == (int32_t)(group & ~15)) {
+    LaunchPlan roomy = plan;
+    roomy.groupBytes = (int32_t)(std::min<int64_t>({group + meet, 65536, 256LL * plan.ThreadsPerBlock()}) & ~15);
+    if (PacksOwnClasses(forest, roomy)) plan = roomy;
+  }
   return plan;
 }
 
