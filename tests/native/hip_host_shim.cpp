@@ -727,7 +727,7 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
         DeviceStreamHead heads[2];
         std::memcpy(heads, p.words + begin, sizeof(heads));
         const uint32_t depth = heads[0].depth, words = heads[0].words;
-        if (heads[1].depth != depth || heads[1].words != words || words * 4 > kStreamBundleBytes) std::abort();
+        if (depth < 1 || heads[1].depth != depth || heads[1].words != words || words * 4 > kStreamBundleBytes) std::abort();
         if (b + 1 < p.numBundles && p.bundles[b + 1] != begin + words) std::abort();
         if (p.words[begin + kStreamBundleBytes / 4 - 1] == 0xFFFFFFFFu) std::abort(); // (the copy reads that far)
         for (int k = 0; k < 2 * p.chains; ++k) {
@@ -735,8 +735,10 @@ hipError_t LaunchRankStream(const RankStreamParams &p, hipStream_t stream) {
           if (root % 2) std::abort(); // (children are read two words at a time)
           uint32_t at = 0;
           for (uint32_t d = 0; d < depth; ++d) {
-            if (root + at >= words) std::abort(); // a node outside the bundle
-            const uint32_t node = p.words[begin + root + at], f = node >> 5 & 0x7FFu;
+            // a node outside the bundle's trees (the root is the head's; a leaf that is a tree has it as a word too)
+            if (d > 0 && (root + at < kStreamHeadWords || root + at >= words)) std::abort();
+            const uint32_t node = d > 0 ? p.words[begin + root + at] : heads[k & 1].rootWords[k / 2], f = node >> 5 & 0x7FFu;
+            if (d > 0 && at == 0 && node != heads[k & 1].rootWords[k / 2]) std::abort();
             if ((int)f > F || (node & 31u)) std::abort();
             const uint32_t rank = (int)f == F ? 0u : p.ranks[((row / 64) * F + f) * 64 + row % 64];
             at = 2 * (node >> 16 & 0xFFu) + (rank < node >> 24 ? 0u : 1u);

@@ -69,3 +69,23 @@ def test_workgroups_that_take_several_row_blocks(tmp_path, trees):
     assert counts
     for count in counts:
         close(forest, gpu_predict(runner, x[:count]), expected[:count])
+
+
+@pytest.mark.parametrize("depths", [[0] * 19 + [1] * 3 + [8], [1] * 9, [0] * 17 + [2], [8] * 5 + [0, 1, 2], [0] * 3 + [3] * 30])
+def test_bundles_of_the_smallest_trees(tmp_path, depths):
+    """Bundles that are walked no level, one and two: their trees' roots stand in the bundle's head, those that split only there."""
+    rng = np.random.Generator(np.random.PCG64(len(depths)))
+    features, levels = 600, 60
+    grid = np.sort(rng.standard_normal(levels)).astype(np.float32)
+    forest_trees = [synth._grow_tree(rng, depth, lambda d, s: 1.0, lambda: (rng.integers(0, features), grid[rng.integers(0, levels)]),
+                                     rng.normal, force_root=depth > 0) for depth in depths]
+    path = str(tmp_path / "small.json")
+    synth.write_xgboost_json(path, forest_trees, features)
+    forest = model_io.load_xgboost_json(path)
+    runner = make_runner(path, 20000)
+    rows = max(limit_of(runner), 2000) + 33
+    x = rng.standard_normal((rows, features), dtype=np.float32)
+    x[::3] = grid[rng.integers(0, levels, (len(x[::3]), features))]
+    x[rows - 1, :] = np.nan
+    x[rows - 2, :] = np.inf
+    close(forest, gpu_predict(runner, x), cpu_oracle.predict(forest, x)[0])

@@ -158,7 +158,8 @@ constexpr uint32_t kFewRowsLeaf = 0xFFFFu;
 
 // Rank-quantised rows of up to 2047 features, trees of up to 255 splits: 4-byte nodes that a wave streams through LDS of
 // its own.  node = test << 24 | child pair << 16 | feature << 5: a row whose rank is below `test` (threshold index + 1)
-// goes to word 2 * pair of the tree, the others to word 2 * pair + 1; word 0 is the root, word 1 unused.  A leaf holds
+// goes to word 2 * pair of the tree, the others to word 2 * pair + 1; word 0 is the root, word 1 unused: the bundle's head
+// holds the root, and only a tree that is one leaf has the two.  A leaf holds
 // its place: as a left child it tests the pad feature (rank 0) against 1, as a right child anything against 0.  The
 // leaves a walk of the bundle's depth reaches with its last step are never read as nodes: they have no words.
 // Predictions stand in an array of their own, one place per word (the last leaves' included).
@@ -166,12 +167,13 @@ constexpr uint32_t kFewRowsLeaf = 0xFFFFu;
 // A bundle's image begins with a DeviceStreamHead for each half of the wave that walks it, then the trees; it starts on a
 // 16-byte piece and the copy takes kStreamBundleBytes whatever its size (the words end with as many that belong to none).
 struct alignas(16) DeviceStreamHead {
-  uint16_t roots[4];      // byte offsets of the half's trees in the image
-  uint32_t depth;         // of the deepest tree of the bundle
+  uint16_t roots[4];      // byte offsets of the half's trees in the image (of their word 0, which may lie in front of their words)
+  uint32_t depth;         // of the deepest tree of the bundle, at least 1
   uint32_t words;         // of the image (what reads it on the host checks against)
+  uint32_t rootWords[4];  // word 0 of every tree
   uint32_t valueBegin[4]; // of every tree, in the array of predictions (entry 0 is 0.0: the empty places')
 };
-static_assert(sizeof(DeviceStreamHead) == 32, "two 16-byte LDS reads");
+static_assert(sizeof(DeviceStreamHead) == 48, "three 16-byte LDS reads");
 constexpr uint32_t kStreamHeadWords = 2 * sizeof(DeviceStreamHead) / 4;
 constexpr int kStreamMaxChains = 4;          // trees a lane walks side by side (2 or 4); two lanes share a bundle's trees
 constexpr uint32_t kStreamBundleBytes = 4096;

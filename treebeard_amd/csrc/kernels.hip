@@ -1660,6 +1660,13 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
     FinishClasses([&](int c) { return sums[r * Cn + c]; }, Cn, row0 + r, p.out, p.classOut, p.margins, p.probabilities);
 }
 
+// Address of the two children of a stream's word: the pair's index is the word's third byte, eight bytes a pair, from `tree` on.
+// (A sum of four byte products and the third operand: one instruction for the two
+// that pick the byte and add it: 262144 rows x 2000 features, 1000 trees 1226 -> 1190 us.)
+__device__ __forceinline__ uint32_t StreamChildren(uint32_t word, uint32_t tree) {
+  return __builtin_amdgcn_udot4(word, 0x00080000u, tree, false);
+}
+
 // ---------------------------------------------------------------------------
 // Wide rows, rank-quantised: a block keeps 32 rows of one byte per feature in LDS (64 KB at 2000 features) and every
 // wave streams its own bundles of eight trees through 8 KB of its own, two bundles deep: while one is walked the next is
@@ -1672,12 +1679,13 @@ __global__ void __launch_bounds__(1024) FewRowsKernel(const FewRowsParams p, int
 //
 // With three waves a SIMD every wait in a wave's chain is seen.  So: the lane holds the word it stands on and reads both
 // children (8 bytes side by side, at the price of 4) together with the rank, one LDS round trip a level instead of two; a
-// bundle's roots and depth stand in its image, its place comes through a vector load (a scalar load took its latency every
-// bundle); and a workgroup stays, with the next rows' ranks on their way to registers while its last bundle is walked (it
-// has its compute unit's LDS to itself: nothing else walks while it loads).  Walk of 262144 rows x 2000 features, 1000 trees
-// of depth 8, on the same ranks, traced: 1.33 ms with tree groups, 0.80 with two trips a level and a workgroup per 32 rows, 0.73
-// here (LDS pipes 52 % busy, a quarter of that conflicts of the rank reads, VALUs 58 %), and the whole call 1.308 -> 1.223; 20000
-// rows 126 -> 120 us.
+// bundle's depth and its trees' roots stand in the head of its image, its place comes through a vector load (a scalar load took
+// its latency every bundle); chains ask for their next level two by two, while the other two's reads are on their way; and a
+// workgroup stays, with the next rows' ranks on their way to registers while its last bundle is walked (it
+// has its compute unit's LDS to itself: nothing else walks while it loads).  Whole calls of 262144 rows x 2000 features, 1000
+// trees of depth 8: 1308 us with two trips a level and a workgroup per 32 rows, 1223 with one trip and workgroups that stay, 1190
+// with one instruction to a child's address (StreamChildren), 1152 with the roots in the heads and chains that wait for their
+// own reads only, 1131 with chains two by two (fewer instructions between the waits and the next reads); all four at once 1190.
 // ---------------------------------------------------------------------------
 // kStays: workgroups go on with other rows.  Where none does, what that takes (76 VGPRs and 1700 bytes of code) is left out: 3644
 // rows x 167 trees of 896 features 16.8 -> 16.2 us, 5504 x 92 of 1401 21.7 -> 21.2, 7713 x 46 of 672 15.2 -> 14.5.
@@ -1772,42 +1780,52 @@ RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__
       if (b + waves < last || more) TBAMD_STREAM_BUNDLE(follows, other)
       nextBegin = bundles[(uint32_t)after(after(b)) + zero];
       if (b + waves >= last && more) TBAMD_STREAM_NEXT_ROWS
-      const U32x4 head = LdsLoadQuad(buffer + (upper ? (uint32_t)sizeof(DeviceStreamHead) : 0u));
-      const U32x4 valueBegin = LdsLoadQuad(buffer + (upper ? (uint32_t)sizeof(DeviceStreamHead) : 0u) + 16u);
+      const uint32_t headAt = buffer + (upper ? (uint32_t)sizeof(DeviceStreamHead) : 0u);
+      const U32x4 head = LdsLoadQuad(headAt), rootWords = LdsLoadQuad(headAt + 16u), valueBegin = LdsLoadQuad(headAt + 32u);
       const int depth = (int)__builtin_amdgcn_readfirstlane(head.z);
       uint32_t tree[K], node[K]; // where the words of a tree lie, and the word the lane stands on
 #pragma unroll
       for (int k = 0; k < K; ++k) {
         tree[k] = buffer + (k & 1 ? head[k / 2] >> 16 : head[k / 2] & 0xFFFFu);
-        node[k] = *(const __attribute__((address_space(3))) uint32_t *)(uintptr_t)tree[k];
+        node[k] = rootWords[k];
       }
-      // (awaited here: in the loop the compiler would wait for them, and so for other chains' reads, at every level)
+      // Two chains ask for their next level as soon as their own reads are there, the others' still on their way.  (Left to itself
+      // the compiler waits for all chains before the first compares, and reads one child, when the rank is there.)
+      U32x2 children[K];
+      uint32_t rank[K];
+      const auto ask = [&](int k, bool both) {
+        rank[k] = LdsLoadByte(AddChild(node[k], row));
+        if (both) children[k] = LdsLoadNode(StreamChildren(node[k], tree[k]));
+      };
+      const auto step = [&](int k) {
+        asm volatile("" : "+v"(rank[k]), "+v"(children[k]));
+        node[k] = rank[k] < (node[k] >> 24) ? children[k].x : children[k].y;
+      };
+      if (depth > 1) {
 #pragma unroll
-      for (int k = 0; k < K; ++k) asm volatile("" : "+v"(node[k]));
-#pragma unroll 2
-      for (int d = 1; d < depth; ++d) {
-        U32x2 children[K];
-        uint32_t rank[K];
+        for (int k = 0; k < K; ++k) ask(k, true);
+        for (int d = 2; d < depth; ++d) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
-          rank[k] = LdsLoadByte((node[k] & 0xFFE0u) | row);
-          children[k] = LdsLoadNode((((node[k] >> 16) & 0xFFu) << 3) + tree[k]);
+          for (int k = 0; k < K; k += 2) {
+            __builtin_amdgcn_sched_barrier(0);
+            step(k);
+            step(k + 1);
+            ask(k, true);
+            ask(k + 1, true);
+          }
         }
 #pragma unroll
         for (int k = 0; k < K; ++k) {
-          // (both children are read: left to itself the compiler reads one, when the rank is there)
-          asm volatile("" : "+v"(rank[k]), "+v"(children[k]));
-          node[k] = rank[k] < (node[k] >> 24) ? children[k].x : children[k].y;
+          __builtin_amdgcn_sched_barrier(0);
+          step(k);
+          ask(k, false); // (the last level's words are not there: only which they are counts)
         }
+      } else {
+#pragma unroll
+        for (int k = 0; k < K; ++k) ask(k, false);
       }
-      uint32_t rank[K]; // (the last level's words are not there: only which they are counts)
 #pragma unroll
-      for (int k = 0; k < K; ++k) rank[k] = LdsLoadByte((node[k] & 0xFFE0u) | row);
-#pragma unroll
-      for (int k = 0; k < K; ++k) asm volatile("" : "+v"(rank[k]));
-#pragma unroll
-      for (int k = 0; k < K; ++k)
-        at[k] = valueBegin[k] + (depth > 0 ? ((node[k] >> 15) & 0x1FEu) + (rank[k] < (node[k] >> 24) ? 0u : 1u) : 0u);
+      for (int k = 0; k < K; ++k) at[k] = valueBegin[k] + ((node[k] >> 15) & 0x1FEu) + (rank[k] < (node[k] >> 24) ? 0u : 1u);
       buffer = other;
     }
 #pragma unroll

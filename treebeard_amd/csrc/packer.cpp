@@ -448,7 +448,7 @@ RankStreamModel PackRankStream(const Forest &input) {
                                                 : forest.trees[(size_t)a].NumNodes() < forest.trees[(size_t)b].NumNodes();
   });
   auto leafWord = [&](uint32_t pair, bool right) { return (right ? 0u : 1u << 24) | pair << 16 | (uint32_t)forest.numFeatures << 5; };
-  // words of a tree's image in a bundle of `deepest` levels: the children of level deepest - 1 have none
+  // words of a tree's image in a bundle of `deepest` levels: the children of level deepest - 1 have none, nor has a root that splits
   auto wordsOf = [&](int32_t t, int32_t deepest) {
     const Tree &tree = forest.trees[(size_t)t];
     std::vector<int32_t> level{0};
@@ -460,7 +460,7 @@ RankStreamModel PackRankStream(const Forest &input) {
       words += (uint32_t)below.size();
       level.swap(below);
     }
-    return words;
+    return tree.IsLeaf(0) ? words : words - 2;
   };
   auto pack = [&](int32_t chains) {
     sm = RankStreamModel();
@@ -475,11 +475,12 @@ RankStreamModel PackRankStream(const Forest &input) {
         if (words * 4 > kStreamBundleBytes && n > 1) break; // (a tree alone always fits)
         count = n;
       }
-      const int32_t deepest = depth[(size_t)order[next + count - 1]];
+      const int32_t deepest = std::max(1, depth[(size_t)order[next + count - 1]]);
       const uint32_t begin = (uint32_t)sm.words.size();
       DeviceStreamHead heads[2]{};
       for (DeviceStreamHead &head : heads) {
         for (uint16_t &root : head.roots) root = kStreamHeadWords * 4; // (the empty tree)
+        for (uint32_t &word : head.rootWords) word = leafWord(0, false);
         head.depth = (uint32_t)deepest;
       }
       sm.words.resize(begin + kStreamHeadWords);
@@ -487,11 +488,11 @@ RankStreamModel PackRankStream(const Forest &input) {
       for (size_t k = 0; k < count; ++k) {
         const int32_t t = order[next + k];
         const Tree &tree = forest.trees[(size_t)t];
-        const size_t at = sm.words.size(), valueAt = sm.values.size();
-        const uint32_t limit = wordsOf(t, deepest);
+        const uint32_t own = wordsOf(t, deepest), inHead = tree.IsLeaf(0) ? 0u : 2u, limit = own + inHead;
+        const size_t at = sm.words.size() - inHead, valueAt = sm.values.size(); // (words 0 and 1 of a root that splits: the head's)
         heads[k & 1].roots[k / 2] = (uint16_t)((at - begin) * 4);
         heads[k & 1].valueBegin[k / 2] = (uint32_t)valueAt;
-        sm.words.resize(at + limit, 0u);
+        sm.words.resize(sm.words.size() + own, 0u);
         sm.values.resize(valueAt + tree.NumNodes() + 1, 0.0f);
         struct Place { int32_t node; uint32_t word; };
         std::vector<Place> queue{{0, 0}};
@@ -500,13 +501,15 @@ RankStreamModel PackRankStream(const Forest &input) {
           const auto [n, word] = queue[head];
           if (tree.IsLeaf(n)) {
             if (word < limit) sm.words[at + word] = leafWord(word / 2, word & 1u);
+            if (word == 0) heads[k & 1].rootWords[k / 2] = leafWord(0, false);
             sm.values[valueAt + word] = tree.value[(size_t)n];
             continue;
           }
           const auto &sorted = ranks[(size_t)tree.feature[(size_t)n]];
           const uint32_t test = (uint32_t)(std::lower_bound(sorted.begin(), sorted.end(), tree.value[(size_t)n]) - sorted.begin()) + 1;
           if (word >= limit) throw Error("internal error: a split without a word");
-          sm.words[at + word] = test << 24 | pairs << 16 | (uint32_t)tree.feature[(size_t)n] << 5;
+          (word == 0 ? heads[k & 1].rootWords[k / 2] : sm.words[at + word]) =
+              test << 24 | pairs << 16 | (uint32_t)tree.feature[(size_t)n] << 5;
           queue.push_back({tree.left[(size_t)n], 2 * pairs});
           queue.push_back({tree.right[(size_t)n], 2 * pairs + 1});
           ++pairs;
