@@ -1685,7 +1685,8 @@ __device__ __forceinline__ uint32_t StreamChildren(uint32_t word, uint32_t tree)
 // has its compute unit's LDS to itself: nothing else walks while it loads).  Whole calls of 262144 rows x 2000 features, 1000
 // trees of depth 8: 1308 us with two trips a level and a workgroup per 32 rows, 1223 with one trip and workgroups that stay, 1190
 // with one instruction to a child's address (StreamChildren), 1152 with the roots in the heads and chains that wait for their
-// own reads only, 1131 with chains two by two (fewer instructions between the waits and the next reads); all four at once 1190.
+// own reads only, 1131 with chains two by two (fewer instructions between the waits and the next reads; all four at once 1190), 1114 with
+// their compares and addresses ordered so that no instruction waits for the one before.
 // ---------------------------------------------------------------------------
 // kStays: workgroups go on with other rows.  Where none does, what that takes (76 VGPRs and 1700 bytes of code) is left out: 3644
 // rows x 167 trees of 896 features 16.8 -> 16.2 us, 5504 x 92 of 1401 21.7 -> 21.2, 7713 x 46 of 672 15.2 -> 14.5.
@@ -1794,35 +1795,51 @@ RankStreamKernel(const uint8_t *__restrict__ ranks, const uint32_t *__restrict__
       U32x2 children[K];
       uint32_t rank[K];
       const auto ask = [&](int k, bool both) {
-        rank[k] = LdsLoadByte(AddChild(node[k], row));
-        if (both) children[k] = LdsLoadNode(StreamChildren(node[k], tree[k]));
+        uint32_t below[2], at[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+          below[i] = both ? StreamChildren(node[k + i], tree[k + i]) : 0u;
+          at[i] = AddChild(node[k + i], row);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) rank[k + i] = LdsLoadByte(at[i]);
+        if (both) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i) children[k + i] = LdsLoadNode(below[i]);
+        }
       };
       const auto step = [&](int k) {
-        asm volatile("" : "+v"(rank[k]), "+v"(children[k]));
-        node[k] = rank[k] < (node[k] >> 24) ? children[k].x : children[k].y;
+        uint64_t second; // (a mask may be read two instructions after it is written: the second compare stands in the first one's wait)
+        asm("v_cmp_lt_u32_sdwa vcc, %3, %0 src0_sel:DWORD src1_sel:BYTE_3\n\t"
+            "v_cmp_lt_u32_sdwa %2, %4, %1 src0_sel:DWORD src1_sel:BYTE_3\n\t"
+            "s_nop 0\n\t"
+            "v_cndmask_b32_e32 %0, %6, %5, vcc\n\t"
+            "v_cndmask_b32_e64 %1, %8, %7, %2"
+            : "+&v"(node[k]), "+&v"(node[k + 1]), "=&s"(second)
+            : "v"(rank[k]), "v"(rank[k + 1]), "v"(children[k].x), "v"(children[k].y), "v"(children[k + 1].x), "v"(children[k + 1].y)
+            : "vcc");
       };
       if (depth > 1) {
 #pragma unroll
-        for (int k = 0; k < K; ++k) ask(k, true);
+        for (int k = 0; k < K; k += 2) ask(k, true);
         for (int d = 2; d < depth; ++d) {
 #pragma unroll
           for (int k = 0; k < K; k += 2) {
             __builtin_amdgcn_sched_barrier(0);
             step(k);
-            step(k + 1);
             ask(k, true);
-            ask(k + 1, true);
           }
         }
 #pragma unroll
-        for (int k = 0; k < K; ++k) {
+        for (int k = 0; k < K; k += 2) {
           __builtin_amdgcn_sched_barrier(0);
           step(k);
           ask(k, false); // (the last level's words are not there: only which they are counts)
         }
       } else {
 #pragma unroll
-        for (int k = 0; k < K; ++k) ask(k, false);
+        for (int k = 0; k < K; k += 2) ask(k, false);
       }
 #pragma unroll
       for (int k = 0; k < K; ++k) at[k] = valueBegin[k] + ((node[k] >> 15) & 0x1FEu) + (rank[k] < (node[k] >> 24) ? 0u : 1u);
