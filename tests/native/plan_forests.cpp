@@ -273,6 +273,28 @@ static void TwoTreesOfSlices() {
   EXPECT(two > 0 && kept > 0, "%ld, %ld", two, kept);
 }
 
+// Numbers of features that files can hold: too many for any row in LDS, and the last ones that can be counted.
+static void MostFeatures() {
+  const DeviceLimits limits;
+  const int32_t last = std::numeric_limits<int32_t>::max();
+  for (int32_t features : {16384, 65536, 1 << 24, last - 3, last - 2, last - 1, last}) {
+    Forest forest = ForestOf(100, 4, 63);
+    forest.numFeatures = features;
+    bool valid = true;
+    try {
+      forest.Validate();
+    } catch (const Error &) {
+      valid = false;
+    }
+    EXPECT(valid == (features <= last - 2), "%d features", features);
+    if (!valid) continue;
+    for (int64_t batch : {1, 1000, 1 << 20}) {
+      const LaunchPlan plan = ChoosePlan(forest, batch, nullptr, limits);
+      EXPECT(plan.kernel == LaunchPlan::Kernel::kGlobalWalk && PackForest(forest, plan).globalTrees.size() == 4, "%d features, %lld rows", features, (long long)batch);
+    }
+  }
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
@@ -283,6 +305,7 @@ int main(int argc, char **argv) {
   if (asked("small_batches")) SmallBatches();
   if (asked("two_trees_of_classes")) TwoTreesOfClasses();
   if (asked("two_trees_of_slices")) TwoTreesOfSlices();
+  if (asked("most_features")) MostFeatures();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

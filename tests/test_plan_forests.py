@@ -58,3 +58,7 @@ def test_two_trees_side_by_side_of_classifiers(driver):
 
 def test_two_trees_side_by_side_of_sliced_forests(driver):
     run(driver, "two_trees_of_slices")
+
+
+def test_as_many_features_as_can_be_counted(driver):
+    run(driver, "most_features")

@@ -1,6 +1,7 @@
 #include "forest.h"
 
 #include <cmath>
+#include <limits>
 
 namespace tbamd {
 
@@ -54,6 +55,7 @@ void Tree::Validate(int32_t numFeatures, size_t treeIndex) const {
 
 void Forest::Validate() const {
   if (numFeatures <= 0) throw Error("model has no features");
+  if (numFeatures > std::numeric_limits<int32_t>::max() - 2) throw Error("model has too many features"); // (a pad feature and its pair are counted behind them)
   if (numClasses < 0 || numClasses > 127) throw Error("unsupported number of classes");
   for (size_t t = 0; t < trees.size(); ++t) {
     trees[t].Validate(numFeatures, t);
