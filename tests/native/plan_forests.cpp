@@ -295,6 +295,55 @@ static void MostFeatures() {
   }
 }
 
+// Classifiers under every order that a profile gives their trees: what the planner took to be the tree threads' own classes may meet
+// after all, and then finds its room, two blocks to a compute unit where the plan was made for two.
+static void RoomOfOwnClasses() {
+  const DeviceLimits limits;
+  uint64_t state = 1;
+  const auto pick = [&](int32_t low, int32_t high) {
+    state = state * 6364136223846793005ull + 1442695040888963407ull;
+    return low + (int32_t)((state >> 33) % (uint64_t)(high - low + 1));
+  };
+  long roomy = 0, meet = 0;
+  for (int32_t i = 0; i < 400; ++i) {
+    const bool wide = i % 2; // (one block per compute unit, and two)
+    const int32_t features = wide ? pick(380, 520) : pick(20, 110), classes = wide ? pick(10, 16) : pick(3, 9), trees = pick(40, 110);
+    Forest forest = ForestOf(features, trees, 3);
+    forest.numClasses = classes;
+    HitCountProfile profile;
+    profile.numRows = 1000;
+    const int32_t biggest = wide ? pick(190, 255) : pick(330, 511);
+    for (int32_t t = 0; t < trees; ++t) { // of one depth and many sizes, which the profile brings into order
+      Tree &tree = forest.trees[(size_t)t] = FullTree(pick(wide ? 131 : 257, biggest) / 2 * 2 + 1, features);
+      tree.classId = t % classes;
+      std::vector<int64_t> hits(tree.NumNodes(), 0);
+      hits[0] = profile.numRows;
+      const bool big = (int32_t)tree.NumNodes() * 4 > biggest * 3;
+      for (size_t n = 0; n < tree.NumNodes(); ++n)
+        if (!tree.IsLeaf((int32_t)n)) {
+          hits[(size_t)tree.left[n]] = big ? 0 : hits[n]; // (the deeper side)
+          hits[(size_t)tree.right[n]] = big ? hits[n] : 0;
+        }
+      profile.hits.push_back(hits);
+    }
+    const int64_t batch = pick(2000, 600000);
+    WalkOptions walk;
+    walk.peelWalks = true;
+    LaunchPlan later = ChoosePlan(forest, batch, nullptr, limits);
+    const PackedModel plain = PackForest(forest, later);
+    later.peelWalks = true; // (asked for when the runner is there)
+    for (const LaunchPlan &plan : {ChoosePlan(forest, batch, nullptr, limits, walk), later}) {
+      if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.quantizedRows) continue;
+      const PackedModel pm = PackForest(forest, plan, &profile);
+      EXPECT(pm.LdsBytes() <= (size_t)limits.ldsBytesPerBlock && (plain.LdsBytes() * 2 > (size_t)limits.ldsBytesPerBlock || pm.LdsBytes() * 2 <= (size_t)limits.ldsBytesPerBlock),
+             "%d features, %d classes, %d trees, %lld rows: %zu and %zu bytes of LDS, own classes %d and %d", features, classes, trees, (long long)batch,
+             plain.LdsBytes(), pm.LdsBytes(), plain.ownClasses, pm.ownClasses);
+      if (plain.ownClasses && plan.ownGroupBytes > 0 && plain.groupBytes == plan.ownGroupBytes) ++(pm.ownClasses ? roomy : meet);
+    }
+  }
+  EXPECT(roomy > 0 && meet > 0, "%ld, %ld", roomy, meet);
+}
+
 int main(int argc, char **argv) {
   const auto asked = [&](const char *name) { return argc < 2 || std::strcmp(argv[1], name) == 0; };
   if (asked("big_trees")) BigTrees();
@@ -306,6 +355,7 @@ int main(int argc, char **argv) {
   if (asked("two_trees_of_classes")) TwoTreesOfClasses();
   if (asked("two_trees_of_slices")) TwoTreesOfSlices();
   if (asked("most_features")) MostFeatures();
+  if (asked("room_of_own_classes")) RoomOfOwnClasses();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

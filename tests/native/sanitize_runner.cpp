@@ -558,6 +558,52 @@ static int MutatedCompiledModels(const char *path, int iterations) {
   return gFailures;
 }
 
+// A classifier whose tree threads' own classes leave their meeting place to the groups: shapes in which they meet again, pinned with
+// the group size kept, find that place free - straight away, from a compiled-model file, and with the fields of an older file.
+void KeptGroupSize(const Case &c) {
+  const auto field = [](const std::string &text, const char *name) {
+    const size_t at = text.find(std::string(" ") + name + "=");
+    return at == std::string::npos ? -1 : std::atoi(text.c_str() + at + std::strlen(name) + 2);
+  };
+  const std::string file = std::string(std::getenv("TMPDIR") ? std::getenv("TMPDIR") : "/tmp") + "/kept_group_size.tbamd";
+  std::vector<float> out((size_t)c.rows);
+  int meet = 0, own = 0;
+  for (int from = 0; from < 3; ++from) {
+    intptr_t runner = MakeRunner(c, 40731, false);
+    const std::string chosen = Describe(runner);
+    const int threads = field(chosen, "treeThreads"), group = field(chosen, "groupBytes");
+    if (from > 0) {
+      EXPECT(tbmi_save_compiled_model(runner, file.c_str()) == 0, "tbmi_save_compiled_model");
+      DeleteInferenceRunner(runner);
+      if (from == 2) { // version 5: 14 words of plan behind 48 bytes
+        std::ifstream in(file, std::ios::binary);
+        std::string bytes((std::istreambuf_iterator<char>(in)), std::istreambuf_iterator<char>());
+        in.close();
+        bytes[8] = 5;
+        bytes.erase(48 + 14 * 4, 4);
+        std::ofstream(file, std::ios::binary) << bytes;
+      }
+      runner = tbmi_load_compiled_model(file.c_str(), 0);
+      EXPECT(runner != 0, "tbmi_load_compiled_model");
+      const std::string loaded = Describe(runner);
+      EXPECT((loaded == chosen) == (from == 1) && field(loaded, "groupBytes") <= group, "%s\n%s", chosen.c_str(), loaded.c_str());
+    }
+    for (int k : {1, 2, 4, 8})
+      for (int slices : {1, 4}) {
+        EXPECT(tbmi_set_plan(runner, 0, threads, k, 0, slices) == 0, "interleave %d, %d slices", k, slices);
+        const std::string plan = Describe(runner);
+        ++(field(plan, "ownClasses") ? own : meet);
+        EXPECT(field(plan, "interleave") == k && field(plan, "ldsBytes") <= 160 * 1024, "%s", plan.c_str());
+        EXPECT(tbmi_run_host(runner, c.x.data(), out.data(), c.rows) == 0, "tbmi_run_host");
+        Compare(c, out.data(), 0, c.rows, "a plan of another interleave");
+      }
+    // a size that the caller names is kept whoever the classes are
+    EXPECT(tbmi_set_plan(runner, 0, threads, 2, 16384, 1) == 0 && field(Describe(runner), "groupBytes") == 16384, "%s", Describe(runner).c_str());
+    DeleteInferenceRunner(runner);
+  }
+  EXPECT(meet > 0 && own > 0, "%d plans with classes that meet, %d without", meet, own);
+}
+
 int main(int argc, char **argv) {
   // argv: pairs of <model.json> <rows>, or --mutate <compiled model> <iterations>
   if (argc == 4 && std::strcmp(argv[1], "--mutate") == 0) {
@@ -580,6 +626,10 @@ int main(int argc, char **argv) {
     for (int64_t r = 0; r < c.rows; ++r) c.expected[r] = Predict(c.forest, c.x.data() + r * F, nullptr);
     if (std::getenv("SANITIZE_NOALLOC")) {
       NoAllocOfManySums(c);
+      continue;
+    }
+    if (std::getenv("SANITIZE_SHAPES")) {
+      KeptGroupSize(c);
       continue;
     }
     HostEntryPoints(c);

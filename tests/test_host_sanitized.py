@@ -213,6 +213,21 @@ def test_no_alloc_calls_of_many_class_sums(tmp_path, address_driver):
 
 
 @pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_plans_of_classes_with_the_group_size_kept(tmp_path, address_driver):
+    """65 trees of depth 9 voting for 7 classes over 463 features: one block per compute unit, whose LDS the row tile and the tree
+    groups fill while the classes are the tree threads' own."""
+    import numpy as np
+    rng = np.random.Generator(np.random.PCG64(12))
+    trees = [synth._grow_tree(rng, 9, lambda d, s: 0.8, lambda: (rng.integers(0, 463), rng.normal()), lambda: rng.normal(0.0, 0.1))
+             for _ in range(65)]
+    path = str(tmp_path / "classes463.json")
+    synth.write_xgboost_json(path, trees, 463, objective="multi:softmax", num_class=7, tree_info=[t % 7 for t in range(65)])
+    env = dict(os.environ, SANITIZE_SHAPES="1", ASAN_OPTIONS="detect_leaks=1:abort_on_error=0", TMPDIR=str(tmp_path))
+    run = subprocess.run([address_driver, path, "70"], capture_output=True, text=True, env=env, timeout=600)
+    assert run.returncode == 0, (run.stdout + run.stderr)[-4000:]
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
 def test_runner_survives_mutated_compiled_models(tmp_path, synth_model, address_driver):
     """tbmi_load_compiled_model on compiled-model files whose header words (plan, batch size, return type, counts) and
     body were overwritten: refused with a message or loaded and run on a few rows, under ASan + UBSan."""

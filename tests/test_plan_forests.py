@@ -62,3 +62,7 @@ def test_two_trees_side_by_side_of_sliced_forests(driver):
 
 def test_as_many_features_as_can_be_counted(driver):
     run(driver, "most_features")
+
+
+def test_room_that_own_classes_leave(driver):
+    run(driver, "room_of_own_classes")

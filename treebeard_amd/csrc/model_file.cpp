@@ -21,7 +21,7 @@ namespace tbamd {
 namespace {
 
 constexpr char kMagic[8] = {'T', 'B', 'A', 'M', 'D', 'M', 'D', 'L'};
-constexpr uint32_t kVersion = 5;
+constexpr uint32_t kVersion = 6, kVersionWithoutOwnGroups = 5; // (the older one ends its plan at deferTails)
 
 struct Writer {
   std::string bytes;
@@ -81,6 +81,7 @@ void SaveCompiledModel(const std::string &path, const Forest &forest, const Laun
   w.Put<int32_t>(plan.tiling);
   w.Put<int32_t>(plan.peelWalks ? 1 : 0);
   w.Put<int32_t>(plan.deferTails ? 1 : 0);
+  w.Put<int32_t>(plan.ownGroupBytes);
   w.Put<uint64_t>(forest.trees.size());
   for (const Tree &t : forest.trees) {
     w.Put<int32_t>(t.classId);
@@ -103,7 +104,8 @@ CompiledModel LoadCompiledModel(const std::string &path) {
   if (bytes.size() < sizeof(kMagic) || std::memcmp(bytes.data(), kMagic, sizeof(kMagic)) != 0)
     throw Error(path + " is not a compiled model file");
   Reader r{bytes, sizeof(kMagic)};
-  if (r.Get<uint32_t>() != kVersion) throw Error("unsupported compiled model version");
+  const uint32_t version = r.Get<uint32_t>();
+  if (version != kVersion && version != kVersionWithoutOwnGroups) throw Error("unsupported compiled model version");
   CompiledModel m;
   m.batchSize = r.Get<int32_t>();
   m.returnTypeWidth = r.Get<int32_t>();
@@ -127,6 +129,7 @@ CompiledModel LoadCompiledModel(const std::string &path) {
   m.plan.tiling = r.Get<int32_t>();
   m.plan.peelWalks = r.Get<int32_t>() != 0;
   m.plan.deferTails = r.Get<int32_t>() != 0;
+  if (version != kVersionWithoutOwnGroups) m.plan.ownGroupBytes = r.Get<int32_t>();
   const uint64_t trees = r.Get<uint64_t>();
   if (trees > (bytes.size() - r.pos) / 36) throw Error("model file is truncated"); // (a tree takes 36 bytes at least)
   m.forest.trees.resize(trees);

@@ -643,6 +643,13 @@ std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &pl
 }
 
 namespace {
+// The plan with the group sizes that PackForest tries, in that order: the first only if it makes classes the tree threads' own.
+std::vector<LaunchPlan> GroupSizes(const LaunchPlan &plan) {
+  std::vector<LaunchPlan> tried(plan.ownGroupBytes > 0 ? 2 : 1, plan);
+  if (plan.ownGroupBytes > 0) tried[0].groupBytes = plan.ownGroupBytes;
+  return tried;
+}
+
 // What PackForest goes by of a scalar plan without a profile: the trees' depths and sizes, in its order.
 struct PlainTrees {
   std::vector<int32_t> depth, order;
@@ -664,9 +671,12 @@ struct PlainTrees {
 } // namespace
 
 bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan) {
-  const PlainTrees trees(forest, plan);
-  std::vector<std::vector<int32_t>> rounds;
-  return OwnClassRounds(forest, plan, trees.depth, trees.units, trees.order, &rounds);
+  for (const LaunchPlan &tried : GroupSizes(plan)) {
+    const PlainTrees trees(forest, tried);
+    std::vector<std::vector<int32_t>> rounds;
+    if (OwnClassRounds(forest, tried, trees.depth, trees.units, trees.order, &rounds)) return true;
+  }
+  return false;
 }
 
 int64_t TreeBytesInLds(const Forest &forest, bool leavesOutside) {
@@ -800,7 +810,8 @@ std::vector<BundleTrees> LayOutGroups(const Forest &forest, const LaunchPlan &pl
 
 constexpr uint32_t kPeeledTailNodes = 1u << 20; // below the cuts of a plan with a profile (8 MB: they stay in the caches)
 
-PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCountProfile *profile, const std::vector<int32_t> *cuts) {
+PackedModel PackPlan(const Forest &input, const LaunchPlan &asked, const HitCountProfile *profile, const std::vector<int32_t> *cuts) {
+  LaunchPlan plan = asked; // (of its groups' two sizes the one that is taken, once that is known)
   // Plans also come out of files: every field is brought into its range before anything is computed from it.
   if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds && plan.kernel != LaunchPlan::Kernel::kTreeParallel &&
       plan.kernel != LaunchPlan::Kernel::kGlobalWalk)
@@ -832,6 +843,9 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
   if (plan.groupBytes > 256 * plan.ThreadsPerBlock())
     throw Error("groupBytes must not exceed 256 bytes per lane of the block (group prefetch registers)");
   if (plan.groupBytes < 1024 || plan.groupBytes > 65536) throw Error("groupBytes must be in [1024, 65536]");
+  if (plan.ownGroupBytes != 0 && (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || forest.numClasses < 2 || plan.ownGroupBytes < plan.groupBytes ||
+                                  plan.ownGroupBytes > std::min(65536, 256 * plan.ThreadsPerBlock())))
+    throw Error("launch plan: groups of the tree threads' own classes are no smaller than others and keep their limits");
 
   if (plan.quantizedRows && (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.rowsPerBlock != 64))
     throw Error("rank-quantised rows need the row-parallel kernel with 64 rows per block");
@@ -850,11 +864,10 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     throw Error("tile sizes above 1 need a row tile below 64 KB (tiles hold byte offsets): fewer rows per block");
 
   PackedModel pm;
-  pm.plan = plan;
+  pm.plan = asked;
   pm.numFeatures = forest.numFeatures;
   pm.numClasses = forest.numClasses;
   pm.numTrees = (int32_t)forest.trees.size();
-  pm.leavesOutside = LeavesOutside(forest, plan);
   if (plan.deferTails) { // tail node 0: a leaf of value 0, what a lane without a queue entry walks
     pm.tailNodes.push_back(DeviceNode{0.0f, (0u << kTailFeatureBits) | (uint32_t)forest.numFeatures});
     pm.tailOrigin.push_back(-1);
@@ -864,7 +877,6 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     throw Error("feature offsets do not fit 16 bits for this rowsPerBlock / feature count");
   const uint32_t featureStride = plan.FeatureStride();
   if (plan.rankRows16 && pm.RowTileBytes() > 0x10000u) throw Error("two-byte rank rows: the row tile must stay below 64 KB (byte offsets)");
-  const uint32_t groupCapacity = (uint32_t)plan.groupBytes / kNodeBytes; // in 8-byte units
   const uint32_t tileUnits = TileBytes(T) / kNodeBytes;                    // units per tile (1 for scalar nodes)
 
   // Rank quantisation: x < t_j  <=>  #{t : t <= x} <= j for the sorted distinct thresholds t_0 < t_1 < ...
@@ -945,6 +957,7 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
   std::vector<int32_t> fullDepth(numTrees, 0); // deferred tails: the tree's own depth (depth[] is then where its walk stops)
   int64_t tailBudget = plan.deferTails && forest.numFeatures + 1 < (1 << kTailFeatureBits) ? (int64_t)(cuts ? kMaxTailNodes : kPeeledTailNodes) - 1 : 0;
   std::vector<TreeUnits> units(numTrees);
+  std::vector<std::vector<uint32_t>> levels(T > 1 ? 0 : numTrees); // (of the nodes that walks reach: pruned models keep others)
   for (size_t t = 0; t < numTrees; ++t) {
     const Tree &tree = forest.trees[t];
     const std::vector<int64_t> *hits = profile ? &profile->hits[t] : nullptr;
@@ -960,7 +973,8 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
         if (tile.count == 0) leafLevel[tile.leafNode] = tile.level;
     } else {
       depth[t] = tree.Depth();
-      units[t] = UnitsOfTree(NodesPerLevel(tree), pm.leavesOutside); // (of the nodes that walks reach: pruned models keep others)
+      levels[t] = NodesPerLevel(tree);
+      units[t] = UnitsOfTree(levels[t], false);
       std::vector<int32_t> stack{0};
       leafLevel[0] = 0;
       while (!stack.empty()) { // (the level of every node; only the leaves' entries are used)
@@ -1047,6 +1061,20 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     if (depth[a] != depth[b]) return depth[a] < depth[b];
     return peel[a] < peel[b];
   });
+
+  // The groups' size, what stays out of them, and whose the classes are.
+  std::vector<std::vector<int32_t>> rounds; // classes of the tree threads' own: treeThreads * K trees each, -1: none
+  for (const LaunchPlan &tried : GroupSizes(asked)) {
+    plan = tried;
+    pm.groupBytes = plan.groupBytes;
+    pm.leavesOutside = LeavesOutside(forest, plan);
+    if (T > 1) continue;
+    for (size_t t = 0; t < numTrees && !plan.deferTails; ++t) units[t] = UnitsOfTree(levels[t], pm.leavesOutside);
+    rounds.clear();
+    pm.ownClasses = OwnClassRounds(forest, plan, depth, units, order, &rounds);
+    if (pm.ownClasses) break;
+  }
+  const uint32_t groupCapacity = (uint32_t)plan.groupBytes / kNodeBytes; // in 8-byte units
 
   const auto pushUnit = [&](const DeviceNode &node, int32_t origin, int32_t second = -1) {
     pm.nodes.push_back(node);
@@ -1231,8 +1259,6 @@ PackedModel PackPlan(const Forest &input, const LaunchPlan &plan, const HitCount
     }
   };
 
-  std::vector<std::vector<int32_t>> rounds; // classes of the tree threads' own: treeThreads * K trees each, -1: none
-  if (T == 1) pm.ownClasses = OwnClassRounds(forest, plan, depth, units, order, &rounds);
   if (pm.ownClasses) {
     const size_t TT = (size_t)plan.treeThreads;
     for (size_t next = 0; next < rounds.size();) {

@@ -27,6 +27,10 @@ struct LaunchPlan {
   int32_t treeLanes = 1;        // tree-parallel: lanes per row, power of two; block = rowsPerBlock * treeLanes
   int32_t interleave = 4;       // K: trees walked concurrently by one lane (1, 2, 4, 8)
   int32_t groupBytes = 48 * 1024; // LDS bytes for one tree group's nodes (<= 65536)
+  // What they are where classes are the tree threads' own (PackedModel::ownClasses): those never meet, and their meeting place
+  // behind the rows goes to the groups.  Beside groupBytes, not in its place: whether classes are the threads' own is the packer's
+  // to find out, for every shape this plan is changed into.  0: groupBytes either way.
+  int32_t ownGroupBytes = 0;
   int32_t treeSlices = 1;       // grid.y: how many blocks share one row block's trees
   bool featureOffsetInWords = false;
   // Row-parallel kernel on rank-quantised rows: a separate kernel first replaces every feature value
@@ -59,6 +63,13 @@ struct LaunchPlan {
   // stubs, the rows that reach one are queued per wave as (row, node) and walked on densely, 64 queue entries
   // at a time, whatever trees they come from.  Needs a profile; set by ChoosePlan where the kernel has the form.
   bool deferTails = false;
+
+  // A block of another shape: the meeting place that ownGroupBytes counts on is that of the old one.
+  void Reshape(int32_t rows, int32_t threads) {
+    if (rows != rowsPerBlock || threads != treeThreads) ownGroupBytes = 0;
+    rowsPerBlock = rows;
+    treeThreads = threads;
+  }
 
   int32_t ThreadsPerBlock() const {
     if (kernel == Kernel::kGlobalWalk) return rowsPerBlock;
@@ -96,6 +107,7 @@ struct PackedModel {
   // the f32 row-parallel walk takes level 0 from scalar registers instead of an LDS node read.
   std::vector<DeviceNode> bundleRoots;
   uint32_t maxGroupNodes = 0;
+  int32_t groupBytes = 0; // that the groups were filled to: the plan's groupBytes or ownGroupBytes
   // Classifiers on scalar row-parallel plans: every class is one tree thread's, so that class sums need no meeting of the tree
   // threads.  Groups are whole rounds of a bundle for every tree thread, bundles without trees among them.
   bool ownClasses = false;

@@ -1108,7 +1108,7 @@ std::string InferenceRunner::DescribePlan() const {
                                                        : "rows_lds")
      << " rowsPerBlock=" << p.rowsPerBlock << " treeThreads=" << p.treeThreads << " treeLanes=" << p.treeLanes
      << " interleave=" << p.interleave
-     << " groupBytes=" << p.groupBytes << " treeSlices=" << p.treeSlices
+     << " groupBytes=" << (m_model.groupBytes > 0 ? m_model.groupBytes : p.groupBytes) << " treeSlices=" << p.treeSlices
      << " offsetsInWords=" << (p.featureOffsetInWords ? 1 : 0) << " quantizedRows=" << (p.quantizedRows ? 1 : 0) << " rankRows16=" << (p.rankRows16 ? 1 : 0)
      << " groups=" << m_model.groups.size()
      << " bundles=" << m_model.bundles.size() << " nodes=" << m_model.nodes.size()

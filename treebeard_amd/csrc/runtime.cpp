@@ -379,10 +379,9 @@ int32_t tbmi_set_plan(intptr_t h, int32_t rowsPerBlock, int32_t treeThreads, int
         plan.treeLanes = 1;
         plan.quantizedRows = false;
         plan.rankRows16 = false;
-        if (rowsPerBlock > 0) plan.rowsPerBlock = rowsPerBlock;
-        plan.treeThreads = treeThreads > 0 ? treeThreads : 1;
+        plan.Reshape(rowsPerBlock > 0 ? rowsPerBlock : plan.rowsPerBlock, treeThreads > 0 ? treeThreads : 1);
         if (interleave > 0) plan.interleave = interleave;
-        if (groupBytes > 0) plan.groupBytes = groupBytes;
+        if (groupBytes > 0) plan.groupBytes = groupBytes, plan.ownGroupBytes = 0;
         if (treeSlices > 0) plan.treeSlices = treeSlices;
         const int64_t words = (int64_t)(r->RowSize() + 1) * plan.rowsPerBlock;
         plan.featureOffsetInWords = words * 4 > 0xFFFF;
@@ -402,6 +401,7 @@ int32_t tbmi_set_tree_parallel_plan(intptr_t h, int32_t rowsPerBlock, int32_t tr
       [&] {
         InferenceRunner *r = Runner(h);
         LaunchPlan plan = r->Model().plan;
+        plan.ownGroupBytes = 0;
         plan.kernel = LaunchPlan::Kernel::kTreeParallel;
         plan.deferTails = false;
         plan.featureOffsetInWords = false;
@@ -446,6 +446,7 @@ int32_t tbmi_set_quantized_plan(intptr_t h, int32_t treeThreads, int32_t interle
       [&] {
         InferenceRunner *r = Runner(h);
         LaunchPlan plan = r->Model().plan;
+        plan.ownGroupBytes = 0;
         plan.kernel = LaunchPlan::Kernel::kRowParallelLds;
         plan.quantizedRows = true;
         plan.rankRows16 = false;
@@ -470,6 +471,7 @@ int32_t tbmi_set_rank16_plan(intptr_t h, int32_t rowsPerBlock, int32_t treeThrea
       [&] {
         InferenceRunner *r = Runner(h);
         LaunchPlan plan = r->Model().plan;
+        plan.ownGroupBytes = 0;
         plan.kernel = LaunchPlan::Kernel::kRowParallelLds;
         plan.rankRows16 = true;
         plan.quantizedRows = false;

@@ -461,11 +461,11 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
     if (own < forest.numClasses * (std::ceil(ofClass / (4 * threads)) * 4 * levels + 20.0) && PacksOwnClasses(forest, two)) plan.interleave = 2;
   }
   // Tree threads with classes of their own never meet: their place behind the rows goes to the groups (2^20 rows x 54 features, 800
-  // trees of depth 6, 8 classes: 25 groups and 17, 778 -> 741 us; 65537 rows with sums 81.6 -> 79.7).
+  // trees of depth 6, 8 classes: 25 groups and 17, 778 -> 741 us; 65537 rows with sums 81.6 -> 79.7).  The packer takes it where it
+  // finds the classes to be theirs.
   if (meet > 0 && plan.groupBytes == (int32_t)(group & ~15)) {
-    LaunchPlan roomy = plan;
-    roomy.groupBytes = (int32_t)(std::min<int64_t>({group + meet, 65536, 256LL * plan.ThreadsPerBlock()}) & ~15);
-    if (PacksOwnClasses(forest, roomy)) plan = roomy;
+    const int32_t roomy = (int32_t)(std::min<int64_t>({group + meet, 65536, 256LL * plan.ThreadsPerBlock()}) & ~15);
+    if (forest.numClasses > 1 && plan.treeThreads > 1 && roomy > plan.groupBytes) plan.ownGroupBytes = roomy;
   }
   return plan;
 }
@@ -530,6 +530,7 @@ std::vector<LaunchPlan> CandidatePlans(const Forest &forest, int64_t batchSize, 
           LaunchPlan p = base;
           p.rowsPerBlock = rb;
           p.treeThreads = tt;
+          p.ownGroupBytes = 0; // (what its groups may take is said below)
           p.featureOffsetInWords = words;
           p.interleave = k;
           const int64_t rowTile = (int64_t)(forest.numFeatures + 1) * rb * 4;
@@ -561,6 +562,7 @@ std::vector<LaunchPlan> CandidatePlans(const Forest &forest, int64_t batchSize, 
       p.featureOffsetInWords = false;
       p.rowsPerBlock = rb;
       p.treeThreads = 1024 / rb;
+      p.ownGroupBytes = 0;
       p.interleave = 4;
       int64_t group = std::min<int64_t>(65536, limits.ldsBytesPerBlock / 2 - rowTile - (forest.numClasses > 0 ? 1024 * 8 : 0) - 2048);
       if (group < need || group < 8192) continue;
