@@ -273,6 +273,49 @@ static void TwoTreesOfSlices() {
   EXPECT(two > 0 && kept > 0, "%ld, %ld", two, kept);
 }
 
+// Peeled walks that end in no deferred tails (classes, rows of word offsets, no room for the queues) are laid out as others are, and
+// so planned; those with deferred tails keep all leaves in LDS, and the slices' turns are counted that way.
+static void PlansOfPeeledWalks() {
+  const DeviceLimits limits;
+  WalkOptions walk;
+  walk.peelWalks = true;
+  long whole = 0, tails = 0, outside = 0, two = 0;
+  for (int32_t features : {8, 33, 57, 90, 130, 300})
+    for (int32_t classes : {0, 0, 3, 8})
+      for (int32_t trees : {61, 80, 89, 161, 300})
+        for (int32_t nodes : {63, 127, 255, 511})
+          for (int64_t batch : {4000, 7414, 12708, 16925, 30000, 262144}) {
+            Forest forest = ForestOf(features, trees, nodes);
+            forest.numClasses = classes;
+            for (int32_t t = 0; t < trees; ++t) {
+              if (t % 3 == 0) forest.trees[(size_t)t] = FullTree(nodes / 4 * 2 + 1, features);
+              forest.trees[(size_t)t].classId = classes ? t % classes : 0;
+            }
+            const LaunchPlan plain = ChoosePlan(forest, batch, nullptr, limits), peeled = ChoosePlan(forest, batch, nullptr, limits, walk);
+            if (plain.kernel != LaunchPlan::Kernel::kRowParallelLds || plain.quantizedRows) continue;
+            if (!peeled.deferTails) {
+              ++whole;
+              outside += PackForest(forest, plain).leavesOutside;
+              EXPECT(peeled.interleave == plain.interleave && peeled.groupBytes == plain.groupBytes && peeled.treeSlices == plain.treeSlices,
+                     "%d features, %d classes, %d trees of %d nodes, %lld rows: %d and %d trees a lane", features, classes, trees, nodes, (long long)batch,
+                     plain.interleave, peeled.interleave);
+            } else if (peeled.treeSlices > 1 && peeled.interleave == 2) {
+              ++two;
+              LaunchPlan p = peeled; // (as it was when the trees a lane were chosen: no room given to the queues yet)
+              p.groupBytes = plain.groupBytes;
+              int64_t turns[2];
+              for (int32_t k : {2, 4}) {
+                p.interleave = k;
+                turns[k / 4] = (CountTreeGroups(forest, p) + p.treeSlices - 1) / p.treeSlices;
+              }
+              EXPECT(turns[0] * 2 < turns[1] * 3, "%d features, %d trees of %d nodes, %lld rows: %lld and %lld groups a slice", features, trees, nodes,
+                     (long long)batch, (long long)turns[0], (long long)turns[1]);
+            }
+            tails += peeled.deferTails;
+          }
+  EXPECT(whole > 0 && tails > 0 && outside > 0 && two > 0, "%ld, %ld, %ld, %ld", whole, tails, outside, two);
+}
+
 // Numbers of features that files can hold: too many for any row in LDS, and the last ones that can be counted.
 static void MostFeatures() {
   const DeviceLimits limits;
@@ -356,6 +399,7 @@ int main(int argc, char **argv) {
   if (asked("two_trees_of_slices")) TwoTreesOfSlices();
   if (asked("most_features")) MostFeatures();
   if (asked("room_of_own_classes")) RoomOfOwnClasses();
+  if (asked("plans_of_peeled_walks")) PlansOfPeeledWalks();
   if (gFailures) return 1;
   std::printf("ok\n");
   return 0;

@@ -66,3 +66,7 @@ def test_as_many_features_as_can_be_counted(driver):
 
 def test_room_that_own_classes_leave(driver):
     run(driver, "room_of_own_classes")
+
+
+def test_plans_of_peeled_walks(driver):
+    run(driver, "plans_of_peeled_walks")

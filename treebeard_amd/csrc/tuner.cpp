@@ -437,12 +437,14 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // two and three 4814 x 193 in five 10.2 -> 11.3, 15744 x 80 in four 10.6 -> 10.9; three and four 11.8 and 11.5, 14.8 and 15.0,
   // five and six 19.8 -> 19.0, 14.9 -> 14.2, alike 13.2 -> 12.1.
   plan.treeSlices = (int32_t)std::max<int64_t>(1, slices);
-  const int64_t inLds = !peelWalks && LeavesOutside(forest, plan) ? TreeBytesInLds(forest, true) : totalBytes; // (peeled walks keep all in LDS)
+  LaunchPlan walked = plan, queued = plan; // (as it will be packed: deferred tails keep all leaves in LDS)
+  walked.deferTails = peelWalks && DeferTailsFit(forest, &queued);
+  const int64_t inLds = LeavesOutside(forest, walked) ? TreeBytesInLds(forest, true) : totalBytes;
   if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)plan.groupBytes * (double)forest.trees.size() < fewInGroup * (double)inLds) {
-    LaunchPlan two = plan;
+    LaunchPlan two = walked;
     two.interleave = 2;
     const auto turns = [&](const LaunchPlan &p) { return (CountTreeGroups(forest, p) + slices - 1) / slices; };
-    if (slices == 1 || (forest.numClasses > 1 && PacksOwnClasses(forest, two)) || turns(two) * 2 < turns(plan) * 3) plan.interleave = 2;
+    if (slices == 1 || (forest.numClasses > 1 && PacksOwnClasses(forest, two)) || turns(two) * 2 < turns(walked) * 3) plan.interleave = 2;
   }
   // Classes of the tree threads' own (PackForest) need groups of a bundle for every tree thread: bundles of two where four do
   // not fit, that way costs less (the packer's costs), and the packer will take it: where it does not, two side by side lose (607
