@@ -28,6 +28,27 @@ static Tree FullTree(int32_t nodes, int32_t numFeatures) {
   return tree;
 }
 
+// The same with a spine on the left down to `depth`: few of its leaves are on the last level.
+static Tree SpinedTree(int32_t nodes, int32_t depth, int32_t numFeatures) {
+  Tree tree = FullTree(nodes, numFeatures);
+  size_t at = 0;
+  int32_t level = 0;
+  for (; !tree.IsLeaf((int32_t)at); ++level) at = (size_t)tree.left[at];
+  for (; level < depth; ++level) {
+    const int32_t child = (int32_t)tree.NumNodes();
+    tree.left[at] = child;
+    tree.right[at] = child + 1;
+    for (int i = 0; i < 2; ++i) {
+      tree.value.push_back(0.5f);
+      tree.feature.push_back(0);
+      tree.left.push_back(-1);
+      tree.right.push_back(-1);
+    }
+    at = (size_t)child;
+  }
+  return tree;
+}
+
 static Forest ForestOf(int32_t numFeatures, int32_t trees, int32_t nodes) {
   Forest forest;
   forest.numFeatures = numFeatures;
@@ -348,8 +369,9 @@ static void RoomOfOwnClasses() {
     return low + (int32_t)((state >> 33) % (uint64_t)(high - low + 1));
   };
   long roomy = 0, meet = 0;
-  for (int32_t i = 0; i < 400; ++i) {
+  for (int32_t i = 0; i < 800; ++i) {
     const bool wide = i % 2; // (one block per compute unit, and two)
+    const bool spined = i % 4 / 2; // (all leaves of these stay in LDS)
     const int32_t features = wide ? pick(380, 520) : pick(20, 110), classes = wide ? pick(10, 16) : pick(3, 9), trees = pick(40, 110);
     Forest forest = ForestOf(features, trees, 3);
     forest.numClasses = classes;
@@ -357,7 +379,8 @@ static void RoomOfOwnClasses() {
     profile.numRows = 1000;
     const int32_t biggest = wide ? pick(190, 255) : pick(330, 511);
     for (int32_t t = 0; t < trees; ++t) { // of one depth and many sizes, which the profile brings into order
-      Tree &tree = forest.trees[(size_t)t] = FullTree(pick(wide ? 131 : 257, biggest) / 2 * 2 + 1, features);
+      const int32_t nodes = pick(spined ? biggest / 3 : wide ? 131 : 257, biggest) / 2 * 2 + 1;
+      Tree &tree = forest.trees[(size_t)t] = spined ? SpinedTree(nodes, 12, features) : FullTree(nodes, features);
       tree.classId = t % classes;
       std::vector<int64_t> hits(tree.NumNodes(), 0);
       hits[0] = profile.numRows;
