@@ -398,6 +398,7 @@ hipError_t LaunchWalkRowsLds(const WalkParams &p, int interleave, int tileMode, 
   if (p.s.deferTails) ++shimDeferred;
   if (tileMode < 0 || tileMode > 3 || (tileMode == 3 && p.splitBlocks)) return hipErrorInvalidValue;
   if (tileMode == 3 && (int64_t)((p.s.numFeatures + 2) / 2) * RB * 4 > 0x10000) return hipErrorInvalidValue;
+  if (tileMode >= 2 && p.s.leavesOutside && !p.leafIds) return hipErrorInvalidValue; // (rank tiles: always in LDS)
   const uint32_t stride = tileMode == 0 || tileMode == 3 ? (uint32_t)RB * 4u : tileMode == 1 ? (uint32_t)RB : (uint32_t)RB / 4u;
   return WalkLds(p, interleave, stride, tileMode == 3 ? 2 : tileMode == 2 ? 1 : 0, p.s.leavesOutside != 0, stream);
 }

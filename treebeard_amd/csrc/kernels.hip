@@ -1936,19 +1936,26 @@ hipError_t LaunchSplitVariant(const WalkParams &p, dim3 block, size_t ldsBytes, 
                      p.bundleRoots, p.groups, p.s, p.partial);
 }
 
+// The variants for where the last level's leaves are (rank tiles: always in LDS).
+template <int K, int W, int V>
+hipError_t LaunchSplitLeaves(const WalkParams &p, dim3 block, size_t ldsBytes, hipStream_t stream) {
+  if constexpr (IsRankTile(W)) {
+    return p.s.leavesOutside ? hipErrorInvalidValue : LaunchSplitVariant<K, W, V>(p, block, ldsBytes, stream);
+  } else {
+    return p.s.leavesOutside ? LaunchSplitVariant<K, W, V | kWalkOutside>(p, block, ldsBytes, stream)
+                             : LaunchSplitVariant<K, W, V>(p, block, ldsBytes, stream);
+  }
+}
+
 template <int K, int W>
 hipError_t LaunchSplit(const WalkParams &p, dim3 block, size_t ldsBytes, hipStream_t stream) {
   const int64_t rowBlocks = (p.s.rows + p.s.rowsPerBlock - 1) / p.s.rowsPerBlock;
   if (p.splitBlocks < 1 || p.splitBlocks > rowBlocks * p.s.numGroups || !p.partial || p.leafIds || p.s.deferTails || p.s.fuseArgmax)
     return hipErrorInvalidValue;
-  if (p.s.ownClasses)
-    return p.s.leavesOutside && !IsRankTile(W) ? LaunchSplitVariant<K, W, kWalkOwn | kWalkOutside>(p, block, ldsBytes, stream)
-                                               : LaunchSplitVariant<K, W, kWalkOwn>(p, block, ldsBytes, stream);
-  return p.s.leavesOutside && !IsRankTile(W) ? LaunchSplitVariant<K, W, kWalkPlain | kWalkOutside>(p, block, ldsBytes, stream)
-                                             : LaunchSplitVariant<K, W, kWalkPlain>(p, block, ldsBytes, stream);
+  return p.s.ownClasses ? LaunchSplitLeaves<K, W, kWalkOwn>(p, block, ldsBytes, stream)
+                        : LaunchSplitLeaves<K, W, kWalkPlain>(p, block, ldsBytes, stream);
 }
 
-// The variant for where the last level's leaves are (rank tiles: always in LDS).
 template <int K, int PF, int W, int V>
 hipError_t LaunchWalkLeaves(const WalkParams &p, dim3 grid, dim3 block, size_t ldsBytes, hipStream_t stream) {
   if constexpr (IsRankTile(W)) {
