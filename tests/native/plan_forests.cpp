@@ -301,11 +301,11 @@ static void PlansOfPeeledWalks() {
   WalkOptions walk;
   walk.peelWalks = true;
   long whole = 0, tails = 0, outside = 0, two = 0;
-  for (int32_t features : {8, 33, 57, 90, 130, 300})
-    for (int32_t classes : {0, 0, 3, 8})
-      for (int32_t trees : {61, 80, 89, 161, 300})
-        for (int32_t nodes : {63, 127, 255, 511})
-          for (int64_t batch : {4000, 7414, 12708, 16925, 30000, 262144}) {
+  for (int32_t features : {8, 33, 57, 130, 300})
+    for (int32_t classes : {0, 3})
+      for (int32_t trees : {61, 89, 161})
+        for (int32_t nodes : {127, 511})
+          for (int64_t batch : {7414, 12708, 30000, 262144}) {
             Forest forest = ForestOf(features, trees, nodes);
             forest.numClasses = classes;
             for (int32_t t = 0; t < trees; ++t) {
