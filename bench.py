@@ -46,11 +46,20 @@ def print_lds_read_costs():
 
 
 def plan_key(plan):
-    """The fields of a plan description that decide which kernel runs and how (what a traffic figure is tied to)."""
-    keep = ("kernel", "rowsPerBlock", "treeThreads", "treeLanes", "interleave", "groupBytes", "treeSlices", "quantizedRows",
-            "rankRows16", "tileSize", "staging", "peelWalks", "batchKernel")
+    """The fields of a plan description that decide which kernel runs and how, on which packed model (what a traffic figure is tied to)."""
+    keep = ("kernel", "rowsPerBlock", "treeThreads", "treeLanes", "interleave", "treeSlices", "quantizedRows", "rankRows16", "groups",
+            "bundles", "nodes", "ldsBytes", "tileSize", "staging", "peelWalks", "batchKernel", "treesDeferred", "ownClasses", "leavesOutside")
     fields = dict(item.split("=", 1) for item in plan.split() if "=" in item)
     return " ".join("%s=%s" % (k, fields[k]) for k in keep if k in fields)
+
+
+def lds_reads(kernel, plan_fields, trees, levels):
+    """LDS reads of one row that walks `levels` levels of `trees` trees: nodes, feature values, leaves.  The row-parallel walks
+    get the roots through scalar registers (not on one-byte ranks) and, where leavesOutside=1, the leaves out of the caches."""
+    row_walk = kernel in ("WalkRowsLdsKernel", "WalkRowsSplitKernel")
+    roots = trees if not row_walk or plan_fields["quantizedRows"] == "1" else 0
+    leaves = trees if not row_walk or plan_fields["leavesOutside"] == "0" else 0
+    return levels - trees + roots, levels, leaves
 
 
 def main():
@@ -156,15 +165,12 @@ def main():
     # algorithmic bytes per row.  HBM: the row once (4 F) + the output.  LDS: every visited internal node reads
     # 6 B of node (f32 threshold + i16 feature index) and the 4 B feature value from the LDS row tile, every tree
     # ends with a 4 B leaf read; the visit count is measured exactly by the oracle on a sample of the same rows.
+    # What the kernel of this plan does not read from LDS is not counted (lds_reads).
     from oracle import cpu_oracle, model_io
     forest = model_io.load_xgboost_json(model)
     sample = min(rows, 8192)
     steps_per_row = cpu_oracle.total_steps(forest, x[:sample]) / sample
     hbm_bytes_row = 4 * cfg.num_features + (1 if multiclass else 4)
-    lds_bytes_row = steps_per_row * 10 + 4 * forest.num_trees
-    hbm_time = hbm_bytes_row * rows / (HBM_PEAK_GBS * 1e9)
-    lds_time = lds_bytes_row * rows / (LDS_PEAK_GBS * 1e9)
-    binding = "lds" if lds_time > hbm_time else "hbm"
     plan = runner.describe_plan()
     quantized = "quantizedRows=1" in plan or "rankRows16=1" in plan       # a ranking kernel runs in front of the walk
     plan_fields = dict(item.split("=", 1) for item in plan.split() if "=" in item)
@@ -172,6 +178,11 @@ def main():
               "rows_lds": "WalkRowsLdsKernel", "rows_tiled": "WalkRowsTiledKernel", "tree_parallel": "WalkTreeParallelKernel",
               "global_walk": "WalkGlobalKernel", "deep_walk": "WalkRowsLdsKernel"}[plan_fields["batchKernel"]]
     quantized = quantized and kernel != "FewRowsKernel"
+    nodes, values, leaves = lds_reads(kernel, plan_fields, forest.num_trees, steps_per_row)
+    lds_bytes_row = 6 * nodes + 4 * values + 4 * leaves
+    hbm_time = hbm_bytes_row * rows / (HBM_PEAK_GBS * 1e9)
+    lds_time = lds_bytes_row * rows / (LDS_PEAK_GBS * 1e9)
+    binding = "lds" if lds_time > hbm_time else "hbm"
     # the rank-quantised path reads the f32 rows in its binning kernel: both kernels count for the HBM roofline
     hbm_ms = walk_ms + bin_ms if quantized else walk_ms
     hbm_gbs = hbm_bytes_row * rows / (hbm_ms * 1e-3) / 1e9
@@ -197,16 +208,17 @@ def main():
         from treebeard_amd.runtime_api import lds_read_bandwidth      # the bench-only library libtbamd_bench.so
         lds_measured = {"b%d" % (8 * width): lds_read_bandwidth(width) / 1e9 for width in (4, 8, 16)}
     # What the LDS pipes need at those measured rates for this kernel's own mix (an 8-byte node read and a 4-byte
-    # feature read per level, a 4-byte leaf read per tree): for the visited nodes only, and for the lock-step walk
-    # that takes every row through the depth of each tree (the depth of the deepest tree of a bundle, in fact).
+    # feature read per level, a 4-byte leaf read per tree, as far as it makes them): for the visited nodes only, and for
+    # the lock-step walk that takes every row through the depth of each tree (the depth of the deepest tree of a bundle,
+    # in fact).
     lds_floor = None
     if lds_measured and binding == "lds":
-        per_level = 8.0 / (lds_measured["b64"] * 1e9) + 4.0 / (lds_measured["b32"] * 1e9)
-        per_leaf = 4.0 / (lds_measured["b32"] * 1e9)
+        def floor_ms(levels):
+            nodes, values, leaves = lds_reads(kernel, plan_fields, forest.num_trees, levels)
+            return rows * (nodes * 8.0 / (lds_measured["b64"] * 1e9) + (values + leaves) * 4.0 / (lds_measured["b32"] * 1e9)) * 1e3
         # (peeled walks stop trees early: the plan says how many levels its lock-step walk takes per row)
         depth_sum = float(plan_fields.get("deepLockStepSteps") or plan_fields.get("lockStepSteps") or sum(forest.depth(t) for t in range(forest.num_trees)))
-        visited_ms = rows * (steps_per_row * per_level + forest.num_trees * per_leaf) * 1e3
-        lockstep_ms = rows * (depth_sum * per_level + forest.num_trees * per_leaf) * 1e3
+        visited_ms, lockstep_ms = floor_ms(steps_per_row), floor_ms(depth_sum)
         lds_floor = {"visited_nodes_ms": visited_ms, "frac_of_visited_floor": visited_ms / walk_ms,
                      "lockstep_levels_per_row": depth_sum, "lockstep_ms": lockstep_ms,
                      "frac_of_lockstep_floor": lockstep_ms / walk_ms}

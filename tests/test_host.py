@@ -351,3 +351,18 @@ def test_c_client_builds_against_the_header_and_sees_documented_errors(tmp_path,
     run = subprocess.run([exe, synth_model(1)], capture_output=True, text=True, timeout=120)
     assert run.returncode == 0, (run.returncode, run.stdout, run.stderr)
     assert "trees=100 features=8 classes=0" in run.stdout
+
+
+@pytest.mark.parametrize("kernel,quantized,outside,expected", [
+    ("WalkRowsLdsKernel", 0, 1, (6577, 7577, 0)),           # 14154 of the 14331 LDS instructions a wave was counted to issue
+    ("WalkRowsLdsKernel", 0, 0, (6577, 7577, 1000)), ("WalkRowsSplitKernel", 0, 1, (6577, 7577, 0)),
+    ("WalkRowsLdsKernel", 1, 0, (7577, 7577, 1000)), ("WalkRowsTiledKernel", 0, 0, (7577, 7577, 1000)),
+    ("FewRowsKernel", 0, 1, (7577, 7577, 1000))])
+def test_bench_counts_the_lds_reads_that_are_made(kernel, quantized, outside, expected):
+    import importlib.util
+    spec = importlib.util.spec_from_file_location("bench", os.path.join(ROOT, "bench.py"))
+    bench = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(bench)
+    assert bench.lds_reads(kernel, {"quantizedRows": str(quantized), "leavesOutside": str(outside)}, 1000, 7577) == expected
+    plans = [bench.plan_key("kernel=rows_lds groups=15 leavesOutside=%d" % n) for n in (0, 1)]
+    assert plans[0] != plans[1]
