@@ -35,7 +35,7 @@ typedef const __attribute__((address_space(3))) uint16_t *LdsHalfPtr;
 __device__ __forceinline__ uint32_t LdsLoadHalf(uint32_t address) { return *(LdsHalfPtr)(uintptr_t)address; }
 
 // A node's child pointer (the low half of its meta word) plus `more`: a 16-bit addition leaves the upper half of the result zero and
-// takes 2.6 cycles of a SIMD where one that selects a half (SDWA), a compare or a conditional move takes 4.3.
+// takes 2.2 cycles of a SIMD that eight waves share (2.5: four), where one that selects a half (SDWA) or a compare takes 4.1 to 4.4.
 __device__ __forceinline__ uint32_t AddChild(uint32_t meta, uint32_t more) {
   uint32_t address;
   asm("v_add_u16_e32 %0, %1, %2" : "=v"(address) : "v"(meta), "v"(more));
@@ -176,8 +176,9 @@ __device__ __forceinline__ void StageRows(const float *__restrict__ src, int val
 // leaves hold the walk in place (see device_model.h), so the loop body has no
 // leaf test and no divergence.  Where leaves stay out of the groups (kWalkOutside) their values are gathered from L2,
 // asked for when a bundle ends and added when the next one does: 16 address cycles per wave and tree on a path the walk
-// leaves idle, for two cycles of the LDS pipe and 15 to 50 % of a group's room (2^20 rows x 28 features, 1000 trees of
-// depth 8 1162 -> 1069 us: LDS pipes 83 -> 79 % busy, conflicts 0.30 -> 0.16 cycles a read).  `treeThreads` lanes (in different waves) share
+// leaves idle, for two cycles of the LDS pipe and 20 to 50 % of a group's room (2^20 rows x 28 features, 1000 trees of
+// depth 8 1162 -> 1069 us; conflicts 0.28 -> 0.16 cycles an LDS instruction, LDS pipes 83 -> 81 % and VALUs 81 -> 90 % busy, the last with the
+// additions above too).  `treeThreads` lanes (in different waves) share
 // one row and split each group's bundles between them, which buys occupancy
 // without growing the row tile; their sums meet in an LDS cross-wave pass.
 // Sums are kept in double; trees are added in packed order.

@@ -690,9 +690,15 @@ int64_t TreeBytesInLds(const Forest &forest, bool leavesOutside) {
 
 // What stays out of LDS makes room for more trees between two barriers and takes the leaf reads off the LDS pipes, and costs a
 // gather from L2 per tree.  2^20 rows x 1000 trees of depth 8 (30 % of the nodes are such leaves) 27 groups and 16: 1162 -> 1069
-// us; 800 complete trees of depth 6 in 8 classes (half of the nodes) 50 and 25: 849 -> 790.  Not where no group is saved: one
-// group either way, 338838 rows x 52 trees of depth 5 22.3 and 22.9, 32 slices of a group, 4096 rows x 1000 trees 12.8 and 13.4;
-// nor for the few leaves of skewed trees: 800 of depth 12 in 20 groups and 17 1213 and 1239.
+// us; 800 complete trees of depth 6 in 8 classes (half of the nodes) 50 and 25: 849 -> 790.  Not where their bytes are no group
+// less: one group either way, 338838 rows x 52 trees of depth 5 22.3 and 22.9, 32 slices of a group, 4096 rows x 1000 trees 12.8 and
+// 13.4; nor for the few leaves of skewed trees: 800 of depth 12 in 20 groups and 17 1213 and 1239.
+// Between: a 26 % share, 12 groups and 9, 1005 -> 959 us; 28 %, 6 and 4, 86.5 -> 85.0; 29 %, 21 and 14, 1061 -> 989; 35 %, 18 and 12, 1072 ->
+// 981; at 19 %, with rows of all kinds through skewed trees, 27 groups and 20 would win too: 1132 and 1086.
+// By bytes and not by groups as packed: those can come to as many (a group's addresses reach 64 KB with the leaves outside, and tree
+// threads take whole rounds of bundles), and yet half of the copies and the leaf reads are saved.  33 such forests, inside and outside,
+// 2 to 41 groups and 50 to 900 trees: complete trees 0.90 to 1.01 of the time (28 groups 139.0 -> 125.5, 41 491 -> 462, 2 339 and 342), shares of
+// 26 to 44 % 0.95 to 1.025 (3 groups 445 -> 428, 2 80 -> 78; 2 groups of 163 features 180 -> 184, of 274 47.8 -> 48.8), 0.99 in the mean.
 bool LeavesOutside(const Forest &forest, const LaunchPlan &plan) {
   if (plan.kernel != LaunchPlan::Kernel::kRowParallelLds || plan.WalkTile() > 1 || plan.deferTails || plan.quantizedRows || plan.rankRows16)
     return false;

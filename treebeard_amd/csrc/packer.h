@@ -202,7 +202,7 @@ PackedModel PackWithCuts(const Forest &forest, const LaunchPlan &plan, const std
 bool PacksOwnClasses(const Forest &forest, const LaunchPlan &plan);
 // LDS bytes of all trees of a forest under a scalar row-parallel plan, with the leaves of the trees' last levels or without.
 int64_t TreeBytesInLds(const Forest &forest, bool leavesOutside);
-// Whether PackForest leaves those out (PackedModel::leavesOutside): where that saves tree groups.
+// Whether PackForest leaves those out (PackedModel::leavesOutside): where they are more than a fifth of the bytes and the rest would fill fewer groups.
 bool LeavesOutside(const Forest &forest, const LaunchPlan &plan);
 // How many tree groups PackForest makes under a scalar plan, classes of the tree threads' own aside.
 int32_t CountTreeGroups(const Forest &forest, const LaunchPlan &plan);
