@@ -129,7 +129,8 @@ CompiledModel LoadCompiledModel(const std::string &path) {
   m.plan.tiling = r.Get<int32_t>();
   m.plan.peelWalks = r.Get<int32_t>() != 0;
   m.plan.deferTails = r.Get<int32_t>() != 0;
-  if (version != kVersionWithoutOwnGroups) m.plan.ownGroupBytes = r.Get<int32_t>();
+  m.oneGroupSize = version == kVersionWithoutOwnGroups;
+  if (!m.oneGroupSize) m.plan.ownGroupBytes = r.Get<int32_t>();
   const uint64_t trees = r.Get<uint64_t>();
   if (trees > (bytes.size() - r.pos) / 36) throw Error("model file is truncated"); // (a tree takes 36 bytes at least)
   m.forest.trees.resize(trees);

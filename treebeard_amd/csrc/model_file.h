@@ -12,6 +12,7 @@ namespace tbamd {
 struct CompiledModel {
   Forest forest;
   LaunchPlan plan;
+  bool oneGroupSize = false; // an older file: plan.groupBytes may be what own classes leave room for (SeparateGroupSizes)
   int32_t batchSize = 0;
   int32_t returnTypeWidth = 32;
   bool returnTypeFloatType = true;

@@ -527,6 +527,7 @@ intptr_t tbmi_load_compiled_model(const char *path, int32_t batchSize) {
   return Guard(
       [&]() -> intptr_t {
         CompiledModel m = LoadCompiledModel(path ? path : "");
+        if (m.oneGroupSize) SeparateGroupSizes(m.forest, m.profile.get(), DeviceLimits(), &m.plan);
         CompilerOptions options;
         options.batchSize = batchSize > 0 ? batchSize : m.batchSize;
         options.returnTypeWidth = m.returnTypeWidth;

@@ -474,6 +474,22 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
 
 } // namespace
 
+void SeparateGroupSizes(const Forest &forest, const HitCountProfile *profile, const DeviceLimits &limits, LaunchPlan *plan) {
+  if (forest.numClasses < 2 || plan->kernel != LaunchPlan::Kernel::kRowParallelLds) return;
+  const PackedModel pm = PackForest(forest, *plan, profile); // (which refuses what a damaged file may hold)
+  if (!pm.ownClasses) return;
+  const int64_t place = plan->ThreadsPerBlock() * 8, need = (BiggestTreeNodes(forest) + 2) * kNodeBytes;
+  for (const int64_t budget : {limits.ldsBytesPerBlock / 2, limits.ldsBytesPerBlock}) { // (the planner's)
+    const int64_t room = budget - (int64_t)pm.RowTileBytes() - 512;
+    if (plan->groupBytes > room) continue;
+    const int64_t beside = (room - place) & ~15LL;
+    if (beside >= plan->groupBytes || beside < std::max<int64_t>(need, 1024)) return;
+    plan->ownGroupBytes = plan->groupBytes;
+    plan->groupBytes = (int32_t)beside;
+    return;
+  }
+}
+
 std::vector<LaunchPlan> CandidatePlans(const Forest &forest, int64_t batchSize, const DeviceLimits &limits,
                                        const WalkOptions &walk) {
   std::vector<LaunchPlan> out;

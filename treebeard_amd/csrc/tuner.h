@@ -60,6 +60,10 @@ bool ChooseDeepWalk(const Forest &forest, const DeviceLimits &limits, LaunchPlan
 // How many blocks share a row block's tree groups.
 int32_t DeepWalkSlices(int64_t rowBlocks, int64_t groups, const DeviceLimits &limits);
 
+// A plan of one group size out of a file: where its classes are the tree threads' own and it counts on the meeting place that they
+// leave, that size becomes LaunchPlan::ownGroupBytes and groupBytes the one beside the place.  The packed groups stay the same.
+void SeparateGroupSizes(const Forest &forest, const HitCountProfile *profile, const DeviceLimits &limits, LaunchPlan *plan);
+
 // Candidate plans for the timed search (the analytic choice comes first).
 std::vector<LaunchPlan> CandidatePlans(const Forest &forest, int64_t batchSize, const DeviceLimits &limits,
                                        const WalkOptions &walk = WalkOptions());
