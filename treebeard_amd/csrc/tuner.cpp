@@ -437,7 +437,10 @@ LaunchPlan ChooseScalarPlan(const Forest &forest, int64_t batchSize, const GPUAu
   // two and three 4814 x 193 in five 10.2 -> 11.3, 15744 x 80 in four 10.6 -> 10.9; three and four 11.8 and 11.5, 14.8 and 15.0,
   // five and six 19.8 -> 19.0, 14.9 -> 14.2, alike 13.2 -> 12.1.
   plan.treeSlices = (int32_t)std::max<int64_t>(1, slices);
-  LaunchPlan walked = plan, queued = plan; // (as it will be packed: deferred tails keep all leaves in LDS)
+  // As it will be packed: deferred tails keep all leaves in LDS, peeled walks without them need not.  Three classes, trees of depth 8, two
+  // trees a lane (what counting whole trees asks for) and four: 30000 rows x 61 trees of 33 features 15.6 and 13.1 us, 2^18 x 161 79.9 and
+  // 73.4, 2^20 x 89 190 and 170, 2^18 x 89 of 57 features 79.0 and 72.9; but 2^18 x 61 of 130 features 112.5 and 117.4.
+  LaunchPlan walked = plan, queued = plan;
   walked.deferTails = peelWalks && DeferTailsFit(forest, &queued);
   const int64_t inLds = LeavesOutside(forest, walked) ? TreeBytesInLds(forest, true) : totalBytes;
   if (!(ov && ov->treeWalkInterleaveFactor > 0) && (double)plan.groupBytes * (double)forest.trees.size() < fewInGroup * (double)inLds) {
